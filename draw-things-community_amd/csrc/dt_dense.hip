@@ -11,52 +11,10 @@
 // Tile: BM x BN outputs per 512-thread workgroup (8 waves, two per SIMD, each
 // a BN/2 x BM/4 slice), K-tiles of 32 processed in pairs; one barrier per K-tile
 // (per pair with plain fp16 weights, which no wave writes to LDS itself).
+#include "dt_dense_any.h"
 #include "dt_dense_launch.h"
 
 namespace dt {
-
-// Any shape / alignment: one thread per output element.  Slow; keeps odd
-// shapes (K not a multiple of 32, nib not a multiple of 32, unaligned rows)
-// correct rather than unsupported.
-__global__ void __launch_bounds__(256) dense_qx_generic_kernel(const uint16_t* __restrict__ x, int64_t ldx, int64_t m,
-                                                             int64_t n, int64_t k, const uint8_t* __restrict__ wdata,
-                                                             int qbits, int nib, const uint16_t* __restrict__ bias,
-                                                             uint16_t* y, int64_t ldy, float scale,
-                                                             const uint16_t* add, int64_t ld_add, int act,
-                                                             const uint16_t* __restrict__ gate, float* __restrict__ res,
-                                                             int64_t ld_res, const float* __restrict__ gate32,
-                                                             const uint16_t* mul, int64_t ld_mul) {
-  int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= m * n) return;
-  int64_t mi = o / n, ni = o - mi * n;
-  const uint16_t* xr = x + mi * ldx;
-  float acc = 0.f;
-  if (qbits == 16) {
-    const uint16_t* wr = reinterpret_cast<const uint16_t*>(wdata) + ni * k;
-    for (int64_t kk = 0; kk < k; kk++) acc += (float)bits_to_half(xr[kk]) * (float)bits_to_half(wr[kk]);
-  } else {
-    const QxLayout l = make_layout(qbits, nib);
-    for (int64_t kk = 0; kk < k; kk++) {
-      int64_t e = ni * k + kk;
-      int64_t b = e / nib, r = e - b * nib;
-      const uint8_t* base = wdata + palette_offset(l, b);
-      const uint16_t* pal = reinterpret_cast<const uint16_t*>(base);
-      uint16_t wv = pal[load_index(base + l.pal_bytes, r, qbits)];
-      acc += (float)bits_to_half(xr[kk]) * (float)bits_to_half(wv);
-    }
-  }
-  if (bias) acc += (float)bits_to_half(bias[ni]);
-  float v = round_f16(acc);
-  v = post_value(v, scale, add != nullptr, add ? (float)bits_to_half(add[mi * ld_add + ni]) : 0.f, mul != nullptr,
-                 mul ? (float)bits_to_half(mul[mi * ld_mul + ni]) : 1.f, act, gate != nullptr,
-                 gate ? (float)bits_to_half(gate[ni]) : 1.0f);
-  if (res) {
-    float pr = gate32 ? v * gate32[ni] : v;
-    asm volatile("" : "+v"(pr));  // no fused multiply-add: the product is rounded first
-    res[mi * ld_res + ni] += pr;
-  }
-  if (y) y[mi * ldy + ni] = half_to_bits((half_t)v);
-}
 
 extern template dt_status launch_dense_q<4>(hipStream_t, const DenseArgs&, int, bool, int);
 extern template dt_status launch_dense_q<5>(hipStream_t, const DenseArgs&, int, bool, int);
@@ -233,7 +191,7 @@ static void finish_args(DenseArgs& a, int n_groups, int n_w, int64_t K, const dt
 
 // One validated problem with M > 0: weights that share (qbits, nib) and meet the
 // tiled kernel's alignment go out in runs of up to kMaxWeights per launch; the
-// rest take the generic kernel.
+// rest take the any-shape kernel.
 // Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
 constexpr int64_t kFillTiles = 192;
 
@@ -246,17 +204,33 @@ static dt_status run_group(hipStream_t s, const HostGroup& h) {
     const int64_t n_rows0 = w0.count / K;
     if (!(x_ok && h.w_tiled(i))) {
       if (n_rows0 > 0) {
-        int64_t outs = M * n_rows0;
-        if ((outs + 255) / 256 > 0x7fffffff) return DT_NO_KERNEL;
-        hipLaunchKernelGGL(dense_qx_generic_kernel, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s, h.X, h.ldx,
-                           M, n_rows0, K, static_cast<const uint8_t*>(w0.data), w0.qbits, w0.nib,
-                           h.bias ? h.bias[i] : nullptr, h.Y[i], h.ldy[i], post_scale(h, i),
-                           h.post ? h.post[i].addend : nullptr, h.post ? h.post[i].ld_addend : 0,
-                           h.post ? h.post[i].activation : DT_ACT_NONE,
-                           h.post ? h.post[i].gate : nullptr, h.post ? h.post[i].residual : nullptr,
-                           h.post ? h.post[i].ld_residual : 0, h.post ? h.post[i].gate_f32 : nullptr,
-                           h.post ? h.post[i].multiplicand : nullptr, h.post ? h.post[i].ld_multiplicand : 0);
-        dt_status st = launch_status();
+        DenseAnyArgs g = {};
+        g.x = h.X;
+        g.ldx = h.ldx;
+        g.m = M;
+        g.n = n_rows0;
+        g.k = K;
+        g.w = static_cast<const uint8_t*>(w0.data);
+        g.w_bytes = w0.qbits == 16 ? w0.count * 2 : dt_qx_bytes(w0.qbits, w0.nib, w0.count);
+        g.qbits = w0.qbits;
+        g.nib = w0.nib;
+        g.bias = h.bias ? h.bias[i] : nullptr;
+        g.y = h.Y[i];
+        g.ldy = h.ldy[i];
+        g.scale = post_scale(h, i);
+        if (h.post) {
+          const dt_dense_post& p = h.post[i];
+          g.add = p.addend;
+          g.ld_add = p.ld_addend;
+          g.act = p.activation;
+          g.gate = p.gate;
+          g.res = p.residual;
+          g.ld_res = p.ld_residual;
+          g.gate32 = p.gate_f32;
+          g.mul = p.multiplicand;
+          g.ld_mul = p.ld_multiplicand;
+        }
+        dt_status st = dense_any_launch(s, g);
         if (st != DT_OK) return st;
         if (h.wants_epi(i)) {
           st = epilogue_pass(s, h, i);

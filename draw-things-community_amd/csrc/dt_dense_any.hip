@@ -1,0 +1,307 @@
+// K1a: Dense for the shapes the tiled kernel (dt_dense_kernel.h) does not take -- K no multiple of 64, blocks that are
+// no multiple of 32, rows or weights off the 16-byte grid -- on the matrix instruction all the same.
+//
+// What bounds it: the launches are small (odd widths come with small layers), so it is latency: of the index and X
+// loads, hidden by fetching a K-tile ahead into registers, and of the K loop, kept short by giving the four waves of a
+// small tile a quarter of every K-tile each (their sums meet in LDS).  231 x 1000 -> 1001 q8p: 12.6 us (8.0 with plain
+// fp16 weights), where one thread per output, walking K on its own, took 1105.
+#include "dt_dense_any.h"
+
+#include "dt_dense_kernel.h"
+#include "dt_layout.h"
+
+namespace dt {
+
+// (the part reads words at any address, one instruction each)
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
+// 16 halfs of a row; with CUT those from `left` on are zero and not read.  (Two forms because a lane's partial load
+// would make every other lane wait for its whole one: they write the same registers.)
+template <bool CUT>
+__device__ __forceinline__ void load_halfs16(const uint16_t* p, int left, uint32_t (&raw)[8]) {
+  if constexpr (!CUT) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const u32x4_any v = *reinterpret_cast<const u32x4_any*>(p + 8 * c);
+#pragma unroll
+      for (int i = 0; i < 4; i++) raw[4 * c + i] = v[i];
+    }
+  } else {
+    uint32_t h[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) h[i] = p[i < left ? i : 0];
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      raw[i] = (2 * i < left ? h[2 * i] : 0) | (2 * i + 1 < left ? h[2 * i + 1] << 16 : 0);
+  }
+}
+
+constexpr int kAnyPalBytes = 16384;  // LDS for the palettes of a tile's rows (with the tiles below: three workgroups per CU)
+
+// BT x BT outputs per 256-thread workgroup (BT = 64: 2 x 2 waves of 32 x 32; BT = 32: every wave computes the whole
+// tile over its own quarter of each K-tile).  A K-tile is 4096 / BT wide, so that a thread always stages 16 consecutive
+// k of one X row and of one weight row.
+template <int Q, int BT>
+__global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
+  constexpr int BKA = 4096 / BT, RUNS = BKA / 16;
+  constexpr int LDR = BKA + 8;                 // halfs per LDS row: 16 consecutive rows start on 16 different bank groups
+  constexpr int BUF = BT * LDR;                // halfs per operand and stage
+  constexpr int HW = Q == 16 ? 8 : (Q + 1) / 2;  // dwords that hold a thread's 16 weights or indices
+  constexpr int NRAW = Q == 16 ? 8 : HW + 1;     // ... at any byte offset
+  constexpr int OUT_LD = BT + 1;
+  constexpr int OUT_BYTES = (BT == 32 ? 4 : 1) * BT * OUT_LD * 4;
+  static_assert(OUT_BYTES <= 4 * BUF * 2, "the output tile reuses the operand buffers");
+  __shared__ __attribute__((aligned(16))) half_t tiles[4 * BUF];
+  __shared__ uint16_t pal_lds[Q == 16 ? 1 : kAnyPalBytes / 2];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int l32 = lane & 31, hi = lane >> 5;
+  const int64_t m0 = (blockIdx.x % a.tiles_m) * BT, n0 = (blockIdx.x / a.tiles_m) * BT;
+  const int row = tid / RUNS, run = tid % RUNS;
+  const int64_t gm = m0 + row, gn = n0 + row;
+  const uint16_t* xr = a.x + (gm < a.m ? gm : 0) * a.ldx;
+  const QxLayout lay = make_layout(Q == 16 ? 8 : Q, Q == 16 ? 32 : a.nib);
+  const int nib = lay.nib;
+
+  // palettes of every block the tile's rows touch
+  int64_t blk0 = 0;
+  if constexpr (Q != 16) {
+    if (a.pal_shared) {
+      blk0 = n0 * a.k / nib;
+      const int64_t last_row = n0 + BT <= a.n ? n0 + BT - 1 : a.n - 1;
+      const int n_pal = (int)((last_row * a.k + a.k - 1) / nib - blk0 + 1);
+      for (int i = tid; i < n_pal << Q; i += 256)
+        pal_lds[i] = reinterpret_cast<const u16_any*>(a.w + palette_offset(lay, blk0 + (i >> Q)))[i & ((1 << Q) - 1)];
+    }
+  }
+
+  // Whole runs are fetched as words, unless blocks are shorter than a run (one may then touch more than two) or the
+  // buffer is shorter than a run's words: then index by index.
+  const bool runs_ok = nib >= 16 && a.w_bytes >= 4 * NRAW;
+
+  // cursor of this thread's weight run: block and position inside it
+  int64_t blk = 0;
+  uint32_t r = 0;
+  if constexpr (Q != 16) {
+    const int64_t e = (gn < a.n ? gn : 0) * a.k + run * 16;
+    blk = e / nib;
+    r = (uint32_t)(e - blk * nib);
+  }
+
+  // NRAW dwords from byte p of the packed buffer on.  The last runs of the buffer are read from further ahead instead
+  // of past its end; the result is the number of bytes by which their words are early.
+  auto load_raw = [&](int64_t p, uint32_t (&raw)[NRAW]) {
+    const int64_t q = p + 4 * NRAW <= a.w_bytes ? p : a.w_bytes - 4 * NRAW;
+    const u32_any* src = reinterpret_cast<const u32_any*>(a.w + q);
+#pragma unroll
+    for (int i = 0; i < NRAW; i++) raw[i] = src[i];
+    return (int)(p - q);
+  };
+  auto drop_bytes = [&](uint32_t (&raw)[NRAW], int n) {
+    if (n <= 0) return;
+    for (; n >= 4; n -= 4) {
+#pragma unroll
+      for (int i = 0; i + 1 < NRAW; i++) raw[i] = raw[i + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < NRAW; i++)
+      raw[i] = (uint32_t)((((uint64_t)(i + 1 < NRAW ? raw[i + 1] : 0) << 32) | raw[i]) >> (8 * n));
+  };
+  // ... as the big-endian bit string that starts `sh` (0 .. 7) bits in
+  auto bit_string = [&](const uint32_t (&raw)[NRAW], int sh, uint32_t (&be)[HW + 1]) {
+    if constexpr (Q != 16) {
+#pragma unroll
+      for (int i = 0; i < HW; i++) {
+        const uint64_t two = ((uint64_t)__builtin_bswap32(raw[i]) << 32) | __builtin_bswap32(raw[i + 1]);
+        be[i] = (uint32_t)(two >> (32 - sh));
+      }
+      be[HW] = 0;
+    }
+  };
+
+  uint32_t xraw[8], wraw[NRAW], wraw2[NRAW];
+  int w_left = 0;  // weights of the fetched run that exist
+  int w_head = 0;  // ... of which this many lie in block cur_blk, the others in the next one
+  int early = 0, early2 = 0, sh2 = 0;
+  bool two = false;  // some lane's run crosses into another block
+  int64_t cur_blk = 0;
+  uint32_t cur_r = 0;
+  auto fetch = [&](int kt) {
+    const int64_t k0 = (int64_t)kt * BKA + run * 16;
+    w_left = k0 >= a.k ? 0 : (a.k - k0 < 16 ? (int)(a.k - k0) : 16);
+    const bool whole = (int64_t)(kt + 1) * BKA <= a.k;  // uniform
+    if (whole) load_halfs16<false>(xr + k0, 16, xraw);
+    else load_halfs16<true>(xr + (w_left ? k0 : 0), w_left, xraw);
+    if constexpr (Q == 16) {
+      const uint16_t* wr = reinterpret_cast<const uint16_t*>(a.w) + (gn < a.n ? gn : 0) * a.k;
+      if (whole) load_halfs16<false>(wr + k0, 16, wraw);
+      else load_halfs16<true>(wr + (w_left ? k0 : 0), w_left, wraw);
+    } else {
+      cur_blk = blk;
+      cur_r = r;
+      w_head = (uint32_t)nib - r < (uint32_t)w_left ? (int)((uint32_t)nib - r) : w_left;
+      if (runs_ok) {
+        early = load_raw(index_byte_offset(lay, w_left ? blk : 0, w_left ? r : 0), wraw);
+        two = __builtin_amdgcn_ballot_w64(w_head < w_left) != 0;
+        if (two) {
+          // The rest of the run, as the string in which it has the same place: from w_head indices ahead of the
+          // next block's first one (the bits in between, palette bytes, are not looked at).
+          const int64_t bit = w_head < w_left ? (palette_offset(lay, blk + 1) + lay.pal_bytes) * 8 - w_head * Q : 0;
+          sh2 = (int)(bit & 7);
+          early2 = load_raw(bit >> 3, wraw2);
+        }
+      }
+      r += BKA;
+      if (r >= (uint32_t)nib) {
+        const uint32_t q = r / (uint32_t)nib;
+        blk += q;
+        r -= q * (uint32_t)nib;
+      }
+    }
+  };
+  auto stage = [&](int buf) {
+    half_t* xs = tiles + buf * 2 * BUF + row * LDR + run * 16;
+    half_t* ws = xs + BUF;
+    *reinterpret_cast<uint4_t*>(xs) = uint4_t{xraw[0], xraw[1], xraw[2], xraw[3]};
+    *reinterpret_cast<uint4_t*>(xs + 8) = uint4_t{xraw[4], xraw[5], xraw[6], xraw[7]};
+    if constexpr (Q == 16) {
+      *reinterpret_cast<uint4_t*>(ws) = uint4_t{wraw[0], wraw[1], wraw[2], wraw[3]};
+      *reinterpret_cast<uint4_t*>(ws + 8) = uint4_t{wraw[4], wraw[5], wraw[6], wraw[7]};
+    } else {
+      uint32_t v[16];
+#pragma unroll
+      for (int j = 0; j < 16; j++) v[j] = 0;
+      // weights [from, to) of the run from the palette of block b
+      auto look_up = [&](const uint32_t (&raw)[NRAW], int sh, int64_t b, int from, int to) {
+        uint32_t be[HW + 1];
+        bit_string(raw, sh, be);
+        uint32_t got[16];
+        if (a.pal_shared) {  // uniform
+          const uint16_t* lp = pal_lds + ((int)(b - blk0) << Q);
+#pragma unroll
+          for (int j = 0; j < 16; j++) got[j] = lp[own_index<Q, HW>(be, j)];
+        } else {
+          const u16_any* gp = reinterpret_cast<const u16_any*>(a.w + palette_offset(lay, b));
+#pragma unroll
+          for (int j = 0; j < 16; j++) got[j] = gp[own_index<Q, HW>(be, j)];
+        }
+#pragma unroll
+        for (int j = 0; j < 16; j++) v[j] = j >= from && j < to ? got[j] : v[j];
+      };
+      if (runs_ok) {
+        drop_bytes(wraw, early);
+        look_up(wraw, (int)((cur_r * Q) & 7), w_left ? cur_blk : blk0, 0, w_head);
+        if (two) {
+          drop_bytes(wraw2, early2);
+          look_up(wraw2, sh2, w_head < w_left ? cur_blk + 1 : blk0, w_head, w_left);
+        }
+      } else {
+        int64_t b = cur_blk;
+        uint32_t rr = cur_r;
+#pragma unroll
+        for (int j = 0; j < 16; j++)
+          if (j < w_left) {
+            const uint8_t* base = a.w + palette_offset(lay, b);
+            v[j] = reinterpret_cast<const u16_any*>(base)[load_index(base + lay.pal_bytes, rr, Q)];
+            if (++rr == (uint32_t)nib) {
+              rr = 0;
+              b++;
+            }
+          }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        *reinterpret_cast<uint4_t*>(ws + 8 * h) =
+            uint4_t{v[8 * h] | (v[8 * h + 1] << 16), v[8 * h + 2] | (v[8 * h + 3] << 16),
+                    v[8 * h + 4] | (v[8 * h + 5] << 16), v[8 * h + 6] | (v[8 * h + 7] << 16)};
+    }
+  };
+
+  float16_t acc;
+#pragma unroll
+  for (int v = 0; v < 16; v++) acc[v] = 0.f;
+  const int wn = BT == 64 ? wave & 1 : 0, wm = BT == 64 ? wave >> 1 : 0;
+  const int ks0 = BT == 64 ? 0 : 2 * wave;
+  constexpr int NKS = BT == 64 ? 4 : 2;
+  const int nkt = (int)((a.k + BKA - 1) / BKA);
+  fetch(0);
+  __syncthreads();  // palettes visible
+  stage(0);
+  __syncthreads();
+  for (int kt = 0; kt < nkt; kt++) {
+    const bool more = kt + 1 < nkt;
+    if (more) fetch(kt + 1);
+    const half_t* xs = tiles + (kt & 1) * 2 * BUF + (wm * 32 + l32) * LDR + 8 * hi;
+    const half_t* ws = tiles + (kt & 1) * 2 * BUF + BUF + (wn * 32 + l32) * LDR + 8 * hi;
+#pragma unroll
+    for (int s = 0; s < NKS; s++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const half8_t*>(ws + 16 * (ks0 + s)),
+                                                   *reinterpret_cast<const half8_t*>(xs + 16 * (ks0 + s)), acc, 0, 0, 0);
+    if (more) stage((kt + 1) & 1);
+    __syncthreads();
+  }
+
+  // Sums to LDS as [token][feature], then element by element with consecutive features in consecutive lanes.
+  float* outs = reinterpret_cast<float*>(tiles) + (BT == 32 ? wave * BT * OUT_LD : 0);
+#pragma unroll
+  for (int v = 0; v < 16; v++)
+    outs[(wm * 32 + l32) * OUT_LD + wn * 32 + 8 * (v >> 2) + 4 * hi + (v & 3)] = acc[v];
+  __syncthreads();
+  const float* sums = reinterpret_cast<const float*>(tiles);
+  for (int i = tid; i < BT * BT; i += 256) {
+    const int t = i / BT, f = i % BT;
+    const int64_t mi = m0 + t, ni = n0 + f;
+    if (mi >= a.m || ni >= a.n) continue;
+    float s = sums[t * OUT_LD + f];
+    if constexpr (BT == 32) {
+#pragma unroll
+      for (int p = 1; p < 4; p++) s += sums[(p * BT + t) * OUT_LD + f];
+    }
+    if (a.bias) s += (float)bits_to_half(a.bias[ni]);
+    float v = round_f16(s);
+    v = post_value(v, a.scale, a.add != nullptr, a.add ? (float)bits_to_half(a.add[mi * a.ld_add + ni]) : 0.f,
+                   a.mul != nullptr, a.mul ? (float)bits_to_half(a.mul[mi * a.ld_mul + ni]) : 1.f, a.act,
+                   a.gate != nullptr, a.gate ? (float)bits_to_half(a.gate[ni]) : 1.0f);
+    if (a.res) {
+      float pr = a.gate32 ? v * a.gate32[ni] : v;
+      asm volatile("" : "+v"(pr));  // no fused multiply-add: the product is rounded first
+      a.res[mi * a.ld_res + ni] += pr;
+    }
+    if (a.y) a.y[mi * a.ldy + ni] = half_to_bits((half_t)v);
+  }
+}
+
+template <int Q>
+static void launch_any(hipStream_t s, const DenseAnyArgs& a, bool big, unsigned grid) {
+  if (big) hipLaunchKernelGGL((dense_any_kernel<Q, 64>), dim3(grid), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((dense_any_kernel<Q, 32>), dim3(grid), dim3(256), 0, s, a);
+}
+
+dt_status dense_any_launch(hipStream_t s, DenseAnyArgs a) {
+  if (a.m <= 0 || a.n <= 0) return DT_OK;
+  const auto tiles = [&](int t) { return ((a.m + t - 1) / t) * ((a.n + t - 1) / t); };
+  // The 64 x 64 tile halves what is read and unpacked per output but takes twice as long for a K-tile pair; it wins once
+  // there is one for every compute unit.  1000 -> 1001, 32 against 64 wide, us: 500 rows (128 tiles of 64) 14.9 / 23.9
+  // q8p and 9.7 / 14.8 fp16; 1000 rows (256 tiles) 26.2 / 24.0 and 15.2 / 15.1; 2000 rows (512) 48.2 / 27.7 and
+  // 31.7 / 18.6.
+  const bool big = tiles(64) >= 256;
+  const int BT = big ? 64 : 32;
+  const int64_t grid = tiles(BT);
+  if (grid > 0x7fffffff) return DT_NO_KERNEL;
+  a.tiles_m = (a.m + BT - 1) / BT;
+  a.pal_shared = a.qbits != 16 && ((BT * a.k) / a.nib + 2) * ((int64_t)2 << a.qbits) <= kAnyPalBytes;
+  switch (a.qbits) {
+    case 4: launch_any<4>(s, a, big, (unsigned)grid); break;
+    case 5: launch_any<5>(s, a, big, (unsigned)grid); break;
+    case 6: launch_any<6>(s, a, big, (unsigned)grid); break;
+    case 7: launch_any<7>(s, a, big, (unsigned)grid); break;
+    case 8: launch_any<8>(s, a, big, (unsigned)grid); break;
+    case 16: launch_any<16>(s, a, big, (unsigned)grid); break;
+    default: return DT_INVALID;
+  }
+  return launch_status();
+}
+
+}  // namespace dt

@@ -1,0 +1,56 @@
+"""GPU parity of the Dense kernels that serve what the 128- and 256-wide tiles do not: any shape and alignment.
+
+Bound of every comparison: the fp32 sum of K products in any order is off by at most K 2^-24 sum |x w|, and one rounding
+to fp16 adds half an ulp of the result (2^-11 relative, 2^-25 below the normal range)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    import torch
+
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def make(dthip, oracle, rng, N, K, q, nib):
+    """(QxTensor, its weights as float64)."""
+    if q == 16:
+        w = (rng.standard_normal((N, K)) * 0.05).astype(np.float16)
+        return dthip.QxTensor.from_f16(w), w.astype(np.float64)
+    packed, _, _ = oracle.synth_qx_weight(rng, N, K, q, nib, 0.05)
+    return dthip.QxTensor.from_packed(packed, q, nib, (N, K)), oracle.C.depalettize(q, nib, N * K, packed).reshape(N, K).astype(np.float64)
+
+
+def check(got, X, W, bias=None):
+    X = X.astype(np.float64)
+    want = X @ W.T + (0 if bias is None else bias.astype(np.float64))
+    sums = X.shape[1] * 2.0 ** -24 * (np.abs(X) @ np.abs(W).T + (0 if bias is None else np.abs(bias.astype(np.float64))))
+    tol = (np.abs(want) + sums) * 2.0 ** -11 + 2.0 ** -25 + sums
+    bad = np.abs(got.astype(np.float64) - want) > tol
+    assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4])
+
+
+@pytest.mark.parametrize("M,N,K,q,nib", [
+    (1, 1, 1, 6, 1),            # the smallest there is: one block per weight
+    (33, 31, 100, 6, 32),       # blocks that end inside a thread's run of 16
+    (32, 32, 128, 5, 24),       # a block stride that is no multiple of 4
+    (31, 65, 129, 7, 4096),     # an odd row length: every row starts at another bit
+    (5, 40, 16, 4, 512),        # less than a K-tile
+    (231, 1001, 1000, 8, 16384),
+    (130, 70, 127, 16, 0), (40, 33, 72, 16, 0),  # plain fp16, without and with 16-byte rows
+    (70, 90, 2500, 8, 512),     # more palettes than the LDS holds: looked up in memory
+    (1500, 1400, 200, 6, 4096), (1450, 1470, 77, 4, 64), (1500, 1400, 100, 16, 0),  # enough tiles for the 64 x 64 form
+])
+def test_dense_any_shape(dthip, oracle, M, N, K, q, nib):
+    rng = np.random.default_rng(M * 7 + N * 5 + K + q)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    w, W = make(dthip, oracle, rng, N, K, q, nib)
+    bias = (rng.standard_normal(N) * 0.1).astype(np.float16)
+    print("dense any shape", M, N, K, q, nib, flush=True)
+    check(dthip.dense_multi(dev(X), [w], [dev(bias)])[0].cpu().numpy(), X, W, bias)
+    # X as a view that starts at an odd element of rows of odd length
+    wide = np.zeros((M, K + 3 - (K & 1)), np.float16)
+    wide[:, 1:1 + K] = X
+    check(dthip.dense_multi(dev(wide)[:, 1:1 + K], [w], [None])[0].cpu().numpy(), X, W)
