@@ -13,6 +13,7 @@
 // (per pair with plain fp16 weights, which no wave writes to LDS itself).
 #include "dt_dense_any.h"
 #include "dt_dense_launch.h"
+#include "dt_dense_rows.h"
 
 namespace dt {
 
@@ -238,6 +239,36 @@ static dt_status run_group(hipStream_t s, const HostGroup& h) {
         }
       }
       i++;
+      continue;
+    }
+    // few rows: the kernel that streams the weights
+    int64_t run_features = 0;
+    int run_end = i;
+    for (; run_end < h.n_weights && run_end - i < kMaxWeights; run_end++) {
+      const dt_qx_weight& wj = h.W[run_end];
+      if (wj.qbits != w0.qbits || (wj.qbits != 16 && wj.nib != w0.nib) || !h.w_tiled(run_end)) break;
+      run_features += wj.count / K;
+    }
+    if (const int fb = dense_rows_features(M, K, w0.qbits, w0.nib, run_features); fb > 0) {
+      DenseArgs a;
+      DenseGroup& g = a.g[0];
+      g.x = h.X;
+      g.ldx = h.ldx;
+      g.m = (int32_t)M;
+      g.tiles_m = 1;
+      g.tile_begin = 0;
+      g.w_begin = 0;
+      int64_t tiles = 0;
+      const int first = i;
+      for (; i < run_end; i++) tiles += add_weight(a, i - first, h, i, (int)tiles, fb, false);
+      if (tiles > 0x7fffffff) return DT_NO_KERNEL;
+      g.w_end = i - first;
+      g.tiles_n = a.total_tiles = (int32_t)tiles;
+      finish_args(a, 1, i - first, K, w0);
+      dt_status st = dense_rows_launch(s, a, w0.qbits, fb);
+      for (int j = first; j < i && st == DT_OK; j++)
+        if (h.wants_epi(j)) st = epilogue_pass(s, h, j);
+      if (st != DT_OK) return st;
       continue;
     }
     // tile shape: big tiles when there is enough work to fill 256 CUs with them

@@ -260,16 +260,7 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
       for (int p = 1; p < 4; p++) s += sums[(p * BT + t) * OUT_LD + f];
     }
     if (a.bias) s += (float)bits_to_half(a.bias[ni]);
-    float v = round_f16(s);
-    v = post_value(v, a.scale, a.add != nullptr, a.add ? (float)bits_to_half(a.add[mi * a.ld_add + ni]) : 0.f,
-                   a.mul != nullptr, a.mul ? (float)bits_to_half(a.mul[mi * a.ld_mul + ni]) : 1.f, a.act,
-                   a.gate != nullptr, a.gate ? (float)bits_to_half(a.gate[ni]) : 1.0f);
-    if (a.res) {
-      float pr = a.gate32 ? v * a.gate32[ni] : v;
-      asm volatile("" : "+v"(pr));  // no fused multiply-add: the product is rounded first
-      a.res[mi * a.ld_res + ni] += pr;
-    }
-    if (a.y) a.y[mi * a.ldy + ni] = half_to_bits((half_t)v);
+    store_post(a, mi, ni, round_f16(s));
   }
 }
 

@@ -99,6 +99,20 @@ struct DenseArgs {
   DenseWeight w[kMaxWeights];
 };
 
+// The tail of output (mi, ni) element by element: v is the Dense's own result, rounded to fp16.
+template <typename W>
+__device__ __forceinline__ void store_post(const W& w, int64_t mi, int64_t ni, float v) {
+  v = post_value(v, w.scale, w.add != nullptr, w.add ? (float)bits_to_half(w.add[mi * w.ld_add + ni]) : 0.f,
+                 w.mul != nullptr, w.mul ? (float)bits_to_half(w.mul[mi * w.ld_mul + ni]) : 1.f, w.act,
+                 w.gate != nullptr, w.gate ? (float)bits_to_half(w.gate[ni]) : 1.0f);
+  if (w.res) {
+    float pr = w.gate32 ? v * w.gate32[ni] : v;
+    asm volatile("" : "+v"(pr));  // no fused multiply-add: the product is rounded first
+    w.res[mi * w.ld_res + ni] += pr;
+  }
+  if (w.y) w.y[mi * w.ldy + ni] = half_to_bits((half_t)v);
+}
+
 __device__ __forceinline__ uint4_t ld_global_16(const void* p) {
   return *reinterpret_cast<const uint4_t*>(p);
 }

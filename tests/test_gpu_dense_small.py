@@ -54,3 +54,30 @@ def test_dense_any_shape(dthip, oracle, M, N, K, q, nib):
     wide = np.zeros((M, K + 3 - (K & 1)), np.float16)
     wide[:, 1:1 + K] = X
     check(dthip.dense_multi(dev(wide)[:, 1:1 + K], [w], [None])[0].cpu().numpy(), X, W)
+
+
+@pytest.mark.parametrize("M,N,K,q,nib", [
+    (1, 1, 64, 6, 64),             # one output; half of a 128-wide stretch of K
+    (1, 3072, 3072, 8, 16384), (16, 17, 128, 4, 512), (17, 33, 192, 5, 1024), (33, 100, 1216, 6, 4096),
+    (64, 48, 2112, 7, 8192), (64, 70, 64, 16, 0), (3, 9000, 320, 6, 4096),  # (the last: 32 features per workgroup)
+    (20, 8200, 192, 16, 0),
+    (2, 40, 3072, 8, 64),          # palettes that do not fit: the tiled kernel
+])
+def test_dense_few_rows(dthip, oracle, M, N, K, q, nib):
+    rng = np.random.default_rng(M * 7 + N * 5 + K + q)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    wide = np.zeros((M, K + 8), np.float16)  # rows that do not follow each other
+    wide[:, :K] = X
+    pairs = [make(dthip, oracle, rng, n, K, q, nib) for n in (N, 16, N)]
+    bias = [(rng.standard_normal(w.shape[0]) * 0.1).astype(np.float16) for w, _ in pairs]
+    print("dense few rows", M, N, K, q, nib, flush=True)
+    outs = dthip.dense_multi(dev(wide)[:, :K], [w for w, _ in pairs], [dev(bias[0]), None, dev(bias[2])])
+    for i, (_, W) in enumerate(pairs):
+        check(outs[i].cpu().numpy(), X, W, None if i == 1 else bias[i])
+    # the tails act on the same Dense results, bit for bit
+    gate = dev((1 + 0.3 * rng.standard_normal(N)).astype(np.float16))
+    res = dev(rng.standard_normal((M, N)).astype(np.float32))
+    want = res + (outs[0].float() * gate.float()).half().float()
+    dthip.dense_post(dev(X), [w for w, _ in pairs], [dev(bias[0]), None, dev(bias[2])],
+                     [dthip.DensePost(gate=gate, residual=res, keep_output=False), None, None])
+    assert bool((res == want).all())
