@@ -81,3 +81,30 @@ def test_dense_few_rows(dthip, oracle, M, N, K, q, nib):
     dthip.dense_post(dev(X), [w for w, _ in pairs], [dev(bias[0]), None, dev(bias[2])],
                      [dthip.DensePost(gate=gate, residual=res, keep_output=False), None, None])
     assert bool((res == want).all())
+
+
+@pytest.mark.parametrize("M,K,rank,N", [(1, 1, 1, 1), (15, 33, 3, 7), (17, 100, 16, 129), (65, 320, 17, 128), (130, 257, 33, 200),
+                                        (300, 3072, 128, 96), (33, 64, 70, 1001), (4099, 96, 20, 136), (4100, 40, 130, 130)])
+def test_lora_branch_fp32_shapes(dthip, M, K, rank, N):
+    """fp16(up(scale * down(float(x)))) at the edges of both kernels' blocks and of their K steps, X an unaligned view:
+    both sums in fp32 (K 2^-24 and rank 2^-24 of the sums of magnitudes), one rounding to fp16."""
+    import torch
+
+    rng = np.random.default_rng(M + K + rank + N)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    wide = np.zeros((M, K + 2 + (K & 1)), np.float16)
+    wide[:, 1:1 + K] = X
+    down = (rng.standard_normal((rank, K)) * 0.1).astype(np.float32)
+    up = (rng.standard_normal((N, rank)) * 0.1).astype(np.float32)
+    xd, dd, ud = dev(wide), dev(down), dev(up)
+    T = torch.empty((M, rank), dtype=torch.float32, device="cuda")
+    out = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    print("lora branch", M, K, rank, N, flush=True)
+    st = dthip.lib().dt_lora_branch_f32_f16(None, M, K, xd.data_ptr() + 2, wide.shape[1], dd.data_ptr(), rank, ud.data_ptr(), N, 0.75,
+                                            T.data_ptr(), out.data_ptr(), N)
+    assert st == 0
+    X, down, up = (a.astype(np.float64) for a in (X, down, up))
+    t, t_abs = 0.75 * (X @ down.T), 0.75 * (np.abs(X) @ np.abs(down).T)
+    assert np.all(np.abs(T.cpu().numpy() - t) <= (K + 2) * 2.0 ** -24 * t_abs)
+    want, sums = t @ up.T, (K + rank + 2) * 2.0 ** -24 * (t_abs @ np.abs(up).T)
+    assert np.all(np.abs(out.cpu().numpy().astype(np.float64) - want) <= sums + (np.abs(want) + sums) * 2.0 ** -11 + 2.0 ** -25)
