@@ -53,14 +53,14 @@ __device__ __forceinline__ int v_unit_swz(int row, int u) {
   return u ^ ((row >> 1) & 1);
 }
 
-// SPLIT: the (task, key tile) pairs of the whole launch -- a task being the 256 query rows of one (batch, head) --
-// are laid end to end and cut into one equal run per workgroup, so that a launch whose task count is no multiple
-// of the compute units still keeps all of them busy to the end.  A workgroup walks its run task by task.  A piece
-// that covers a whole task is finished as usual.  Any other piece leaves its unnormalised fp32 output, reference
-// maximum and row sums in a workspace slot and adds its tile count to the task's counter; the piece that brings the
-// counter to the task's tile count -- the last to arrive, whichever that is -- folds all the task's pieces together,
-// in the fixed order of their workgroups, and writes the output.  Nobody waits for anybody: there is no spinning
-// anywhere, and the result does not depend on which piece arrives last.
+// SPLIT: for launches whose task count -- a task being the 256 query rows of one (batch, head) -- leaves the last round
+// of workgroups mostly empty.  The first whole_tasks tasks, full rounds of them, go to a workgroup each; each of the
+// others is cut along its keys into `shares` equal parts.  A workgroup with a part holds its unnormalised fp32 output,
+// reference maximum and row sums, and the parts meet in pairs, the pairs in pairs, and so on: of two that meet, the
+// first leaves what it holds in its workspace slot, counts itself in and ends; the other one folds it into its own
+// registers and goes on to the next meeting, the last of them to the output.  Nobody waits for anybody, and the fold is
+// the same whichever came first.  (Runs of several tasks' parts per workgroup, folded one after the other by the last
+// to arrive, balance better on paper; that kernel needed 370 registers, and its spills made a tile 1.8 times as long.)
 template <int DP, bool PREMUL, bool ONESEG, bool SPLIT>
 __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   constexpr int ROWB = DP * 2;                 // bytes per tile row
@@ -86,11 +86,15 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
 
   // XCD-aware order: tiles of one (batch, head) are consecutive, and each XCD
   // gets a contiguous run, so a head's K/V stay in one XCD's L2.
+  auto xcd_order = [](int i, int total) __attribute__((always_inline)) {
+    const int per = total / 8;
+    return i < per * 8 ? (i & 7) * per + (i >> 3) : i;
+  };
+  // SPLIT: the first whole_tasks workgroups take a task each, bid counts the others
   int bid = blockIdx.x;
-  {
-    const int per = a.total_blocks / 8;
-    if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
-  }
+  const bool takes_whole = SPLIT && bid < a.whole_tasks;
+  if constexpr (SPLIT) bid = takes_whole ? xcd_order(bid, a.whole_tasks) : xcd_order(bid - a.whole_tasks, a.total_blocks);
+  else bid = xcd_order(bid, a.total_blocks);
   const int64_t Sq = a.Sq, Skv = a.Skv;
   const int D = a.D;
   const int n_tiles = (int)((Skv + BKV - 1) / BKV);
@@ -141,22 +145,16 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   }
   const float c = PREMUL ? 1.0f : a.scale_log2e;
 
-  // ---- the run of work of this workgroup ----------------------------------
-  // Not SPLIT: one task, all of its key tiles.  SPLIT: units [u, u_end) of the launch's (task, key tile) pairs.
-  int u = 0, u_end = 0;  // (a split launch holds fewer than 2^31 units)
+  // ---- the work of this workgroup: key tiles [t_lo, t_hi) of a task --------------------------------
+  int task = bid, t_lo = 0, t_hi = n_tiles, share = 0;
   if constexpr (SPLIT) {
-    u = (int)((int64_t)bid * a.units / a.total_blocks);
-    u_end = (int)((int64_t)(bid + 1) * a.units / a.total_blocks);
-  }
-  [[maybe_unused]] int piece_no = 0;
-  [[maybe_unused]] __shared__ int s_last;
-  for (;;) {
-  int task = bid, t_lo = 0, t_hi = n_tiles;
-  if constexpr (SPLIT) {
-    if (u >= u_end) break;
-    task = u / n_tiles;
-    t_lo = u - task * n_tiles;
-    t_hi = (u_end - u) < (n_tiles - t_lo) ? t_lo + (u_end - u) : n_tiles;
+    if (!takes_whole) {
+      // part by part: the workgroups that run together on a die read the same keys of neighbouring tasks
+      share = bid / a.cut_tasks;
+      task = a.whole_tasks + (bid - share * a.cut_tasks);
+      t_lo = (int)((int64_t)share * n_tiles / a.shares);
+      t_hi = (int)((int64_t)(share + 1) * n_tiles / a.shares);
+    }
   }
   const int qt = task % a.q_tiles;
   const int bh = task / a.q_tiles;
@@ -568,88 +566,76 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     }
   };
 
-  if constexpr (!SPLIT) {
-    store_output();
-    break;
-  } else {
-    if (t_lo == 0 && t_hi == n_tiles) {
-      store_output();  // the piece is the whole task
-    } else {
-      // ---- a piece of a task: leave it for, or fold in, the task's other pieces ----------------------------
-      // Slot layout (floats): [DB * 16 accumulators][512 threads], then [512] reference maxima, then [512]
-      // row-sum shares: a wave's access covers 256 consecutive bytes.  A workgroup owns two slots: its first piece
-      // goes to the even one, a later piece -- which can only be its last -- to the odd one.
-      // The pieces of a task run on any compute units of the device, whose L2 caches (one per die) do not see each
-      // other's ordinary stores.  Partial results are therefore written and read with device-scope accesses
-      // (relaxed atomics: write-through stores, loads that do not trust a die's cached copy) instead of
-      // bracketing ordinary accesses with cache-wide write-backs and invalidations, which cost far more than the
-      // 130 KB they would protect.
+  if constexpr (SPLIT) {
+    if (!takes_whole) {
+      __shared__ int s_seen;
+      // Slot layout (floats): [DB * 16 accumulators][512 threads], then [512] reference maxima, then [512] row-sum
+      // shares: a wave's access covers 256 consecutive bytes.  The parts of a task run on any compute units of the
+      // device, whose L2 caches (one per die) do not see each other's ordinary stores: slots are written and read with
+      // device-scope accesses (relaxed atomics: write-through stores, loads that do not trust a die's cached copy)
+      // instead of bracketing ordinary accesses with cache-wide write-backs and invalidations, which cost far more than
+      // the 130 KB they would protect.
       constexpr int SLOT_F = sdpa_split_slot_floats(DP);
-      const int P = a.total_blocks;
-      float* slot = a.partials + (size_t)(2 * bid + (piece_no > 0 ? 1 : 0)) * SLOT_F;
+      const int cut = task - a.whole_tasks;
+      float* const slots = a.partials + (size_t)cut * SLOT_F + tid;
+      const size_t slot_step = (size_t)a.cut_tasks * SLOT_F;
+      int32_t* const counters = a.counters + cut * kSdpaSplitNodes;
+      int node0 = 0;  // counters of this level
+      for (int level = 0; (1 << level) < a.shares; level++) {
+        const int me = share >> level, other = me ^ 1;
+        if ((other << level) < a.shares) {  // uniform; otherwise nobody to meet on this level
+          int32_t* const met = counters + node0 + (me >> 1);
+          if (tid == 0) s_seen = __hip_atomic_load(met, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __syncthreads();
+          if (s_seen == 0) {  // uniform: the other one is not there yet
+            float* const own = slots + (me << level) * slot_step;
 #pragma unroll
-      for (int db = 0; db < DB; db++)
+            for (int db = 0; db < DB; db++)
 #pragma unroll
-        for (int v = 0; v < 16; v++)
-          __hip_atomic_store(slot + (db * 16 + v) * 512 + tid, oacc[db][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(slot + DB * 16 * 512 + tid, m_ref, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(slot + DB * 16 * 512 + 512 + tid, l_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // every wave's stores have been acknowledged before the barrier, hence before the one thread's count that
-      // publishes the piece
-      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-      __syncthreads();
-      if (tid == 0) {
-        const int done = t_hi - t_lo;
-        const int before = __hip_atomic_fetch_add(a.counters + task, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = (before + done == n_tiles) ? 1 : 0;
-      }
-      __syncthreads();
-      if (s_last != 0) {  // uniform: every other piece of the task has been published
-        const int64_t ua = (int64_t)task * n_tiles, ub = ua + n_tiles;
-        // the workgroup whose run holds unit x is the largest p with p * units < (x + 1) * P
-        const int p_lo = (int)(((ua + 1) * P - 1) / a.units), p_hi = (int)((ub * P - 1) / a.units);
-        // The pieces are folded in the order of their workgroups, this one's own included (re-read from its slot),
-        // whichever of them happens to be the one doing it: the result does not depend on the order of arrival.
-        for (int p = p_lo; p <= p_hi; p++) {
-          const int64_t first_unit = (int64_t)p * a.units / P;
-          const float* other = a.partials + (size_t)(2 * p + (first_unit < ua ? 1 : 0)) * SLOT_F;
-          auto ld = [&](int i) __attribute__((always_inline)) {
-            return __hip_atomic_load(other + i * 512 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          };
-          // all of the slot's loads go out before the first of them is waited for
-          const float m_o = ld(DB * 16), l_o = ld(DB * 16 + 1);
-          float16_t got[DB];
-#pragma unroll
-          for (int db = 0; db < DB; db++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) got[db][v] = ld(db * 16 + v);
-          __builtin_amdgcn_sched_barrier(0);
-          if (p == p_lo) {
-            m_ref = m_o;
-            l_run = l_o;
-#pragma unroll
-            for (int db = 0; db < DB; db++) oacc[db] = got[db];
-            continue;
+              for (int v = 0; v < 16; v++)
+                __hip_atomic_store(own + (db * 16 + v) * 512, oacc[db][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(own + DB * 16 * 512, m_ref, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(own + DB * 16 * 512 + 512, l_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // every wave's stores have been acknowledged before the barrier, hence before the count that publishes them
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+            __syncthreads();
+            if (tid == 0) s_seen = __hip_atomic_fetch_add(met, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (s_seen == 0) return;  // uniform: the other one goes on
           }
+          const float* const theirs = slots + (other << level) * slot_step;
+          auto ld = [&](int i) __attribute__((always_inline)) {
+            return __hip_atomic_load(theirs + i * 512, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          };
+          const float m_o = ld(DB * 16), l_o = ld(DB * 16 + 1);
           const float m_new = fmaxf(m_ref, m_o);
           const float wa = fast_exp2((m_ref - m_new) * c), wb = fast_exp2((m_o - m_new) * c);
+          // a wa + b wb with both products rounded: the same for either order
+          auto fold = [&](float mine, float got) __attribute__((always_inline)) {
+            float x = mine * wa, y = got * wb;
+            asm volatile("" : "+v"(x), "+v"(y));
+            return x + y;
+          };
           m_ref = m_new;
-          l_run = l_run * wa + l_o * wb;
+          l_run = fold(l_run, l_o);
 #pragma unroll
-          for (int db = 0; db < DB; db++)
+          for (int db = 0; db < DB; db++) {
+            float16_t got;
 #pragma unroll
-            for (int v = 0; v < 16; v++) oacc[db][v] = oacc[db][v] * wa + got[db][v] * wb;
+            for (int v = 0; v < 16; v++) got[v] = ld(db * 16 + v);
+#pragma unroll
+            for (int v = 0; v < 16; v++) oacc[db][v] = fold(oacc[db][v], got[v]);
+          }
+          __syncthreads();  // s_seen may be written again
         }
-        store_output();
+        node0 += kSdpaSplitNodes >> (level + 1);
       }
     }
-    u += t_hi - t_lo;
-    piece_no++;
   }
-  }  // the workgroup's run
+  store_output();
 }
 
-// Zeroes the per-task tile counters of a SPLIT launch (a fill kernel, so that the launch can be captured in a graph).
+// Zeroes the counters of a SPLIT launch (a fill kernel, so that the launch can be captured in a graph).
 __global__ void sdpa_zero_counters_kernel(int32_t* counters, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) counters[i] = 0;
@@ -684,35 +670,33 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
   if (never) return false;
   const int64_t tasks = (int64_t)B * Hq * ((Sq + QROWS - 1) / QROWS);
   const int64_t n_tiles = (Skv + BKV - 1) / BKV;
-  const int64_t units = tasks * n_tiles;
-  if (tasks > (1 << 20) || units >= (1LL << 31)) return false;  // (the kernel counts units in 32 bits)
+  if (tasks > (1 << 20) || tasks * n_tiles >= (1LL << 31)) return false;  // (the kernel counts units in 32 bits)
   const int cus = compute_units();
-  // at most 8 pieces per task (the piece that arrives last folds the others in one after the other), at least
-  // `min_tiles` key tiles per workgroup
-  const int64_t min_tiles = always ? 2 : 8;
-  int64_t wgs = cus;
-  if (wgs > tasks * 8) wgs = tasks * 8;
-  if (wgs > units / min_tiles) wgs = units / min_tiles;
-  if (wgs < 2 || n_tiles < 2) return false;
+  const int64_t whole = tasks / cus * cus, cut = tasks - whole;  // full rounds of tasks, and what is left
+  // as many parts per task as the round takes (of at least two key tiles)
+  int64_t shares = cut > 0 ? cus / cut : 0;
+  if (shares > kSdpaSplitNodes) shares = kSdpaSplitNodes;
+  if (shares > n_tiles / 2) shares = n_tiles / 2;
+  if (always && shares < 2 && n_tiles >= 2) shares = 2;
+  if (cut == 0 || shares < 2) return false;
   if (!always) {
-    // Measured on this part (head size 128): the card delivers about the same attention throughput whether all of
-    // its compute units are busy or only 70-85 % of them -- a compute unit runs a key tile in ~1.4 us when a third
-    // of the card idles and in ~1.9 us when none does -- so a launch of 1.69 or 6.19 rounds of workgroups gains
-    // nothing from being cut into equal runs (0.276 against 0.248 ms at 24 heads x 4608 tokens).  What does gain
-    // is a launch that fills well under one round: there the unsplit time is one task at the fast rate, the split
-    // time the mean load at the slow rate plus ~25 us of fixed cost per workgroup (counter reset, pipeline refill,
-    // partial results out and in).
-    const double rounds = (double)tasks / cus;
-    if (rounds >= 1.0) return false;
-    const double fixed = 25.0 / (1.9 * (double)n_tiles);  // in task times
-    if (1.0 / 1.35 <= rounds * (double)cus / (double)wgs + fixed) return false;
+    // Measured on this part: a key tile of the last, partial round takes 1.4 us at head size 128 (1.0 at 64 and below)
+    // while most of the card idles and 1.9 us (1.2) when none of it does, and cutting costs 20 us (12): the counters'
+    // launch, the parts' way out and in.  Head size 128, us before / after: 264 tasks of 42 key tiles 150 / 120, of 72
+    // 244 / 181; 320 of 72 244 / 208; 384 of 42 151 / 150 (not cut); 64 of 72 98 / 64.  Head size 64: 264 of 42 100 / 77,
+    // 64 of 72 72 / 42; 384 of 18 49 / 51 (not cut).
+    const bool small = D <= 64;
+    const double idle = small ? 1.0 : 1.4, full = small ? 1.2 : 1.9, fixed = small ? 12.0 : 20.0;
+    const double busy = (double)(cut * shares) / cus;
+    const double cut_time = (double)((n_tiles + shares - 1) / shares) * (idle + (full - idle) * busy) + fixed;
+    if ((double)n_tiles * idle < cut_time + 4.0) return false;
   }
   if (plan) {
-    plan->workgroups = (int32_t)wgs;
-    plan->tasks = (int32_t)tasks;
-    plan->units = units;
-    plan->counter_bytes = ((size_t)tasks * 4 + 255) & ~(size_t)255;
-    plan->partial_bytes = (size_t)2 * wgs * sdpa_split_slot_floats(D <= 64 ? 64 : 128) * 4;
+    plan->shares = (int32_t)shares;
+    plan->cut_tasks = (int32_t)cut;
+    plan->whole_tasks = (int32_t)whole;
+    plan->counter_bytes = ((size_t)cut * kSdpaSplitNodes * 4 + 255) & ~(size_t)255;
+    plan->partial_bytes = (size_t)(cut * shares) * sdpa_split_slot_floats(D <= 64 ? 64 : 128) * 4;
   }
   return true;
 }
@@ -729,12 +713,12 @@ static dt_status launch(hipStream_t s, SdpaArgs a) {
                       (a.Skv + 2 * BKV) * a.k[0].ss * 2 < 0x7fffffffLL && (a.Skv + 2 * BKV) * a.v[0].ss * 2 < 0x7fffffffLL;
   dim3 block(512);
   if (a.partials) {
-    // key-split launch: the counters start at zero, then one workgroup per equal run of units
-    hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a.counters,
-                       (int)total);
+    // key-split launch: the counters start at zero
+    const int n = a.cut_tasks * kSdpaSplitNodes;
+    hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
     if (const dt_status st = launch_status(); st != DT_OK) return st;
-    a.total_blocks = a.split_workgroups;
-    dim3 grid((unsigned)a.split_workgroups);
+    a.total_blocks = a.cut_tasks * a.shares;  // (of the cut tasks)
+    dim3 grid((unsigned)(a.whole_tasks + a.total_blocks));
     if (oneseg) {
       if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, true, true, true>), grid, block, 0, s, a);
       else hipLaunchKernelGGL((sdpa_kernel<DP, false, true, true>), grid, block, 0, s, a);

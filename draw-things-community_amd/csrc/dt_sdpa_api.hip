@@ -214,8 +214,9 @@ static dt_status sdpa_enqueue(dt_stream stream, int32_t B, int32_t Hq, int32_t H
     if (workspace_bytes < used + plan.bytes() || (reinterpret_cast<uintptr_t>(workspace) & 255)) return;
     a.counters = reinterpret_cast<int32_t*>(free_ws);
     a.partials = reinterpret_cast<float*>(free_ws + plan.counter_bytes);
-    a.units = plan.units;
-    a.split_workgroups = plan.workgroups;
+    a.whole_tasks = plan.whole_tasks;
+    a.cut_tasks = plan.cut_tasks;
+    a.shares = plan.shares;
   };
   if (Wo) {
     uint16_t* ow = reinterpret_cast<uint16_t*>(ws);

@@ -704,6 +704,30 @@ def test_sdpa_key_split_vs_oracle(dthip, oracle, torch_cuda, monkeypatch, B, Sq,
     assert float((got.float() - plain.float()).abs().max()) <= 2e-3
 
 
+@pytest.mark.parametrize("D,Skv,n_seg", [(128, 1100, 1), (128, 1100, 2), (64, 450, 1), (40, 130, 2)])
+def test_sdpa_key_split_last_round(dthip, oracle, torch_cuda, monkeypatch, D, Skv, n_seg):
+    """264 tasks: 256 stay whole, the last 8 -- of the last head -- are cut into 8, 8, 4 and 2 parts."""
+    torch = torch_cuda
+    rng = np.random.default_rng(D + Skv + n_seg)
+    B, H, Sq = 1, 33, 2000
+    q, k, v = rand_qkv(rng, B, Sq, Skv, H, H, D)
+    scale = 1 / np.sqrt(D)
+    parts = lambda t: [to_dev(torch, np.ascontiguousarray(t[:, a:b])) for a, b in ([(0, Skv)] if n_seg == 1 else [(0, 77), (77, Skv)])]
+    args = ([to_dev(torch, q)], parts(k), parts(v), scale)
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "always")
+    print("sdpa key split, last round", D, Skv, n_seg, flush=True)
+    got = dthip.sdpa_segments(*args)
+    again = dthip.sdpa_segments(*args)
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "never")
+    plain = dthip.sdpa_segments(*args)
+    assert torch.equal(got, again) and torch.equal(got[:, :, :32], plain[:, :, :32])  # whole tasks: the same bits
+    rows = np.sort(rng.choice(Sq, size=24, replace=False))
+    rows[0], rows[-1] = 0, Sq - 1
+    want = oracle.C.sdpa(np.ascontiguousarray(q[:, rows, 32:]), np.ascontiguousarray(k[:, :, 32:]), np.ascontiguousarray(v[:, :, 32:]), scale)
+    mx, rr = oracle.err_stats(got[:, rows, 32:].cpu().numpy(), want)
+    assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+
+
 def test_sdpa_key_split_joint_segments_fused_prep(dthip, oracle, torch_cuda, monkeypatch):
     """Key-split with text || image segments, fused per-head RMSNorm + RoPE staging and the static-scratch entry
     point: all three forms agree bit for bit with each other and with the oracle within the attention bar."""
