@@ -43,10 +43,13 @@ static dt_status launch_dense(hipStream_t s, const DenseArgs& a, int tile, int q
 static int choose_pal_mode(int qbits, int nib, int64_t K, int BM, int BN) {
   if (qbits == 16) return kPlainF16;
   const int64_t pal_bytes = (int64_t)2 << qbits;
-  const int64_t budget = pal_lds_bytes(BM, BN);
-  if ((int64_t)BN * pal_bytes <= budget) return kPalRow;
   const int64_t shared_count = ((int64_t)BN * K) / nib + 2;
-  if (shared_count * pal_bytes <= budget) return kPalShared;
+  const bool row = (int64_t)BN * pal_bytes <= pal_lds_bytes(BM, BN, kPalRow);
+  const bool shared = !(BM == 256 && BN == 128) && shared_count * pal_bytes <= pal_lds_bytes(BM, BN, kPalShared);
+  // a per-row table has no bank conflicts, but 128- and 256-entry palettes make one of 32 or 64 KB: the 128 x 128 tile
+  // takes it only where the palettes of its blocks would not fit the 24 KB that let two workgroups share a compute unit
+  if (row && !(shared && BM == 128 && BN == 128 && qbits >= 7)) return kPalRow;
+  if (shared) return kPalShared;
   return kPalGlobal;
 }
 

@@ -13,18 +13,20 @@ namespace dt {
 constexpr int kMaxWeights = 8;
 constexpr int kMaxGroups = 4;
 constexpr int BK = 32;
-constexpr int kPalLdsBytes = 32768;
-// LDS a tile shape can spare for palettes: the tiles of 128 features have a weight ring half the size of the
-// 256-feature tiles' (and the 128 x 128 tile X slots half the size too), which leaves room for a per-row table of
-// 256-entry palettes (128 rows x 512 B = 64 KB; with 256 tokens: 64 KB of X slots + 24 KB of ring + 64 KB = 152 KB).
-constexpr int pal_lds_bytes(int BM, int BN) { return BN == 128 ? 65536 : kPalLdsBytes; }
-
 enum PalMode : int {
   kPalShared = 0,  // palettes of every block the tile's rows touch, loaded once, slot = block - first block
   kPalRow = 1,     // one palette per row in a transposed table, a row's column rewritten where its block changes
   kPalGlobal = 2,  // lookups go to global memory (any layout)
   kPlainF16 = 3    // weight is plain fp16, no palette
 };
+
+// LDS a tile shape can spare for palettes.  The tiles of 128 features have a weight ring half the size of the
+// 256-feature tiles', which leaves room for a per-row table of 256-entry palettes (128 rows x 512 B = 64 KB; with 256
+// tokens: 64 KB of X slots + 24 KB of ring + 64 KB = 152 KB).  Where the 128 x 128 tile can do with 24 KB it takes no
+// more: two workgroups then share a compute unit (2 x (32 KB of X slots + 24 KB of ring + 24 KB)).
+constexpr int pal_lds_bytes(int BM, int BN, int mode) {
+  return BN == 256 ? 32768 : BM == 128 && mode == kPalShared ? 24576 : 65536;
+}
 
 struct DenseWeight {
   const uint8_t* data;
@@ -492,7 +494,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // their addresses then fit an instruction offset.  X (and a plain fp16 W) lives in two pair slots, each
   // holding two K-tiles as [rows][64 halfs]: one is read while the next pair is in flight into the other.
   constexpr bool HAS_PAL = MODE == kPalShared || MODE == kPalRow;
-  constexpr int PAL_BYTES = HAS_PAL ? pal_lds_bytes(BM, BN) : 0;
+  constexpr int PAL_BYTES = MODE == kPalRow ? BN << (Q + 1) : HAS_PAL ? pal_lds_bytes(BM, BN, MODE) : 0;
   constexpr int XS_BYTES = BM * PROW * 2;
   constexpr int WP_BYTES = MODE == kPlainF16 ? BN * PROW * 2 : 0;
   constexpr int BS_BYTES = MODE == kPlainF16 ? 0 : NST * B_STAGE * 2;
