@@ -33,6 +33,8 @@ ABI_SYMBOLS = (
     "dt_dense_qx_f16",
     "dt_dense_qx_heads_f16",
     "dt_dense_qx_grouped_f16",
+    "dt_dense_workspace_bytes",
+    "dt_dense_qx_grouped_ws_f16",
     "dt_dense_qx_post_f16",
     "dt_qk_norm_rope_f16",
     "dt_layernorm_modulate_f16",
@@ -131,6 +133,10 @@ def lib():
                                            ctypes.POINTER(_DensePost), ctypes.c_uint32]
         L.dt_dense_qx_grouped_f16.restype = i32
         L.dt_dense_qx_grouped_f16.argtypes = [vp, i32, ctypes.POINTER(_DenseGroup), ctypes.c_uint32]
+        L.dt_dense_workspace_bytes.restype = ctypes.c_size_t
+        L.dt_dense_workspace_bytes.argtypes = [i32, ctypes.POINTER(_DenseGroup)]
+        L.dt_dense_qx_grouped_ws_f16.restype = i32
+        L.dt_dense_qx_grouped_ws_f16.argtypes = [vp, i32, ctypes.POINTER(_DenseGroup), ctypes.c_uint32, vp, ctypes.c_size_t]
         L.dt_qk_norm_rope_f16.argtypes = [vp, _View4, i32, i64, i32, i32, vp, f32, i32, vp, i64, f32]
         L.dt_layernorm_modulate_f16.restype = i32
         L.dt_layernorm_modulate_f16.argtypes = [vp, i64, i64, vp, i64, vp, vp, i32, f32, vp, i64]
@@ -390,6 +396,24 @@ def _marshal_dense(x, weights, biases, outs, epilogues):
     return (x2, M, K, n, W, B, Y, LDY, E, outs)
 
 
+_ROWS_MAX = 64  # rows up to which the library streams the weights and needs no workspace
+
+
+def _addr(a):
+    return None if a is None else ctypes.addressof(a)
+
+
+def _enqueue_dense(groups, flags, stream, device):
+    """Enqueues an array of _DenseGroup, with the scratch memory that lets the library cut tiles along K where there are
+    too few of them for the chip.  (Caller: the arrays that the groups point to stay alive until this returns.)"""
+    n = len(groups)
+    need = lib().dt_dense_workspace_bytes(n, groups)
+    # torch's allocator hands the block out again in stream order, so it may be dropped as soon as the call is enqueued
+    ws = _torch().empty(need, dtype=_torch().uint8, device=device) if need else None
+    st = lib().dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, None if ws is None else ws.data_ptr(), need)
+    _check("dt_dense_qx_grouped_ws_f16", st)
+
+
 def _shape_outs(x, M, outs):
     lead = tuple(x.shape[:-1])
     return [o.reshape(lead + (o.shape[-1],)) if o.shape[0] == M and o.is_contiguous() else o for o in outs]
@@ -401,7 +425,11 @@ def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object
     per-head RMSNorm / RoPE that follows projection i."""
     with _on(stream):
         x2, M, K, n, W, B, Y, LDY, E, outs = _marshal_dense(x, weights, biases, outs, epilogues)
-        if E is None:
+        if M > _ROWS_MAX:
+            G = (_DenseGroup * 1)(_DenseGroup(M, K, x2.data_ptr(), x2.stride(0), _addr(W), n, _addr(B), _addr(Y), _addr(LDY),
+                                              _addr(E), None))
+            _enqueue_dense(G, flags, stream, x.device)
+        elif E is None:
             st = lib().dt_dense_qx_f16(_stream_ptr(stream), M, K, x2.data_ptr(), x2.stride(0), W, n, B, Y, LDY, flags)
             _check("dt_dense_qx_f16", st)
         else:
@@ -490,8 +518,13 @@ def dense_post(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]
     with _on(stream):
         x2, M, K, n, W, B, Y, LDY, _, outs = _marshal_dense(x, weights, biases, outs, None)
         P = _marshal_posts(posts, weights, M, Y, outs)
-        st = lib().dt_dense_qx_post_f16(_stream_ptr(stream), M, K, x2.data_ptr(), x2.stride(0), W, n, B, Y, LDY, P, flags)
-        _check("dt_dense_qx_post_f16", st)
+        if M > _ROWS_MAX:
+            G = (_DenseGroup * 1)(_DenseGroup(M, K, x2.data_ptr(), x2.stride(0), _addr(W), n, _addr(B), _addr(Y), _addr(LDY),
+                                              None, _addr(P)))
+            _enqueue_dense(G, flags, stream, x.device)
+        else:
+            st = lib().dt_dense_qx_post_f16(_stream_ptr(stream), M, K, x2.data_ptr(), x2.stride(0), W, n, B, Y, LDY, P, flags)
+            _check("dt_dense_qx_post_f16", st)
     lead = tuple(x.shape[:-1])
     return [None if o is None else (o.reshape(lead + (o.shape[-1],)) if o.shape[0] == M and o.is_contiguous() else o)
             for o in outs]
@@ -509,16 +542,16 @@ def dense_grouped(problems: Sequence[dict], flags: int = 0, stream=None):
 def _dense_grouped(problems, flags, stream):
     keep = [_marshal_dense(p["x"], p["weights"], p["biases"], p.get("outs"), p.get("epilogues")) for p in problems]
     G = (_DenseGroup * len(keep))()
-    cast = lambda a: None if a is None else ctypes.addressof(a)  # the arrays stay alive in `keep` until the call returns
     posts = []
     for i, (x2, M, K, n, W, B, Y, LDY, E, outs) in enumerate(keep):
         P = None
         if problems[i].get("posts") is not None:
             P = _marshal_posts(problems[i]["posts"], problems[i]["weights"], M, Y, outs)
         posts.append(P)
-        G[i] = _DenseGroup(M, K, x2.data_ptr(), x2.stride(0), cast(W), n, cast(B), cast(Y), cast(LDY), cast(E), cast(P))
-    st = lib().dt_dense_qx_grouped_f16(_stream_ptr(stream), len(keep), G, flags)
-    _check("dt_dense_qx_grouped_f16", st)
+        G[i] = _DenseGroup(M, K, x2.data_ptr(), x2.stride(0), _addr(W), n, _addr(B), _addr(Y), _addr(LDY), _addr(E), _addr(P))
+    # (the arrays stay alive in `keep` until the call returns)
+    if keep:
+        _enqueue_dense(G, flags, stream, problems[0]["x"].device)
     return [[None if o is None else _shape_outs(p["x"], k[1], [o])[0] for o in k[9]] for p, k in zip(problems, keep)]
 
 

@@ -11,6 +11,10 @@
 // Tile: BM x BN outputs per 512-thread workgroup (8 waves, two per SIMD, each
 // a BN/2 x BM/4 slice), K-tiles of 32 processed in pairs; one barrier per K-tile
 // (per pair with plain fp16 weights, which no wave writes to LDS itself).
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+
 #include "dt_dense_any.h"
 #include "dt_dense_launch.h"
 #include "dt_dense_rows.h"
@@ -193,13 +197,189 @@ static void finish_args(DenseArgs& a, int n_groups, int n_w, int64_t K, const dt
   a.pal_step = (int32_t)(std::gcd((int64_t)K, (int64_t)a.nib) / BK);
 }
 
+// How a launch of the tiled kernel is laid out: its tile and, where the tiles do not fill the compute units evenly, how
+// many of them are cut along K into how many shares.
+struct TilePlan {
+  int tile = kTile256x256, BM = 256, BN = 256;
+  int64_t tiles = 0;
+  int64_t whole = 0;  // tiles that stay whole; the rest is cut into `split` shares each
+  int split = 1;
+  // workspace of the split tiles: their counters, then their slots
+  size_t counter_bytes() const { return split > 1 ? ((size_t)(tiles - whole) * kSplitNodes * 4 + 255) & ~(size_t)255 : 0; }
+  size_t bytes() const { return split > 1 ? counter_bytes() + (size_t)((tiles - whole) * split * dense_split_slot_bytes(BM, BN)) : 0; }
+};
+
+constexpr int kDenseCUs = 256;
+// Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
+constexpr int64_t kFillTiles = 192;
+constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
+
+// Estimated time (us) of a launch, from what this part measures.  Per K-tile and workgroup: 256 x 256 tiles 0.80 us
+// while a third of the compute units work and 1.02 us when all do (the card is limited as a whole), 7 % more with 7-
+// and 8-bit palettes, a third less with plain fp16 weights; 128 x 256 tiles 0.63 .. 0.73 us (the unpacking, which
+// bounds them, is the same as for 256 rows); 256 x 128 tiles 0.72.  Two 128 x 128 tiles share a compute unit, except
+// with 64 KB of palettes: 0.57 us for a few of them, 0.75 us with one on every compute unit, 1.0 us for both of a pair.
+// A workgroup spends 7 us outside its K loop.  Cutting costs the launch that zeroes the counters and, for each level of
+// meetings, a way out and in for the sums: 2 shares of 72 tiles (36 MB) 15 us, 3 of them 29, 6 shares of 36 tiles 45.
+static double plan_cost(const TilePlan& p, int qbits, int mode, int nk) {
+  const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8;
+  const bool pairs_of_tiles = p.tile == kTile128x128 && !(mode == kPalRow && qbits == 8);
+  // one workgroup's K-tile with the share `busy` of the compute units at work
+  const auto k_tile = [&](double busy) -> double {
+    switch (p.tile) {
+      case kTile256x256: return plain ? 0.58 + 0.14 * busy : (0.72 + 0.30 * busy) * (wide ? 1.07 : 1.0);
+      case kTile128x256: return plain ? 0.42 + 0.08 * busy : (0.61 + 0.12 * busy) * (wide ? 1.2 : 1.0);
+      case kTile128x128: return plain ? 0.28 + 0.06 * busy : (0.53 + 0.22 * busy) * (wide ? 1.15 : 1.0);
+    }
+    return 0.72;
+  };
+  // `n` workgroups of `kt` K-tiles each
+  const auto time = [&](int64_t n, int kt) -> double {
+    if (n == 0) return 0.0;
+    if (pairs_of_tiles) {
+      const double rounds = (double)n / (2 * kDenseCUs), both = plain ? 0.5 : wide ? 1.15 : 1.0;
+      return std::max(rounds * both, k_tile(std::min(1.0, 2 * rounds))) * kt + 7.0 * std::ceil(rounds);
+    }
+    const int64_t full = n / kDenseCUs, rest = n % kDenseCUs;
+    return (double)full * (kt * k_tile(1.0) + 7.0) + (rest ? kt * k_tile((double)rest / kDenseCUs) + 7.0 : 0.0);
+  };
+  if (p.split == 1) return time(p.tiles, nk);
+  const int64_t shares = (p.tiles - p.whole) * p.split;
+  const int levels = p.split > 4 ? 3 : p.split > 2 ? 2 : 1;
+  const double mb = 1e-6 * (double)(shares * dense_split_slot_bytes(p.BM, p.BN));
+  return time(p.whole, nk) + time(shares, 2 * ((nk / 2 + p.split - 1) / p.split)) + 5.0 + levels * (5.0 + 0.15 * mb);
+}
+
+// The best way to cut tiles of `base`'s shape that `ws_bytes` of workspace allow: all of them, or those of the last,
+// unfilled round of workgroups.
+static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, size_t ws_bytes, double* cost) {
+  TilePlan best = base;
+  best.split = 1;
+  best.whole = base.tiles;
+  *cost = plan_cost(best, qbits, mode, nk);
+  for (int s = 2; s <= kMaxSplit && nk / s >= 8; s++)
+    for (const int64_t whole : {(int64_t)0, base.tiles / kDenseCUs * kDenseCUs}) {
+      TilePlan p = base;
+      p.split = s;
+      p.whole = whole;
+      if (p.whole >= p.tiles || p.bytes() > ws_bytes || p.bytes() > kDenseMaxWorkspace) continue;
+      const double t = plan_cost(p, qbits, mode, nk);
+      if (t < *cost) {
+        *cost = t;
+        best = p;
+      }
+    }
+  return best;
+}
+
+// The layout of one launch over problems hs[0 .. n) (weights [w_begin, w_end) of each; they share K and the weight
+// format).  `wide`: a fused head epilogue needs tiles of 256 features.
+static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws_bytes) {
+  const dt_qx_weight& w0 = hs[0].W[w_begin];
+  const int64_t K = hs[0].K;
+  const int nk = (int)(K / BK);
+  const auto shape = [&](int tile, int BM, int BN) {
+    TilePlan p;
+    p.tile = tile;
+    p.BM = BM;
+    p.BN = BN;
+    for (int gi = 0; gi < n; gi++)
+      for (int j = w_begin; j < (n > 1 ? hs[gi].n_weights : w_end); j++)
+        p.tiles += ((hs[gi].M + BM - 1) / BM) * ((hs[gi].W[j].count / K + BN - 1) / BN);
+    p.whole = p.tiles;
+    return p;
+  };
+  int64_t m_max = 0, n_max = 0;
+  for (int gi = 0; gi < n; gi++) {
+    m_max = std::max(m_max, hs[gi].M);
+    n_max = std::max(n_max, hs[gi].W[w_begin].count / K);
+  }
+  // (palettes that fit beside no big tile -- 256-entry palettes with small blocks -- would be looked up in memory:
+  // the small tile holds a per-row table of them and is several times faster, unless a fused epilogue needs the big one)
+  const bool pal_fits_big = choose_pal_mode(w0.qbits, w0.nib, K, 256, 256) != kPalGlobal ||
+                            choose_pal_mode(w0.qbits, w0.nib, K, 128, 128) == kPalGlobal;
+  const TilePlan t256 = shape(kTile256x256, 256, 256), tnarrow = shape(kTile128x256, 128, 256);
+  const TilePlan ttall = shape(kTile256x128, 256, 128), tsmall = shape(kTile128x128, 128, 128);
+  const bool tall_ok = (w0.qbits == 7 || w0.qbits == 8) && choose_pal_mode(w0.qbits, w0.nib, K, 256, 128) == kPalRow;
+  const bool big = (((m_max >= 1024) && (n_max >= 256) && t256.tiles >= kFillTiles) && pal_fits_big) || wide;
+  TilePlan base = big ? (m_max < 1024 ? tnarrow : t256) : (!pal_fits_big && tall_ok && m_max >= 1024 && n_max >= 128 && t256.tiles * 2 >= kFillTiles) ? ttall : tsmall;
+  const auto pal_mode = [&](const TilePlan& p) { return choose_pal_mode(w0.qbits, w0.qbits == 16 ? 32 : w0.nib, K, p.BM, p.BN); };
+  // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate, whose error
+  // is up to a tenth, sees a clear gain.
+  const char* knob = getenv("DT_DENSE_SPLIT");  // "never" | "always" (as often as can be; for tests); read at every call
+  if (ws_bytes == 0 || (knob && knob[0] == 'n')) return base;
+  if (knob && knob[0] == 'a') {
+    TilePlan p = pal_fits_big ? (m_max <= 128 ? tnarrow : t256) : tall_ok && !wide ? ttall : base;
+    if (p.tile == kTile128x128) return base;
+    p.whole = 0;
+    p.split = std::min(kMaxSplit, nk / 2);
+    return p.split > 1 && p.bytes() <= std::min(ws_bytes, kDenseMaxWorkspace) ? p : base;
+  }
+  TilePlan best = base;
+  const double start = plan_cost(base, w0.qbits, pal_mode(base), nk);
+  double least = std::min(0.92 * start, start - 8.0);
+  const auto consider = [&](const TilePlan& shape) {
+    double t;
+    const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, ws_bytes, &t);
+    if (t < least) {
+      least = t;
+      best = p;
+    }
+  };
+  if (pal_fits_big) {
+    consider(t256);
+    consider(tnarrow);
+  } else if (tall_ok && !wide) {
+    consider(ttall);
+  }
+  return best;
+}
+
+// End of the run of weights from i on that share a launch: at most kMaxWeights, of one format, all within the tiled
+// kernels' alignment.  *fused: one of them wants its head epilogue fused.
+static int weight_run(const HostGroup& h, int i, bool* fused) {
+  const dt_qx_weight& w0 = h.W[i];
+  int end = i;
+  for (; end < h.n_weights && end - i < kMaxWeights; end++) {
+    const dt_qx_weight& w = h.W[end];
+    if (w.qbits != w0.qbits || (w.qbits != 16 && w.nib != w0.nib) || !h.w_tiled(end)) break;
+    *fused = *fused || (h.wants_epi(end) && h.fusable(end));
+  }
+  return end;
+}
+
 // One validated problem with M > 0: weights that share (qbits, nib) and meet the
 // tiled kernel's alignment go out in runs of up to kMaxWeights per launch; the
 // rest take the any-shape kernel.
-// Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
-constexpr int64_t kFillTiles = 192;
 
-static dt_status run_group(hipStream_t s, const HostGroup& h) {
+// Scratch memory of a call, or none.
+struct Workspace {
+  uint8_t* ptr = nullptr;
+  size_t bytes = 0;
+};
+
+// Zeroes the counters of a K-split launch (a fill kernel, so that the launch can be captured in a graph).
+__global__ void dense_zero_counters_kernel(int32_t* counters, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) counters[i] = 0;
+}
+
+static dt_status launch_plan(hipStream_t s, DenseArgs& a, const TilePlan& plan, const Workspace& ws, int qbits, int mode) {
+  a.whole_tiles = (int32_t)plan.whole;
+  a.split = plan.split;
+  a.partials = nullptr;
+  a.counters = nullptr;
+  if (plan.split > 1) {
+    a.counters = reinterpret_cast<int32_t*>(ws.ptr);
+    a.partials = reinterpret_cast<float*>(ws.ptr + plan.counter_bytes());
+    const int n = (int)(plan.tiles - plan.whole) * kSplitNodes;
+    hipLaunchKernelGGL(dense_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
+    if (const dt_status st = launch_status(); st != DT_OK) return st;
+  }
+  return launch_dense(s, a, plan.tile, qbits, mode);
+}
+
+static dt_status run_group(hipStream_t s, const HostGroup& h, const Workspace& ws) {
   const int64_t M = h.M, K = h.K;
   const bool x_ok = h.x_ok();
   int i = 0;
@@ -245,13 +425,10 @@ static dt_status run_group(hipStream_t s, const HostGroup& h) {
       continue;
     }
     // few rows: the kernel that streams the weights
+    bool any_fused = false;
+    const int run_end = weight_run(h, i, &any_fused);
     int64_t run_features = 0;
-    int run_end = i;
-    for (; run_end < h.n_weights && run_end - i < kMaxWeights; run_end++) {
-      const dt_qx_weight& wj = h.W[run_end];
-      if (wj.qbits != w0.qbits || (wj.qbits != 16 && wj.nib != w0.nib) || !h.w_tiled(run_end)) break;
-      run_features += wj.count / K;
-    }
+    for (int j = i; j < run_end; j++) run_features += h.W[j].count / K;
     if (const int fb = dense_rows_features(M, K, w0.qbits, w0.nib, run_features); fb > 0) {
       DenseArgs a;
       DenseGroup& g = a.g[0];
@@ -274,29 +451,9 @@ static dt_status run_group(hipStream_t s, const HostGroup& h) {
       if (st != DT_OK) return st;
       continue;
     }
-    // tile shape: big tiles when there is enough work to fill 256 CUs with them
-    bool any_fused = false;
-    for (int j = i; j < h.n_weights && j < i + kMaxWeights; j++)
-      any_fused = any_fused || (h.wants_epi(j) && h.fusable(j));
-    // (the fused epilogue needs the 128-feature wave slice of the big tile)
-    int64_t big_tiles = 0;  // 256 x 256 tiles this launch would have
-    for (int j = i, cnt = 0; j < h.n_weights && cnt < kMaxWeights; j++, cnt++) {
-      const dt_qx_weight& wj = h.W[j];
-      if (wj.qbits != w0.qbits || (wj.qbits != 16 && wj.nib != w0.nib) || !h.w_tiled(j)) break;
-      big_tiles += ((M + 255) / 256) * ((wj.count / K + 255) / 256);
-    }
-    // (palettes that fit beside no big tile -- 256-entry palettes with small blocks -- would be looked up in memory:
-    // the small tile holds a per-row table of them and is several times faster, unless a fused epilogue needs the big one)
-    const bool pal_fits_big = choose_pal_mode(w0.qbits, w0.nib, K, 256, 256) != kPalGlobal ||
-                              choose_pal_mode(w0.qbits, w0.nib, K, 128, 128) == kPalGlobal;
-    const bool big = (((M >= 1024) && (n_rows0 >= 256) && big_tiles >= kFillTiles) && pal_fits_big) || any_fused;
-    // few token rows: halve the token tile so that more workgroups share the work
-    const bool narrow = big && M < 1024;
-    // palettes that only fit beside a 128-feature tile, and enough work for tall tiles: 256 tokens x 128 features
-    // (twice the MFMAs per unpacked weight of the 128 x 128 tile)
-    const bool tall = !big && !pal_fits_big && (w0.qbits == 7 || w0.qbits == 8) && M >= 1024 && n_rows0 >= 128 &&
-                      big_tiles * 2 >= kFillTiles;
-    const int BM = big ? (narrow ? 128 : 256) : (tall ? 256 : 128), BN = big ? 256 : 128;
+    const TilePlan plan = plan_tiles(&h, 1, i, run_end, any_fused, ws.bytes);
+    const int BM = plan.BM, BN = plan.BN;
+    const bool big = BN == 256;
     DenseArgs a;
     DenseGroup& g = a.g[0];
     g.x = h.X;
@@ -307,21 +464,14 @@ static dt_status run_group(hipStream_t s, const HostGroup& h) {
     g.w_begin = 0;
     int tiles_n = 0, cnt = 0;
     const int first = i;
-    while (i < h.n_weights && cnt < kMaxWeights) {
-      const dt_qx_weight& w = h.W[i];
-      if (w.qbits != w0.qbits || (w.qbits != 16 && w.nib != w0.nib) || !h.w_tiled(i)) break;
-      tiles_n += add_weight(a, cnt, h, i, tiles_n, BN, big && h.wants_epi(i) && h.fusable(i));
-      cnt++;
-      i++;
-    }
+    for (; i < run_end; i++, cnt++) tiles_n += add_weight(a, cnt, h, i, tiles_n, BN, big && h.wants_epi(i) && h.fusable(i));
     g.w_end = cnt;
     g.tiles_n = tiles_n;
     if ((int64_t)g.tiles_m * tiles_n > 0x7fffffff) return DT_NO_KERNEL;
     a.total_tiles = g.tiles_m * tiles_n;
     finish_args(a, 1, cnt, K, w0);
     const int mode = choose_pal_mode(w0.qbits, a.nib, K, BM, BN);
-    dt_status st = launch_dense(s, a, tall ? kTile256x128 : !big ? kTile128x128 : narrow ? kTile128x256 : kTile256x256,
-                                w0.qbits, mode);
+    dt_status st = launch_plan(s, a, plan, ws, w0.qbits, mode);
     if (st != DT_OK) return st;
     for (int j = first; j < i; j++)
       if (h.wants_epi(j) && !(big && h.fusable(j))) {
@@ -332,10 +482,9 @@ static dt_status run_group(hipStream_t s, const HostGroup& h) {
   return DT_OK;
 }
 
-// All problems in one launch of 256 x 256 tiles, when every X and weight meets
-// the tiled kernel's alignment, they share K and the weight format, and at least
-// one of them is large enough for that tile.  Returns false if they do not fit.
-static bool run_groups_fused(hipStream_t s, const HostGroup* hs, int n, dt_status* status) {
+// All problems in one launch, when every X and weight meets the tiled kernel's alignment, they share K and the weight
+// format, and at least one of them is large enough for a tile of 256.  Returns false if they do not fit.
+static bool groups_fuse(const HostGroup* hs, int n) {
   if (n < 2 || n > kMaxGroups) return false;
   const dt_qx_weight& w0 = hs[0].W[0];
   int total_w = 0;
@@ -361,7 +510,16 @@ static bool run_groups_fused(hipStream_t s, const HostGroup* hs, int n, dt_statu
     for (int i = 0; i < hs[gi].n_weights; i++) any_epi = any_epi || hs[gi].wants_epi(i);
   }
   if (any_post && any_epi) return false;
-  constexpr int BM = 256, BN = 256;
+  int64_t tiles = 0;
+  for (int gi = 0; gi < n; gi++)
+    for (int i = 0; i < hs[gi].n_weights; i++) tiles += ((hs[gi].M + 127) / 128) * ((hs[gi].W[i].count / hs[gi].K + 127) / 128);
+  return tiles <= 0x7fffffff / 8;
+}
+
+static dt_status run_groups_fused(hipStream_t s, const HostGroup* hs, int n, const Workspace& ws) {
+  const dt_qx_weight& w0 = hs[0].W[0];
+  const TilePlan plan = plan_tiles(hs, n, 0, 0, true, ws.bytes);
+  const int BM = plan.BM, BN = plan.BN;
   DenseArgs a;
   int cnt = 0;
   int64_t tiles = 0;
@@ -380,17 +538,65 @@ static bool run_groups_fused(hipStream_t s, const HostGroup* hs, int n, dt_statu
     g.w_end = cnt;
     g.tiles_n = tiles_n;
     tiles += (int64_t)g.tiles_m * tiles_n;
-    if (tiles > 0x7fffffff) return false;
   }
   a.total_tiles = (int32_t)tiles;
   finish_args(a, n, cnt, hs[0].K, w0);
   const int mode = choose_pal_mode(w0.qbits, a.nib, hs[0].K, BM, BN);
-  dt_status st = launch_dense(s, a, kTile256x256, w0.qbits, mode);
+  dt_status st = launch_plan(s, a, plan, ws, w0.qbits, mode);
   for (int gi = 0; gi < n && st == DT_OK; gi++)
     for (int i = 0; i < hs[gi].n_weights && st == DT_OK; i++)
       if (hs[gi].wants_epi(i) && !hs[gi].fusable(i)) st = epilogue_pass(s, hs[gi], i);
-  *status = st;
-  return true;
+  return st;
+}
+
+// The workspace that run_group would use for h.
+static size_t group_workspace(const HostGroup& h) {
+  size_t need = 0;
+  if (!h.x_ok()) return 0;
+  for (int i = 0; i < h.n_weights;) {
+    if (!h.w_tiled(i)) {
+      i++;
+      continue;
+    }
+    bool wide = false;
+    const int end = weight_run(h, i, &wide);
+    int64_t features = 0;
+    for (int j = i; j < end; j++) features += h.W[j].count / h.K;
+    if (dense_rows_features(h.M, h.K, h.W[i].qbits, h.W[i].nib, features) == 0)
+      need = std::max(need, plan_tiles(&h, 1, i, end, wide, kDenseMaxWorkspace).bytes());
+    i = end;
+  }
+  return need;
+}
+
+// The problems of a grouped call that have rows, validated.
+static dt_status gather_groups(int32_t n_groups, const dt_dense_group* groups, HostGroup (&hs)[64], int& n) {
+  if (n_groups < 0 || (n_groups > 0 && !groups)) return DT_INVALID;
+  if (n_groups > 64) return DT_INVALID;
+  n = 0;
+  for (int i = 0; i < n_groups; i++) {
+    const dt_dense_group& d = groups[i];
+    const HostGroup h{d.M, d.K, d.X, d.ldx, d.W, d.n_weights, d.bias, d.Y, d.ldy, d.epi, d.post};
+    dt_status st = validate_group(h);
+    if (st != DT_OK) return st;
+    if (h.M > 0) hs[n++] = h;
+  }
+  return DT_OK;
+}
+
+static dt_status run_groups(dt_stream stream, int32_t n_groups, const dt_dense_group* groups, const Workspace& ws) {
+  HostGroup hs[64];
+  int n = 0;
+  if (const dt_status st = gather_groups(n_groups, groups, hs, n); st != DT_OK) return st;
+  if (n == 0) return DT_OK;
+  if (const dt_status ready = device_ready(); ready != DT_OK) return ready;
+  hipStream_t s = as_stream(stream);
+  if (groups_fuse(hs, n)) return run_groups_fused(s, hs, n, ws);
+  for (int i = 0; i < n; i++) {
+    const dt_status st = run_group(s, hs[i], ws);
+    if (st != DT_OK) return st;
+  }
+  return DT_OK;
 }
 
 }  // namespace dt
@@ -412,7 +618,7 @@ DT_EXPORT dt_status dt_dense_qx_heads_f16(dt_stream stream, int64_t M, int64_t K
   if (st != DT_OK) return st;
   if (M == 0) return DT_OK;
   if (const dt_status ready = device_ready(); ready != DT_OK) return ready;
-  return run_group(as_stream(stream), h);
+  return run_group(as_stream(stream), h, Workspace{});
 }
 
 DT_EXPORT dt_status dt_dense_qx_post_f16(dt_stream stream, int64_t M, int64_t K, const uint16_t* X, int64_t ldx,
@@ -426,32 +632,30 @@ DT_EXPORT dt_status dt_dense_qx_post_f16(dt_stream stream, int64_t M, int64_t K,
   if (st != DT_OK) return st;
   if (M == 0) return DT_OK;
   if (const dt_status ready = device_ready(); ready != DT_OK) return ready;
-  return run_group(as_stream(stream), h);
+  return run_group(as_stream(stream), h, Workspace{});
 }
 
 DT_EXPORT dt_status dt_dense_qx_grouped_f16(dt_stream stream, int32_t n_groups, const dt_dense_group* groups,
                                             uint32_t flags) {
-  using namespace dt;
   (void)flags;
-  if (n_groups < 0 || (n_groups > 0 && !groups)) return DT_INVALID;
-  if (n_groups > 64) return DT_INVALID;
+  return dt::run_groups(stream, n_groups, groups, dt::Workspace{});
+}
+
+DT_EXPORT size_t dt_dense_workspace_bytes(int32_t n_groups, const dt_dense_group* groups) {
+  using namespace dt;
   HostGroup hs[64];
   int n = 0;
-  for (int i = 0; i < n_groups; i++) {
-    const dt_dense_group& d = groups[i];
-    const HostGroup h{d.M, d.K, d.X, d.ldx, d.W, d.n_weights, d.bias, d.Y, d.ldy, d.epi, d.post};
-    dt_status st = validate_group(h);
-    if (st != DT_OK) return st;
-    if (h.M > 0) hs[n++] = h;
-  }
-  if (n == 0) return DT_OK;
-  if (const dt_status ready = device_ready(); ready != DT_OK) return ready;
-  hipStream_t s = as_stream(stream);
-  dt_status st = DT_OK;
-  if (run_groups_fused(s, hs, n, &st)) return st;
-  for (int i = 0; i < n; i++) {
-    st = run_group(s, hs[i]);
-    if (st != DT_OK) return st;
-  }
-  return DT_OK;
+  if (gather_groups(n_groups, groups, hs, n) != DT_OK || n == 0) return 0;
+  if (groups_fuse(hs, n)) return plan_tiles(hs, n, 0, 0, true, kDenseMaxWorkspace).bytes();
+  size_t need = 0;
+  for (int i = 0; i < n; i++) need = std::max(need, group_workspace(hs[i]));
+  return need;
+}
+
+DT_EXPORT dt_status dt_dense_qx_grouped_ws_f16(dt_stream stream, int32_t n_groups, const dt_dense_group* groups,
+                                               uint32_t flags, void* workspace, size_t workspace_bytes) {
+  (void)flags;
+  if (reinterpret_cast<uintptr_t>(workspace) & 255) return DT_INVALID;
+  return dt::run_groups(stream, n_groups, groups,
+                        dt::Workspace{static_cast<uint8_t*>(workspace), workspace ? workspace_bytes : 0});
 }

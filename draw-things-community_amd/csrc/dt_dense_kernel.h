@@ -99,7 +99,19 @@ struct DenseArgs {
   int32_t total_tiles;
   DenseGroup g[kMaxGroups];
   DenseWeight w[kMaxWeights];
+  // K-split launch (SPLIT kernels only): the first `whole_tiles` tiles are one workgroup's work each, every other tile
+  // that of `split` workgroups, each summing a share of K.  `partials`: a slot per share (share-major); `counters`:
+  // kSplitNodes per split tile, zeroed in front of the launch.
+  int32_t whole_tiles;
+  int32_t split;
+  float* partials;
+  int32_t* counters;
 };
+
+constexpr int kMaxSplit = 8;
+constexpr int kSplitNodes = kMaxSplit;  // meetings of a tile's shares: 4 + 2 + 1
+// Bytes of one slot of `partials`: a tile's fp32 sums.
+constexpr int64_t dense_split_slot_bytes(int BM, int BN) { return (int64_t)BM * BN * 4; }
 
 // The tail of output (mi, ni) element by element: v is the Dense's own result, rounded to fp16.
 template <typename W>
@@ -477,7 +489,16 @@ __device__ __forceinline__ void dense_epilogue(float16_t (&acc)[WN / 32][WM / 32
 // are held transposed (rows = output features n, columns = tokens m) so that
 // each lane ends up with runs of consecutive n for one token: 16-byte stores.
 // POST selects the epilogue with the elementwise tail.
-template <int Q, int BM, int BN, int MODE, bool POST>
+//
+// SPLIT: launches whose tiles do not fill the compute units (or fill them a little more than once) cut the tiles of
+// the unfilled round along K.  A workgroup then holds the fp32 sums of a share of K-tile pairs, and the shares meet in
+// pairs, the pairs in pairs, and so on: of two that meet, the first leaves its sums in its slot, counts itself in and
+// ends; the other one adds them to its own registers and goes on to the next meeting, the last of them to the epilogue.
+// Nobody waits for anybody, and a + b being b + a the result does not depend on who came first.  Shares of one tile run
+// on different dies, whose L2 caches do not see each other's ordinary stores: slots are written and read with
+// device-scope accesses.  (The last to arrive adding up all slots in turn, its own among them, took 32 us for three
+// shares of 80 tiles; two that meet take 7.)
+template <int Q, int BM, int BN, int MODE, bool POST, bool SPLIT>
 __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   constexpr int WN = BN / 2, WM = BM / 4;   // per-wave slice: WN features x WM tokens
   constexpr int TN = WN / 32, TM = WM / 32;
@@ -529,11 +550,25 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // feature tiles at 32 CUs: an X slice is 16 KB per K-tile, a packed W slice 4-8 KB),
   // so every X and W panel slice is fetched into that XCD's L2 once per block
   // instead of once per tile column.
-  const int total = a.total_tiles;
-  int bid = blockIdx.x;
-  {
+  auto xcd_order = [](int i, int total) {
     const int per = total / 8;
-    if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
+    return i < per * 8 ? (i & 7) * per + (i >> 3) : i;
+  };
+  int bid = blockIdx.x, share = 0, split_tile = -1;  // share: which part of K (split tiles)
+  if constexpr (SPLIT) {
+    // split tiles follow the whole ones, share by share: the workgroups that run together on a die walk the same
+    // stretch of K of neighbouring tiles
+    if (bid >= a.whole_tiles) {
+      const int rest = a.total_tiles - a.whole_tiles;
+      const int i = xcd_order(bid - a.whole_tiles, rest * a.split);
+      share = i / rest;
+      split_tile = i - share * rest;
+      bid = a.whole_tiles + split_tile;
+    } else {
+      bid = xcd_order(bid, a.whole_tiles);
+    }
+  } else {
+    bid = xcd_order(bid, a.total_tiles);
   }
   int gi = 0;
 #pragma unroll
@@ -560,7 +595,15 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   const int n0 = (tn - w.tile_begin) * BN;
   const int m0 = tm * BM;
   const int K = a.k;
-  const int nk = K / BK;
+  // this workgroup's K-tiles: [t_lo, nk), both even
+  int t_lo = 0, nk = K / BK;
+  if constexpr (SPLIT) {
+    if (split_tile >= 0) {
+      const int pairs = nk / 2;
+      t_lo = 2 * (int)((int64_t)share * pairs / a.split);
+      nk = 2 * (int)((int64_t)(share + 1) * pairs / a.split);
+    }
+  }
   const QxLayout lay = make_layout(Q, a.nib);
   const uint32_t pal_bytes = (uint32_t)lay.pal_bytes;
   // ---- per-thread load coordinates (32-bit byte offsets from uniform bases) ----
@@ -589,7 +632,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   if constexpr (MODE != kPlainF16) {
     int gn = n0 + b_row;
     if (gn >= w.n) gn = w.n - 1;
-    const int64_t e = (int64_t)gn * K;
+    const int64_t e = (int64_t)gn * K + (SPLIT ? t_lo * BK : 0);
     const int64_t blk = e / a.nib;
     const int64_t r = e - blk * a.nib;
     cur.off = (uint32_t)index_byte_offset(lay, blk, r);
@@ -651,7 +694,8 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     if (e == blk * a.nib) fill_pal_column(blk);
   };
   int next_pal_tile = a.pal_step;  // next K-tile at which some row may change block
-  if constexpr (MODE == kPalRow) fill_pal_column(((int64_t)gn_row * K) / a.nib);
+  if constexpr (SPLIT) next_pal_tile = (t_lo / a.pal_step + 1) * a.pal_step;
+  if constexpr (MODE == kPalRow) fill_pal_column(((int64_t)gn_row * K + (SPLIT ? t_lo * BK : 0)) / a.nib);
 
   // ---- staging --------------------------------------------------------------
   struct IdxSet {
@@ -681,7 +725,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 
   // Loads the indices of the tile the cursor points at (the last tile is re-read
   // harmlessly by the final iterations) and moves the cursor on by one tile.
-  int issued = 0;  // tiles loaded so far
+  int issued = SPLIT ? t_lo : 0;  // tile that the cursor points at
   auto issue_idx = [&](IdxSet& R) {
     if constexpr (MODE != kPlainF16) {
       if (!stager) return;
@@ -800,16 +844,16 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   };
 
   // ---- prologue: pair 0 in slot A, weights of tiles 0 and 1 in the ring --------
-  issue_pair(XsA, WpA, 0);
-  issue_idx(WS[0]);  // tile 0
+  issue_pair(XsA, WpA, SPLIT ? t_lo / 2 : 0);
+  issue_idx(WS[0]);  // tile 0 (of this workgroup's)
   issue_idx(WS[1]);  // tile 1
   __syncthreads();   // palettes visible
   stage_to_lds(WS[0], 0);
   issue_idx(WS[0]);  // tile 2
   if constexpr (MODE == kPalRow) {
-    if (next_pal_tile == 1) {  // tile 1 may already start a new palette block
+    if (next_pal_tile == (SPLIT ? t_lo : 0) + 1) {  // tile 1 may already start a new palette block
       __syncthreads();
-      refresh_pal_column(1);
+      refresh_pal_column((SPLIT ? t_lo : 0) + 1);
       next_pal_tile += a.pal_step;
       __syncthreads();
     }
@@ -818,7 +862,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   issue_idx(WS[1]);  // tile 3
   __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
   __syncthreads();
-  if constexpr (MODE == kPlainF16) issue_pair(XsB, WpB, 1);  // (the loop issues pair q + 2 from the middle of pair q)
+  if constexpr (MODE == kPlainF16) issue_pair(XsB, WpB, (SPLIT ? t_lo / 2 : 0) + 1);  // (the loop issues pair q + 2 from the middle of pair q)
 #pragma unroll
   for (int i = 0; i < TN; i++) read_w(0, i, WpA, 0, 0, 0);
 #pragma unroll
@@ -967,7 +1011,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     s_fill = s;
   };
 
-  int t = 0;
+  int t = SPLIT ? t_lo : 0;
   for (; t + 3 < nk; t += 4) {
     iteration(t, 0, XsA, WpA, XsB, WpB);
     iteration(t + 1, 1, XsA, WpA, XsB, WpB);
@@ -983,6 +1027,62 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     // the loop's last barrier lies before the last reads (and every transfer was waited for ahead of it)
     __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
     __syncthreads();
+  }
+  if constexpr (SPLIT) {
+    if (split_tile >= 0) {
+      __shared__ int s_seen;
+      const int64_t slot_step = (int64_t)(a.total_tiles - a.whole_tiles) * (BM * BN);
+      // slot: [TN * TM * 16][512 threads] floats, so that a wave's access covers 256 consecutive bytes
+      float* const slots = a.partials + (int64_t)split_tile * (BM * BN) + tid;
+      int32_t* const counters = a.counters + split_tile * kSplitNodes;
+      int node0 = 0;  // counters of this level
+      for (int level = 0; (1 << level) < a.split; level++) {
+        const int me = share >> level, other = me ^ 1;
+        if ((other << level) < a.split) {  // uniform; otherwise nothing to meet on this level
+          int32_t* const met = counters + node0 + (me >> 1);
+          if (tid == 0) s_seen = __hip_atomic_load(met, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __syncthreads();
+          if (s_seen == 0) {  // uniform: the other sum is not there yet
+            float* const own = slots + (me << level) * slot_step;
+#pragma unroll
+            for (int i = 0; i < TN; i++)
+#pragma unroll
+              for (int j = 0; j < TM; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                  __hip_atomic_store(own + ((i * TM + j) * 16 + v) * 512, acc[i][j][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // every wave's stores have been acknowledged before the barrier, hence before the count that publishes them
+            __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
+            __syncthreads();
+            if (tid == 0) s_seen = __hip_atomic_fetch_add(met, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (s_seen == 0) return;  // uniform: the other one goes on
+          }
+          const float* const theirs = slots + (other << level) * slot_step;
+          constexpr int NH = TN * TM > 4 ? 2 : 1;  // in halves where a whole slot would not fit beside the sums
+#pragma unroll
+          for (int h = 0; h < NH; h++) {
+            float16_t got[TN / NH][TM];
+#pragma unroll
+            for (int i = 0; i < TN / NH; i++)
+#pragma unroll
+              for (int j = 0; j < TM; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++)
+                  got[i][j][v] = __hip_atomic_load(theirs + (((h * (TN / NH) + i) * TM + j) * 16 + v) * 512, __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < TN / NH; i++)
+#pragma unroll
+              for (int j = 0; j < TM; j++) acc[h * (TN / NH) + i][j] += got[i][j];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          __syncthreads();  // s_seen may be written again
+        }
+        node0 += kSplitNodes >> (level + 1);
+      }
+    }
   }
   dense_epilogue<WN, WM, POST>(acc, smem, wave, lane, n0 + wn * WN, (int64_t)m0 + wm * WM, w, g.m);
 }

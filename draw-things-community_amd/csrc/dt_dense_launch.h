@@ -9,23 +9,29 @@ namespace dt {
 // 128 and 256 entries -- and is instantiated for those index widths only)
 enum DenseTile : int { kTile128x128 = 0, kTile128x256 = 1, kTile256x256 = 2, kTile256x128 = 3 };
 
-template <int Q, int BM, int BN, bool POST>
+template <int Q, int BM, int BN, bool POST, bool SPLIT>
 static dt_status launch_tiled(hipStream_t s, const DenseArgs& a, int mode) {
-  dim3 grid((unsigned)a.total_tiles), block(512);
+  const int64_t rest = SPLIT ? a.total_tiles - a.whole_tiles : 0;
+  dim3 grid((unsigned)(a.total_tiles - rest + rest * a.split)), block(512);
   if constexpr (Q == 16) {  // plain fp16 weight
-    hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT>), grid, block, 0, s, a);
     return launch_status();
   } else {
     switch (mode) {
-      case kPalShared: hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalShared, POST>), grid, block, 0, s, a); break;
+      case kPalShared:
+        if constexpr (BM == 256 && BN == 128) return DT_NO_KERNEL;
+        else hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalShared, POST, SPLIT>), grid, block, 0, s, a);
+        break;
       case kPalRow:
         if constexpr ((BN << (Q + 1)) <= pal_lds_bytes(BM, BN, kPalRow)) {
-          hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalRow, POST>), grid, block, 0, s, a);
+          hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalRow, POST, SPLIT>), grid, block, 0, s, a);
           break;
         } else {
           return DT_NO_KERNEL;  // choose_pal_mode never picks per-row palettes that do not fit
         }
-      default: hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalGlobal, POST>), grid, block, 0, s, a); break;
+      default:
+        if constexpr (BM == 256 && BN == 128) return DT_NO_KERNEL;
+        else hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalGlobal, POST, SPLIT>), grid, block, 0, s, a);
     }
     return launch_status();
   }
@@ -34,17 +40,18 @@ static dt_status launch_tiled(hipStream_t s, const DenseArgs& a, int mode) {
 template <int Q, bool POST>
 static dt_status launch_dense_qp(hipStream_t s, const DenseArgs& a, int tile, int mode) {
   switch (tile) {
-    case kTile128x128: return launch_tiled<Q, 128, 128, POST>(s, a, mode);
-    case kTile128x256: return launch_tiled<Q, 128, 256, POST>(s, a, mode);
+    case kTile128x128: return launch_tiled<Q, 128, 128, POST, false>(s, a, mode);
+    case kTile128x256:
+      return a.partials ? launch_tiled<Q, 128, 256, POST, true>(s, a, mode) : launch_tiled<Q, 128, 256, POST, false>(s, a, mode);
     case kTile256x128:
       if constexpr (Q == 7 || Q == 8) {
         if (mode != kPalRow) return DT_NO_KERNEL;
-        hipLaunchKernelGGL((dense_qx_kernel<Q, 256, 128, kPalRow, POST>), dim3((unsigned)a.total_tiles), dim3(512), 0, s, a);
-        return launch_status();
+        return a.partials ? launch_tiled<Q, 256, 128, POST, true>(s, a, mode) : launch_tiled<Q, 256, 128, POST, false>(s, a, mode);
       } else {
         return DT_NO_KERNEL;  // the host side picks this tile for 7- and 8-bit indices only
       }
-    default: return launch_tiled<Q, 256, 256, POST>(s, a, mode);
+    default:
+      return a.partials ? launch_tiled<Q, 256, 256, POST, true>(s, a, mode) : launch_tiled<Q, 256, 256, POST, false>(s, a, mode);
   }
 }
 

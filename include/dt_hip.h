@@ -276,6 +276,17 @@ dt_status dt_dense_qx_grouped_f16(dt_stream stream, int32_t n_groups, const dt_d
                                   uint32_t flags);
 
 /*
+ * The same with scratch memory: where a launch has too few tiles for the chip (or a few more than it runs at once),
+ * tiles are cut along K, their shares' fp32 sums kept in the workspace and added up in a fixed order.
+ * dt_dense_workspace_bytes() says how much the call can use (0 = it would not cut anything, or the arguments are not
+ * valid); with less, or none, it cuts less or nothing.  workspace: device memory, 256-byte aligned (DT_INVALID
+ * otherwise), its contents do not matter; calls that may overlap in time need one each.
+ */
+size_t dt_dense_workspace_bytes(int32_t n_groups, const dt_dense_group* groups);
+dt_status dt_dense_qx_grouped_ws_f16(dt_stream stream, int32_t n_groups, const dt_dense_group* groups,
+                                     uint32_t flags, void* workspace, size_t workspace_bytes);
+
+/*
  * In place on a [B, S, H, D] view: optional RMSNorm, then optional RoPE.
  *   gamma       : RMSNorm weight, [D] when norm_per_head != 0 (Flux:
  *                 RMSNorm(axis: [3]), Models/Flux1.swift:165), [H*D] when 0

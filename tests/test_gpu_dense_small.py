@@ -108,3 +108,114 @@ def test_lora_branch_fp32_shapes(dthip, M, K, rank, N):
     assert np.all(np.abs(T.cpu().numpy() - t) <= (K + 2) * 2.0 ** -24 * t_abs)
     want, sums = t @ up.T, (K + rank + 2) * 2.0 ** -24 * (t_abs @ np.abs(up).T)
     assert np.all(np.abs(out.cpu().numpy().astype(np.float64) - want) <= sums + (np.abs(want) + sums) * 2.0 ** -11 + 2.0 ** -25)
+
+
+@pytest.mark.parametrize("M,N,K,q,nib", [
+    (65, 256, 128, 6, 4096), (128, 300, 192, 5, 1024),    # 128 x 256 tiles; 2 and 3 shares
+    (129, 257, 320, 4, 512), (300, 600, 448, 6, 64),      # 256 x 256 tiles; 5 and 7 shares, ragged edges, a block per 64 columns
+    (257, 256, 576, 8, 16384), (200, 130, 704, 16, 0),    # 8 shares of unequal length; shared palettes, plain fp16
+    (200, 140, 512, 8, 512), (130, 300, 1088, 7, 4096),   # palettes that only fit beside 256 x 128 tiles
+])
+def test_dense_cut_along_k(dthip, oracle, monkeypatch, M, N, K, q, nib):
+    import torch
+
+    rng = np.random.default_rng(M * 7 + N * 5 + K + q)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    pairs = [make(dthip, oracle, rng, n, K, q, nib) for n in (N, 128)]
+    ws, bias = [w for w, _ in pairs], dev((rng.standard_normal(N) * 0.1).astype(np.float16))
+    x, gate = dev(X), dev((1 + 0.3 * rng.standard_normal(N)).astype(np.float16))
+    gamma, rot = dev((1 + 0.1 * rng.standard_normal(128)).astype(np.float16)), dev(rng.standard_normal((M + 3, 128)).astype(np.float16))
+    epi = [None, dthip.HeadEpilogue(gamma, rot, 3)]
+    print("dense cut along K", M, N, K, q, nib, flush=True)
+    monkeypatch.setenv("DT_DENSE_SPLIT", "always")
+    outs = dthip.dense_multi(x, ws, [bias, None])
+    again = dthip.dense_multi(x, ws, [bias, None])
+    check(outs[0].cpu().numpy(), X, pairs[0][1], bias.cpu().numpy())
+    check(outs[1].cpu().numpy(), X, pairs[1][1])
+    assert all(torch.equal(a, b) for a, b in zip(outs, again))
+    # the tails act on the same sums, bit for bit
+    res = dev(rng.standard_normal((M, N)).astype(np.float32))
+    want = res + (outs[0].float() * gate.float()).half().float()
+    dthip.dense_post(x, ws, [bias, None], [dthip.DensePost(gate=gate, residual=res, keep_output=False), None])
+    assert torch.equal(res, want)
+    if q == 16 or K * 2 ** q * 2 * 256 // nib <= 32768 or q <= 6:  # (the head epilogue's tiles are 256 wide)
+        fused = dthip.dense_multi(x, ws, [bias, None], epilogues=epi)
+        lead = dthip.dense_multi(x, ws, [bias, None])[1]
+        assert torch.equal(fused[0], outs[0])
+        v = lead.float()
+        n = (v * torch.rsqrt((v * v).mean(-1, keepdim=True) + 1e-6) * gamma.float()).half().float()
+        r = rot[3:].float()
+        turned = torch.stack([n[:, ::2] * r[:, ::2] - n[:, 1::2] * r[:, 1::2], n[:, ::2] * r[:, 1::2] + n[:, 1::2] * r[:, ::2]], -1).reshape(M, 128)
+        # one fp16 rounding more or less of a normalised value, turned: 2^-10 of the pair's magnitude, plus the last rounding
+        mag = torch.hypot(n[:, ::2], n[:, 1::2]).repeat_interleave(2, -1) * torch.hypot(r[:, ::2], r[:, 1::2]).repeat_interleave(2, -1)
+        assert bool(((fused[1].float() - turned).abs() <= mag * 2.0 ** -9 + 2.0 ** -24).all())
+
+
+def _groups(dthip, x, w, out):
+    """One problem as the C entry points take it, and what keeps it alive."""
+    import ctypes
+
+    W = (dthip._QxWeight * 1)(w._c())
+    Y, LDY = (ctypes.c_void_p * 1)(out.data_ptr()), (ctypes.c_int64 * 1)(out.stride(0))
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(x.shape[0], x.shape[1], x.data_ptr(), x.stride(0), ctypes.addressof(W), 1, None,
+                                                  ctypes.addressof(Y), ctypes.addressof(LDY), None, None))
+    return G, (W, Y, LDY)
+
+
+def test_dense_workspace_is_optional(dthip, oracle, monkeypatch):
+    """A launch of few tiles is cut without being told to; too little workspace, or none, gives the uncut result, a
+    misaligned one is refused; and a captured graph replays the cut launch, its counters zeroed each time."""
+    import torch
+
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    rng = np.random.default_rng(12)
+    X = rng.standard_normal((300, 3072)).astype(np.float16)
+    w, W = make(dthip, oracle, rng, 512, 3072, 6, 4096)
+    x, out = dev(X), torch.zeros((300, 512), dtype=torch.float16, device="cuda")
+    G, keep = _groups(dthip, x, w, out)
+    L, s = dthip.lib(), torch.cuda.current_stream().cuda_stream
+    need = L.dt_dense_workspace_bytes(1, G)
+    assert need > 0
+    ws = torch.full((need + 256,), 0xff, dtype=torch.uint8, device="cuda")
+    assert L.dt_dense_qx_grouped_f16(s, 1, G, 0) == 0
+    whole = out.clone()
+    check(whole.cpu().numpy(), X, W)
+    for give in (0, 256):
+        out.zero_()
+        assert L.dt_dense_qx_grouped_ws_f16(s, 1, G, 0, ws.data_ptr() if give else None, give) == 0
+        assert torch.equal(out, whole)
+    assert L.dt_dense_qx_grouped_ws_f16(s, 1, G, 0, ws.data_ptr() + 64, need) == dthip.DT_INVALID
+    assert L.dt_dense_qx_grouped_ws_f16(s, 1, G, 0, ws.data_ptr(), need) == 0
+    cut = out.clone()
+    check(cut.cpu().numpy(), X, W)
+    print("dense cut along K as hip graph", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        L.dt_dense_qx_grouped_ws_f16(torch.cuda.current_stream().cuda_stream, 1, G, 0, ws.data_ptr(), need)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, cut)
+        assert L.dt_dense_qx_grouped_ws_f16(s, 1, G, 0, ws.data_ptr(), need) == 0
+
+
+def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
+    """288 tiles: 256 stay whole, the 32 of the second round are cut; against the uncut launch, one fp16 rounding apart."""
+    import torch
+
+    rng = np.random.default_rng(13)
+    M, N, K = 1530, 12288, 3072
+    w, _ = make(dthip, oracle, rng, N, K, 6, 4096)
+    x = dev(rng.standard_normal((M, K)).astype(np.float16))
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    whole = dthip.dense_multi(x, [w], [None])[0].float()
+    monkeypatch.delenv("DT_DENSE_SPLIT")
+    G, keep = _groups(dthip, x, w, torch.empty((M, N), dtype=torch.float16, device="cuda"))
+    print("dense last round cut along K", flush=True)
+    assert dthip.lib().dt_dense_workspace_bytes(1, G) > 0
+    cut = dthip.dense_multi(x, [w], [None])[0].float()
+    # the two sums differ by at most 2 K 2^-24 sum |x w| <= 2 K 2^-24 |x| |w| (row norms), the roundings by 2^-10 of the value
+    sums = 2 * K * 2.0 ** -24 * x.float().norm(dim=1)[:, None] * w.dequantize().float().norm(dim=1)[None]
+    assert bool(((cut - whole).abs() <= whole.abs() * 2.0 ** -10 + sums + 2.0 ** -24).all())
+    assert not torch.equal(cut, whole)
