@@ -51,6 +51,7 @@ struct SdpaSplit {
   int32_t shares;         // this many parts
   size_t counter_bytes;   // counters of the cut tasks (256-byte aligned), followed by
   size_t partial_bytes;   // a slot per part
+  size_t room;            // workspace to ask callers for (at least bytes())
   size_t bytes() const { return counter_bytes + partial_bytes; }
 };
 // True when splitting pays: the task count leaves a good part of the last round of workgroups idle and there are enough

@@ -17,6 +17,7 @@
 // the V^T operand (head dimension along lanes, keys along registers) comes
 // from ds_read_b64_tr_b16, which hands lane j of a 16-lane group the element
 // column (j % 4) of the rows addressed by lanes (j / 4) + {0, 4, 8, 12}.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 
@@ -680,6 +681,8 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
   if (always && shares < 2 && n_tiles >= 2) shares = 2;
   if (cut == 0 || shares < 2) return false;
   if (!always) {
+    // (launches of six rounds and more keep asking for no workspace: a seventh of their time at most is the last round)
+    if (tasks >= 6LL * cus) return false;
     // Measured on this part: a key tile of the last, partial round takes 1.4 us at head size 128 (1.0 at 64 and below)
     // while most of the card idles and 1.9 us (1.2) when none of it does, and cutting costs 20 us (12): the counters'
     // launch, the parts' way out and in.  Head size 128, us before / after: 264 tasks of 42 key tiles 150 / 120, of 72
@@ -696,7 +699,11 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
     plan->cut_tasks = (int32_t)cut;
     plan->whole_tasks = (int32_t)whole;
     plan->counter_bytes = ((size_t)cut * kSdpaSplitNodes * 4 + 255) & ~(size_t)255;
-    plan->partial_bytes = (size_t)(cut * shares) * sdpa_split_slot_floats(D <= 64 ? 64 : 128) * 4;
+    const size_t slot = (size_t)sdpa_split_slot_floats(D <= 64 ? 64 : 128) * 4;
+    plan->partial_bytes = (size_t)(cut * shares) * slot;
+    // What callers are asked to bring: two slots for each of up to 8 workgroups per task, at most one per compute unit.
+    // The parts need no more than that (2 cut < 2 cus slots, or cut * shares <= cus of them and 32 bytes per task).
+    plan->room = (((size_t)tasks * 4 + 255) & ~(size_t)255) + 2 * (size_t)std::min<int64_t>(cus, tasks * kSdpaSplitNodes) * slot;
   }
   return true;
 }

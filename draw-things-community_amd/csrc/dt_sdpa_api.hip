@@ -31,7 +31,7 @@ DT_EXPORT size_t dt_sdpa_workspace_bytes(int32_t B, int32_t Hq, int32_t Hk, int3
   // counters), for launches whose workgroup count leaves a good part of the last round of compute units idle.  A
   // call that is handed less than this, but at least the staging bytes above, runs unsplit.
   SdpaSplit plan;
-  if (sdpa_split_plan(B, Hq, D, Sq, Skv, &plan)) bytes += align256(plan.bytes());
+  if (sdpa_split_plan(B, Hq, D, Sq, Skv, &plan)) bytes += align256(plan.room);
   return bytes;
 }
 
