@@ -245,75 +245,68 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       v_off[i] = (uint32_t)((ld_row[i] * a.v[0].ss + v_ch[i] * 8) * 2) + (uint32_t)t_lo * v_step;
     }
   }
-  // General case: a uniform cursor holds the segment the next tile starts in --
-  // address of the tile's first row, row stride, last row of the segment --
-  // and is re-read from the argument block only when a tile starts past that
-  // segment's end.  Tiles inside the segment are fetched with per-lane 32-bit
-  // offsets from the cursor; a tile that straddles segments goes row by row.
+  // General case: a uniform cursor holds the address of the next tile's first row, the step to the tile behind it and
+  // the first tile that does not lie wholly inside the segment.  Up to there a tile costs one scalar comparison and one
+  // addition, and its lanes fetch with 32-bit offsets from the cursor; a tile that straddles segments or ends the
+  // sequence goes row by row and moves the cursor to the segment the next tile starts in.
   struct SegCursor {
-    const char* base;  // first row of the next tile (this batch and head)
-    int64_t ss;        // row stride, elements
-    int64_t end;       // first joint row past the segment
-    int64_t row0;      // first joint row of the next tile
+    const char* base;
+    int64_t step;
+    int inside;  // tiles below this one lie inside the segment
   };
-  // (an end of 0 makes the first tile look its segment up)
-  SegCursor kcur{nullptr, 0, 0, (int64_t)t_lo * BKV}, vcur{nullptr, 0, 0, (int64_t)t_lo * BKV};
-  auto seek = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[LOADS], const int (&chs)[LOADS])
+  auto seek = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[LOADS], const int (&chs)[LOADS], int t)
                   __attribute__((always_inline)) {
+    const int64_t row0 = (int64_t)t * BKV;
     int sg = 0;
 #pragma unroll
     for (int i = 1; i < kMaxSeg; i++)
-      if (i < a.n_kvseg && c.row0 >= segs[i].start) sg = i;
-    c.ss = segs[sg].ss;
-    c.end = (sg + 1 < a.n_kvseg) ? segs[sg + 1].start : Skv;
-    c.base = reinterpret_cast<const char*>(segs[sg].ptr + b * segs[sg].sb + hk * segs[sg].sh +
-                                           (c.row0 - segs[sg].start) * c.ss);
+      if (i < a.n_kvseg && row0 >= segs[i].start) sg = i;
+    const int64_t ss = segs[sg].ss, end = (sg + 1 < a.n_kvseg) ? segs[sg + 1].start : Skv;
+    c.inside = ss > 0 && ss < (1 << 24) ? (int)(end / BKV) : 0;
+    c.step = ss * (BKV * 2);
+    c.base = reinterpret_cast<const char*>(segs[sg].ptr + b * segs[sg].sb + hk * segs[sg].sh + (row0 - segs[sg].start) * ss);
 #pragma unroll
-    for (int i = 0; i < LOADS; i++) off[i] = (uint32_t)((ld_row[i] * c.ss + chs[i] * 8) * 2);
+    for (int i = 0; i < LOADS; i++) off[i] = (uint32_t)((ld_row[i] * ss + chs[i] * 8) * 2);
   };
+  SegCursor kcur{nullptr, 0, 0}, vcur{nullptr, 0, 0};
+  if constexpr (!ONESEG) {
+    seek(a.k, kcur, k_off, k_ch, t_lo);
+    seek(a.v, vcur, v_off, v_ch, t_lo);
+  }
   // (zero_tail: rows of the tile past the last key get zeros instead of keeping an earlier tile's bytes -- for V,
   // whose stale rows would otherwise meet a probability of exactly zero in the second MFMA: 0 x Inf = NaN)
   auto zero_slot = [&](unsigned char* dst, int i) __attribute__((always_inline)) {
     *reinterpret_cast<uint4_t*>(dst + (wave * LOADS + i) * 1024 + lane * 16) = uint4_t{0, 0, 0, 0};
   };
   auto issue_general = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[LOADS], const int (&chs)[LOADS],
-                           unsigned char* dst, bool zero_tail) __attribute__((always_inline)) {
-    if (c.row0 < Skv) {
-      if (c.row0 >= c.end) seek(segs, c, off, chs);  // uniform
-      const int64_t last = c.row0 + BKV < Skv ? c.row0 + BKV : Skv;
-      if (zero_tail && last - c.row0 < BKV) {  // uniform: the ragged last tile
+                           unsigned char* dst, int t, bool zero_tail) __attribute__((always_inline)) {
+    if (t < c.inside) {  // uniform
 #pragma unroll
-        for (int i = 0; i < LOADS; i++)
-          if (c.row0 + ld_row[i] >= Skv) zero_slot(dst, i);
-      }
-      if (last <= c.end && c.ss > 0 && c.ss < (1 << 24)) {
-        const int n_rows = (int)(last - c.row0);
-        const void* base = c.base;
+      for (int i = 0; i < LOADS; i++)
+        if (chs[i] * 8 < D) load_to_lds_16(c.base, off[i], lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
+      c.base += c.step;
+      return;
+    }
+    const int64_t row0 = (int64_t)t * BKV;
 #pragma unroll
-        for (int i = 0; i < LOADS; i++)
-          if (ld_row[i] < n_rows && chs[i] * 8 < D)
-            load_to_lds_16(base, off[i], lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
-      } else {
+    for (int i = 0; i < LOADS; i++) {
+      const int64_t kj = row0 + ld_row[i];
+      if (kj >= Skv) {
+        if (zero_tail) zero_slot(dst, i);
+      } else if (chs[i] * 8 < D) {
+        int sl = 0;
 #pragma unroll
-        for (int i = 0; i < LOADS; i++) {
-          const int64_t kj = c.row0 + ld_row[i];
-          if (kj < Skv && chs[i] * 8 < D) {
-            int sl = 0;
-#pragma unroll
-            for (int u = 1; u < kMaxSeg; u++)
-              if (u < a.n_kvseg && kj >= segs[u].start) sl = u;
-            const uint16_t* src =
-                segs[sl].ptr + b * segs[sl].sb + (kj - segs[sl].start) * segs[sl].ss + hk * segs[sl].sh + chs[i] * 8;
-            load_to_lds_16(src, lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
-          }
-        }
+        for (int u = 1; u < kMaxSeg; u++)
+          if (u < a.n_kvseg && kj >= segs[u].start) sl = u;
+        const uint16_t* src =
+            segs[sl].ptr + b * segs[sl].sb + (kj - segs[sl].start) * segs[sl].ss + hk * segs[sl].sh + chs[i] * 8;
+        load_to_lds_16(src, lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
       }
     }
-    c.base += c.ss * (BKV * 2);
-    c.row0 += BKV;
+    if (t + 1 < n_tiles) seek(segs, c, off, chs, t + 1);
   };
   // starts the transfer of the next K (or V) tile and moves on by one tile
-  auto issue_k = [&](unsigned char* dst) __attribute__((always_inline)) {
+  auto issue_k = [&](unsigned char* dst, [[maybe_unused]] int t) __attribute__((always_inline)) {
     if constexpr (ONESEG) {
 #pragma unroll
       for (int i = 0; i < LOADS; i++) {
@@ -323,10 +316,10 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       }
       rows_left -= BKV;
     } else {
-      issue_general(a.k, kcur, k_off, k_ch, dst, false);
+      issue_general(a.k, kcur, k_off, k_ch, dst, t, false);
     }
   };
-  auto issue_v = [&](unsigned char* dst) __attribute__((always_inline)) {
+  auto issue_v = [&](unsigned char* dst, [[maybe_unused]] int t) __attribute__((always_inline)) {
     if constexpr (ONESEG) {
       if (rows_left_v < BKV) {  // uniform: the ragged last tile
 #pragma unroll
@@ -341,7 +334,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       }
       rows_left_v -= BKV;
     } else {
-      issue_general(a.v, vcur, v_off, v_ch, dst, true);
+      issue_general(a.v, vcur, v_off, v_ch, dst, t, true);
     }
   };
   // ---- running state -----------------------------------------------------
@@ -486,7 +479,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   // one starts each interval with the softmax of the scores it produced in the
   // previous interval, so one wave's exponentials overlap the other's MFMAs.
   const bool second = wave >= 4;
-  issue_k(Ks0);  // K(0)
+  issue_k(Ks0, t_lo);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the tile has landed
   __syncthreads();
 
@@ -494,8 +487,8 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   // k_next, V(t) to v_cur
   auto interval = [&](int t, const unsigned char* k_cur, unsigned char* k_next, const unsigned char* v_prev,
                       unsigned char* v_cur) __attribute__((always_inline)) {
-    if (t + 1 < t_hi) issue_k(k_next);
-    if (t < t_hi) issue_v(v_cur);
+    if (t + 1 < t_hi) issue_k(k_next, t + 1);
+    if (t < t_hi) issue_v(v_cur, t);
     // the wave doing softmax arithmetic gets issue priority: its exponentials only make progress in
     // the gaps the other wave's MFMA stream leaves (measured: +1 %; the opposite assignment -2 %)
     if (!second) {
