@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import subprocess
 from dataclasses import dataclass
 from typing import Optional, Sequence
@@ -82,6 +83,13 @@ class _DenseGroup(ctypes.Structure):
                 ("post", ctypes.c_void_p)]
 
 
+# The same four as struct formats: a launch's arrays are packed in one go (a ctypes structure costs a microsecond each,
+# which for a conditioning row's six projections is more than the kernel takes).
+_FMT_WEIGHT, _FMT_EPI, _FMT_POST, _FMT_GROUP = "Qiiq", "QQqfi", "i4xQQqf4xQqQQq", "qqQqQi4xQQQQQ"
+for _fmt, _cls in ((_FMT_WEIGHT, _QxWeight), (_FMT_EPI, _HeadEpilogue), (_FMT_POST, _DensePost), (_FMT_GROUP, _DenseGroup)):
+    assert struct.calcsize("=" + _fmt) == ctypes.sizeof(_cls)
+
+
 class _Segment(ctypes.Structure):
     _fields_ = [("view", _View4), ("len", ctypes.c_int64), ("gamma", ctypes.c_void_p)]
 
@@ -134,9 +142,9 @@ def lib():
         L.dt_dense_qx_grouped_f16.restype = i32
         L.dt_dense_qx_grouped_f16.argtypes = [vp, i32, ctypes.POINTER(_DenseGroup), ctypes.c_uint32]
         L.dt_dense_workspace_bytes.restype = ctypes.c_size_t
-        L.dt_dense_workspace_bytes.argtypes = [i32, ctypes.POINTER(_DenseGroup)]
+        L.dt_dense_workspace_bytes.argtypes = [i32, vp]
         L.dt_dense_qx_grouped_ws_f16.restype = i32
-        L.dt_dense_qx_grouped_ws_f16.argtypes = [vp, i32, ctypes.POINTER(_DenseGroup), ctypes.c_uint32, vp, ctypes.c_size_t]
+        L.dt_dense_qx_grouped_ws_f16.argtypes = [vp, i32, vp, ctypes.c_uint32, vp, ctypes.c_size_t]
         L.dt_qk_norm_rope_f16.argtypes = [vp, _View4, i32, i64, i32, i32, vp, f32, i32, vp, i64, f32]
         L.dt_layernorm_modulate_f16.restype = i32
         L.dt_layernorm_modulate_f16.argtypes = [vp, i64, i64, vp, i64, vp, vp, i32, f32, vp, i64]
@@ -357,66 +365,76 @@ class HeadEpilogue:
     head_dim: int = 128
 
 
-def _marshal_dense(x, weights, biases, outs, epilogues):
-    """ctypes arguments of one Dense problem; returns (keepalive, fields, outs, M, x2)."""
-    torch = _torch()
+def _pack_epilogues(epilogues, M):
+    vals = []
+    for e in epilogues:
+        if e is None:
+            vals += (0, 0, 0, 0.0, 128)
+            continue
+        if e.rot is not None:
+            _f16_cuda(e.rot, "rot")
+            if e.rot.dim() != 2 or e.rot.shape[1] != e.head_dim or not e.rot.is_contiguous() \
+                    or e.rot.shape[0] < e.rot_pos0 + M:
+                raise ValueError("rot must be a contiguous [>= rot_pos0 + M, head_dim] table")
+        if e.gamma is not None and (_f16_cuda(e.gamma, "gamma").numel() != e.head_dim or not e.gamma.is_contiguous()):
+            raise ValueError("gamma must hold head_dim elements")
+        vals += (0 if e.gamma is None else e.gamma.data_ptr(), 0 if e.rot is None else e.rot.data_ptr(), e.rot_pos0, e.eps,
+                 e.head_dim)
+    return struct.pack("=" + _FMT_EPI * len(epilogues), *vals)
+
+
+def _marshal_dense(x, weights, biases, outs, epilogues, posts):
+    """One Dense problem: (what it keeps alive, its packed dt_dense_group, its outputs, M)."""
     _f16_cuda(x, "x")
     K = x.shape[-1]
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
     M = x2.shape[0]
     n = len(weights)
-    W = (_QxWeight * n)(*[w._c() for w in weights])
+    vals = []
     for w in weights:
         if w.shape[1] != K:
             raise ValueError(f"weight {w.shape} does not match input width {K}")
-    if outs is None:
-        outs = [torch.empty((M, w.shape[0]), dtype=torch.float16, device=x.device) for w in weights]
-    vp = ctypes.c_void_p
-    B = (vp * n)(*[None if b is None else _f16_cuda(b, "bias").data_ptr() for b in biases])
-    Y = (vp * n)(*[o.data_ptr() for o in outs])
-    LDY = (ctypes.c_int64 * n)(*[o.stride(0) for o in outs])
-    E = None
-    if epilogues is not None:
-        E = (_HeadEpilogue * n)()
-        for i, e in enumerate(epilogues):
-            if e is None:
-                E[i] = _HeadEpilogue(None, None, 0, 0.0, 128)
-                continue
-            if e.rot is not None:
-                _f16_cuda(e.rot, "rot")
-                if e.rot.dim() != 2 or e.rot.shape[1] != e.head_dim or not e.rot.is_contiguous() \
-                        or e.rot.shape[0] < e.rot_pos0 + M:
-                    raise ValueError("rot must be a contiguous [>= rot_pos0 + M, head_dim] table")
-            if e.gamma is not None and (_f16_cuda(e.gamma, "gamma").numel() != e.head_dim or not e.gamma.is_contiguous()):
-                raise ValueError("gamma must hold head_dim elements")
-            E[i] = _HeadEpilogue(None if e.gamma is None else e.gamma.data_ptr(),
-                                 None if e.rot is None else e.rot.data_ptr(), e.rot_pos0, e.eps, e.head_dim)
-    return (x2, M, K, n, W, B, Y, LDY, E, outs)
+        vals += (w.data.data_ptr(), w.qbits, w.nib, w.count)
+    outs = [x.new_empty((M, w.shape[0])) for w in weights] if outs is None else list(outs)
+    ptrs = [0 if b is None else _f16_cuda(b, "bias").data_ptr() for b in biases]
+    if len(ptrs) != n or len(outs) != n:
+        raise ValueError("weights, biases and outs must be of one length")
+    ys = [o.data_ptr() for o in outs]
+    strides = [o.stride(0) for o in outs]
+    # (a problem with both is for the library to refuse)
+    epi = b"" if epilogues is None else _pack_epilogues(epilogues, M)
+    post = b"" if posts is None else _pack_posts(posts, weights, M, ys, outs)
+    arrays = ctypes.create_string_buffer(struct.pack(f"={_FMT_WEIGHT * n}{2 * n}Q{n}q", *vals, *ptrs, *ys, *strides) + epi + post)
+    base = ctypes.addressof(arrays)
+    tails = base + 48 * n
+    group = struct.pack("=" + _FMT_GROUP, M, K, x2.data_ptr(), x2.stride(0), base, n, base + 24 * n, base + 32 * n, base + 40 * n,
+                        0 if epilogues is None else tails, 0 if posts is None else tails + len(epi))
+    return (x2, arrays), group, outs, M
 
 
 _ROWS_MAX = 64  # rows up to which the library streams the weights and needs no workspace
 
 
-def _addr(a):
-    return None if a is None else ctypes.addressof(a)
-
-
-def _enqueue_dense(groups, flags, stream, device):
-    """Enqueues an array of _DenseGroup, with the scratch memory that lets the library cut tiles along K where there are
-    too few of them for the chip.  (Caller: the arrays that the groups point to stay alive until this returns.)"""
-    n = len(groups)
-    need = lib().dt_dense_workspace_bytes(n, groups)
+def _enqueue_dense(fn, problems, flags, stream):
+    """Enqueues Dense problems -- (x, weights, biases, outs, epilogues, posts) each -- together, with the scratch memory
+    that lets the library cut tiles along K where there are too few of them for the chip.  Returns their outputs."""
+    packed = [_marshal_dense(*p) for p in problems]
+    groups = b"".join(g for _, g, _, _ in packed)  # (what they point to lives in `packed` until the call returns)
+    n, L = len(packed), lib()
+    need = L.dt_dense_workspace_bytes(n, groups) if any(M > _ROWS_MAX for _, _, _, M in packed) else 0
     # torch's allocator hands the block out again in stream order, so it may be dropped as soon as the call is enqueued
-    ws = _torch().empty(need, dtype=_torch().uint8, device=device) if need else None
-    st = lib().dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, None if ws is None else ws.data_ptr(), need)
-    _check("dt_dense_qx_grouped_ws_f16", st)
+    ws = problems[0][0].new_empty(need, dtype=_torch().uint8) if need else None
+    _check(fn, L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, None if ws is None else ws.data_ptr(), need))
+    return [_shape_outs(p[0], M, outs) for p, (_, _, outs, M) in zip(problems, packed)]
 
 
 def _shape_outs(x, M, outs):
+    if x.dim() == 2:
+        return outs
     lead = tuple(x.shape[:-1])
-    return [o.reshape(lead + (o.shape[-1],)) if o.shape[0] == M and o.is_contiguous() else o for o in outs]
+    return [o if o is None or o.shape[0] != M or not o.is_contiguous() else o.reshape(lead + (o.shape[-1],)) for o in outs]
 
 
 def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]], outs=None, flags: int = 0,
@@ -424,18 +442,8 @@ def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object
     """Several Dense ops that share the input, one launch (x_q / x_k / x_v).  `epilogues[i]` (optional) fuses the
     per-head RMSNorm / RoPE that follows projection i."""
     with _on(stream):
-        x2, M, K, n, W, B, Y, LDY, E, outs = _marshal_dense(x, weights, biases, outs, epilogues)
-        if M > _ROWS_MAX:
-            G = (_DenseGroup * 1)(_DenseGroup(M, K, x2.data_ptr(), x2.stride(0), _addr(W), n, _addr(B), _addr(Y), _addr(LDY),
-                                              _addr(E), None))
-            _enqueue_dense(G, flags, stream, x.device)
-        elif E is None:
-            st = lib().dt_dense_qx_f16(_stream_ptr(stream), M, K, x2.data_ptr(), x2.stride(0), W, n, B, Y, LDY, flags)
-            _check("dt_dense_qx_f16", st)
-        else:
-            st = lib().dt_dense_qx_heads_f16(_stream_ptr(stream), M, K, x2.data_ptr(), x2.stride(0), W, n, B, Y, LDY, E, flags)
-            _check("dt_dense_qx_heads_f16", st)
-        return _shape_outs(x, M, outs)
+        fn = "dt_dense_qx_f16" if epilogues is None else "dt_dense_qx_heads_f16"
+        return _enqueue_dense(fn, [(x, weights, biases, outs, epilogues, None)], flags, stream)[0]
 
 
 ACT_NONE, ACT_GELU_TANH, ACT_SWISH, ACT_GELU_ERF = 0, 1, 2, 3
@@ -455,14 +463,13 @@ class DensePost:
         self.scale, self.addend, self.multiplicand = scale, addend, multiplicand
 
 
-def _marshal_posts(posts, weights, M, Y, outs):
+def _pack_posts(posts, weights, M, Y, outs):
     """dt_dense_post array for the DensePost tails of one problem; clears Y / outs entries that only accumulate."""
     torch = _torch()
-    n = len(weights)
-    P = (_DensePost * n)()
+    vals = []
     for i, p in enumerate(posts):
         if p is None:
-            P[i] = _DensePost(ACT_NONE, None, None, 0, 1.0, None, 0, None, None, 0)
+            vals += (ACT_NONE, 0, 0, 0, 1.0, 0, 0, 0, 0, 0)
             continue
         N = weights[i].shape[0]
         if float(p.scale) == 0.0:
@@ -479,7 +486,7 @@ def _marshal_posts(posts, weights, M, Y, outs):
                 g16 = _f16_cuda(p.gate, "gate")
             if p.gate.numel() != N or not p.gate.is_contiguous():
                 raise ValueError("gate must hold one value per output feature")
-        rp, ldr = None, 0
+        rp, ldr = 0, 0
         if p.residual is not None:
             r = p.residual
             if not (isinstance(r, torch.Tensor) and r.is_cuda and r.dtype == torch.float32):
@@ -489,25 +496,25 @@ def _marshal_posts(posts, weights, M, Y, outs):
                 raise ValueError("residual must be an [M, N] view with contiguous rows")
             rp, ldr = r2.data_ptr(), r2.stride(0)
             if not p.keep_output:
-                Y[i] = None
+                Y[i] = 0
                 outs[i] = None
-        ap, lda = None, 0
+        ap, lda = 0, 0
         if p.addend is not None:
             a2 = _f16_cuda(p.addend, "addend")
             a2 = a2.reshape(-1, N) if a2.dim() != 2 else a2
             if a2.shape != (M, N) or a2.stride(1) != 1 or a2.data_ptr() != p.addend.data_ptr():
                 raise ValueError("addend must be an [M, N] view with contiguous rows")
             ap, lda = a2.data_ptr(), a2.stride(0)
-        mp, ldm = None, 0
+        mp, ldm = 0, 0
         if p.multiplicand is not None:
             m2 = _f16_cuda(p.multiplicand, "multiplicand")
             m2 = m2.reshape(-1, N) if m2.dim() != 2 else m2
             if m2.shape != (M, N) or m2.stride(1) != 1 or m2.data_ptr() != p.multiplicand.data_ptr():
                 raise ValueError("multiplicand must be an [M, N] view with contiguous rows")
             mp, ldm = m2.data_ptr(), m2.stride(0)
-        P[i] = _DensePost(p.activation, None if g16 is None else g16.data_ptr(), rp, ldr, float(p.scale), ap, lda,
-                          None if g32 is None else g32.data_ptr(), mp, ldm)
-    return P
+        vals += (p.activation, 0 if g16 is None else g16.data_ptr(), rp, ldr, float(p.scale), ap, lda,
+                 0 if g32 is None else g32.data_ptr(), mp, ldm)
+    return struct.pack("=" + _FMT_POST * len(weights), *vals)
 
 
 def dense_post(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]], posts: Sequence[Optional[DensePost]],
@@ -516,18 +523,7 @@ def dense_post(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]
     linear1 -> GELU and the gated residual additions of a transformer block).  Returns the fp16 outputs (None where
     a projection only accumulates into its residual)."""
     with _on(stream):
-        x2, M, K, n, W, B, Y, LDY, _, outs = _marshal_dense(x, weights, biases, outs, None)
-        P = _marshal_posts(posts, weights, M, Y, outs)
-        if M > _ROWS_MAX:
-            G = (_DenseGroup * 1)(_DenseGroup(M, K, x2.data_ptr(), x2.stride(0), _addr(W), n, _addr(B), _addr(Y), _addr(LDY),
-                                              None, _addr(P)))
-            _enqueue_dense(G, flags, stream, x.device)
-        else:
-            st = lib().dt_dense_qx_post_f16(_stream_ptr(stream), M, K, x2.data_ptr(), x2.stride(0), W, n, B, Y, LDY, P, flags)
-            _check("dt_dense_qx_post_f16", st)
-    lead = tuple(x.shape[:-1])
-    return [None if o is None else (o.reshape(lead + (o.shape[-1],)) if o.shape[0] == M and o.is_contiguous() else o)
-            for o in outs]
+        return _enqueue_dense("dt_dense_qx_post_f16", [(x, weights, biases, outs, None, posts)], flags, stream)[0]
 
 
 def dense_grouped(problems: Sequence[dict], flags: int = 0, stream=None):
@@ -535,24 +531,12 @@ def dense_grouped(problems: Sequence[dict], flags: int = 0, stream=None):
     problem is a dict with the arguments of dense_multi or dense_post: x, weights, biases, and optionally outs and
     either epilogues or posts.  Returns one list of outputs per problem (None where a projection only accumulates
     into its residual)."""
+    if not problems:
+        return []
     with _on(stream):
-        return _dense_grouped(problems, flags, stream)
-
-
-def _dense_grouped(problems, flags, stream):
-    keep = [_marshal_dense(p["x"], p["weights"], p["biases"], p.get("outs"), p.get("epilogues")) for p in problems]
-    G = (_DenseGroup * len(keep))()
-    posts = []
-    for i, (x2, M, K, n, W, B, Y, LDY, E, outs) in enumerate(keep):
-        P = None
-        if problems[i].get("posts") is not None:
-            P = _marshal_posts(problems[i]["posts"], problems[i]["weights"], M, Y, outs)
-        posts.append(P)
-        G[i] = _DenseGroup(M, K, x2.data_ptr(), x2.stride(0), _addr(W), n, _addr(B), _addr(Y), _addr(LDY), _addr(E), _addr(P))
-    # (the arrays stay alive in `keep` until the call returns)
-    if keep:
-        _enqueue_dense(G, flags, stream, problems[0]["x"].device)
-    return [[None if o is None else _shape_outs(p["x"], k[1], [o])[0] for o in k[9]] for p, k in zip(problems, keep)]
+        return _enqueue_dense("dt_dense_qx_grouped_f16",
+                              [(p["x"], p["weights"], p["biases"], p.get("outs"), p.get("epilogues"), p.get("posts")) for p in problems],
+                              flags, stream)
 
 
 class Dense:
