@@ -3,6 +3,8 @@
 // Dense of a DiT block.  HBM-bound: 4 bytes read and 2 written per element.
 // One wave per row; the row stays in registers between the mean, the variance
 // and the output pass, so memory is touched once.
+#include <type_traits>
+
 #include "dt_common.h"
 
 namespace dt {
@@ -37,15 +39,15 @@ __device__ __forceinline__ float mod_at(const void* p, int64_t c) {
   if constexpr (MOD == DT_MOD_F16) return (float)bits_to_half(static_cast<const uint16_t*>(p)[c]);
   else return static_cast<const float*>(p)[c];
 }
-// four consecutive values starting at element c (c % 4 == 0, vector aligned)
+// four consecutive values as they lie in memory, and widened
 template <int MOD>
-__device__ __forceinline__ void mod_at4(const void* p, int c, float (&o)[4]) {
+using Mod4 = std::conditional_t<MOD == DT_MOD_F16, uint2_t, float4_t>;
+template <int MOD>
+__device__ __forceinline__ void widen4(const Mod4<MOD>& t, float (&o)[4]) {
   if constexpr (MOD == DT_MOD_F16) {
-    const uint2_t t = *reinterpret_cast<const uint2_t*>(static_cast<const uint16_t*>(p) + c);
     o[0] = (float)bits_to_half((uint16_t)t[0]); o[1] = (float)bits_to_half((uint16_t)(t[0] >> 16));
     o[2] = (float)bits_to_half((uint16_t)t[1]); o[3] = (float)bits_to_half((uint16_t)(t[1] >> 16));
   } else {
-    const float4_t t = *reinterpret_cast<const float4_t*>(static_cast<const float*>(p) + c);
     o[0] = t[0]; o[1] = t[1]; o[2] = t[2]; o[3] = t[3];
   }
 }
@@ -62,9 +64,11 @@ struct AdaLnArgs {
 };
 
 // Rows of up to NV * 256 elements, C % 4 == 0, 16-byte aligned rows: lane l
-// holds the float4 at element 256 i + 4 l of every 256-element chunk i.
+// holds the float4 at element 256 i + 4 l of every 256-element chunk i.  A lane past the row's end reads the row's
+// first chunk and drops it: behind a test of their own, the chunks' loads (and the scale's and shift's, two chunks ahead
+// of their use here) were each waited for before the next went out, 20 us for however few rows (512 x 3072 beside 4096 x 3072: 20.7 -> 15.5 and 25.1 -> 18.9 us; 1376 x 3072: 21.4 -> 13.6).
 template <int NV, int MOD>
-__global__ void __launch_bounds__(256) adaln_rows_kernel(const AdaLnArgs a) {
+__global__ void __launch_bounds__(256, NV <= 20 ? 3 : 2) adaln_rows_kernel(const AdaLnArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= a.m) return;
@@ -72,42 +76,55 @@ __global__ void __launch_bounds__(256) adaln_rows_kernel(const AdaLnArgs a) {
   uint16_t* yr = a.y + row * a.ldy;
   const int c = (int)a.c;
   float4_t v[NV];
-  float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const int e = i * 256 + lane * 4;
-    v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-    if (e < c) v[i] = *reinterpret_cast<const float4_t*>(xr + e);
+    v[i] = *reinterpret_cast<const float4_t*>(xr + (e < c ? e : 0));
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    if (i * 256 + lane * 4 >= c) v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
     s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
   }
   const float mean = wave_sum64(s) / (float)c;
   float q = 0.f;
 #pragma unroll
-  for (int i = 0; i < NV; i++) {
-    const int e = i * 256 + lane * 4;
-    if (e < c) {
+  for (int i = 0; i < NV; i++)
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        v[i][j] -= mean;
-        q += v[i][j] * v[i][j];
-      }
+    for (int j = 0; j < 4; j++) {
+      v[i][j] = i * 256 + lane * 4 < c ? v[i][j] - mean : 0.f;
+      q += v[i][j] * v[i][j];
     }
-  }
   const float inv = 1.0f / sqrtf(wave_sum64(q) / (float)c + a.eps);
+  constexpr int G = 2;  // chunks whose scale and shift are fetched together, one group ahead
+  using Raw = Mod4<MOD>;
+  Raw sc[2][G], sh[2][G];
+  auto fetch = [&](int buf, int i0) {
+#pragma unroll
+    for (int k = 0; k < G; k++) {
+      const int e = (i0 + k) * 256 + lane * 4, ec = e < c ? e : 0;
+      constexpr int W = MOD == DT_MOD_F16 ? 2 : 4;
+      if (a.scale) sc[buf][k] = *reinterpret_cast<const Raw*>(static_cast<const char*>(a.scale) + ec * W);
+      if (a.shift) sh[buf][k] = *reinterpret_cast<const Raw*>(static_cast<const char*>(a.shift) + ec * W);
+    }
+  };
+  fetch(0, 0);
 #pragma unroll
   for (int i = 0; i < NV; i++) {
+    const int buf = i / G % 2, k = i % G;
+    if (k == 0 && i + G < NV) fetch(buf ^ 1, i + G);
     const int e = i * 256 + lane * 4;
-    if (e < c) {
-      uint16_t o[4];
-      float sc[4] = {0.f, 0.f, 0.f, 0.f}, sh[4] = {0.f, 0.f, 0.f, 0.f};
-      if (a.scale) mod_at4<MOD>(a.scale, e, sc);
-      if (a.shift) mod_at4<MOD>(a.shift, e, sh);
+    uint16_t o[4];
+    float fs[4] = {0.f, 0.f, 0.f, 0.f}, ft[4] = {0.f, 0.f, 0.f, 0.f};
+    if (a.scale) widen4<MOD>(sc[buf][k], fs);
+    if (a.shift) widen4<MOD>(sh[buf][k], ft);
 #pragma unroll
-      for (int j = 0; j < 4; j++)
-        o[j] = modulate<MOD>(v[i][j] * inv, a.scale != nullptr, sc[j], a.shift != nullptr, sh[j]);
+    for (int j = 0; j < 4; j++)
+      o[j] = modulate<MOD>(v[i][j] * inv, a.scale != nullptr, fs[j], a.shift != nullptr, ft[j]);
+    if (e < c)
       *reinterpret_cast<uint2_t*>(yr + e) =
           uint2_t{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
-    }
   }
 }
 

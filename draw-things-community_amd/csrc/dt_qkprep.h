@@ -23,6 +23,11 @@ struct QkPrepArgs {
 
 dt_status qk_prep_launch(hipStream_t s, const QkPrepArgs& a);
 
+// Several tensors of one head size in one launch, which also zeroes `n_zero` counters.  False -- nothing launched --
+// unless all of them take the per-head form with 16-byte accesses.
+constexpr int kQkPrepParts = 4;
+bool qk_prep_launch_parts(hipStream_t s, const QkPrepArgs* parts, int n, int32_t* zero, int n_zero, dt_status* status);
+
 #if defined(__HIPCC__)
 // The pass's arithmetic on one 16-byte chunk (8 elements = 4 complex pairs), shared with the attention kernel, which
 // applies it to the query fragments it holds in registers.

@@ -34,6 +34,7 @@ struct SdpaArgs {
   int32_t whole_tasks;  // tasks with a workgroup each
   int32_t cut_tasks;    // the ones behind them, each cut along its keys into
   int32_t shares;       // this many parts
+  int32_t counters_zeroed;  // by an earlier launch
   int32_t q_tiles, total_blocks;  // filled by the launcher
 };
 

@@ -714,9 +714,11 @@ static dt_status launch(hipStream_t s, SdpaArgs a) {
   dim3 block(512);
   if (a.partials) {
     // key-split launch: the counters start at zero
-    const int n = a.cut_tasks * kSdpaSplitNodes;
-    hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
-    if (const dt_status st = launch_status(); st != DT_OK) return st;
+    if (!a.counters_zeroed) {
+      const int n = a.cut_tasks * kSdpaSplitNodes;
+      hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
+      if (const dt_status st = launch_status(); st != DT_OK) return st;
+    }
     a.total_blocks = a.cut_tasks * a.shares;  // (of the cut tasks)
     dim3 grid((unsigned)(a.whole_tasks + a.total_blocks));
     if (oneseg) {

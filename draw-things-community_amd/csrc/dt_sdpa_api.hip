@@ -140,13 +140,15 @@ static dt_status sdpa_enqueue(dt_stream stream, int32_t B, int32_t Hq, int32_t H
   // Keys: RMSNorm -> cmul staged into one contiguous copy when asked for (the kernel moves K tiles from memory
   // straight into LDS, so there is no register stage to do it in); otherwise read in place.  V is read in place.
   const bool kprep = sh.kprep;
+  QkPrepArgs prep[kMaxSeg];
+  int n_prep = 0;
   if (kprep) {
     uint16_t* kw = reinterpret_cast<uint16_t*>(ws);
     ws += align256((size_t)B * Skv * Hk * D * 2);
     int64_t pos = 0;
     for (int i = 0; i < n_kvseg; i++) {
       if (k_seg[i].len == 0) continue;
-      QkPrepArgs p;
+      QkPrepArgs& p = prep[n_prep++];
       p.src = static_cast<const uint16_t*>(k_seg[i].view.ptr);
       p.src_sb = k_seg[i].view.stride_b;
       p.src_ss = k_seg[i].view.stride_s;
@@ -165,8 +167,6 @@ static dt_status sdpa_enqueue(dt_stream stream, int32_t B, int32_t Hq, int32_t H
       p.rot = rot_k;
       p.rot_pos0 = pos;
       p.post_scale = 1.0f;
-      dt_status st = qk_prep_launch(s, p);
-      if (st != DT_OK) return st;
       pos += k_seg[i].len;
     }
     a.n_kvseg = 1;
@@ -218,6 +218,19 @@ static dt_status sdpa_enqueue(dt_stream stream, int32_t B, int32_t Hq, int32_t H
     a.cut_tasks = plan.cut_tasks;
     a.shares = plan.shares;
   };
+  // The pass over K, in front of the kernel: all segments in one launch, which also zeroes the counters of cut tasks, if
+  // their layout allows it.
+  auto run_prep = [&]() -> dt_status {
+    if (n_prep == 0) return DT_OK;
+    dt_status st = DT_OK;
+    const int n_zero = a.partials ? a.cut_tasks * kSdpaSplitNodes : 0;
+    if (qk_prep_launch_parts(s, prep, n_prep, a.counters, n_zero, &st)) {
+      a.counters_zeroed = 1;
+      return st;
+    }
+    for (int i = 0; i < n_prep && st == DT_OK; i++) st = qk_prep_launch(s, prep[i]);
+    return st;
+  };
   if (Wo) {
     uint16_t* ow = reinterpret_cast<uint16_t*>(ws);
     ws += align256((size_t)B * Sq * Hq * D * 2);
@@ -226,7 +239,8 @@ static dt_status sdpa_enqueue(dt_stream stream, int32_t B, int32_t Hq, int32_t H
     a.o_sb = Sq * Hq * D;
     a.o_ss = (int64_t)Hq * D;
     a.o_sh = D;
-    dt_status st = sdpa_launch(s, a);
+    dt_status st = run_prep();
+    if (st == DT_OK) st = sdpa_launch(s, a);
     if (st != DT_OK) return st;
     // unify-heads projection on the staged attention output: one Dense over all batches when the output's
     // batches follow each other at the row stride, else batch by batch
@@ -252,6 +266,7 @@ static dt_status sdpa_enqueue(dt_stream stream, int32_t B, int32_t Hq, int32_t H
   a.o_sb = o.stride_b;
   a.o_ss = o.stride_s;
   a.o_sh = o.stride_h;
+  if (const dt_status st = run_prep(); st != DT_OK) return st;
   return sdpa_launch(s, a);
 }
 
