@@ -498,7 +498,11 @@ __device__ __forceinline__ void dense_epilogue(float16_t (&acc)[WN / 32][WM / 32
 // on different dies, whose L2 caches do not see each other's ordinary stores: slots are written and read with
 // device-scope accesses.  (The last to arrive adding up all slots in turn, its own among them, took 32 us for three
 // shares of 80 tiles; two that meet take 7.)
-template <int Q, int BM, int BN, int MODE, bool POST, bool SPLIT>
+//
+// NS: pair slots.  Two, or more of them with plain fp16 weights: every pair then has NS - 1 pairs of K-tiles to arrive,
+// which a workgroup that has a compute unit to itself needs (128 x 128 tiles with two and with four slots: 2016 x 5120 ->
+// 1280 57.8 / 48.7 us, 4608 x 3072 -> 64 31.7 / 23.9; two tiles on a compute unit hide the latency for each other).
+template <int Q, int BM, int BN, int MODE, bool POST, bool SPLIT, int NS>
 __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   constexpr int WN = BN / 2, WM = BM / 4;   // per-wave slice: WN features x WM tokens
   constexpr int TN = WN / 32, TM = WM / 32;
@@ -510,6 +514,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   constexpr int B_STAGE = BN * BK;
   constexpr int PROW = 2 * BK;                   // halfs per row of a pair slot
   static_assert(BM % 128 == 0 && BN % 128 == 0 && BN <= 256, "tile");
+  static_assert(NS == 2 || (MODE == kPlainF16 && NS > 2 && (NS - 1) * (AP + BP) < 16), "pair slots");
 
   // One LDS array, carved up by hand so that the epilogue can reuse all of it.  The palettes come first:
   // their addresses then fit an instruction offset.  X (and a plain fp16 W) lives in two pair slots, each
@@ -519,8 +524,8 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   constexpr int XS_BYTES = BM * PROW * 2;
   constexpr int WP_BYTES = MODE == kPlainF16 ? BN * PROW * 2 : 0;
   constexpr int BS_BYTES = MODE == kPlainF16 ? 0 : NST * B_STAGE * 2;
-  constexpr int OFF_XA = PAL_BYTES, OFF_XB = OFF_XA + XS_BYTES, OFF_WA = OFF_XB + XS_BYTES, OFF_WB = OFF_WA + WP_BYTES;
-  constexpr int OFF_BS = OFF_WB + WP_BYTES, LOOP_BYTES = OFF_BS + BS_BYTES;
+  constexpr int OFF_XA = PAL_BYTES, OFF_XB = OFF_XA + XS_BYTES, OFF_WA = OFF_XA + NS * XS_BYTES, OFF_WB = OFF_WA + WP_BYTES;
+  constexpr int OFF_BS = OFF_WA + NS * WP_BYTES, LOOP_BYTES = OFF_BS + BS_BYTES;
   constexpr int OUT_BYTES = BM * BN * 2;  // the fp16 output tile, parked here by the epilogue
   constexpr int LDS_BYTES = LOOP_BYTES > OUT_BYTES ? LOOP_BYTES : OUT_BYTES;
   __shared__ __attribute__((aligned(4096))) unsigned char smem[LDS_BYTES];
@@ -845,6 +850,10 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 
   // ---- prologue: pair 0 in slot A, weights of tiles 0 and 1 in the ring --------
   issue_pair(XsA, WpA, SPLIT ? t_lo / 2 : 0);
+  if constexpr (NS > 2) {
+#pragma unroll
+    for (int i = 1; i < NS; i++) issue_pair(XsA + i * (XS_BYTES / 2), WpA + i * (WP_BYTES / 2), (SPLIT ? t_lo / 2 : 0) + i);
+  }
   issue_idx(WS[0]);  // tile 0 (of this workgroup's)
   issue_idx(WS[1]);  // tile 1
   __syncthreads();   // palettes visible
@@ -860,9 +869,9 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   }
   stage_to_lds(WS[1], 1);
   issue_idx(WS[1]);  // tile 3
-  __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
+  __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0 | (NS > 2 ? (NS - 1) * (AP + BP) : 0));  // the first pair
   __syncthreads();
-  if constexpr (MODE == kPlainF16) issue_pair(XsB, WpB, (SPLIT ? t_lo / 2 : 0) + 1);  // (the loop issues pair q + 2 from the middle of pair q)
+  if constexpr (MODE == kPlainF16 && NS == 2) issue_pair(XsB, WpB, (SPLIT ? t_lo / 2 : 0) + 1);  // (the loop issues pair q + NS from the middle of pair q)
 #pragma unroll
   for (int i = 0; i < TN; i++) read_w(0, i, WpA, 0, 0, 0);
 #pragma unroll
@@ -963,7 +972,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       }
       if (par) {
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
+        __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0 | (NS - 2) * (AP + BP));  // the next pair
         __syncthreads();
       }
 #pragma unroll
@@ -974,10 +983,10 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
         for (int r = m * RPS; r < (m + 1) * RPS; r++)
           if (r < NF) read1(r);
         if (par) {
-          // this iteration's slot is free from the barrier on: the pair after next goes into it
+          // this iteration's slot is free from the barrier on: pair q + NS goes into it
 #pragma unroll
           for (int q = m * PPS; q < (m + 1) * PPS; q++)
-            if (q < AP + BP) issue_pair_part(xs, wp, (t >> 1) + 2, q);
+            if (q < AP + BP) issue_pair_part(xs, wp, (t >> 1) + NS, q);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1012,15 +1021,28 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   };
 
   int t = SPLIT ? t_lo : 0;
-  for (; t + 3 < nk; t += 4) {
-    iteration(t, 0, XsA, WpA, XsB, WpB);
-    iteration(t + 1, 1, XsA, WpA, XsB, WpB);
-    iteration(t + 2, 0, XsB, WpB, XsA, WpA);
-    iteration(t + 3, 1, XsB, WpB, XsA, WpA);
-  }
-  if (t < nk) {  // nk is even: two iterations left
-    iteration(t, 0, XsA, WpA, XsB, WpB);
-    iteration(t + 1, 1, XsA, WpA, XsB, WpB);
+  if constexpr (NS > 2) {
+    for (int slot = 0; t < nk; t += 2) {
+      const int next = slot + 1 < NS ? slot + 1 : 0;
+      half_t* const xs = XsA + slot * (XS_BYTES / 2);
+      half_t* const wp = WpA + slot * (WP_BYTES / 2);
+      half_t* const xn = XsA + next * (XS_BYTES / 2);
+      half_t* const wn_ = WpA + next * (WP_BYTES / 2);
+      iteration(t, 0, xs, wp, xn, wn_);
+      iteration(t + 1, 1, xs, wp, xn, wn_);
+      slot = next;
+    }
+  } else {
+    for (; t + 3 < nk; t += 4) {
+      iteration(t, 0, XsA, WpA, XsB, WpB);
+      iteration(t + 1, 1, XsA, WpA, XsB, WpB);
+      iteration(t + 2, 0, XsB, WpB, XsA, WpA);
+      iteration(t + 3, 1, XsB, WpB, XsA, WpA);
+    }
+    if (t < nk) {  // nk is even: two iterations left
+      iteration(t, 0, XsA, WpA, XsB, WpB);
+      iteration(t + 1, 1, XsA, WpA, XsB, WpB);
+    }
   }
 
   if constexpr (MODE == kPlainF16) {

@@ -14,24 +14,33 @@ static dt_status launch_tiled(hipStream_t s, const DenseArgs& a, int mode) {
   const int64_t rest = SPLIT ? a.total_tiles - a.whole_tiles : 0;
   dim3 grid((unsigned)(a.total_tiles - rest + rest * a.split)), block(512);
   if constexpr (Q == 16) {  // plain fp16 weight
-    hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT>), grid, block, 0, s, a);
+    // pair slots: as many as fit where a workgroup has a compute unit to itself (up to 256 tiles of 128 x 128; beyond,
+    // two slots let two of them share one)
+    if constexpr (BM == 128 && BN == 256) {
+      hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 3>), grid, block, 0, s, a);
+    } else if constexpr (BM == 128 && BN == 128) {
+      if (grid.x <= 256) hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 4>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 2>), grid, block, 0, s, a);
+    } else {
+      hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 2>), grid, block, 0, s, a);
+    }
     return launch_status();
   } else {
     switch (mode) {
       case kPalShared:
         if constexpr (BM == 256 && BN == 128) return DT_NO_KERNEL;
-        else hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalShared, POST, SPLIT>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalShared, POST, SPLIT, 2>), grid, block, 0, s, a);
         break;
       case kPalRow:
         if constexpr ((BN << (Q + 1)) <= pal_lds_bytes(BM, BN, kPalRow)) {
-          hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalRow, POST, SPLIT>), grid, block, 0, s, a);
+          hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalRow, POST, SPLIT, 2>), grid, block, 0, s, a);
           break;
         } else {
           return DT_NO_KERNEL;  // choose_pal_mode never picks per-row palettes that do not fit
         }
       default:
         if constexpr (BM == 256 && BN == 128) return DT_NO_KERNEL;
-        else hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalGlobal, POST, SPLIT>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((dense_qx_kernel<Q, BM, BN, kPalGlobal, POST, SPLIT, 2>), grid, block, 0, s, a);
     }
     return launch_status();
   }

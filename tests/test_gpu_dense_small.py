@@ -151,6 +151,21 @@ def test_dense_cut_along_k(dthip, oracle, monkeypatch, M, N, K, q, nib):
         assert bool(((fused[1].float() - turned).abs() <= mag * 2.0 ** -9 + 2.0 ** -24).all())
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 704])
+def test_dense_plain_pair_slots(dthip, oracle, K):
+    """Plain fp16 weights with fewer K-tile pairs than the 128 x 128 tile's four slots, as many, and more; the 128 x 256
+    tile's three, which a fused head epilogue beside it asks for; and the two that launches of many tiles keep."""
+    rng = np.random.default_rng(K)
+    print("dense plain pair slots", K, flush=True)
+    for M, N in ((130, 200), (300, 256), (2050, 2100)):
+        X = rng.standard_normal((M, K)).astype(np.float16)
+        (w, W), (head, _) = make(dthip, oracle, rng, N, K, 16, 0), make(dthip, oracle, rng, 128, K, 16, 0)
+        check(dthip.dense_multi(dev(X), [w], [None])[0].cpu().numpy(), X, W)
+        if M < 1024:
+            epi = dthip.HeadEpilogue(dev(np.ones(128, np.float16)), None, 0)
+            check(dthip.dense_multi(dev(X), [head, w], [None, None], epilogues=[epi, None])[1].cpu().numpy(), X, W)
+
+
 def _groups(dthip, x, w, out):
     """One problem as the C entry points take it, and what keeps it alive."""
     import ctypes
