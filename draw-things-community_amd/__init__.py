@@ -369,6 +369,14 @@ class HeadEpilogue:
     head_dim: int = 128
 
 
+def _per_weight(entries, n, what):
+    """One entry per weight: a shorter list leaves the rest None."""
+    entries = list(entries)
+    if len(entries) > n:
+        raise IndexError(f"{len(entries)} {what} for {n} weights")
+    return entries + [None] * (n - len(entries))
+
+
 def _pack_epilogues(epilogues, M):
     vals = []
     for e in epilogues:
@@ -402,14 +410,14 @@ def _marshal_dense(x, weights, biases, outs, epilogues, posts):
             raise ValueError(f"weight {w.shape} does not match input width {K}")
         vals += (w.data.data_ptr(), w.qbits, w.nib, w.count)
     outs = [x.new_empty((M, w.shape[0])) for w in weights] if outs is None else list(outs)
-    ptrs = [0 if b is None else _f16_cuda(b, "bias").data_ptr() for b in biases]
-    if len(ptrs) != n or len(outs) != n:
-        raise ValueError("weights, biases and outs must be of one length")
+    ptrs = [0 if b is None else _f16_cuda(b, "bias").data_ptr() for b in _per_weight(biases, n, "biases")]
+    if len(outs) != n:
+        raise ValueError("weights and outs must be of one length")
     ys = [o.data_ptr() for o in outs]
     strides = [o.stride(0) for o in outs]
     # (a problem with both is for the library to refuse)
-    epi = b"" if epilogues is None else _pack_epilogues(epilogues, M)
-    post = b"" if posts is None else _pack_posts(posts, weights, M, ys, outs)
+    epi = b"" if epilogues is None else _pack_epilogues(_per_weight(epilogues, n, "epilogues"), M)
+    post = b"" if posts is None else _pack_posts(_per_weight(posts, n, "posts"), weights, M, ys, outs)
     arrays = ctypes.create_string_buffer(struct.pack(f"={_FMT_WEIGHT * n}{2 * n}Q{n}q", *vals, *ptrs, *ys, *strides) + epi + post)
     base = ctypes.addressof(arrays)
     tails = base + 48 * n

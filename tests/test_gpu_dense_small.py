@@ -234,3 +234,28 @@ def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     sums = 2 * K * 2.0 ** -24 * x.float().norm(dim=1)[:, None] * w.dequantize().float().norm(dim=1)[None]
     assert bool(((cut - whole).abs() <= whole.abs() * 2.0 ** -10 + sums + 2.0 ** -24).all())
     assert not torch.equal(cut, whole)
+
+
+def test_lists_shorter_than_the_weights(dthip, oracle):
+    """Biases, head epilogues and tails that are not given stand for none; more of them than weights are refused."""
+    import torch
+
+    rng = np.random.default_rng(23)
+    M, K, N = 70, 128, 256
+    x = dev(rng.standard_normal((M, K)).astype(np.float16))
+    ws = [make(dthip, oracle, rng, N, K, 6, 4096)[0] for _ in range(3)]
+    b = dev((rng.standard_normal(N) * 0.1).astype(np.float16))
+    gamma = dev((1 + 0.1 * rng.standard_normal(128)).astype(np.float16))
+    e, p = dthip.HeadEpilogue(gamma), dthip.DensePost(dthip.ACT_GELU_TANH)
+    for short, full in [
+        (dthip.dense_multi(x, ws, [b]), dthip.dense_multi(x, ws, [b, None, None])),
+        (dthip.dense_multi(x, ws, [b, b], epilogues=[e]), dthip.dense_multi(x, ws, [b, b, None], epilogues=[e, None, None])),
+        (dthip.dense_post(x, ws, [], [p]), dthip.dense_post(x, ws, [None] * 3, [p, None, None])),
+    ]:
+        assert len(short) == 3 and all(torch.equal(s, f) for s, f in zip(short, full))
+    with pytest.raises(IndexError):
+        dthip.dense_multi(x, ws[:1], [b, b])
+    with pytest.raises(IndexError):
+        dthip.dense_multi(x, ws[:1], [b], epilogues=[e, e])
+    with pytest.raises(IndexError):
+        dthip.dense_post(x, ws[:1], [b], [p, p])
