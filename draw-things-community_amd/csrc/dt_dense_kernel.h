@@ -658,20 +658,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     }
   }
 
-  // ---- palettes -> LDS --------------------------------------------------
-  if constexpr (MODE == kPalShared) {
-    int last_row = n0 + BN - 1;
-    if (last_row >= w.n) last_row = w.n - 1;
-    int64_t last_block = ((int64_t)last_row * K + (K - 1)) / a.nib;
-    int n_pal = (int)(last_block - pal_first_block + 1);
-    const int per_pal = 1 << (Q - 1);  // dwords per palette
-    for (int i = tid; i < n_pal * per_pal; i += 512) {
-      int p = i / per_pal, e = i - p * per_pal;
-      const uint32_t* src =
-          reinterpret_cast<const uint32_t*>(w.data + palette_offset(lay, pal_first_block + p));
-      reinterpret_cast<uint32_t*>(Pal)[i] = src[e];
-    }
-  }
+  // ---- per-row palettes ---------------------------------------------------
   // kPalRow: Pal is a table [128-row group][entry][row % 64][row / 64 % 2] of
   // fp16: rows r and r + 64 share a dword, so the 64 lanes of a wave (64
   // consecutive rows, one entry each) hit 64 different banks whatever entries
@@ -700,7 +687,6 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   };
   int next_pal_tile = a.pal_step;  // next K-tile at which some row may change block
   if constexpr (SPLIT) next_pal_tile = (t_lo / a.pal_step + 1) * a.pal_step;
-  if constexpr (MODE == kPalRow) fill_pal_column(((int64_t)gn_row * K + (SPLIT ? t_lo * BK : 0)) / a.nib);
 
   // ---- staging --------------------------------------------------------------
   struct IdxSet {
@@ -708,7 +694,14 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     uint32_t poff;
     int32_t slot;
   };
-  IdxSet WS[2];  // tile T travels in WS[T % 2]
+  // Tile T travels in WS[T % 2].  MID: a 128 x 128 tile has a quarter of the MFMA work to hide latency behind, and waiting
+  // for X in even iterations and for the indices in odd ones cost it two latencies per pair of K-tiles.  It asks for
+  // all that a pair needs in the middle of an odd iteration and waits for it in the middle of the next one, so that tile
+  // T travels in WS[(T - 2) % 4] (us before / after: 8192 x 1280 -> 320 q6p 35.4 / 32.1, 2016 x 1280 -> 1280 q8p 34.9 /
+  // 33.0, q6p 29.3 / 28.2, 8192 x 320 -> 1280 q6p 27.1 / 26.4).  The big tiles keep the shorter loop.
+  constexpr bool MID = HAS_PAL && BM == 128 && BN == 128;
+  constexpr int NW = MID ? 4 : 2;
+  IdxSet WS[NW];
   const int last_pair = nk / 2 - 1;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 
@@ -854,11 +847,32 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 #pragma unroll
     for (int i = 1; i < NS; i++) issue_pair(XsA + i * (XS_BYTES / 2), WpA + i * (WP_BYTES / 2), (SPLIT ? t_lo / 2 : 0) + i);
   }
-  issue_idx(WS[0]);  // tile 0 (of this workgroup's)
-  issue_idx(WS[1]);  // tile 1
+  IdxSet& tile0 = WS[NW - 2];
+  IdxSet& tile1 = WS[NW - 1];
+  issue_idx(tile0);  // tile 0 (of this workgroup's)
+  issue_idx(tile1);
+  if constexpr (MID) {
+    issue_idx(WS[0]);  // tile 2
+    issue_idx(WS[1]);  // tile 3
+  }
+  // the palettes are asked for last: what they wait for is on its way with them
+  if constexpr (MODE == kPalShared) {
+    int last_row = n0 + BN - 1;
+    if (last_row >= w.n) last_row = w.n - 1;
+    int64_t last_block = ((int64_t)last_row * K + (K - 1)) / a.nib;
+    int n_pal = (int)(last_block - pal_first_block + 1);
+    const int per_pal = 1 << (Q - 1);  // dwords per palette
+    for (int i = tid; i < n_pal * per_pal; i += 512) {
+      int p = i / per_pal, e = i - p * per_pal;
+      const uint32_t* src =
+          reinterpret_cast<const uint32_t*>(w.data + palette_offset(lay, pal_first_block + p));
+      reinterpret_cast<uint32_t*>(Pal)[i] = src[e];
+    }
+  }
+  if constexpr (MODE == kPalRow) fill_pal_column(((int64_t)gn_row * K + (SPLIT ? t_lo * BK : 0)) / a.nib);
   __syncthreads();   // palettes visible
-  stage_to_lds(WS[0], 0);
-  issue_idx(WS[0]);  // tile 2
+  stage_to_lds(tile0, 0);
+  if constexpr (!MID) issue_idx(WS[0]);  // tile 2
   if constexpr (MODE == kPalRow) {
     if (next_pal_tile == (SPLIT ? t_lo : 0) + 1) {  // tile 1 may already start a new palette block
       __syncthreads();
@@ -867,11 +881,15 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       __syncthreads();
     }
   }
-  stage_to_lds(WS[1], 1);
-  issue_idx(WS[1]);  // tile 3
+  stage_to_lds(tile1, 1);
+  if constexpr (!MID) issue_idx(WS[1]);  // tile 3
   __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0 | (NS > 2 ? (NS - 1) * (AP + BP) : 0));  // the first pair
   __syncthreads();
-  if constexpr (MODE == kPlainF16 && NS == 2) issue_pair(XsB, WpB, (SPLIT ? t_lo / 2 : 0) + 1);  // (the loop issues pair q + NS from the middle of pair q)
+  if constexpr ((MODE == kPlainF16 || MID) && NS == 2) issue_pair(XsB, WpB, (SPLIT ? t_lo / 2 : 0) + 1);  // (the loop issues pair q + NS from the middle of pair q)
+  if constexpr (MID) {
+    issue_idx(WS[2]);  // tile 4
+    issue_idx(WS[3]);  // tile 5
+  }
 #pragma unroll
   for (int i = 0; i < TN; i++) read_w(0, i, WpA, 0, 0, 0);
 #pragma unroll
@@ -884,6 +902,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // the odd iteration reads one k-step ahead into that pair.  Index registers
   // are refilled in odd iterations only, so the even iteration's wait covers
   // nothing that was issued just before it.
+  // (MID: the closing barriers wait for the LDS only; pair and indices are waited for in the middle of odd iterations.)
   //
   // A wave issues in order, and an LDS instruction occupies it for tens of
   // clocks, so the iteration is written as 16 slots of one MFMA followed by
@@ -891,7 +910,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // the palette lookups and the weight writes all issue while an MFMA of the
   // same wave (or of the wave it shares the SIMD with) is executing.
   int s_cur = 0, s_nxt = 1, s_fill = 2;
-  auto iteration = [&](int t, int par, half_t* xs, half_t* wp, half_t* xs_other, half_t* wp_other) {
+  auto iteration = [&](int t, int par, half_t* xs, half_t* wp, half_t* xs_other, half_t* wp_other, int set = 0) {
     if constexpr (MODE == kPalRow) {
       if (t + 2 == next_pal_tile) {
         // lookups of tile t+1 finished before the last barrier
@@ -900,12 +919,12 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
         __syncthreads();
       }
     }
-    IdxSet& R = WS[par];
+    IdxSet& R = WS[MID ? 2 * set + par : par];
     // the wait for the indices comes here, before the transfer goes out: vector
     // memory loads return in order, so a wait with the transfer outstanding
     // would last until it lands
     touch(R);
-    if (par) issue_idx(WS[0]);  // tile t+3
+    if (par && !MID) issue_idx(WS[0]);  // tile t+3
     const half_t* xs_n = par == 0 ? xs : xs_other;  // fragments of tile t+1, k-step 0
     const half_t* wp_n = par == 0 ? wp : wp_other;
     constexpr int NM = TN * TM;  // MFMAs per k-step = slots per phase
@@ -914,15 +933,15 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     // Phase 0 (k-step 0): the fragments of k-step 1, one every third place;
     // between them the parts of the transfer (even iterations), the unpacking,
     // the refill of the index registers (odd iterations), the first 8 lookups.
-    const int nd = par == 0 ? AP + BP : 0;
-    const int ns0 = nd + (packed ? 4 + par + 8 : 0);
+    const int nd = par == 0 && !MID ? AP + BP : 0;
+    const int ns0 = nd + (packed ? 4 + (MID ? 0 : par) + 8 : 0);
     auto stage0 = [&](int s) {
       if (s < nd) { issue_pair_part(xs_other, wp_other, (t >> 1) + 1, s); return; }
       s -= nd;
       if (!packed) return;
       if (s < 4) { unpack_piece(R, s); return; }
       s -= 4;
-      if (par) {
+      if (par && !MID) {
         if (s == 0) { issue_idx(WS[1]); return; }  // tile t+4
         s -= 1;
       }
@@ -931,9 +950,16 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     // Phase 1 (k-step 1): the next tile's first fragments (every k-step 0
     // MFMA has been issued, so their registers are free), the other lookups,
     // the two weight writes.
-    const int ns1 = packed ? 10 : 0;
+    const int nd1 = MID && par ? AP + 2 : 0;
+    const int ns1 = packed ? nd1 + 10 : 0;
     auto stage1 = [&](int s) {
       if (!packed) return;
+      if (s < nd1) {
+        if (s < AP) issue_pair_part(xs, wp, (t >> 1) + NS, s);
+        else issue_idx(WS[MID ? 2 * set + s - AP : 0]);  // tiles t+5, t+6
+        return;
+      }
+      s -= nd1;
       if (s < 8) lookup(8 + s);
       else if (s < 10) write_weights(s_fill, s - 8);
     };
@@ -1001,6 +1027,12 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 #pragma unroll
       for (int k = m * n0 / NM; k < (m + 1) * n0 / NM; k++) place(k, ns0, read0, stage0);
     }
+    if (MID && par) {
+      // the next pair and the indices of the one after it; this pair's slot is free from here on
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
+      __syncthreads();
+    }
 #pragma unroll
     for (int m = 0; m < NM; m++) {
       __builtin_amdgcn_sched_barrier(0);
@@ -1009,7 +1041,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       for (int k = m * n1 / NM; k < (m + 1) * n1 / NM; k++) place(k, ns1, read1, stage1);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (par == 0)
+    if (par == 0 && !MID)
       __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
     else
       __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
@@ -1036,8 +1068,8 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     for (; t + 3 < nk; t += 4) {
       iteration(t, 0, XsA, WpA, XsB, WpB);
       iteration(t + 1, 1, XsA, WpA, XsB, WpB);
-      iteration(t + 2, 0, XsB, WpB, XsA, WpA);
-      iteration(t + 3, 1, XsB, WpB, XsA, WpA);
+      iteration(t + 2, 0, XsB, WpB, XsA, WpA, 1);
+      iteration(t + 3, 1, XsB, WpB, XsA, WpA, 1);
     }
     if (t < nk) {  // nk is even: two iterations left
       iteration(t, 0, XsA, WpA, XsB, WpB);
@@ -1045,7 +1077,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     }
   }
 
-  if constexpr (MODE == kPlainF16) {
+  if constexpr (MODE == kPlainF16 || MID) {
     // the loop's last barrier lies before the last reads (and every transfer was waited for ahead of it)
     __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
     __syncthreads();

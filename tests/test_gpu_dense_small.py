@@ -166,6 +166,18 @@ def test_dense_plain_pair_slots(dthip, oracle, K):
             check(dthip.dense_multi(dev(X), [head, w], [None, None], epilogues=[epi, None])[1].cpu().numpy(), X, W)
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 704])
+@pytest.mark.parametrize("q,nib", [(4, 512), (5, 1024), (6, 4096), (7, 8192), (8, 16384), (8, 512)])
+def test_dense_small_tile_pairs(dthip, oracle, K, q, nib):
+    """The 128 x 128 tile's K-tile pairs, from one to several rounds of its index registers, palettes per row and shared,
+    one workgroup per compute unit and two."""
+    rng = np.random.default_rng(K + q + nib)
+    for M, N in ((131, 260), (1300, 4096)) if K in (64, 320) else ((131, 260),):
+        X = rng.standard_normal((M, K)).astype(np.float16)
+        w, W = make(dthip, oracle, rng, N, K, q, nib)
+        check(dthip.dense_multi(dev(X), [w], [None])[0].cpu().numpy(), X, W)
+
+
 def _groups(dthip, x, w, out):
     """One problem as the C entry points take it, and what keeps it alive."""
     import ctypes
