@@ -52,7 +52,17 @@ static int choose_pal_mode(int qbits, int nib, int64_t K, int BM, int BN) {
   const bool shared = !(BM == 256 && BN == 128) && shared_count * pal_bytes <= pal_lds_bytes(BM, BN, kPalShared);
   // a per-row table has no bank conflicts, but 128- and 256-entry palettes make one of 32 or 64 KB: the 128 x 128 tile
   // takes it only where the palettes of its blocks would not fit the 24 KB that let two workgroups share a compute unit
-  if (row && !(shared && BM == 128 && BN == 128 && qbits >= 7)) return kPalRow;
+  const bool small = BM == 128 && BN == 128;
+  if (shared && small && qbits >= 7) return kPalShared;
+  // And where some row may enter a new block at every second K-tile (K an odd multiple of 64), that check, its barrier
+  // and the 64 entries to rewrite cost more than conflicts do (us, per row / shared: 8192 x 320 -> 960 19.1 / 17.7,
+  // 4608 x 960 -> 3072 48.0 / 42.8, 2048 x 1344 -> 4096 51.5 / 43.8, on 128 x 128 tiles 2016 x 1600 -> 1280 42.6 / 35.8);
+  // at every fourth they are even on the small tile (4096 x 640 -> 640 17.9 / 17.5), at every eighth the table is
+  // ahead (2016 x 1280 -> 1280 28.2 / 29.8).  Palettes of 16 and 32 entries are rewritten fast enough (4096 x 320 ->
+  // 1280: q5p 16.5 / 16.4, q4p 16.2 / 16.4).
+  const int64_t step = std::gcd(K, (int64_t)nib) / BK;
+  if (shared && qbits == 6 && (small ? step <= 4 : BN == 256 && step <= 2)) return kPalShared;
+  if (row) return kPalRow;
   if (shared) return kPalShared;
   return kPalGlobal;
 }

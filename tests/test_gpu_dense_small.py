@@ -178,6 +178,24 @@ def test_dense_small_tile_pairs(dthip, oracle, K, q, nib):
         check(dthip.dense_multi(dev(X), [w], [None])[0].cpu().numpy(), X, W)
 
 
+@pytest.mark.parametrize("M,N,K,nib", [
+    (200, 300, 64, 4096), (200, 300, 1600, 4096),  # 128 x 128 tiles, a block's end at every second K-tile
+    (200, 300, 640, 4096), (200, 300, 768, 4096),  # at every fourth: shared palettes still; every eighth: per row
+    (200, 300, 6080, 4096), (200, 300, 6208, 4096),  # as many palettes as 24 KB hold, and more
+    (70, 300, 320, 64),                            # small blocks
+    (8100, 1600, 192, 4096), (6200, 2000, 4032, 4096), (6200, 2000, 4160, 4096),  # 256 x 256 tiles: up to 32 KB, and beyond
+])
+def test_dense_shared_palettes_of_64(dthip, oracle, M, N, K, nib):
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    w, W = make(dthip, oracle, rng, N, K, 6, nib)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    got = dthip.dense_multi(dev(X), [w], [None])[0]
+    rows = np.unique(np.concatenate([np.arange(min(M, 130)), np.arange(M - 130, M).clip(0)]))
+    check(got[torch.from_numpy(rows).cuda()].cpu().numpy(), X[rows], W)
+
+
 def _groups(dthip, x, w, out):
     """One problem as the C entry points take it, and what keeps it alive."""
     import ctypes
