@@ -311,7 +311,11 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   const TilePlan t256 = shape(kTile256x256, 256, 256), tnarrow = shape(kTile128x256, 128, 256);
   const TilePlan ttall = shape(kTile256x128, 256, 128), tsmall = shape(kTile128x128, 128, 128);
   const bool tall_ok = (w0.qbits == 7 || w0.qbits == 8) && choose_pal_mode(w0.qbits, w0.nib, K, 256, 128) == kPalRow;
-  const bool big = (((m_max >= 1024) && (n_max >= 256) && t256.tiles >= kFillTiles) && pal_fits_big) || wide;
+  // (plain fp16 weights with one or two pairs of K-tiles -- a LoRA's up projection -- are all prologue and output, which two
+  // small tiles on a compute unit hide for each other: us, 256 x 256 / 128 x 128, 4608 x 64 -> 3072 with an addend 22.9 /
+  // 21.0, -> 12288 81.5 / 66.7, 1900 x 128 -> 9216 25.3 / 19.3; 8192 x 64 -> 2048 14.9 / 14.7)
+  const bool brief = w0.qbits == 16 && K <= 128;
+  const bool big = (((m_max >= 1024) && (n_max >= 256) && t256.tiles >= kFillTiles) && pal_fits_big && !brief) || wide;
   TilePlan base = big ? (m_max < 1024 ? tnarrow : t256) : (!pal_fits_big && tall_ok && m_max >= 1024 && n_max >= 128 && t256.tiles * 2 >= kFillTiles) ? ttall : tsmall;
   const auto pal_mode = [&](const TilePlan& p) { return choose_pal_mode(w0.qbits, w0.qbits == 16 ? 32 : w0.nib, K, p.BM, p.BN); };
   // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate, whose error

@@ -166,6 +166,15 @@ def test_dense_plain_pair_slots(dthip, oracle, K):
             check(dthip.dense_multi(dev(X), [head, w], [None, None], epilogues=[epi, None])[1].cpu().numpy(), X, W)
 
 
+@pytest.mark.parametrize("K", [64, 128, 192])
+def test_dense_plain_brief(dthip, oracle, K):
+    """Many tiles of one or two K-tile pairs stay 128 x 128; with three they are 256 x 256."""
+    rng = np.random.default_rng(K)
+    X = rng.standard_normal((4099, K)).astype(np.float16)
+    w, W = make(dthip, oracle, rng, 3080, K, 16, 0)
+    check(dthip.dense_multi(dev(X), [w], [None])[0].cpu().numpy(), X, W)
+
+
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 704])
 @pytest.mark.parametrize("q,nib", [(4, 512), (5, 1024), (6, 4096), (7, 8192), (8, 16384), (8, 512)])
 def test_dense_small_tile_pairs(dthip, oracle, K, q, nib):
