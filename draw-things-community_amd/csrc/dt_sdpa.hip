@@ -426,7 +426,10 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
 #pragma unroll
         for (int v = (kb == 0 ? 1 : 0); v < 16; v++) mx = fmaxf(mx, sacc[kb][v]);
       mx = max32(mx);
-      const float m_new = fmaxf(m_ref, mx);
+      // (Finite even where every score so far is -inf -- keys masked through the dot product itself: against a
+      // reference of -inf the probabilities would be NaN, in a part of the keys that counts for nothing.  No finite
+      // score lies below: |q k| <= 128 * 65504^2 = 5.5e11, and PREMUL's own scale has the whole range of fp32.)
+      const float m_new = fmaxf(fmaxf(m_ref, mx), PREMUL ? -3e38f : -1e12f);
       const float alpha = fast_exp2((m_ref - m_new) * c);  // first tile: exp2(-inf) = 0
       m_ref = m_new;
       l_run *= alpha;

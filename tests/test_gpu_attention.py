@@ -728,6 +728,35 @@ def test_sdpa_key_split_last_round(dthip, oracle, torch_cuda, monkeypatch, D, Sk
     assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
 
 
+@pytest.mark.parametrize("D,n_seg,sign", [(128, 1, 1), (128, 2, 1), (64, 1, 1), (40, 2, 1), (128, 1, -1)])
+@pytest.mark.parametrize("masked", ["tail", "head"])
+def test_sdpa_key_split_masked_part(dthip, oracle, torch_cuda, monkeypatch, D, n_seg, sign, masked):
+    """Keys masked through the dot product -- one component of -inf, so that their scores are -inf -- fill whole parts of
+    the cut tasks (264 tasks, 8 of them in 8 parts of 4 key tiles): they weigh nothing, as if they were not there."""
+    torch = torch_cuda
+    rng = np.random.default_rng(D + n_seg)
+    B, H, S, live = 1, 33, 2000, slice(0, 700) if masked == "tail" else slice(1300, 2000)
+    q, k, v = rand_qkv(rng, B, S, S, H, H, D)
+    scale = sign / np.sqrt(D)
+    q[..., 0], k[..., 0] = sign, -np.inf
+    k[:, live, :, 0] = 0
+    parts = lambda t: [to_dev(torch, np.ascontiguousarray(t[:, a:b])) for a, b in ([(0, S)] if n_seg == 1 else [(0, 77), (77, S)])]
+    args = ([to_dev(torch, q)], parts(k), parts(v), scale)
+    print("sdpa key split, masked part", D, n_seg, sign, masked, flush=True)
+    monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
+    assert dthip.lib().dt_sdpa_workspace_bytes(B, H, H, D, S, S, 0, 0) > 0  # cut by its own estimate
+    got = dthip.sdpa_segments(*args)
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "never")
+    plain = dthip.sdpa_segments(*args)
+    rows = [0, 777, S - 1]
+    want = oracle.C.sdpa(np.ascontiguousarray(q[:, rows, 31:]), np.ascontiguousarray(k[:, live, 31:]),
+                         np.ascontiguousarray(v[:, live, 31:]), scale)
+    for out in (got, plain):
+        mx, rr = oracle.err_stats(out[:, rows, 31:].cpu().numpy(), want)
+        assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+    assert float((got.float() - plain.float()).abs().max()) <= 2e-3
+
+
 def test_sdpa_key_split_joint_segments_fused_prep(dthip, oracle, torch_cuda, monkeypatch):
     """Key-split with text || image segments, fused per-head RMSNorm + RoPE staging and the static-scratch entry
     point: all three forms agree bit for bit with each other and with the oracle within the attention bar."""
