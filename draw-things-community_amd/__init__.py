@@ -421,7 +421,8 @@ def _marshal_dense(x, weights, biases, outs, epilogues, posts):
     arrays = ctypes.create_string_buffer(struct.pack(f"={_FMT_WEIGHT * n}{2 * n}Q{n}q", *vals, *ptrs, *ys, *strides) + epi + post)
     base = ctypes.addressof(arrays)
     tails = base + 48 * n
-    group = struct.pack("=" + _FMT_GROUP, M, K, x2.data_ptr(), x2.stride(0), base, n, base + 24 * n, base + 32 * n, base + 40 * n,
+    # (the stride of a single row says nothing: that of a [K, 1] tensor's transpose is 1)
+    group = struct.pack("=" + _FMT_GROUP, M, K, x2.data_ptr(), x2.stride(0) if M > 1 else K, base, n, base + 24 * n, base + 32 * n, base + 40 * n,
                         0 if epilogues is None else tails, 0 if posts is None else tails + len(epi))
     return (x2, arrays), group, outs, M
 

@@ -298,3 +298,18 @@ def test_lists_shorter_than_the_weights(dthip, oracle):
         dthip.dense_multi(x, ws[:1], [b], epilogues=[e, e])
     with pytest.raises(IndexError):
         dthip.dense_post(x, ws[:1], [b], [p, p])
+
+
+@pytest.mark.parametrize("K,N", [(64, 96), (77, 33)])
+def test_single_row_of_any_stride(dthip, oracle, K, N):
+    """One row of X: its stride, which torch leaves at any value (1 in a [K, 1] tensor's transpose), does not matter."""
+    import torch
+
+    rng = np.random.default_rng(K)
+    w, W = make(dthip, oracle, rng, N, K, 6, 4096)
+    X = rng.standard_normal((1, K)).astype(np.float16)
+    for x in (dev(X.reshape(K, 1)).t(), torch.as_strided(dev(X), (1, K), (7, 1)), dev(X)[:, None].transpose(0, 1)):
+        check(dthip.dense_multi(x, [w], [None])[0].reshape(1, N).cpu().numpy(), X, W)
+    col = torch.zeros((K, 2), dtype=torch.float16, device="cuda")
+    col[:, :1] = dev(X.reshape(K, 1))
+    check(dthip.dense_multi(col[:, :1].t(), [w], [None])[0].cpu().numpy(), X, W)  # (elements two apart: a copy)
