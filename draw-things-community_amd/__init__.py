@@ -444,10 +444,9 @@ def _enqueue_dense(fn, problems, flags, stream):
 
 
 def _shape_outs(x, M, outs):
-    if x.dim() == 2:
-        return outs
     lead = tuple(x.shape[:-1])
-    return [o if o is None or o.shape[0] != M or not o.is_contiguous() else o.reshape(lead + (o.shape[-1],)) for o in outs]
+    plain = lambda o: o is None or o.shape[0] != M or not o.is_contiguous() or (len(lead) == 1 and o.dim() == 2)
+    return [o if plain(o) else o.reshape(lead + (o.shape[-1],)) for o in outs]
 
 
 def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]], outs=None, flags: int = 0,

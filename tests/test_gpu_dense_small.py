@@ -313,3 +313,19 @@ def test_single_row_of_any_stride(dthip, oracle, K, N):
     col = torch.zeros((K, 2), dtype=torch.float16, device="cuda")
     col[:, :1] = dev(X.reshape(K, 1))
     check(dthip.dense_multi(col[:, :1].t(), [w], [None])[0].cpu().numpy(), X, W)  # (elements two apart: a copy)
+
+
+def test_given_outputs_come_back_in_the_shape_of_x(dthip, oracle):
+    """Contiguous outputs of one row per row of X are returned with X's leading dimensions, for a 2-D X as for any other."""
+    import torch
+
+    rng = np.random.default_rng(3)
+    M, K, N = 6, 64, 40
+    w, W = make(dthip, oracle, rng, N, K, 6, 4096)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    for shape, given in (((M, K), (M, N)), ((M, K), (M, 1, N)), ((2, 3, K), (M, N)), ((2, 3, K), (M, 1, N))):
+        out = torch.zeros(given, dtype=torch.float16, device="cuda")
+        for got in (dthip.dense_multi(dev(X).view(shape), [w], [None], outs=[out]),
+                    dthip.dense_post(dev(X).view(shape), [w], [None], [None], outs=[out])):
+            assert got[0].shape == shape[:-1] + (N,) and got[0].data_ptr() == out.data_ptr()
+        check(out.view(M, N).cpu().numpy(), X, W)
