@@ -440,13 +440,14 @@ def _enqueue_dense(fn, problems, flags, stream):
     # torch's allocator hands the block out again in stream order, so it may be dropped as soon as the call is enqueued
     ws = problems[0][0].new_empty(need, dtype=_torch().uint8) if need else None
     _check(fn, L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, None if ws is None else ws.data_ptr(), need))
-    return [_shape_outs(p[0], M, outs) for p, (_, _, outs, M) in zip(problems, packed)]
+    return [_shape_outs(p[0], M, outs, p[3] is None) for p, (_, _, outs, M) in zip(problems, packed)]
 
 
-def _shape_outs(x, M, outs):
+def _shape_outs(x, M, outs, made):
+    if made and x.dim() == 2:
+        return outs
     lead = tuple(x.shape[:-1])
-    plain = lambda o: o is None or o.shape[0] != M or not o.is_contiguous() or (len(lead) == 1 and o.dim() == 2)
-    return [o if plain(o) else o.reshape(lead + (o.shape[-1],)) for o in outs]
+    return [o if o is None or o.shape[0] != M or not o.is_contiguous() else o.reshape(lead + (o.shape[-1],)) for o in outs]
 
 
 def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]], outs=None, flags: int = 0,
