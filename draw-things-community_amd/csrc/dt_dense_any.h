@@ -1,6 +1,7 @@
 // Argument block and launcher of the any-shape Dense kernel (dt_dense_any.hip).
 #pragma once
 #include "dt_common.h"
+#include "dt_dense_any_index.h"
 
 namespace dt {
 

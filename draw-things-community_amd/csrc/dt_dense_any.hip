@@ -38,8 +38,6 @@ __device__ __forceinline__ void load_halfs16(const uint16_t* p, int left, uint32
   }
 }
 
-constexpr int kAnyPalBytes = 16384;  // LDS for the palettes of a tile's rows (with the tiles below: three workgroups per CU)
-
 // BT x BT outputs per 256-thread workgroup (BT = 64: 2 x 2 waves of 32 x 32; BT = 32: every wave computes the whole
 // tile over its own quarter of each K-tile).  A K-tile is 4096 / BT wide, so that a thread always stages 16 consecutive
 // k of one X row and of one weight row.
@@ -60,7 +58,7 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
   const int l32 = lane & 31, hi = lane >> 5;
   const int64_t m0 = (blockIdx.x % a.tiles_m) * BT, n0 = (blockIdx.x / a.tiles_m) * BT;
   const int row = tid / RUNS, run = tid % RUNS;
-  const int64_t gm = m0 + row, gn = n0 + row;
+  const int64_t gm = m0 + row, gn = any_row(n0 + row, a.n);
   const uint16_t* xr = a.x + (gm < a.m ? gm : 0) * a.ldx;
   const QxLayout lay = make_layout(Q == 16 ? 8 : Q, Q == 16 ? 32 : a.nib);
   const int nib = lay.nib;
@@ -69,31 +67,20 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
   int64_t blk0 = 0;
   if constexpr (Q != 16) {
     if (a.pal_shared) {
-      blk0 = n0 * a.k / nib;
-      const int64_t last_row = n0 + BT <= a.n ? n0 + BT - 1 : a.n - 1;
-      const int n_pal = (int)((last_row * a.k + a.k - 1) / nib - blk0 + 1);
-      for (int i = tid; i < n_pal << Q; i += 256)
+      const AnyBlocks held = any_blocks(n0, BT, a.n, a.k, nib);
+      blk0 = held.first;
+      for (int i = tid; i < held.count << Q; i += 256)
         pal_lds[i] = reinterpret_cast<const u16_any*>(a.w + palette_offset(lay, blk0 + (i >> Q)))[i & ((1 << Q) - 1)];
     }
   }
 
-  // Whole runs are fetched as words, unless blocks are shorter than a run (one may then touch more than two) or the
-  // buffer is shorter than a run's words: then index by index.
-  const bool runs_ok = nib >= 16 && a.w_bytes >= 4 * NRAW;
+  const bool runs_ok = any_by_words(NRAW, a.w_bytes, nib);  // (otherwise index by index)
+  AnyCursor next = {0, 0};  // this thread's next weight run
+  if constexpr (Q != 16) next = any_cursor(gn, a.k, run * 16, nib);
 
-  // cursor of this thread's weight run: block and position inside it
-  int64_t blk = 0;
-  uint32_t r = 0;
-  if constexpr (Q != 16) {
-    const int64_t e = (gn < a.n ? gn : 0) * a.k + run * 16;
-    blk = e / nib;
-    r = (uint32_t)(e - blk * nib);
-  }
-
-  // NRAW dwords from byte p of the packed buffer on.  The last runs of the buffer are read from further ahead instead
-  // of past its end; the result is the number of bytes by which their words are early.
+  // NRAW dwords from byte p of the packed buffer on; the result is the number of bytes by which they are early.
   auto load_raw = [&](int64_t p, uint32_t (&raw)[NRAW]) {
-    const int64_t q = p + 4 * NRAW <= a.w_bytes ? p : a.w_bytes - 4 * NRAW;
+    const int64_t q = any_words_at(p, NRAW, a.w_bytes);
     const u32_any* src = reinterpret_cast<const u32_any*>(a.w + q);
 #pragma unroll
     for (int i = 0; i < NRAW; i++) raw[i] = src[i];
@@ -123,42 +110,33 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
 
   uint32_t xraw[8], wraw[NRAW], wraw2[NRAW];
   int w_left = 0;  // weights of the fetched run that exist
-  int w_head = 0;  // ... of which this many lie in block cur_blk, the others in the next one
+  int w_head = 0;  // ... of which this many lie in its first block, the others in the next one
   int early = 0, early2 = 0, sh2 = 0;
   bool two = false;  // some lane's run crosses into another block
-  int64_t cur_blk = 0;
-  uint32_t cur_r = 0;
+  AnyCursor cur = {0, 0};
   auto fetch = [&](int kt) {
     const int64_t k0 = (int64_t)kt * BKA + run * 16;
-    w_left = k0 >= a.k ? 0 : (a.k - k0 < 16 ? (int)(a.k - k0) : 16);
+    w_left = any_run(k0, a.k);
     const bool whole = (int64_t)(kt + 1) * BKA <= a.k;  // uniform
     if (whole) load_halfs16<false>(xr + k0, 16, xraw);
     else load_halfs16<true>(xr + (w_left ? k0 : 0), w_left, xraw);
     if constexpr (Q == 16) {
-      const uint16_t* wr = reinterpret_cast<const uint16_t*>(a.w) + (gn < a.n ? gn : 0) * a.k;
+      const uint16_t* wr = reinterpret_cast<const uint16_t*>(a.w) + gn * a.k;
       if (whole) load_halfs16<false>(wr + k0, 16, wraw);
       else load_halfs16<true>(wr + (w_left ? k0 : 0), w_left, wraw);
     } else {
-      cur_blk = blk;
-      cur_r = r;
-      w_head = (uint32_t)nib - r < (uint32_t)w_left ? (int)((uint32_t)nib - r) : w_left;
+      cur = next;
+      w_head = any_run_head(cur, w_left, nib);
       if (runs_ok) {
-        early = load_raw(index_byte_offset(lay, w_left ? blk : 0, w_left ? r : 0), wraw);
+        early = load_raw(index_byte_offset(lay, w_left ? cur.blk : 0, w_left ? cur.r : 0), wraw);
         two = __builtin_amdgcn_ballot_w64(w_head < w_left) != 0;
         if (two) {
-          // The rest of the run, as the string in which it has the same place: from w_head indices ahead of the
-          // next block's first one (the bits in between, palette bytes, are not looked at).
-          const int64_t bit = w_head < w_left ? (palette_offset(lay, blk + 1) + lay.pal_bytes) * 8 - w_head * Q : 0;
+          const int64_t bit = w_head < w_left ? any_rest_bit(lay, cur, w_head) : 0;
           sh2 = (int)(bit & 7);
           early2 = load_raw(bit >> 3, wraw2);
         }
       }
-      r += BKA;
-      if (r >= (uint32_t)nib) {
-        const uint32_t q = r / (uint32_t)nib;
-        blk += q;
-        r -= q * (uint32_t)nib;
-      }
+      any_advance(next, BKA, nib);
     }
   };
   auto stage = [&](int buf) {
@@ -192,14 +170,14 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
       };
       if (runs_ok) {
         drop_bytes(wraw, early);
-        look_up(wraw, (int)((cur_r * Q) & 7), w_left ? cur_blk : blk0, 0, w_head);
+        look_up(wraw, (int)((cur.r * Q) & 7), w_left ? cur.blk : blk0, 0, w_head);
         if (two) {
           drop_bytes(wraw2, early2);
-          look_up(wraw2, sh2, w_head < w_left ? cur_blk + 1 : blk0, w_head, w_left);
+          look_up(wraw2, sh2, w_head < w_left ? cur.blk + 1 : blk0, w_head, w_left);
         }
       } else {
-        int64_t b = cur_blk;
-        uint32_t rr = cur_r;
+        int64_t b = cur.blk;
+        uint32_t rr = cur.r;
 #pragma unroll
         for (int j = 0; j < 16; j++)
           if (j < w_left) {
@@ -282,7 +260,7 @@ dt_status dense_any_launch(hipStream_t s, DenseAnyArgs a) {
   const int64_t grid = tiles(BT);
   if (grid > 0x7fffffff) return DT_NO_KERNEL;
   a.tiles_m = (a.m + BT - 1) / BT;
-  a.pal_shared = a.qbits != 16 && ((BT * a.k) / a.nib + 2) * ((int64_t)2 << a.qbits) <= kAnyPalBytes;
+  a.pal_shared = a.qbits != 16 && any_pal_shared(BT, a.k, a.qbits, a.nib);
   switch (a.qbits) {
     case 4: launch_any<4>(s, a, big, (unsigned)grid); break;
     case 5: launch_any<5>(s, a, big, (unsigned)grid); break;

@@ -164,3 +164,74 @@ def test_cpp_operator_mirror_compiles(dthip, tmp_path):
     subprocess.check_call([cxx, "-std=c++17", "-Wall", "-Wextra", "-Werror", "-fsyntax-only", "-I",
                            os.path.join(ROOT, "include"), str(src)])
     assert os.path.exists(os.path.join(os.path.dirname(dthip.LIB_PATH), "dt_cpp_check"))
+
+
+def test_any_shape_dense_stays_inside_its_buffers(tmp_path):
+    """The any-shape Dense kernel's index arithmetic, walked on the host for every tile, row and run of ragged shapes:
+    every palette slot that a thread looks up is one that the tile has loaded into its LDS, which holds them, every word
+    lies in the packed buffer, and a run starts at the weight it stands for."""
+    import shutil
+    import subprocess
+
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no C++ compiler")
+    src = tmp_path / "walk.cpp"
+    src.write_text(r'''
+#include <cstdio>
+#include <cstdlib>
+#include "dt_dense_any_index.h"
+using namespace dt;
+#define CHECK(c) do { if (!(c)) { printf("%s: n %lld k %lld q %d nib %d tile %d row %lld k0 %lld\n", #c, (long long)n, (long long)k, q, nib, bt, (long long)row, (long long)k0); return 1; } } while (0)
+static int walk(int64_t n, int64_t k, int q, int nib, int bt) {
+  const int bka = 4096 / bt, words = (q + 1) / 2 + 1;
+  const QxLayout lay = make_layout(q, nib);
+  const int64_t bytes = qx_total_bytes(q, nib, n * k), last = (n * k - 1) / nib;
+  const bool shared = any_pal_shared(bt, k, q, nib), by_words = any_by_words(words, bytes, nib);
+  for (int64_t n0 = 0; n0 < n; n0 += bt) {
+    const AnyBlocks held = any_blocks(n0, bt, n, k, nib);
+    for (int tr = 0; tr < bt; tr++)
+      for (int run = 0; run < bka / 16; run++) {
+        const int64_t row = any_row(n0 + tr, n);
+        int64_t k0 = run * 16;
+        CHECK(held.first >= 0 && held.first + held.count - 1 <= last && row >= 0 && row < n);
+        CHECK(!shared || (held.count << q) * 2 <= kAnyPalBytes);
+        AnyCursor c = any_cursor(row, k, run * 16, nib);
+        for (int64_t kt = 0; kt * bka < k; kt++, k0 += bka, any_advance(c, bka, nib)) {
+          const int left = any_run(k0, k), head = any_run_head(c, left, nib);
+          CHECK(left >= 0 && left <= 16 && head <= left && (left == 0 || head > 0));
+          if (left == 0) continue;  // (such a lane looks at the tile's first palette)
+          CHECK(c.blk * nib + c.r == row * k + k0);
+          if (!by_words) continue;
+          CHECK(c.blk >= held.first && c.blk < held.first + held.count);
+          int64_t at = any_words_at(index_byte_offset(lay, c.blk, c.r), words, bytes);
+          CHECK(at >= 0 && at + 4 * words <= bytes);
+          if (head < left) {
+            CHECK(c.blk + 1 < held.first + held.count);
+            at = any_words_at(any_rest_bit(lay, c, head) >> 3, words, bytes);
+            CHECK(at >= 0 && at + 4 * words <= bytes);
+          }
+        }
+      }
+  }
+  return 0;
+}
+int main(int argc, char** argv) {
+  for (int i = 1; i + 3 < argc; i += 4)
+    for (int bt = 32; bt <= 64; bt += 32)
+      if (walk(atoll(argv[i]), atoll(argv[i + 1]), atoi(argv[i + 2]), atoi(argv[i + 3]), bt)) return 1;
+  return 0;
+}
+''')
+    exe = tmp_path / "walk"
+    subprocess.check_call([cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-Werror", "-I",
+                           os.path.join(ROOT, "draw-things-community_amd", "csrc"), str(src), "-o", str(exe)])
+    # N, K, index width, block size: the shapes of the GPU's parity test, and random ones
+    shapes = [(1, 1, 6, 1), (31, 100, 6, 32), (32, 128, 5, 24), (65, 129, 7, 4096), (40, 16, 4, 512), (1001, 1000, 8, 16384),
+              (90, 2500, 8, 512), (1400, 200, 6, 4096), (1470, 77, 4, 64), (33, 2560, 8, 16384), (97, 5121, 6, 4096)]
+    rng = np.random.default_rng(88)
+    for _ in range(300):
+        n, k, nib = (int(np.exp(rng.uniform(np.log(lo), np.log(hi)))) for lo, hi in ((1, 600), (1, 1500), (1, 20000)))
+        shapes.append((n, k, int(rng.integers(4, 9)), nib))
+    out = subprocess.run([str(exe)] + [str(v) for s in shapes for v in s], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
