@@ -430,6 +430,22 @@ def _marshal_dense(x, weights, biases, outs, epilogues, posts):
 _ROWS_MAX = 64  # rows up to which the library streams the weights and needs no workspace
 
 
+def _scratch(like, need, least):
+    """(what holds it, address, bytes) of scratch memory on the device of `like`, 256-byte aligned: `need` bytes, or where
+    the device is that full the `least` that the call cannot do without.  torch's allocator hands the block out again in
+    stream order, so it may be dropped as soon as the call is enqueued."""
+    if not need:
+        return None, None, 0
+    torch = _torch()
+    try:
+        ws = like.new_empty(need + 255, dtype=torch.uint8)
+        return ws, (ws.data_ptr() + 255) & ~255, need
+    except torch.OutOfMemoryError:
+        if need == least:
+            raise
+    return _scratch(like, least, least)
+
+
 def _enqueue_dense(fn, problems, flags, stream):
     """Enqueues Dense problems -- (x, weights, biases, outs, epilogues, posts) each -- together, with the scratch memory
     that lets the library cut tiles along K where there are too few of them for the chip.  Returns their outputs."""
@@ -437,9 +453,8 @@ def _enqueue_dense(fn, problems, flags, stream):
     groups = b"".join(g for _, g, _, _ in packed)  # (what they point to lives in `packed` until the call returns)
     n, L = len(packed), lib()
     need = L.dt_dense_workspace_bytes(n, groups) if any(M > _ROWS_MAX for _, _, _, M in packed) else 0
-    # torch's allocator hands the block out again in stream order, so it may be dropped as soon as the call is enqueued
-    ws = problems[0][0].new_empty(need, dtype=_torch().uint8) if need else None
-    _check(fn, L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, None if ws is None else ws.data_ptr(), need))
+    ws, at, need = _scratch(problems[0][0], need, 0)
+    _check(fn, L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, at, need))
     return [_shape_outs(p[0], M, outs, p[3] is None) for p, (_, _, outs, M) in zip(problems, packed)]
 
 
@@ -922,12 +937,9 @@ def sdpa_segments(q_segs, k_segs, v_segs, scale, gamma_q=None, gamma_k=None, rot
         _check("dt_sdpa_f16_static", st)
         return out
     need = L.dt_sdpa_workspace_bytes(B, Hq, Hk, D, Sq, Skv, int(prep), int(fused))
-    ws = torch.empty(max(need, 256) + 256, dtype=torch.uint8, device=out.device) if need else None
-    ws_ptr = None
-    if ws is not None:
-        ws_ptr = (ws.data_ptr() + 255) & ~255
-    st = L.dt_sdpa_f16(
-        _stream_ptr(stream), B, Hq, Hk, D, nq, qa, nk, ka, va, rq, rk, eps, ov, scale, wo, bo_p, ws_ptr, need)
+    staged = sum((b + 255) // 256 * 256 for b in (prep * B * Skv * Hk * D * 2, fused * B * Sq * Hq * D * 2))
+    ws, at, need = _scratch(out, need, staged)
+    st = L.dt_sdpa_f16(_stream_ptr(stream), B, Hq, Hk, D, nq, qa, nk, ka, va, rq, rk, eps, ov, scale, wo, bo_p, at, need)
     _check("dt_sdpa_f16", st)
     return out
 

@@ -329,3 +329,54 @@ def test_given_outputs_come_back_in_the_shape_of_x(dthip, oracle):
                     dthip.dense_post(dev(X).view(shape), [w], [None], [None], outs=[out])):
             assert got[0].shape == shape[:-1] + (N,) and got[0].data_ptr() == out.data_ptr()
         check(out.view(M, N).cpu().numpy(), X, W)
+
+
+@pytest.mark.parametrize("kind", ["dense", "attention", "attention staged"])
+def test_optional_scratch_is_not_insisted_on(dthip, oracle, monkeypatch, kind):
+    """Where torch may not allocate any more, calls run uncut instead of failing: the scratch that cutting takes is
+    optional, the staging of prepared keys is not."""
+    import torch
+
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
+    rng = np.random.default_rng(9)
+    L = dthip.lib()
+    staged = 0
+    if kind == "dense":
+        M, K, N = 512, 5120, 5120
+        w, _ = make(dthip, oracle, rng, N, K, 6, 4096)
+        x, out = dev(rng.standard_normal((M, K)).astype(np.float16)), torch.empty((M, N), dtype=torch.float16, device="cuda")
+        need = L.dt_dense_workspace_bytes(1, _groups(dthip, x, w, out)[0])
+        call = lambda: dthip.dense_multi(x, [w], [None], outs=[out])
+    else:
+        B, S, H, D = 1, 1500, 4, 128
+        q, k, v = (torch.randn((B, S, H, D), device="cuda").half() for _ in range(3))
+        more = {} if kind == "attention" else {"gamma_k": [torch.ones(D, device="cuda").half()]}
+        staged = B * S * H * D * 2 if more else 0
+        need = L.dt_sdpa_workspace_bytes(B, H, H, D, S, S, int(bool(more)), 0)
+        out = torch.empty((B, S, H, D), dtype=torch.float16, device="cuda")
+        call = lambda: dthip.sdpa_segments([q], [k], [v], D ** -0.5, out=out, **more)
+    assert need > (22 << 20) + staged  # (more than torch can have left over in a block)
+    call()
+    cut = out.clone()
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "never")
+    call()
+    whole = out.clone()
+    monkeypatch.delenv("DT_DENSE_SPLIT")
+    monkeypatch.delenv("DT_SDPA_KEY_SPLIT")
+    assert not torch.equal(cut, whole)
+    print("scratch that cannot be had:", kind, flush=True)
+    torch.cuda.empty_cache()
+    total = torch.cuda.mem_get_info()[1]
+    keep = torch.empty(staged, dtype=torch.uint8, device="cuda")
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    try:
+        del keep  # room for the staging, and for no more
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need, dtype=torch.uint8, device="cuda")
+        out.zero_()
+        call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(out, whole)
