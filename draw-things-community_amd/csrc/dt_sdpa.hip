@@ -697,9 +697,13 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
     plan->counter_bytes = ((size_t)cut * kSdpaSplitNodes * 4 + 255) & ~(size_t)255;
     const size_t slot = (size_t)sdpa_split_slot_floats(D <= 64 ? 64 : 128) * 4;
     plan->partial_bytes = (size_t)(cut * shares) * slot;
-    // What callers are asked to bring: two slots for each of up to 8 workgroups per task, at most one per compute unit.
-    // The parts need no more than that (2 cut < 2 cus slots, or cut * shares <= cus of them and 32 bytes per task).
-    plan->room = (((size_t)tasks * 4 + 255) & ~(size_t)255) + 2 * (size_t)std::min<int64_t>(cus, tasks * kSdpaSplitNodes) * slot;
+    // What callers are asked to bring.  With full rounds in front: what the parts take (24 heads x 2637 tokens: 9 MB).
+    // Launches under one round ask for two slots for each of up to 8 workgroups per task, at most one per compute unit,
+    // as the planning test pins it; the parts need no more than that (2 cut < 2 cus slots, or cut * shares <= cus of them
+    // and 32 bytes per task).
+    plan->room = whole > 0 && !always ? plan->bytes()
+                                      : (((size_t)tasks * 4 + 255) & ~(size_t)255) +
+                                            2 * (size_t)std::min<int64_t>(cus, tasks * kSdpaSplitNodes) * slot;
   }
   return true;
 }

@@ -323,9 +323,11 @@ DT_EXPORT dt_status dt_sdpa_f16_static(dt_stream stream, int32_t B, int32_t Hq, 
   if (sh.empty) return DT_OK;
   if (sh.need > (size_t)DT_SDPA_STATIC_SCRATCH_BYTES) return DT_OOM;  // beyond the fixed array: use dt_sdpa_f16
   if (const dt_status ready = device_ready(); ready != DT_OK) return ready;
-  // the staging bytes are a must; the key-split form's room is used if the array still has it
-  size_t give = dt_sdpa_workspace_bytes(B, Hq, Hk, D, sh.Sq, sh.Skv, sh.kprep ? 1 : 0, Wo ? 1 : 0);
-  if (give > (size_t)DT_SDPA_STATIC_SCRATCH_BYTES) give = sh.need;
+  // the staging bytes are a must; the key-split form takes what it needs if the array still has it
+  size_t give = sh.need;
+  SdpaSplit plan;
+  if (sdpa_split_plan(B, Hq, D, sh.Sq, sh.Skv, &plan) && give + plan.bytes() <= (size_t)DT_SDPA_STATIC_SCRATCH_BYTES)
+    give += plan.bytes();
   void* ws = nullptr;
   if (give > 0) {
     ws = sdpa_static_scratch();

@@ -323,11 +323,11 @@ dt_status dt_qk_norm_rope_f16(dt_stream stream, dt_view4 x, int32_t B, int64_t S
  *   workspace : device scratch, 256-byte aligned; may be NULL when nothing is
  *             staged.  dt_sdpa_workspace_bytes(...) is the staging this call
  *             cannot run without (fused_prep / fused_out_proj; less than that
- *             is DT_OOM) plus, for launches that would occupy well under one
- *             round of the card's compute units, room for the key-split form of
- *             the kernel (each task's key tiles shared out over several
- *             workgroups, fp32 partial results folded in a fixed order by the
- *             piece that finishes last).  Given only the staging part, or
+ *             is DT_OOM) plus, for launches that leave much of the card idle in
+ *             their last round of workgroups, room for the key-split form of
+ *             the kernel (the key tiles of that round's tasks shared out over
+ *             several workgroups, whose fp32 partial results are folded in
+ *             pairs, the same whichever comes first).  Given only the staging part, or
  *             nothing, such a launch runs unsplit: same results to within one
  *             rounding of the fp16 output, lower occupancy.
  *             Environment: DT_SDPA_KEY_SPLIT=never|always overrides the
@@ -361,8 +361,8 @@ size_t dt_sdpa_workspace_bytes(int32_t B, int32_t Hq, int32_t Hk, int32_t D, int
  *   The scratch is one fixed array of DT_SDPA_STATIC_SCRATCH_BYTES per GPU, resident on every GPU the library runs
  *   on until the process ends (its device address is looked up once per device, by dt_init or by the first call
  *   with that device current).  A request whose staging exceeds it returns DT_OOM and enqueues nothing: use
- *   dt_sdpa_f16 with a workspace of the caller's then.  (The optional key-split room is used when the array still
- *   has it, exactly as dt_sdpa_f16 uses a workspace of dt_sdpa_workspace_bytes().)  The limit covers the staged K of a joint
+ *   dt_sdpa_f16 with a workspace of the caller's then.  (The key-split form is used where the array still has
+ *   the room that it takes.)  The limit covers the staged K of a joint
  *   sequence of 4608 tokens x 24 heads x 128 with fused QK-norm / RoPE (28.3 MB; up to ~10900 such tokens) and the
  *   fused unify-heads staging of SD 1.5 (5.2 MB).
  *   All calls on one GPU share that GPU's array, whose contents are whatever the last call left (every byte a

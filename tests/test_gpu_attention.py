@@ -794,6 +794,21 @@ def test_sdpa_key_split_joint_segments_fused_prep(dthip, oracle, torch_cuda, mon
     assert float((seg_split.float() - seg_plain.float()).abs().max()) <= 2e-3
 
 
+def test_sdpa_key_split_static_scratch(dthip, torch_cuda, monkeypatch):
+    """The fixed array takes the parts of a launch whose own request for scratch (two slots per workgroup, 69 MB) exceeds
+    it: 64 tasks in 4 parts each need 35 MB."""
+    torch = torch_cuda
+    monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn((1, 4096, 4, 128), generator=g, device="cuda").half() for _ in range(3))
+    args = ([q], [k], [v], 128 ** -0.5)
+    print("sdpa key split, static scratch", flush=True)
+    got = dthip.sdpa_segments(*args, static_scratch=True)
+    assert torch.equal(got, dthip.sdpa_segments(*args))
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "never")
+    assert not torch.equal(got, dthip.sdpa_segments(*args, static_scratch=True))
+
+
 def test_sdpa_key_split_by_its_own_estimate(dthip, oracle, torch_cuda, monkeypatch):
     """A launch that fills a quarter of the card (4 heads x 4096 tokens: 64 workgroups of 64 key tiles) is split
     without being told to; sampled rows against the oracle."""

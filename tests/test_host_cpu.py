@@ -60,6 +60,17 @@ def test_key_split_planning(dthip, monkeypatch):
     assert ws(1, 1, 128, 1, 64) == 0                # a single key tile cannot be cut
 
 
+def test_key_split_room_beside_full_rounds(dthip, monkeypatch):
+    """Launches with full rounds in front bring a slot for every part of their cut tasks and no more."""
+    L = dthip.lib()
+    ws = lambda H, D, S: L.dt_sdpa_workspace_bytes(1, H, H, D, S, S, 0, 0)
+    monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
+    slot = lambda dp: (dp // 32 * 16 * 512 + 2 * 512) * 4
+    assert ws(24, 128, 2637) == 256 + 8 * 8 * slot(128)    # 264 tasks: 8 of them in 8 parts
+    assert ws(20, 128, 4096) == 2048 + 64 * 4 * slot(128)  # 320 tasks: 64 in 4 parts, whose counters fill 2 KB
+    assert ws(33, 64, 2000) == 256 + 8 * 8 * slot(64)
+
+
 def test_missing_library_fails_loudly(dthip, monkeypatch):
     monkeypatch.setattr(dthip, "_lib", None)
     monkeypatch.setattr(dthip, "LIB_PATH", os.path.join(ROOT, "no_such_dir", "libdthip.so"))
