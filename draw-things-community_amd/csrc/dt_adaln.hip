@@ -63,10 +63,13 @@ struct AdaLnArgs {
   int64_t ldy;
 };
 
-// Rows of up to NV * 256 elements, C % 4 == 0, 16-byte aligned rows: lane l
-// holds the float4 at element 256 i + 4 l of every 256-element chunk i.  A lane past the row's end reads the row's
-// first chunk and drops it: behind a test of their own, the chunks' loads (and the scale's and shift's, two chunks ahead
-// of their use here) were each waited for before the next went out, 20 us for however few rows (512 x 3072 beside 4096 x 3072: 20.7 -> 15.5 and 25.1 -> 18.9 us; 1376 x 3072: 21.4 -> 13.6).
+// Rows of (NV - 2) * 256 + 4 .. NV * 256 elements, C % 4 == 0, 16-byte aligned rows: lane l
+// holds the float4 at element 256 i + 4 l of every 256-element chunk i.  Only in the last two chunks can a lane lie past
+// the row's end; it then reads the row's first chunk and drops it: behind a test of their own, the chunks' loads (and the
+// scale's and shift's, two chunks ahead of their use here) were each waited for before the next went out, 20 us for
+// however few rows.  NV goes in steps of two because chunks past the end cost what the others do, and the tests registers:
+// in steps of 4, 12 beyond 20, with a test for every chunk, fp32 modulation of 8700 rows took, us, 4608 wide 55.2 (here
+// 42.9), 5120 63.2 (48.1, 5.6 TB/s), 6144 88.2 (72.8); 512 rows of 5120 10.0 (7.4).
 template <int NV, int MOD>
 __global__ void __launch_bounds__(256, NV <= 20 ? 3 : 2) adaln_rows_kernel(const AdaLnArgs a) {
   const int lane = threadIdx.x & 63;
@@ -79,12 +82,12 @@ __global__ void __launch_bounds__(256, NV <= 20 ? 3 : 2) adaln_rows_kernel(const
 #pragma unroll
   for (int i = 0; i < NV; i++) {
     const int e = i * 256 + lane * 4;
-    v[i] = *reinterpret_cast<const float4_t*>(xr + (e < c ? e : 0));
+    v[i] = *reinterpret_cast<const float4_t*>(xr + (i < NV - 2 || e < c ? e : 0));
   }
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; i++) {
-    if (i * 256 + lane * 4 >= c) v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (i >= NV - 2 && i * 256 + lane * 4 >= c) v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
     s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
   }
   const float mean = wave_sum64(s) / (float)c;
@@ -93,7 +96,7 @@ __global__ void __launch_bounds__(256, NV <= 20 ? 3 : 2) adaln_rows_kernel(const
   for (int i = 0; i < NV; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      v[i][j] = i * 256 + lane * 4 < c ? v[i][j] - mean : 0.f;
+      v[i][j] = i < NV - 2 || i * 256 + lane * 4 < c ? v[i][j] - mean : 0.f;
       q += v[i][j] * v[i][j];
     }
   const float inv = 1.0f / sqrtf(wave_sum64(q) / (float)c + a.eps);
@@ -103,7 +106,7 @@ __global__ void __launch_bounds__(256, NV <= 20 ? 3 : 2) adaln_rows_kernel(const
   auto fetch = [&](int buf, int i0) {
 #pragma unroll
     for (int k = 0; k < G; k++) {
-      const int e = (i0 + k) * 256 + lane * 4, ec = e < c ? e : 0;
+      const int e = (i0 + k) * 256 + lane * 4, ec = i0 + k < NV - 2 || e < c ? e : 0;
       constexpr int W = MOD == DT_MOD_F16 ? 2 : 4;
       if (a.scale) sc[buf][k] = *reinterpret_cast<const Raw*>(static_cast<const char*>(a.scale) + ec * W);
       if (a.shift) sh[buf][k] = *reinterpret_cast<const Raw*>(static_cast<const char*>(a.shift) + ec * W);
@@ -122,7 +125,7 @@ __global__ void __launch_bounds__(256, NV <= 20 ? 3 : 2) adaln_rows_kernel(const
 #pragma unroll
     for (int j = 0; j < 4; j++)
       o[j] = modulate<MOD>(v[i][j] * inv, a.scale != nullptr, fs[j], a.shift != nullptr, ft[j]);
-    if (e < c)
+    if (i < NV - 2 || e < c)
       *reinterpret_cast<uint2_t*>(yr + e) =
           uint2_t{(uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16)};
   }
@@ -245,20 +248,18 @@ __global__ void __launch_bounds__(256) layernorm16_generic_kernel(const LayerNor
   }
 }
 
+// The instantiation for a row of `nv` chunks.
+template <int NV, int MOD>
+static void launch_adaln_rows(hipStream_t s, const AdaLnArgs& a, int nv) {
+  if constexpr (NV < 32)
+    if (nv > NV) return launch_adaln_rows<NV + 2, MOD>(s, a, nv);
+  hipLaunchKernelGGL((adaln_rows_kernel<NV, MOD>), dim3((unsigned)((a.m + 3) / 4)), dim3(256), 0, s, a);
+}
+
 template <int MOD>
 static void launch_adaln(hipStream_t s, const AdaLnArgs& a, bool vec) {
-  const dim3 grid((unsigned)((a.m + 3) / 4)), block(256);
-  if (!vec || a.c > 32 * 256) {
-    hipLaunchKernelGGL((adaln_generic_kernel<MOD>), grid, block, 0, s, a);
-    return;
-  }
-  const int nv = (int)((a.c + 255) / 256);
-  if (nv <= 4) hipLaunchKernelGGL((adaln_rows_kernel<4, MOD>), grid, block, 0, s, a);
-  else if (nv <= 8) hipLaunchKernelGGL((adaln_rows_kernel<8, MOD>), grid, block, 0, s, a);
-  else if (nv <= 12) hipLaunchKernelGGL((adaln_rows_kernel<12, MOD>), grid, block, 0, s, a);
-  else if (nv <= 16) hipLaunchKernelGGL((adaln_rows_kernel<16, MOD>), grid, block, 0, s, a);
-  else if (nv <= 20) hipLaunchKernelGGL((adaln_rows_kernel<20, MOD>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((adaln_rows_kernel<32, MOD>), grid, block, 0, s, a);
+  if (vec && a.c <= 32 * 256) launch_adaln_rows<2, MOD>(s, a, (int)((a.c + 255) / 256));
+  else hipLaunchKernelGGL((adaln_generic_kernel<MOD>), dim3((unsigned)((a.m + 3) / 4)), dim3(256), 0, s, a);
 }
 
 }  // namespace dt

@@ -43,6 +43,24 @@ def test_layernorm_modulate_vs_oracle(dthip, oracle, M, C, mod):
                  oracle.np_layernorm_modulate16(x, None, shift, 1e-6, mod), shift)
 
 
+@pytest.mark.parametrize("mod", ["f16", "f32", "affine"])
+def test_layernorm_modulate_row_lengths(dthip, oracle, mod):
+    """One, two and all lanes of the last chunk of 256, at every pair of chunks a kernel is made for, rows apart from each
+    other by guard values that must not be read into the statistics."""
+    import torch
+    rng = np.random.default_rng(17)
+    dt = np.float16 if mod == "f16" else np.float32
+    for chunks in range(1, 33):
+        for C in (256 * chunks - 252, 256 * chunks - 248, 256 * chunks):
+            x = (rng.standard_normal((3, C)) + 0.5).astype(np.float32)
+            scale, shift = (1 + 0.3 * rng.standard_normal(C)).astype(dt), (0.5 * rng.standard_normal(C)).astype(dt)
+            wide = torch.full((3, C + 4), 1e30, dtype=torch.float32, device="cuda")
+            wide[:, :C] = torch.from_numpy(x)
+            got = dthip.layernorm_modulate(wide[:, :C], torch.from_numpy(scale).cuda(), torch.from_numpy(shift).cuda(), 1e-6,
+                                           affine=mod == "affine")
+            assert close(got.cpu().numpy(), oracle.np_layernorm_modulate16(x, scale, shift, 1e-6, mod), shift), C
+
+
 def test_layernorm_modulate_views_and_edges(dthip, oracle):
     import torch
     rng = np.random.default_rng(3)
