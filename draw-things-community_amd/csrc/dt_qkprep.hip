@@ -116,7 +116,9 @@ struct QkPrepMulti {
   int32_t* zero;
   int32_t n_zero;
 };
-template <int LPR>
+// I counts rows: 32 bits where they do, chosen by the host (32760 x 40 heads of 128: 154.6 us; 171.0 with both divisions
+// in the kernel, behind a test that kept the passes' loads apart; 165.4 with the one of 64 bits).
+template <int LPR, typename I>
 __global__ void __launch_bounds__(256) qk_prep_head16_kernel(const QkPrepMulti all) {
   constexpr int RPP = 256 / LPR;  // rows per pass
   int part = 0;
@@ -139,18 +141,7 @@ __global__ void __launch_bounds__(256) qk_prep_head16_kernel(const QkPrepMulti a
     const int64_t row = row0 + i * RPP;
     on[i] = row < rows;
     const int64_t rc = on[i] ? row : rows - 1;
-    int64_t h, s, b;
-    if (rows <= 0x7fffffff) {  // uniform
-      const uint32_t r32 = (uint32_t)rc, bs = r32 / (uint32_t)a.H, b32 = bs / (uint32_t)a.S;
-      h = r32 - bs * (uint32_t)a.H;
-      s = bs - b32 * (uint32_t)a.S;
-      b = b32;
-    } else {
-      const int64_t bs = rc / a.H;
-      h = rc % a.H;
-      s = bs % a.S;
-      b = bs / a.S;
-    }
+    const I bs = (I)rc / (I)a.H, h = (I)rc - bs * (I)a.H, b = bs / (I)a.S, s = bs - b * (I)a.S;
     v[i] = *reinterpret_cast<const uint4_t*>(a.src + b * a.src_sb + s * a.src_ss + h * a.src_sh + 8 * c);
     dst[i] = a.dst + b * a.dst_sb + s * a.dst_ss + h * a.dst_sh + 8 * c;
     if (a.rot) r[i] = *reinterpret_cast<const uint4_t*>(a.rot + (a.rot_pos0 + s) * a.D + 8 * c);
@@ -229,18 +220,27 @@ static bool chunks_ok(const QkPrepArgs& a) {
          (!a.rot || aligned16(a.rot)) && (!a.gamma || aligned16(a.gamma));
 }
 
+template <int LPR>
+static void launch_head16(hipStream_t s, unsigned blocks, const QkPrepMulti& all, bool wide) {
+  if (wide) hipLaunchKernelGGL((qk_prep_head16_kernel<LPR, int64_t>), dim3(blocks), dim3(256), 0, s, all);
+  else hipLaunchKernelGGL((qk_prep_head16_kernel<LPR, uint32_t>), dim3(blocks), dim3(256), 0, s, all);
+}
+
 bool qk_prep_launch_parts(hipStream_t s, const QkPrepArgs* parts, int n, int32_t* zero, int n_zero, dt_status* status) {
   if (n < 1 || n > kQkPrepParts) return false;
   QkPrepMulti all;
   const int lpr = parts[0].D / 8;
   int64_t blocks = 0;
+  bool wide = false;
   for (int i = 0; i < n; i++) {
     const QkPrepArgs& a = parts[i];
     if (a.B <= 0 || a.S <= 0 || a.H <= 0 || a.D != parts[0].D || !(a.norm_per_head || !a.gamma) || !chunks_ok(a)) return false;
     const int per_block = (256 / lpr) * kHeadPasses;
     all.part[i] = a;
     all.first_block[i] = (int32_t)blocks;
-    blocks += ((int64_t)a.B * a.S * a.H + per_block - 1) / per_block;
+    const int64_t rows = (int64_t)a.B * a.S * a.H;
+    wide = wide || rows > 0x7fffffff;
+    blocks += (rows + per_block - 1) / per_block;
     if (blocks > 0x7ffffffe) return false;
   }
   for (int i = n; i < kQkPrepParts; i++) {
@@ -249,10 +249,9 @@ bool qk_prep_launch_parts(hipStream_t s, const QkPrepArgs* parts, int n, int32_t
   }
   all.zero = zero;
   all.n_zero = n_zero;
-  const dim3 grid((unsigned)blocks);
-  if (lpr == 16) hipLaunchKernelGGL(qk_prep_head16_kernel<16>, grid, dim3(256), 0, s, all);
-  else if (lpr == 8) hipLaunchKernelGGL(qk_prep_head16_kernel<8>, grid, dim3(256), 0, s, all);
-  else if (lpr == 4) hipLaunchKernelGGL(qk_prep_head16_kernel<4>, grid, dim3(256), 0, s, all);
+  if (lpr == 16) launch_head16<16>(s, (unsigned)blocks, all, wide);
+  else if (lpr == 8) launch_head16<8>(s, (unsigned)blocks, all, wide);
+  else if (lpr == 4) launch_head16<4>(s, (unsigned)blocks, all, wide);
   else return false;
   *status = launch_status();
   return true;
