@@ -165,8 +165,11 @@ __global__ void __launch_bounds__(256) qk_prep_head16_kernel(const QkPrepMulti a
 }
 
 // Whole-row norm over H * D <= 8192 elements: one wave per (b, s) row, the row held in registers between the
-// sum of squares and the output -- one read, one write.
-constexpr int kRowChunks = 16;  // 16-byte chunks per lane
+// sum of squares and the output -- one read, one write.  NC 16-byte chunks per lane, in steps of two: only in the last
+// two can a lane lie past the row's end.  (us, 16 chunks whatever the width / here: 32760 rows of 1536 56.1 / 37.4, of 5120
+// 150.4 / 124.5, 5.4 TB/s; 1500 rows of 5120 11.8 / 10.6.)
+constexpr int kRowChunks = 16;
+template <int NC>
 __global__ void __launch_bounds__(256) qk_prep_row16_kernel(const QkPrepArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t bs = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -177,17 +180,17 @@ __global__ void __launch_bounds__(256) qk_prep_row16_kernel(const QkPrepArgs a) 
   const int nc = width / 8;  // chunks in the row
   const uint16_t* src = a.src + b * a.src_sb + s * a.src_ss;
   uint16_t* dst = a.dst + b * a.dst_sb + s * a.dst_ss;
-  uint4_t v[kRowChunks];
+  uint4_t v[NC];
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < kRowChunks; i++) {
+  for (int i = 0; i < NC; i++) {
     const int ch = lane + 64 * i;
     // (a lane past the row's end reads its first chunk: behind a test the loads would be waited for one by one)
-    v[i] = *reinterpret_cast<const uint4_t*>(src + 8 * (ch < nc ? ch : 0));
+    v[i] = *reinterpret_cast<const uint4_t*>(src + 8 * (i < NC - 2 || ch < nc ? ch : 0));
   }
 #pragma unroll
-  for (int i = 0; i < kRowChunks; i++) {
-    if (lane + 64 * i >= nc) v[i] = uint4_t{0, 0, 0, 0};
+  for (int i = 0; i < NC; i++) {
+    if (i >= NC - 2 && lane + 64 * i >= nc) v[i] = uint4_t{0, 0, 0, 0};
     float x[8];
     unpack_chunk(v[i], x);
 #pragma unroll
@@ -197,9 +200,9 @@ __global__ void __launch_bounds__(256) qk_prep_row16_kernel(const QkPrepArgs a) 
   const float inv = 1.0f / sqrtf(ss / (float)width + a.eps);
   const uint16_t* rot_row = a.rot ? a.rot + (a.rot_pos0 + s) * a.D : nullptr;
 #pragma unroll
-  for (int i = 0; i < kRowChunks; i++) {
+  for (int i = 0; i < NC; i++) {
     const int ch = lane + 64 * i;
-    if (ch < nc) {
+    if (i < NC - 2 || ch < nc) {
       float x[8];
       unpack_chunk(v[i], x);
       // the norm weight is indexed over the whole row, the table over the head dimension
@@ -209,6 +212,14 @@ __global__ void __launch_bounds__(256) qk_prep_row16_kernel(const QkPrepArgs a) 
       *reinterpret_cast<uint4_t*>(dst + 8 * ch) = finish_chunk(x, inv, true, g, rot_row != nullptr, r, a.post_scale);
     }
   }
+}
+
+// The instantiation for a row of `nc` chunks per lane.
+template <int NC>
+static void launch_row16(hipStream_t s, unsigned blocks, const QkPrepArgs& a, int nc) {
+  if constexpr (NC < kRowChunks)
+    if (nc > NC) return launch_row16<NC + 2>(s, blocks, a, nc);
+  hipLaunchKernelGGL(qk_prep_row16_kernel<NC>, dim3(blocks), dim3(256), 0, s, a);
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -271,7 +282,7 @@ dt_status qk_prep_launch(hipStream_t s, const QkPrepArgs& a) {
     if (chunks_ok(a) && (int64_t)a.H * a.D <= 8 * 64 * kRowChunks) {
       int64_t blocks = (rows + 3) / 4;
       if (blocks > 0x7fffffff) return DT_NO_KERNEL;
-      hipLaunchKernelGGL(qk_prep_row16_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+      launch_row16<2>(s, (unsigned)blocks, a, (a.H * a.D + 511) / 512);
       return launch_status();
     }
     if (rows > 0x7fffffff) return DT_NO_KERNEL;

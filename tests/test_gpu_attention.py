@@ -625,6 +625,25 @@ def test_qk_row_norm_rope_wan_full_size(dthip, oracle, torch_cuda):
     assert bool(torch.isfinite(y.float()).all()) and float(y.float().abs().max()) < 40.0
 
 
+@pytest.mark.parametrize("C", [8, 512, 520, 1024, 1032, 2048, 2056, 3064, 3072, 4096, 4104, 5128, 6144, 6152, 7168, 7176, 8184, 8192, 8200])
+def test_qk_row_norm_chunks(dthip, oracle, torch_cuda, C):
+    """Row norm and rotation of rows that end at, just past and just ahead of every count of chunks that a lane holds
+    (steps of 1024 elements up to 8192, beyond it the form for any width), inside wider rows of infinities: one ulp for
+    the norm and one for the rotation, and nothing else touched."""
+    torch = torch_cuda
+    rng = np.random.default_rng(C)
+    S, D = 6, 8
+    x, rot, gam = f16(rng.standard_normal((S, C))), f16(rng.standard_normal((S, D))), f16(1 + 0.1 * rng.standard_normal(C))
+    wide = torch.full((1, S, C + 24), float("inf"), dtype=torch.float16, device="cuda")
+    wide[0, :, 8:8 + C] = to_dev(torch, x)
+    print("row norm chunks", C, flush=True)
+    dthip.qk_norm_rope_(wide[:, :, 8:8 + C].unflatten(2, (C // D, D)), to_dev(torch, gam), 1e-6, False, rot=to_dev(torch, rot))
+    assert bool(torch.isinf(wide[:, :, :8]).all()) and bool(torch.isinf(wide[:, :, 8 + C:]).all())
+    want = oracle.C.cmul(oracle.C.rmsnorm(x, gam, 1e-6).reshape(S, C // D, D), rot).astype(np.float64).reshape(S, -1, 2)
+    got = wide[0, :, 8:8 + C].cpu().numpy().astype(np.float64).reshape(S, -1, 2)
+    assert np.all(np.abs(got - want) <= 2 * (np.hypot(want[..., :1], want[..., 1:]) * 2.0 ** -10 + 2.0 ** -24))
+
+
 def test_sdpa_wan_causal_chunked_windows(dthip, oracle, torch_cuda):
     """Wan causal inference (Models/Wan.swift:104-127): the frames are attended in chunks; query chunk i (rows
     [i * frames, (i + 1) * frames)) sees the key / value prefix of min(hw, (i + 1) * frames + padFrames) rows.  Each
