@@ -228,12 +228,14 @@ constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
 // while a third of the compute units work and 1.02 us when all do (the card is limited as a whole), 7 % more with 7-
 // and 8-bit palettes, a third less with plain fp16 weights; 128 x 256 tiles 0.63 .. 0.73 us (the unpacking, which
 // bounds them, is the same as for 256 rows); 256 x 128 tiles 0.72.  Two 128 x 128 tiles share a compute unit, except
-// with 64 KB of palettes: 0.57 us for a few of them, 0.75 us with one on every compute unit, 1.0 us for both of a pair.
+// with per-row palettes of 128 or 256 entries, 32 or 64 KB beside the other 56: 0.57 us for a few of them, 0.75 us with
+// one on every compute unit, 1.0 us for both of a pair; rounds of one with 7-bit per-row palettes 0.70 (0.54 .. 0.87 over
+// K and nib).
 // A workgroup spends 7 us outside its K loop.  Cutting costs the launch that zeroes the counters and, for each level of
 // meetings, a way out and in for the sums: 2 shares of 72 tiles (36 MB) 15 us, 3 of them 29, 6 shares of 36 tiles 45.
 static double plan_cost(const TilePlan& p, int qbits, int mode, int nk) {
   const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8;
-  const bool pairs_of_tiles = p.tile == kTile128x128 && !(mode == kPalRow && qbits == 8);
+  const bool pairs_of_tiles = p.tile == kTile128x128 && !(mode == kPalRow && wide);
   // one workgroup's K-tile with the share `busy` of the compute units at work
   const auto k_tile = [&](double busy) -> double {
     switch (p.tile) {
@@ -251,6 +253,7 @@ static double plan_cost(const TilePlan& p, int qbits, int mode, int nk) {
       return std::max(rounds * both, k_tile(std::min(1.0, 2 * rounds))) * kt + 7.0 * std::ceil(rounds);
     }
     const int64_t full = n / kDenseCUs, rest = n % kDenseCUs;
+    if (full && p.tile == kTile128x128 && qbits == 7) return ((double)full + (rest ? 1 : 0)) * (kt * 0.70 + 7.0);
     return (double)full * (kt * k_tile(1.0) + 7.0) + (rest ? kt * k_tile((double)rest / kDenseCUs) + 7.0 : 0.0);
   };
   if (p.split == 1) return time(p.tiles, nk);

@@ -71,6 +71,23 @@ def test_key_split_room_beside_full_rounds(dthip, monkeypatch):
     assert ws(33, 64, 2000) == 256 + 8 * 8 * slot(64)
 
 
+def test_dense_tiles_that_cannot_share_a_compute_unit_are_cut(dthip, monkeypatch):
+    """Two 128 x 128 tiles with per-row palettes of 128 entries (88 KB of LDS each) do not run side by side: 460 of them are
+    two rounds, where 256 x 128 tiles that are cut take three quarters of the time.  With 64 entries they do, and nothing is cut."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    addr = ctypes.addressof
+    M, K, N, nib = 590, 7936, 5888, 8192
+
+    def ws(q):
+        W = (dthip._QxWeight * 2)(*[dthip._QxWeight(4096, q, nib, N * K)] * 2)  # (addresses are not looked at)
+        Y, ldy = (ctypes.c_void_p * 2)(4096, 4096), (ctypes.c_int64 * 2)(N, N)
+        G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), 2, None, addr(Y), addr(ldy), None, None))
+        return dthip.lib().dt_dense_workspace_bytes(1, G)
+
+    assert ws(7) > 0
+    assert ws(6) == 0
+
+
 def test_missing_library_fails_loudly(dthip, monkeypatch):
     monkeypatch.setattr(dthip, "_lib", None)
     monkeypatch.setattr(dthip, "LIB_PATH", os.path.join(ROOT, "no_such_dir", "libdthip.so"))
