@@ -32,6 +32,20 @@ def check(got, X, W, bias=None):
     assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4])
 
 
+def _groups(dthip, x, ws, outs, bias=None, epi=None, post=None):
+    """One problem as the C entry points take it, and what keeps it alive."""
+    import ctypes
+
+    n, at = len(ws), ctypes.addressof
+    W = (dthip._QxWeight * n)(*[w._c() for w in ws])
+    B = (ctypes.c_void_p * n)(*[None if bias is None or b is None else b.data_ptr() for b in bias or ws])
+    Y, LDY = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs]), (ctypes.c_int64 * n)(*[o.stride(0) for o in outs])
+    tails = [None if t is None else ctypes.create_string_buffer(t, len(t)) for t in (epi, post)]
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(x.shape[0], x.shape[1], x.data_ptr(), x.stride(0), at(W), n, at(B), at(Y), at(LDY),
+                                                  *[None if t is None else at(t) for t in tails]))
+    return G, (W, B, Y, LDY, tails)
+
+
 @pytest.mark.parametrize("M,N,K,q,nib", [
     (1, 1, 1, 6, 1),            # the smallest there is: one block per weight
     (33, 31, 100, 6, 32),       # blocks that end inside a thread's run of 16
@@ -114,7 +128,8 @@ def test_lora_branch_fp32_shapes(dthip, M, K, rank, N):
     (65, 256, 128, 6, 4096), (128, 300, 192, 5, 1024),    # 128 x 256 tiles; 2 and 3 shares
     (129, 257, 320, 4, 512), (300, 600, 448, 6, 64),      # 256 x 256 tiles; 5 and 7 shares, ragged edges, a block per 64 columns
     (257, 256, 576, 8, 16384), (200, 130, 704, 16, 0),    # 8 shares of unequal length; shared palettes, plain fp16
-    (200, 140, 512, 8, 512), (130, 300, 1088, 7, 4096),   # palettes that only fit beside 256 x 128 tiles
+    (200, 140, 512, 8, 512), (130, 300, 512, 7, 512),     # palettes that only fit beside 256 x 128 tiles
+    (130, 300, 1088, 7, 4096),                            # ... and that fit beside 256 x 256 tiles, shared
 ])
 def test_dense_cut_along_k(dthip, oracle, monkeypatch, M, N, K, q, nib):
     import torch
@@ -127,8 +142,17 @@ def test_dense_cut_along_k(dthip, oracle, monkeypatch, M, N, K, q, nib):
     gamma, rot = dev((1 + 0.1 * rng.standard_normal(128)).astype(np.float16)), dev(rng.standard_normal((M + 3, 128)).astype(np.float16))
     epi = [None, dthip.HeadEpilogue(gamma, rot, 3)]
     print("dense cut along K", M, N, K, q, nib, flush=True)
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    whole = dthip.dense_multi(x, ws, [bias, None])
     monkeypatch.setenv("DT_DENSE_SPLIT", "always")
+    # every tile is cut into as many shares as there are pairs of K-tiles, up to eight, of a slot of its fp32 sums each
+    bm = 256 if M > 128 or (q == 7 and nib == 512) or (q == 8 and nib == 512) else 128
+    bn = 128 if (q == 7 and nib == 512) or (q == 8 and nib == 512) else 256
+    tiles, shares = sum(-(-M // bm) * -(-w.shape[0] // bn) for w in ws), min(8, K // 64)
+    G, keep = _groups(dthip, x, ws, [torch.empty((M, w.shape[0]), dtype=torch.float16, device="cuda") for w in ws])
+    assert dthip.lib().dt_dense_workspace_bytes(1, G) == (tiles * 32 + 255) // 256 * 256 + tiles * shares * bm * bn * 4
     outs = dthip.dense_multi(x, ws, [bias, None])
+    assert not all(torch.equal(a, b) for a, b in zip(outs, whole))  # (the sums were added up in another order)
     again = dthip.dense_multi(x, ws, [bias, None])
     check(outs[0].cpu().numpy(), X, pairs[0][1], bias.cpu().numpy())
     check(outs[1].cpu().numpy(), X, pairs[1][1])
@@ -138,7 +162,7 @@ def test_dense_cut_along_k(dthip, oracle, monkeypatch, M, N, K, q, nib):
     want = res + (outs[0].float() * gate.float()).half().float()
     dthip.dense_post(x, ws, [bias, None], [dthip.DensePost(gate=gate, residual=res, keep_output=False), None])
     assert torch.equal(res, want)
-    if q == 16 or K * 2 ** q * 2 * 256 // nib <= 32768 or q <= 6:  # (the head epilogue's tiles are 256 wide)
+    if bn == 256:  # (the head epilogue's tiles are 256 wide)
         fused = dthip.dense_multi(x, ws, [bias, None], epilogues=epi)
         lead = dthip.dense_multi(x, ws, [bias, None])[1]
         assert torch.equal(fused[0], outs[0])
@@ -205,17 +229,6 @@ def test_dense_shared_palettes_of_64(dthip, oracle, M, N, K, nib):
     check(got[torch.from_numpy(rows).cuda()].cpu().numpy(), X[rows], W)
 
 
-def _groups(dthip, x, w, out):
-    """One problem as the C entry points take it, and what keeps it alive."""
-    import ctypes
-
-    W = (dthip._QxWeight * 1)(w._c())
-    Y, LDY = (ctypes.c_void_p * 1)(out.data_ptr()), (ctypes.c_int64 * 1)(out.stride(0))
-    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(x.shape[0], x.shape[1], x.data_ptr(), x.stride(0), ctypes.addressof(W), 1, None,
-                                                  ctypes.addressof(Y), ctypes.addressof(LDY), None, None))
-    return G, (W, Y, LDY)
-
-
 def test_dense_workspace_is_optional(dthip, oracle, monkeypatch):
     """A launch of few tiles is cut without being told to; too little workspace, or none, gives the uncut result, a
     misaligned one is refused; and a captured graph replays the cut launch, its counters zeroed each time."""
@@ -226,7 +239,7 @@ def test_dense_workspace_is_optional(dthip, oracle, monkeypatch):
     X = rng.standard_normal((300, 3072)).astype(np.float16)
     w, W = make(dthip, oracle, rng, 512, 3072, 6, 4096)
     x, out = dev(X), torch.zeros((300, 512), dtype=torch.float16, device="cuda")
-    G, keep = _groups(dthip, x, w, out)
+    G, keep = _groups(dthip, x, [w], [out])
     L, s = dthip.lib(), torch.cuda.current_stream().cuda_stream
     need = L.dt_dense_workspace_bytes(1, G)
     assert need > 0
@@ -254,6 +267,54 @@ def test_dense_workspace_is_optional(dthip, oracle, monkeypatch):
         assert L.dt_dense_qx_grouped_ws_f16(s, 1, G, 0, ws.data_ptr(), need) == 0
 
 
+@pytest.mark.parametrize("M,q,nib", [(5, 6, 4096), (70, 6, 4096), (1100, 8, 16384), (70, 16, 0), (300, 6, 24)])
+def test_dense_c_entry_points_without_workspace(dthip, oracle, monkeypatch, M, q, nib):
+    """The Dense entry points that take no workspace do what the operators, which go through the one that takes it, do when
+    nothing is cut: bit for bit, plain, with head epilogues, with tails, and as a group."""
+    import ctypes
+
+    import torch
+
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    rng = np.random.default_rng(M + q)
+    K, N = 320, 256
+    x = dev(rng.standard_normal((M, K)).astype(np.float16))
+    ws = [make(dthip, oracle, rng, N, K, q, nib)[0] for _ in range(2)]
+    bias = [dev((rng.standard_normal(N) * 0.1).astype(np.float16)), None]
+    gamma, rot = dev((1 + 0.1 * rng.standard_normal(128)).astype(np.float16)), dev(rng.standard_normal((M, 128)).astype(np.float16))
+    epi = [dthip.HeadEpilogue(gamma, rot), None]
+    gate, res0 = dev((1 + 0.3 * rng.standard_normal(N)).astype(np.float16)), dev(rng.standard_normal((M, N)).astype(np.float32))
+    res = [res0.clone(), res0.clone()]
+    posts = [[dthip.DensePost(dthip.ACT_GELU_TANH, gate=gate, residual=r), dthip.DensePost(scale=0.5)] for r in res]
+    want = [dthip.dense_multi(x, ws, bias), dthip.dense_multi(x, ws, bias, epilogues=epi), dthip.dense_post(x, ws, bias, posts[0])]
+    L, s = dthip.lib(), torch.cuda.current_stream().cuda_stream
+    new = lambda: [torch.zeros((M, N), dtype=torch.float16, device="cuda") for _ in ws]
+    packed_epi = dthip._pack_epilogues(epi, M)
+    print("dense entry points without workspace", M, q, nib, flush=True)
+
+    def call(fn, outs, *tail):
+        (g,), keep = _groups(dthip, x, ws, outs, bias)
+        W, B, Y, LDY, _ = keep
+        return fn(s, g.M, g.K, g.X, g.ldx, W, g.n_weights, B, Y, LDY, *tail, 0)
+
+    outs = new()
+    assert call(L.dt_dense_qx_f16, outs) == 0
+    assert all(torch.equal(a, b) for a, b in zip(outs, want[0]))
+    outs, held = new(), ctypes.create_string_buffer(packed_epi, len(packed_epi))
+    assert call(L.dt_dense_qx_heads_f16, outs, ctypes.cast(held, L.dt_dense_qx_heads_f16.argtypes[10])) == 0
+    assert all(torch.equal(a, b) for a, b in zip(outs, want[1]))
+    outs = new()
+    packed_post = dthip._pack_posts(posts[1], ws, M, [o.data_ptr() for o in outs], list(outs))
+    held = ctypes.create_string_buffer(packed_post, len(packed_post))
+    assert call(L.dt_dense_qx_post_f16, outs, ctypes.cast(held, L.dt_dense_qx_post_f16.argtypes[10])) == 0
+    assert all(torch.equal(a, b) for a, b in zip(outs, want[2])) and torch.equal(res[0], res[1])
+    for kind, tails in enumerate([{}, {"epi": packed_epi}]):
+        outs = new()
+        G, keep = _groups(dthip, x, ws, outs, bias, **tails)
+        assert L.dt_dense_qx_grouped_f16(s, 1, G, 0) == 0
+        assert all(torch.equal(a, b) for a, b in zip(outs, want[kind]))
+
+
 def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     """288 tiles: 256 stay whole, the 32 of the second round are cut; against the uncut launch, one fp16 rounding apart."""
     import torch
@@ -265,7 +326,7 @@ def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     monkeypatch.setenv("DT_DENSE_SPLIT", "never")
     whole = dthip.dense_multi(x, [w], [None])[0].float()
     monkeypatch.delenv("DT_DENSE_SPLIT")
-    G, keep = _groups(dthip, x, w, torch.empty((M, N), dtype=torch.float16, device="cuda"))
+    G, keep = _groups(dthip, x, [w], [torch.empty((M, N), dtype=torch.float16, device="cuda")])
     print("dense last round cut along K", flush=True)
     assert dthip.lib().dt_dense_workspace_bytes(1, G) > 0
     cut = dthip.dense_multi(x, [w], [None])[0].float()
@@ -346,7 +407,7 @@ def test_optional_scratch_is_not_insisted_on(dthip, oracle, monkeypatch, kind):
         M, K, N = 512, 5120, 5120
         w, _ = make(dthip, oracle, rng, N, K, 6, 4096)
         x, out = dev(rng.standard_normal((M, K)).astype(np.float16)), torch.empty((M, N), dtype=torch.float16, device="cuda")
-        need = L.dt_dense_workspace_bytes(1, _groups(dthip, x, w, out)[0])
+        need = L.dt_dense_workspace_bytes(1, _groups(dthip, x, [w], [out])[0])
         call = lambda: dthip.dense_multi(x, [w], [None], outs=[out])
     else:
         B, S, H, D = 1, 1500, 4, 128
