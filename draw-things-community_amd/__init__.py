@@ -446,7 +446,7 @@ def _scratch(like, need, least):
     return _scratch(like, least, least)
 
 
-def _enqueue_dense(fn, problems, flags, stream):
+def _enqueue_dense(problems, flags, stream):
     """Enqueues Dense problems -- (x, weights, biases, outs, epilogues, posts) each -- together, with the scratch memory
     that lets the library cut tiles along K where there are too few of them for the chip.  Returns their outputs."""
     packed = [_marshal_dense(*p) for p in problems]
@@ -454,7 +454,7 @@ def _enqueue_dense(fn, problems, flags, stream):
     n, L = len(packed), lib()
     need = L.dt_dense_workspace_bytes(n, groups) if any(M > _ROWS_MAX for _, _, _, M in packed) else 0
     ws, at, need = _scratch(problems[0][0], need, 0)
-    _check(fn, L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, at, need))
+    _check("dt_dense_qx_grouped_ws_f16", L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, at, need))
     return [_shape_outs(p[0], M, outs, p[3] is None) for p, (_, _, outs, M) in zip(problems, packed)]
 
 
@@ -470,8 +470,7 @@ def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object
     """Several Dense ops that share the input, one launch (x_q / x_k / x_v).  `epilogues[i]` (optional) fuses the
     per-head RMSNorm / RoPE that follows projection i."""
     with _on(stream):
-        fn = "dt_dense_qx_f16" if epilogues is None else "dt_dense_qx_heads_f16"
-        return _enqueue_dense(fn, [(x, weights, biases, outs, epilogues, None)], flags, stream)[0]
+        return _enqueue_dense([(x, weights, biases, outs, epilogues, None)], flags, stream)[0]
 
 
 ACT_NONE, ACT_GELU_TANH, ACT_SWISH, ACT_GELU_ERF = 0, 1, 2, 3
@@ -551,7 +550,7 @@ def dense_post(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]
     linear1 -> GELU and the gated residual additions of a transformer block).  Returns the fp16 outputs (None where
     a projection only accumulates into its residual)."""
     with _on(stream):
-        return _enqueue_dense("dt_dense_qx_post_f16", [(x, weights, biases, outs, None, posts)], flags, stream)[0]
+        return _enqueue_dense([(x, weights, biases, outs, None, posts)], flags, stream)[0]
 
 
 def dense_grouped(problems: Sequence[dict], flags: int = 0, stream=None):
@@ -562,9 +561,8 @@ def dense_grouped(problems: Sequence[dict], flags: int = 0, stream=None):
     if not problems:
         return []
     with _on(stream):
-        return _enqueue_dense("dt_dense_qx_grouped_f16",
-                              [(p["x"], p["weights"], p["biases"], p.get("outs"), p.get("epilogues"), p.get("posts")) for p in problems],
-                              flags, stream)
+        return _enqueue_dense([(p["x"], p["weights"], p["biases"], p.get("outs"), p.get("epilogues"), p.get("posts"))
+                               for p in problems], flags, stream)
 
 
 class Dense:

@@ -441,3 +441,11 @@ def test_optional_scratch_is_not_insisted_on(dthip, oracle, monkeypatch, kind):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(out, whole)
+
+
+def test_refused_dense_names_the_call_that_was_made(dthip, oracle):
+    rng = np.random.default_rng(4)
+    w = make(dthip, oracle, rng, 260, 64, 6, 4096)[0]
+    x, gamma = dev(rng.standard_normal((5, 64)).astype(np.float16)), dev(np.ones(130, np.float16))
+    with pytest.raises(dthip.DtError, match="dt_dense_qx_grouped_ws_f16"):
+        dthip.dense_multi(x, [w], [None], epilogues=[dthip.HeadEpilogue(gamma, head_dim=130)])
