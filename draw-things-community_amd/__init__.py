@@ -427,7 +427,10 @@ def _marshal_dense(x, weights, biases, outs, epilogues, posts):
     return (x2, arrays), group, outs, M
 
 
-_ROWS_MAX = 64  # rows up to which the library streams the weights and needs no workspace
+# Rows up to which the library streams the weights (kRowsMax in csrc/dt_dense_rows.h) and uses no workspace, so that it is
+# not asked how much (0.5 us of a conditioning row's 22).  The few such calls that it gives to the tiled kernel after all
+# -- plain fp16 weights with over 16 rows and 8192 features, palettes that do not fit the LDS -- run uncut from here.
+_ROWS_MAX = 64
 
 
 def _scratch(like, need, least):
@@ -609,7 +612,7 @@ class LoRADense:
 
     def _padded(self):
         """The pair with the rank padded by zero rows / columns to the tiled kernel's K granule (64): the zeros add
-        nothing, so the results are the same bit for bit, and the up projection avoids the slow any-shape kernel."""
+        nothing, so the results are the same bit for bit, and the up projection avoids the any-shape kernel."""
         # keyed on the identity of the pair's tensors (held here, so that their addresses cannot be handed to other
         # tensors while the cache lives), their in-place modification counters, the rank and the count
         src = (self.down.data, self.up.data)

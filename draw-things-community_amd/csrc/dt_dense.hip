@@ -10,7 +10,9 @@
 //
 // Tile: BM x BN outputs per 512-thread workgroup (8 waves, two per SIMD, each
 // a BN/2 x BM/4 slice), K-tiles of 32 processed in pairs; one barrier per K-tile
-// (per pair with plain fp16 weights, which no wave writes to LDS itself).
+// (per pair with plain fp16 weights, which no wave writes to LDS itself).  Transfers
+// from memory are waited for once per K-tile, on the 128 x 128 tile with
+// palettes in LDS and with plain fp16 weights once per pair.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -219,6 +221,8 @@ struct TilePlan {
   size_t bytes() const { return split > 1 ? counter_bytes() + (size_t)((tiles - whole) * split * dense_split_slot_bytes(BM, BN)) : 0; }
 };
 
+// Compute units of the whole card, on which the costs below were measured (part of one would need costs of its own; the
+// results do not depend on the layout chosen beyond the order of the sums).
 constexpr int kDenseCUs = 256;
 // Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
 constexpr int64_t kFillTiles = 192;
@@ -365,10 +369,6 @@ static int weight_run(const HostGroup& h, int i, bool* fused) {
   return end;
 }
 
-// One validated problem with M > 0: weights that share (qbits, nib) and meet the
-// tiled kernel's alignment go out in runs of up to kMaxWeights per launch; the
-// rest take the any-shape kernel.
-
 // Scratch memory of a call, or none.
 struct Workspace {
   uint8_t* ptr = nullptr;
@@ -396,6 +396,10 @@ static dt_status launch_plan(hipStream_t s, DenseArgs& a, const TilePlan& plan, 
   return launch_dense(s, a, plan.tile, qbits, mode);
 }
 
+// One validated problem with M > 0: weights that share (qbits, nib) and meet the
+// tiled kernel's alignment go out in runs of up to kMaxWeights per launch, of the
+// kernel that streams the weights where X has few rows, else of the tiled one; the
+// rest take the any-shape kernel.
 static dt_status run_group(hipStream_t s, const HostGroup& h, const Workspace& ws) {
   const int64_t M = h.M, K = h.K;
   const bool x_ok = h.x_ok();

@@ -517,8 +517,8 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   static_assert(NS == 2 || (MODE == kPlainF16 && NS > 2 && (NS - 1) * (AP + BP) < 16), "pair slots");
 
   // One LDS array, carved up by hand so that the epilogue can reuse all of it.  The palettes come first:
-  // their addresses then fit an instruction offset.  X (and a plain fp16 W) lives in two pair slots, each
-  // holding two K-tiles as [rows][64 halfs]: one is read while the next pair is in flight into the other.
+  // their addresses then fit an instruction offset.  X (and a plain fp16 W) lives in NS pair slots, each
+  // holding two K-tiles as [rows][64 halfs]: one is read while the next pairs are in flight into the others.
   constexpr bool HAS_PAL = MODE == kPalShared || MODE == kPalRow;
   constexpr int PAL_BYTES = MODE == kPalRow ? BN << (Q + 1) : HAS_PAL ? pal_lds_bytes(BM, BN, MODE) : 0;
   constexpr int XS_BYTES = BM * PROW * 2;

@@ -88,6 +88,14 @@ def test_dense_tiles_that_cannot_share_a_compute_unit_are_cut(dthip, monkeypatch
     assert ws(6) == 0
 
 
+def test_rows_that_need_no_workspace(dthip):
+    """The operators do not ask for workspace up to the rows that the library's streaming kernel takes: one number, twice."""
+    import re
+
+    header = open(os.path.join(ROOT, "draw-things-community_amd", "csrc", "dt_dense_rows.h")).read()
+    assert dthip._ROWS_MAX == int(re.search(r"kRowsMax = (\d+);", header).group(1))
+
+
 def test_missing_library_fails_loudly(dthip, monkeypatch):
     monkeypatch.setattr(dthip, "_lib", None)
     monkeypatch.setattr(dthip, "LIB_PATH", os.path.join(ROOT, "no_such_dir", "libdthip.so"))
