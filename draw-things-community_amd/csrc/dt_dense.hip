@@ -45,24 +45,30 @@ static dt_status launch_dense(hipStream_t s, const DenseArgs& a, int tile, int q
   return DT_INVALID;
 }
 
-// Palette placement for a BN-row tile (see PalMode).
-static int choose_pal_mode(int qbits, int nib, int64_t K, int BM, int BN) {
+constexpr int kDenseCUs = 256;  // compute units of the whole card
+
+// Palette placement for a BN-row tile (see PalMode) in a launch of `tiles` of them (0: of more than the compute units).
+static int choose_pal_mode(int qbits, int nib, int64_t K, int BM, int BN, int64_t tiles = 0) {
   if (qbits == 16) return kPlainF16;
   const int64_t pal_bytes = (int64_t)2 << qbits;
   const int64_t shared_count = ((int64_t)BN * K) / nib + 2;
   const bool row = (int64_t)BN * pal_bytes <= pal_lds_bytes(BM, BN, kPalRow);
   const bool shared = !(BM == 256 && BN == 128) && shared_count * pal_bytes <= pal_lds_bytes(BM, BN, kPalShared);
   // a per-row table has no bank conflicts, but 128- and 256-entry palettes make one of 32 or 64 KB: the 128 x 128 tile
-  // takes it only where the palettes of its blocks would not fit the 24 KB that let two workgroups share a compute unit
+  // takes it where the palettes of its blocks would not fit the 24 KB that let two workgroups share a compute unit, and
+  // where there is none to share with and rows enter new blocks at every 16th K-tile at most (us, shared / per row, 250
+  // tiles: q7p K = 1024 27.5 / 25.2, 1536 37.7 / 35.2, 2048 48.5 / 42.1, 4096 89.0 / 76.5; q8p 27.2 / 25.6, 37.3 / 37.0,
+  // 47.6 / 42.7, 87.5 / 76.0; at every 8th, K = 1792, q7p 43.2 / 42.9, q8p 42.7 / 46.4; 512 tiles, which do share, K = 2048
+  // q8p 62.9 / 80.4)
   const bool small = BM == 128 && BN == 128;
-  if (shared && small && qbits >= 7) return kPalShared;
+  const int64_t step = std::gcd(K, (int64_t)nib) / BK;
+  if (shared && small && qbits >= 7 && (tiles == 0 || tiles > kDenseCUs || step < 16)) return kPalShared;
   // And where some row may enter a new block at every second K-tile (K an odd multiple of 64), that check, its barrier
   // and the 64 entries to rewrite cost more than conflicts do (us, per row / shared: 8192 x 320 -> 960 19.1 / 17.7,
   // 4608 x 960 -> 3072 48.0 / 42.8, 2048 x 1344 -> 4096 51.5 / 43.8, on 128 x 128 tiles 2016 x 1600 -> 1280 42.6 / 35.8);
   // at every fourth they are even on the small tile (4096 x 640 -> 640 17.9 / 17.5), at every eighth the table is
   // ahead (2016 x 1280 -> 1280 28.2 / 29.8).  Palettes of 16 and 32 entries are rewritten fast enough (4096 x 320 ->
   // 1280: q5p 16.5 / 16.4, q4p 16.2 / 16.4).
-  const int64_t step = std::gcd(K, (int64_t)nib) / BK;
   if (shared && qbits == 6 && (small ? step <= 4 : BN == 256 && step <= 2)) return kPalShared;
   if (row) return kPalRow;
   if (shared) return kPalShared;
@@ -221,14 +227,12 @@ struct TilePlan {
   size_t bytes() const { return split > 1 ? counter_bytes() + (size_t)((tiles - whole) * split * dense_split_slot_bytes(BM, BN)) : 0; }
 };
 
-// Compute units of the whole card, on which the costs below were measured (part of one would need costs of its own; the
-// results do not depend on the layout chosen beyond the order of the sums).
-constexpr int kDenseCUs = 256;
 // Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
 constexpr int64_t kFillTiles = 192;
 constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
 
-// Estimated time (us) of a launch, from what this part measures.  Per K-tile and workgroup: 256 x 256 tiles 0.80 us
+// Estimated time (us) of a launch, from what the whole card measures (part of one would need costs of its own; the
+// results do not depend on the layout chosen beyond the order of the sums).  Per K-tile and workgroup: 256 x 256 tiles 0.80 us
 // while a third of the compute units work and 1.02 us when all do (the card is limited as a whole), 7 % more with 7-
 // and 8-bit palettes, a third less with plain fp16 weights; 128 x 256 tiles 0.63 .. 0.73 us (the unpacking, which
 // bounds them, is the same as for 256 rows); 256 x 128 tiles 0.72.  Two 128 x 128 tiles share a compute unit, except
@@ -324,7 +328,7 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   const bool brief = w0.qbits == 16 && K <= 128;
   const bool big = (((m_max >= 1024) && (n_max >= 256) && t256.tiles >= kFillTiles) && pal_fits_big && !brief) || wide;
   TilePlan base = big ? (m_max < 1024 ? tnarrow : t256) : (!pal_fits_big && tall_ok && m_max >= 1024 && n_max >= 128 && t256.tiles * 2 >= kFillTiles) ? ttall : tsmall;
-  const auto pal_mode = [&](const TilePlan& p) { return choose_pal_mode(w0.qbits, w0.qbits == 16 ? 32 : w0.nib, K, p.BM, p.BN); };
+  const auto pal_mode = [&](const TilePlan& p) { return choose_pal_mode(w0.qbits, w0.qbits == 16 ? 32 : w0.nib, K, p.BM, p.BN, p.tiles); };
   // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate, whose error
   // is up to a tenth, sees a clear gain.
   const char* knob = getenv("DT_DENSE_SPLIT");  // "never" | "always" (as often as can be; for tests); read at every call
@@ -491,7 +495,7 @@ static dt_status run_group(hipStream_t s, const HostGroup& h, const Workspace& w
     if ((int64_t)g.tiles_m * tiles_n > 0x7fffffff) return DT_NO_KERNEL;
     a.total_tiles = g.tiles_m * tiles_n;
     finish_args(a, 1, cnt, K, w0);
-    const int mode = choose_pal_mode(w0.qbits, a.nib, K, BM, BN);
+    const int mode = choose_pal_mode(w0.qbits, a.nib, K, BM, BN, plan.tiles);
     dt_status st = launch_plan(s, a, plan, ws, w0.qbits, mode);
     if (st != DT_OK) return st;
     for (int j = first; j < i; j++)

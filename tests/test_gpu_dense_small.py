@@ -229,6 +229,25 @@ def test_dense_shared_palettes_of_64(dthip, oracle, M, N, K, nib):
     check(got[torch.from_numpy(rows).cuda()].cpu().numpy(), X[rows], W)
 
 
+@pytest.mark.parametrize("K,q", [(512, 7), (1024, 8), (1536, 7), (2048, 8)])
+def test_dense_row_palettes_on_a_unit_of_ones_own(dthip, oracle, monkeypatch, K, q):
+    """128 x 128 tiles with 128- and 256-entry palettes: up to 256 of them look every row's palette up in a table of its
+    own, more share the palettes with a neighbour.  The same bits, at ragged edges of either; and against the oracle."""
+    import torch
+
+    rng = np.random.default_rng(K + q)
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")  # (a cut tile's sums are added up in another order)
+    nib = {7: 8192, 8: 16384}[q]
+    N, few, many = 2433, 200, 1790  # 2 and 14 tiles by 20: 40 and 280
+    X = rng.standard_normal((many, K)).astype(np.float16)
+    w, W = make(dthip, oracle, rng, N, K, q, nib)
+    x = dev(X)
+    print("dense row palettes", K, q, flush=True)
+    got = dthip.dense_multi(x[:few], [w], [None])[0]
+    assert torch.equal(got, dthip.dense_multi(x, [w], [None])[0][:few])
+    check(got[150:].cpu().numpy(), X[150:few], W)
+
+
 def test_dense_workspace_is_optional(dthip, oracle, monkeypatch):
     """A launch of few tiles is cut without being told to; too little workspace, or none, gives the uncut result, a
     misaligned one is refused; and a captured graph replays the cut launch, its counters zeroed each time."""
