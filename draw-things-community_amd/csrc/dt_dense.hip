@@ -47,6 +47,9 @@ static dt_status launch_dense(hipStream_t s, const DenseArgs& a, int tile, int q
 
 constexpr int kDenseCUs = 256;  // compute units of the whole card
 
+// K-tiles from one at which rows may enter new blocks to the next.
+static int64_t pal_step(int64_t K, int nib) { return std::gcd(K, (int64_t)nib) / BK; }
+
 // Palette placement for a BN-row tile (see PalMode) in a launch of `tiles` of them (0: of more than the compute units).
 static int choose_pal_mode(int qbits, int nib, int64_t K, int BM, int BN, int64_t tiles = 0) {
   if (qbits == 16) return kPlainF16;
@@ -61,7 +64,7 @@ static int choose_pal_mode(int qbits, int nib, int64_t K, int BM, int BN, int64_
   // 47.6 / 42.7, 87.5 / 76.0; at every 8th, K = 1792, q7p 43.2 / 42.9, q8p 42.7 / 46.4; 512 tiles, which do share, K = 2048
   // q8p 62.9 / 80.4)
   const bool small = BM == 128 && BN == 128;
-  const int64_t step = std::gcd(K, (int64_t)nib) / BK;
+  const int64_t step = pal_step(K, nib);
   if (shared && small && qbits >= 7 && (tiles == 0 || tiles > kDenseCUs || step < 16)) return kPalShared;
   // And where some row may enter a new block at every second K-tile (K an odd multiple of 64), that check, its barrier
   // and the 64 entries to rewrite cost more than conflicts do (us, per row / shared: 8192 x 320 -> 960 19.1 / 17.7,
@@ -212,7 +215,7 @@ static void finish_args(DenseArgs& a, int n_groups, int n_w, int64_t K, const dt
   a.n_groups = n_groups;
   a.k = (int32_t)K;
   a.nib = w0.qbits == 16 ? 32 : w0.nib;
-  a.pal_step = (int32_t)(std::gcd((int64_t)K, (int64_t)a.nib) / BK);
+  a.pal_step = (int32_t)pal_step(K, a.nib);
 }
 
 // How a launch of the tiled kernel is laid out: its tile and, where the tiles do not fill the compute units evenly, how
@@ -231,61 +234,64 @@ struct TilePlan {
 constexpr int64_t kFillTiles = 192;
 constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
 
-// Estimated time (us) of a launch, from what the whole card measures (part of one would need costs of its own; the
-// results do not depend on the layout chosen beyond the order of the sums).  Per K-tile and workgroup: 256 x 256 tiles 0.80 us
-// while a third of the compute units work and 1.02 us when all do (the card is limited as a whole), 7 % more with 7-
-// and 8-bit palettes, a third less with plain fp16 weights; 128 x 256 tiles 0.63 .. 0.73 us (the unpacking, which
-// bounds them, is the same as for 256 rows); 256 x 128 tiles 0.72.  Two 128 x 128 tiles share a compute unit, except
-// with per-row palettes of 128 or 256 entries, 32 or 64 KB beside the other 56: 0.57 us for a few of them, 0.75 us with
-// one on every compute unit, 1.0 us for both of a pair; rounds of one with 7-bit per-row palettes 0.70 (0.54 .. 0.87 over
-// K and nib).
-// A workgroup spends 7 us outside its K loop.  Cutting costs the launch that zeroes the counters and, for each level of
-// meetings, a way out and in for the sums: 2 shares of 72 tiles (36 MB) 15 us, 3 of them 29, 6 shares of 36 tiles 45.
-static double plan_cost(const TilePlan& p, int qbits, int mode, int nk) {
-  const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8;
-  const bool pairs_of_tiles = p.tile == kTile128x128 && !(mode == kPalRow && wide);
+// Estimated time (us) of a launch whose rows enter new blocks at every `step`-th K-tile at most: a fit to 930 launches of
+// 65 .. 4000 rows on the whole card (part of one would need costs of its own; the results do not depend on the layout
+// chosen beyond the order of the sums), nine tenths of them within a tenth.  Priced are: one workgroup's K-tile on each
+// tile shape, the cheaper the more compute units idle (the card is limited as a whole); what entering new blocks adds to it
+// where every row has a table of its own to rewrite, most for 128 and 256 entries; the time outside the K loop; two
+// 128 x 128 tiles that share a compute unit, except with per-row tables of 32 or 64 KB beside the other 56, which take it in
+// turns; and cutting: the launch that zeroes the counters and, for each level of meetings, a way out and in for the sums.
+// (us, uncut / cut: 512 x 5120 -> 2 x 5120 q5p 126 / 82, 128 x 5120 -> 1152 q8p 92 / 37; and left whole because of these
+// terms: 3 x (571 x 4288 -> 7872) q7p 251 / 342, 1000 x 1792 -> 4096 q7p 42 / 48, 721 x 7168 -> 2560 fp16 46 / 52.)
+static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t step) {
+  const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8, row = mode == kPalRow;
+  const double entering = row ? (wide ? 0.70 : 0.33) / (double)step : 0.0;
   // one workgroup's K-tile with the share `busy` of the compute units at work
   const auto k_tile = [&](double busy) -> double {
     switch (p.tile) {
-      case kTile256x256: return plain ? 0.58 + 0.14 * busy : (0.72 + 0.30 * busy) * (wide ? 1.07 : 1.0);
-      case kTile128x256: return plain ? 0.42 + 0.08 * busy : (0.61 + 0.12 * busy) * (wide ? 1.2 : 1.0);
-      case kTile128x128: return plain ? 0.28 + 0.06 * busy : (0.53 + 0.22 * busy) * (wide ? 1.15 : 1.0);
+      case kTile256x256: return plain ? 0.37 + 0.44 * busy : (wide ? 0.71 + 0.47 * busy : 0.73 + 0.27 * busy) + entering;
+      case kTile128x256: return plain ? 0.28 + 0.14 * busy : wide ? 0.85 + 0.10 * busy : (row ? 0.60 : 0.78) + 0.17 * busy + entering;
+      case kTile128x128: return plain ? 0.145 + 0.09 * busy : row ? 0.49 + 0.06 * busy + entering : wide ? 0.575 + 0.065 * busy : 0.56 + 0.09 * busy;
     }
-    return 0.72;
+    return 0.51 + 0.195 * busy + entering;
   };
+  const double outside = p.tile == kTile256x256 ? 11.3 : p.tile == kTile128x128 ? 7.7 : 7.1;
+  const bool pairs_of_tiles = p.tile == kTile128x128 && !(row && wide);
   // `n` workgroups of `kt` K-tiles each
   const auto time = [&](int64_t n, int kt) -> double {
     if (n == 0) return 0.0;
-    if (pairs_of_tiles) {
-      const double rounds = (double)n / (2 * kDenseCUs), both = plain ? 0.5 : wide ? 1.15 : 1.0;
-      return std::max(rounds * both, k_tile(std::min(1.0, 2 * rounds))) * kt + 7.0 * std::ceil(rounds);
+    if (pairs_of_tiles && n > kDenseCUs) {
+      const double both = (plain ? 0.54 : wide ? 0.97 : 0.90) + entering, gap = plain ? 0.095 : wide ? 0.24 : 0.20;
+      const int64_t full = n / (2 * kDenseCUs), rest = n % (2 * kDenseCUs);
+      const double last = both * (double)rest / (2 * kDenseCUs);
+      if (full == 0) return std::max(k_tile(1.0) + gap, last) * kt + outside;
+      return ((double)full * both + (rest ? std::max(0.35 * both, last) : 0.0)) * kt + outside * (double)(full + (rest ? 1 : 0));
     }
     const int64_t full = n / kDenseCUs, rest = n % kDenseCUs;
-    if (full && p.tile == kTile128x128 && qbits == 7) return ((double)full + (rest ? 1 : 0)) * (kt * 0.70 + 7.0);
-    return (double)full * (kt * k_tile(1.0) + 7.0) + (rest ? kt * k_tile((double)rest / kDenseCUs) + 7.0 : 0.0);
+    return (double)full * (kt * k_tile(1.0) + outside) + (rest ? kt * k_tile((double)rest / kDenseCUs) + outside : 0.0);
   };
   if (p.split == 1) return time(p.tiles, nk);
   const int64_t shares = (p.tiles - p.whole) * p.split;
   const int levels = p.split > 4 ? 3 : p.split > 2 ? 2 : 1;
   const double mb = 1e-6 * (double)(shares * dense_split_slot_bytes(p.BM, p.BN));
-  return time(p.whole, nk) + time(shares, 2 * ((nk / 2 + p.split - 1) / p.split)) + 5.0 + levels * (5.0 + 0.15 * mb);
+  return time(p.whole, nk) + time(shares, 2 * ((nk / 2 + p.split - 1) / p.split)) + 5.0 + levels * (3.5 + 0.095 * mb);
 }
 
 // The best way to cut tiles of `base`'s shape that `ws_bytes` of workspace allow: all of them, or those of the last,
 // unfilled round of workgroups.
-static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, size_t ws_bytes, double* cost) {
+static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, int64_t step, size_t ws_bytes, double* cost) {
   TilePlan best = base;
   best.split = 1;
   best.whole = base.tiles;
-  *cost = plan_cost(best, qbits, mode, nk);
+  *cost = plan_cost(best, qbits, mode, nk, step);
   for (int s = 2; s <= kMaxSplit && nk / s >= 8; s++)
     for (const int64_t whole : {(int64_t)0, base.tiles / kDenseCUs * kDenseCUs}) {
       TilePlan p = base;
       p.split = s;
       p.whole = whole;
       if (p.whole >= p.tiles || p.bytes() > ws_bytes || p.bytes() > kDenseMaxWorkspace) continue;
-      const double t = plan_cost(p, qbits, mode, nk);
-      if (t < *cost) {
+      const double t = plan_cost(p, qbits, mode, nk, step);
+      if (t < (best.split > 1 ? 0.97 : 1.0) * *cost) {  // (a finer cut, of more memory, has to be worth it)
         *cost = t;
         best = p;
       }
@@ -341,11 +347,12 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
     return p.split > 1 && p.bytes() <= std::min(ws_bytes, kDenseMaxWorkspace) ? p : base;
   }
   TilePlan best = base;
-  const double start = plan_cost(base, w0.qbits, pal_mode(base), nk);
-  double least = std::min(0.92 * start, start - 8.0);
+  const int64_t step = pal_step(K, w0.qbits == 16 ? 32 : w0.nib);
+  const double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step);
+  double least = std::min(0.92 * start, start - 4.0);
   const auto consider = [&](const TilePlan& shape) {
     double t;
-    const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, ws_bytes, &t);
+    const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, step, ws_bytes, &t);
     if (t < least) {
       least = t;
       best = p;

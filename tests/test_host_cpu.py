@@ -88,6 +88,24 @@ def test_dense_tiles_that_cannot_share_a_compute_unit_are_cut(dthip, monkeypatch
     assert ws(6) == 0
 
 
+@pytest.mark.parametrize("M,K,N,n,q,nib,cut", [
+    (571, 4288, 7872, 3, 7, 8192, False),   # 256 x 128 tiles would rewrite their palettes at every other K-tile: 342 us against 251
+    (1000, 1792, 4096, 1, 7, 8192, False),  # 48 against 42
+    (721, 7168, 2560, 1, 16, 0, False),     # plain fp16 weights on four pair slots: 52 against 46
+    (2391, 2688, 1600, 1, 6, 4096, False),  # 66 against 61
+    (512, 5120, 5120, 2, 5, 1024, True),    # 82 against 126
+    (128, 5120, 1152, 1, 8, 16384, True),   # 37 against 92
+])
+def test_dense_is_cut_where_that_is_faster(dthip, monkeypatch, M, K, N, n, q, nib, cut):
+    """The plan follows what cut and uncut launches measured (us at the right, cut first)."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    addr = ctypes.addressof
+    W = (dthip._QxWeight * n)(*[dthip._QxWeight(4096, q, nib, N * K)] * n)  # (addresses are not looked at)
+    Y, ldy = (ctypes.c_void_p * n)(*[4096] * n), (ctypes.c_int64 * n)(*[N] * n)
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), n, None, addr(Y), addr(ldy), None, None))
+    assert (dthip.lib().dt_dense_workspace_bytes(1, G) > 0) == cut
+
+
 def test_rows_that_need_no_workspace(dthip):
     """The operators do not ask for workspace up to the rows that the library's streaming kernel takes: one number, twice."""
     import re
