@@ -278,13 +278,13 @@ static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t 
 }
 
 // The best way to cut tiles of `base`'s shape that `ws_bytes` of workspace allow: all of them, or those of the last,
-// unfilled round of workgroups.
+// unfilled round of workgroups.  None of up to 32 K-tiles (K = 1024): a cut would gain a few us of 25 at most.
 static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, int64_t step, size_t ws_bytes, double* cost) {
   TilePlan best = base;
   best.split = 1;
   best.whole = base.tiles;
   *cost = plan_cost(best, qbits, mode, nk, step);
-  for (int s = 2; s <= kMaxSplit && nk / s >= 8; s++)
+  for (int s = 2; nk > 32 && s <= kMaxSplit && nk / s >= 8; s++)
     for (const int64_t whole : {(int64_t)0, base.tiles / kDenseCUs * kDenseCUs}) {
       TilePlan p = base;
       p.split = s;
@@ -349,7 +349,7 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   TilePlan best = base;
   const int64_t step = pal_step(K, w0.qbits == 16 ? 32 : w0.nib);
   const double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step);
-  double least = std::min(0.92 * start, start - 4.0);
+  double least = std::min(0.95 * start, start - 2.0);
   const auto consider = [&](const TilePlan& shape) {
     double t;
     const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, step, ws_bytes, &t);
