@@ -938,8 +938,10 @@ def sdpa_segments(q_segs, k_segs, v_segs, scale, gamma_q=None, gamma_k=None, rot
         _check("dt_sdpa_f16_static", st)
         return out
     need = L.dt_sdpa_workspace_bytes(B, Hq, Hk, D, Sq, Skv, int(prep), int(fused))
-    staged = sum((b + 255) // 256 * 256 for b in (prep * B * Skv * Hk * D * 2, fused * B * Sq * Hq * D * 2))
-    ws, at, need = _scratch(out, need, staged)
+    ws, at = None, None
+    if need:
+        staged = sum((b + 255) // 256 * 256 for b in (prep * B * Skv * Hk * D * 2, fused * B * Sq * Hq * D * 2))
+        ws, at, need = _scratch(out, need, staged)
     st = L.dt_sdpa_f16(_stream_ptr(stream), B, Hq, Hk, D, nq, qa, nk, ka, va, rq, rk, eps, ov, scale, wo, bo_p, at, need)
     _check("dt_sdpa_f16", st)
     return out
