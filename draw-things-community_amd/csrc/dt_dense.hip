@@ -241,7 +241,7 @@ constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
 // where every row has a table of its own to rewrite, most for 128 and 256 entries; the time outside the K loop; two
 // 128 x 128 tiles that share a compute unit, except with per-row tables of 32 or 64 KB beside the other 56, which take it in
 // turns; and cutting: the launch that zeroes the counters and, for each level of meetings, a way out and in for the sums.
-// (us, uncut / cut: 512 x 5120 -> 2 x 5120 q5p 126 / 82, 128 x 5120 -> 1152 q8p 92 / 37; and left whole because of these
+// (us, uncut / cut: 512 x 5120 -> 2 x 5120 q5p 117 / 88, 128 x 5120 -> 1152 q8p 90 / 37; and left whole because of these
 // terms: 3 x (571 x 4288 -> 7872) q7p 251 / 342, 1000 x 1792 -> 4096 q7p 42 / 48, 721 x 7168 -> 2560 fp16 46 / 52.)
 static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t step) {
   const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8, row = mode == kPalRow;
