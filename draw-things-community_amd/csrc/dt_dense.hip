@@ -3,7 +3,7 @@
 // The packed weight never exists dequantized in memory: per K-tile two threads
 // per weight row each pull half of a 32-index granule into registers, unpack
 // it, look the fp16 values up in palettes held in LDS, and write the fp16 row
-// slice into an LDS ring that v_mfma_f32_32x32x16_f16 then consumes; X (and a
+// slice into an LDS ring that v_mfma_f32_16x16x32_f16 then consumes; X (and a
 // plain fp16 weight) goes from memory straight into LDS.  fp32 accumulation,
 // one rounding to fp16, optional fused tails (per-head RMSNorm + RoPE, or
 // activation / gate / fp32 residual).

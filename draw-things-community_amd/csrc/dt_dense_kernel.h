@@ -178,14 +178,14 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 }
 
 // ---- epilogue, shared by the tiled kernels -------------------------------------------------------------------
-// acc: the wave's WN x WM slice as TN x TM blocks of 32 x 32 (rows = features, columns = tokens).  nw / mw: first
+// acc: the wave's WN x WM slice as TN x TM blocks of 16 x 16 (rows = features, columns = tokens).  nw / mw: first
 // feature (inside weight w) and first token of the slice; m_total: rows of X.  smem: the workgroup's LDS, free
 // for reuse (the caller's K loop ended with a barrier); the wave parks its slice at smem + wave * WM * WN halfs.
 template <int WN, int WM, bool POST>
-__device__ __forceinline__ void dense_epilogue(float16_t (&acc)[WN / 32][WM / 32], unsigned char* smem, int wave, int lane,
+__device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16], unsigned char* smem, int wave, int lane,
                                                int nw, int64_t mw, const DenseWeight& w, int m_total) {
-  constexpr int TN = WN / 32, TM = WM / 32;
-  const int l32 = lane & 31, hi = lane >> 5;
+  constexpr int TN = WN / 16, TM = WM / 16;
+  const int l16 = lane & 15, quad = lane >> 4;
   const bool head = WN == 128 && !POST && (w.gamma || w.rot);
   // ---- epilogue --------------------------------------------------------------
   // The K loop ended with a barrier, so its LDS tiles are free.  Every wave parks
@@ -203,14 +203,12 @@ __device__ __forceinline__ void dense_epilogue(float16_t (&acc)[WN / 32][WM / 32
   constexpr int RPI = 64 / CH;  // token rows per trip
   half_t* const park = reinterpret_cast<half_t*>(smem) + wave * (WM * WN);
   {
-    // Accumulator block (i, j): lane holds token (lane & 31) of the block and
-    // features 8 g + 4 (lane / 32) + (0..3), g = 0..3.  Chunk c of token t is
-    // parked at chunk c ^ (t % CH): the 8-byte writes of 32 tokens spread over the banks.
+    // Accumulator block (i, j): lane holds token (lane & 15) of the block and
+    // features 4 (lane / 16) + (0..3).  Chunk c of token t is parked at chunk
+    // c ^ (t % CH): the 8-byte writes of 16 tokens spread over the banks.
 #pragma unroll
-    for (int i = 0; i < TN; i++)
-#pragma unroll
-      for (int gq = 0; gq < 4; gq++) {
-        const int nn = nw + i * 32 + 8 * gq + 4 * hi;
+    for (int i = 0; i < TN; i++) {
+        const int nn = nw + i * 16 + 4 * quad;
         float b4[4] = {0.f, 0.f, 0.f, 0.f};
         if (w.bias) {
           if (nn + 3 < w.n && (reinterpret_cast<uintptr_t>(w.bias) & 7) == 0) {
@@ -227,12 +225,12 @@ __device__ __forceinline__ void dense_epilogue(float16_t (&acc)[WN / 32][WM / 32
         }
 #pragma unroll
         for (int j = 0; j < TM; j++) {
-          const int t = j * 32 + l32;
-          const uint2_t pk = {pack_h2(acc[i][j][4 * gq] + b4[0], acc[i][j][4 * gq + 1] + b4[1]),
-                              pack_h2(acc[i][j][4 * gq + 2] + b4[2], acc[i][j][4 * gq + 3] + b4[3])};
-          *reinterpret_cast<uint2_t*>(park + t * WN + (((i * 4 + gq) ^ (t & (CH - 1))) << 3) + 4 * hi) = pk;
+          const int t = j * 16 + l16;
+          const uint2_t pk = {pack_h2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]),
+                              pack_h2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
+          *reinterpret_cast<uint2_t*>(park + t * WN + (((i * 2 + (quad >> 1)) ^ (t & (CH - 1))) << 3) + 4 * (quad & 1)) = pk;
         }
-      }
+    }
   }
   // a wave's LDS operations execute in order: its reads below see the writes above
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -502,10 +500,15 @@ __device__ __forceinline__ void dense_epilogue(float16_t (&acc)[WN / 32][WM / 32
 // NS: pair slots.  Two, or more of them with plain fp16 weights: every pair then has NS - 1 pairs of K-tiles to arrive,
 // which a workgroup that has a compute unit to itself needs (128 x 128 tiles with two and with four slots: 2016 x 5120 ->
 // 1280 57.8 / 48.7 us, 4608 x 3072 -> 64 31.7 / 23.9; two tiles on a compute unit hide the latency for each other).
+//
+// Where two 128 x 128 tiles fit a compute unit's LDS, their registers have to leave room for both: four waves per SIMD.
+constexpr bool dense_two_per_cu(int Q, int BM, int BN, int mode, int NS) {
+  return BM == 128 && BN == 128 && (mode == kPalShared || (mode == kPalRow && Q <= 6) || (mode == kPlainF16 && NS == 2));
+}
 template <int Q, int BM, int BN, int MODE, bool POST, bool SPLIT, int NS>
-__global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
+__global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 4 : 2)) dense_qx_kernel(const DenseArgs a) {
   constexpr int WN = BN / 2, WM = BM / 4;   // per-wave slice: WN features x WM tokens
-  constexpr int TN = WN / 32, TM = WM / 32;
+  constexpr int TN = WN / 16, TM = WM / 16;  // its 16 x 16 blocks
   constexpr int AP = BM * (BK / 4) / 512;  // 16-byte chunks of X per thread per pair of K-tiles
   constexpr int BP = MODE == kPlainF16 ? BN * (BK / 4) / 512 : 0;  // plain fp16 weight: the same
   constexpr int QW = MODE == kPlainF16 ? 1 : Q;  // dwords per granule
@@ -555,7 +558,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // feature tiles at 32 CUs: an X slice is 16 KB per K-tile, a packed W slice 4-8 KB),
   // so every X and W panel slice is fetched into that XCD's L2 once per block
   // instead of once per tile column.
-  auto xcd_order = [](int i, int total) {
+  auto xcd_order = [](int i, int total) __attribute__((always_inline)) {
     const int per = total / 8;
     return i < per * 8 ? (i & 7) * per + (i >> 3) : i;
   };
@@ -664,7 +667,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // consecutive rows, one entry each) hit 64 different banks whatever entries
   // they ask for.  Each of a row's two threads keeps half of the row's column current.
   const int pal_col = (b_row >> 7) * (256 << Q) + (b_row & 63) * 4 + ((b_row >> 6) & 1) * 2;  // byte offset of this row's column
-  auto fill_pal_column = [&](int64_t blk) {
+  auto fill_pal_column = [&](int64_t blk) __attribute__((always_inline)) {
     if (!stager) return;
     constexpr int ND = (1 << Q) / 4;  // dwords of palette per thread
     const uint32_t* src =
@@ -680,7 +683,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   int gn_row = n0 + b_row;  // this thread's weight row
   if (gn_row >= w.n) gn_row = w.n - 1;
   // rewrites the column if the row enters a new block at K-tile `tile`
-  auto refresh_pal_column = [&](int tile) {
+  auto refresh_pal_column = [&](int tile) __attribute__((always_inline)) {
     const int64_t e = (int64_t)gn_row * K + (int64_t)tile * BK;
     const int64_t blk = e / a.nib;
     if (e == blk * a.nib) fill_pal_column(blk);
@@ -707,7 +710,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 
   // Part i (of AP + BP) of the memory -> LDS transfer of K-tile pair q into a
   // pair slot (pairs past the end re-read the last one, harmlessly).
-  auto issue_pair_part = [&](half_t* xs, half_t* wp, int q, int i) {
+  auto issue_pair_part = [&](half_t* xs, half_t* wp, int q, int i) __attribute__((always_inline)) {
     if (q > last_pair) q = last_pair;
     const int64_t kb = (int64_t)q * (4 * BK);  // byte offset of the pair inside a row
     if (i < AP) {
@@ -716,7 +719,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       load_to_lds_16(wbase + kb, bf_off[i - AP], lds_address(wp) + (uint32_t)((wave_u * BP + i - AP) * 1024));
     }
   };
-  auto issue_pair = [&](half_t* xs, half_t* wp, int q) {
+  auto issue_pair = [&](half_t* xs, half_t* wp, int q) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < AP + BP; i++) issue_pair_part(xs, wp, q, i);
   };
@@ -724,7 +727,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // Loads the indices of the tile the cursor points at (the last tile is re-read
   // harmlessly by the final iterations) and moves the cursor on by one tile.
   int issued = SPLIT ? t_lo : 0;  // tile that the cursor points at
-  auto issue_idx = [&](IdxSet& R) {
+  auto issue_idx = [&](IdxSet& R) __attribute__((always_inline)) {
     if constexpr (MODE != kPlainF16) {
       if (!stager) return;
       const uint32_t* src = reinterpret_cast<const uint32_t*>(wbase + cur.off);
@@ -755,7 +758,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   const char* gpal = nullptr;
   uint32_t pal_base = 0;
   // piece 0 also turns the index dwords into a bit string; piece p yields offsets 4p .. 4p+3
-  auto unpack_piece = [&](IdxSet& R, int p) {
+  auto unpack_piece = [&](IdxSet& R, int p) __attribute__((always_inline)) {
     if constexpr (MODE != kPlainF16) {
       if (!stager) return;
       if (p == 0) {
@@ -769,7 +772,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
         la[j] = own_index_at<Q, HW, (MODE == kPalRow ? 8 : 1)>(be, j, pal_base);
     }
   };
-  auto lookup = [&](int j) {
+  auto lookup = [&](int j) __attribute__((always_inline)) {
     if (!stager) return;
     if constexpr (MODE == kPalGlobal)
       la[j] = *reinterpret_cast<const uint16_t*>(gpal + la[j]);
@@ -781,9 +784,9 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
   // them against anything else.
   // unpacked weight tiles are chunk-major, [4 chunks of 8 k][BN rows][8 halfs]: a wave's 64 rows of one chunk are
   // 1 KB of consecutive addresses, for the row-per-lane writes here and for the row-per-lane operand reads alike
-  auto w_chunk = [](int row, int c) { return (c * BN + row) * 8; };
+  auto w_chunk = [](int row, int c) __attribute__((always_inline)) { return (c * BN + row) * 8; };
   const uint32_t w_dst = lds_address(Bs) + 2u * (uint32_t)w_chunk(b_row, second ? 2 : 0);
-  auto write_weights = [&](int stage, int h) {
+  auto write_weights = [&](int stage, int h) __attribute__((always_inline)) {
     if constexpr (MODE != kPlainF16) {
       if (!stager) return;
       const uint4_t v = {la[8 * h] | (la[8 * h + 1] << 16), la[8 * h + 2] | (la[8 * h + 3] << 16),
@@ -792,7 +795,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       asm volatile("ds_write_b128 %0, %1" : : "v"(addr), "v"(v) : "memory");
     }
   };
-  auto stage_to_lds = [&](IdxSet& R, int stage) {  // all at once (prologue)
+  auto stage_to_lds = [&](IdxSet& R, int stage) __attribute__((always_inline)) {  // all at once (prologue)
 #pragma unroll
     for (int p = 0; p < 4; p++) unpack_piece(R, p);
 #pragma unroll
@@ -801,7 +804,7 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     write_weights(stage, 1);
   };
   // Makes the wait for an index load happen here rather than at its first use.
-  auto touch = [&](IdxSet& R) {
+  auto touch = [&](IdxSet& R) __attribute__((always_inline)) {
     if constexpr (MODE != kPlainF16) {
       if (!stager) return;
 #pragma unroll
@@ -809,36 +812,46 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     }
   };
 
-  float16_t acc[TN][TM];
+  float4_t acc[TN][TM];
 #pragma unroll
   for (int i = 0; i < TN; i++)
 #pragma unroll
-    for (int j = 0; j < TM; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+    for (int j = 0; j < TM; j++) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  // ---- fragment double buffer --------------------------------------------
-  // MFMA A operand = W rows (features), B operand = X rows (tokens); lane holds
-  // row (lane & 31), k-slots 8 * (lane / 32) .. + 7 of the 16-wide k-step.
-  // In a pair slot the 16-byte chunk c (0..7: tile parity * 4 + k-step * 2 +
-  // half) of row r sits at slot c ^ (r / 2 % 8); rows 32 apart share a swizzle.
-  const int l32 = lane & 31, hi = lane >> 5;
-  const int xrow = wm * WM + l32, wrow = wn * WN + l32;
-  const int x_lane = xrow * PROW + ((hi ^ ((xrow >> 1) & 7)) << 3);  // halfs; chunk bits xor'ed per read
-  const int w_lane = wrow * PROW + ((hi ^ ((wrow >> 1) & 7)) << 3);
-  half8_t fw[2][TN], fx[2][TM];
-  // par: tile of the pair (0/1), ks: k-step of the tile, stage: ring stage of the unpacked weights
-  auto read_w = [&](int buf, int i, const half_t* wp, int par, int stage, int ks) {
+  // ---- fragments ----------------------------------------------------------
+  // v_mfma_f32_16x16x32_f16: A operand = W rows (features), B operand = X rows (tokens); lane holds row (lane & 15),
+  // k 8 * (lane / 16) .. + 7 of the K-tile.  (For the same work it moves 8 KB of operands and accumulators through the
+  // register file where 32x32x16 moves 10, and the card is power-limited here: a stream of nothing else reaches 1.95
+  // PFLOP/s against 1.68 on random data, with this kernel's operand reads from LDS beside it 1.58 against 1.44.)
+  // An iteration's MFMAs go in two phases, one per half of the wave's W blocks, so that a half's registers are refilled
+  // while the other half multiplies.  X blocks are refilled behind their last use (XB = 1: 13 MFMAs before the next one)
+  // where a phase is long enough, else there are two sets of them.
+  // In a pair slot the 16-byte chunk c (0..7: tile parity * 4 + lane / 16) of row r sits at slot c ^ (r / 2 % 8); rows
+  // 16 apart share a swizzle.
+  constexpr int HN = TN / 2;
+  constexpr int XB = TM >= 4 ? 1 : 2;
+  const int l16 = lane & 15, quad = lane >> 4;
+  const int xrow = wm * WM + l16, wrow = wn * WN + l16;
+  const int x_lane = xrow * PROW + ((quad ^ ((xrow >> 1) & 7)) << 3);  // halfs; the tile's parity xor'ed per read
+  const int w_lane = wrow * PROW + ((quad ^ ((wrow >> 1) & 7)) << 3);
+  half8_t fw[TN], fx[XB][TM];
+  // par: tile of the pair (0/1), stage: ring stage of the unpacked weights
+  auto read_w = [&](int i, const half_t* wp, int par, int stage) __attribute__((always_inline)) {
     if constexpr (MODE == kPlainF16)
-      fw[buf][i] = *reinterpret_cast<const half8_t*>(wp + (w_lane ^ ((4 * par + 2 * ks) << 3)) + i * 32 * PROW);
+      fw[i] = *reinterpret_cast<const half8_t*>(wp + (w_lane ^ (32 * par)) + i * 16 * PROW);
     else
-      fw[buf][i] = *reinterpret_cast<const half8_t*>(Bs + stage * B_STAGE + ((2 * ks + hi) * BN + wrow + i * 32) * 8);
+      fw[i] = *reinterpret_cast<const half8_t*>(Bs + stage * B_STAGE + (quad * BN + wrow + i * 16) * 8);
   };
-  auto read_x = [&](int buf, int j, const half_t* xs, int par, int ks) {
-    fx[buf][j] = *reinterpret_cast<const half8_t*>(xs + (x_lane ^ ((4 * par + 2 * ks) << 3)) + j * 32 * PROW);
+  auto read_x = [&](int j, const half_t* xs, int par) __attribute__((always_inline)) {
+    fx[XB == 2 ? par : 0][j] = *reinterpret_cast<const half8_t*>(xs + (x_lane ^ (32 * par)) + j * 16 * PROW);
   };
-  auto mfma = [&](int buf, int i, int j) {
-    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[buf][i], fx[buf][j], acc[i][j], 0, 0, 0);
+  // MFMA m of phase `half` of a tile of parity `par`
+  auto mfma = [&](int half, int m, int par) __attribute__((always_inline)) {
+    const int i = half * HN + m % HN, j = m / HN;
+    // (assembly because the sums have to stay where they are: the builtin's result may be any other four registers, and
+    // with 176 of 256 taken by sums and operands the allocator spilled over the moving holes.  Operands come from LDS
+    // reads, whose waits the compiler inserts; a sum's next MFMA is a whole iteration away.)
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(fw[i]), "v"(fx[XB == 2 ? par : 0][j]));
   };
 
   // ---- prologue: pair 0 in slot A, weights of tiles 0 and 1 in the ring --------
@@ -891,26 +904,26 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     issue_idx(WS[3]);  // tile 5
   }
 #pragma unroll
-  for (int i = 0; i < TN; i++) read_w(0, i, WpA, 0, 0, 0);
+  for (int i = 0; i < HN; i++) read_w(i, WpA, 0, 0);
 #pragma unroll
-  for (int j = 0; j < TM; j++) read_x(0, j, XsA, 0, 0);
+  for (int j = 0; j < TM; j++) read_x(j, XsA, 0);
 
   // Iteration t: MFMAs of tile t (pair t / 2) while the weights of tile t+2
   // are unpacked into ring stage (t+2) % 3.  An even iteration starts the
   // transfer of the next pair into the other slot (free since the barrier
   // that ended tile t-1) and waits for it before its closing barrier, because
-  // the odd iteration reads one k-step ahead into that pair.  Index registers
+  // the odd iteration reads the next tile's first operands from that pair.  Index registers
   // are refilled in odd iterations only, so the even iteration's wait covers
   // nothing that was issued just before it.
   // (MID: the closing barriers wait for the LDS only; pair and indices are waited for in the middle of odd iterations.)
   //
   // A wave issues in order, and an LDS instruction occupies it for tens of
-  // clocks, so the iteration is written as 16 slots of one MFMA followed by
-  // a share of the LDS and VALU work: the fragment reads of the next k-step,
+  // clocks, so the iteration is written as slots of one MFMA followed by
+  // a share of the LDS and VALU work: the fragment reads of the next phase,
   // the palette lookups and the weight writes all issue while an MFMA of the
   // same wave (or of the wave it shares the SIMD with) is executing.
   int s_cur = 0, s_nxt = 1, s_fill = 2;
-  auto iteration = [&](int t, int par, half_t* xs, half_t* wp, half_t* xs_other, half_t* wp_other, int set = 0) {
+  auto iteration = [&](int t, int par, half_t* xs, half_t* wp, half_t* xs_other, half_t* wp_other, int set = 0) __attribute__((always_inline)) {
     if constexpr (MODE == kPalRow) {
       if (t + 2 == next_pal_tile) {
         // lookups of tile t+1 finished before the last barrier
@@ -925,17 +938,17 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     // would last until it lands
     touch(R);
     if (par && !MID) issue_idx(WS[0]);  // tile t+3
-    const half_t* xs_n = par == 0 ? xs : xs_other;  // fragments of tile t+1, k-step 0
+    const half_t* xs_n = par == 0 ? xs : xs_other;  // fragments of tile t+1
     const half_t* wp_n = par == 0 ? wp : wp_other;
-    constexpr int NM = TN * TM;  // MFMAs per k-step = slots per phase
-    constexpr int NF = TN + TM;  // fragment reads per phase
+    constexpr int NM = HN * TM;  // MFMAs = slots per phase
+    constexpr int NF0 = HN, NF1 = HN + (XB == 2 ? TM : 0);  // fragment reads per phase (and X behind its last use)
     constexpr bool packed = MODE != kPlainF16;
-    // Phase 0 (k-step 0): the fragments of k-step 1, one every third place;
+    // Phase 0: the other half's W fragments, one every third place;
     // between them the parts of the transfer (even iterations), the unpacking,
     // the refill of the index registers (odd iterations), the first 8 lookups.
     const int nd = par == 0 && !MID ? AP + BP : 0;
     const int ns0 = nd + (packed ? 4 + (MID ? 0 : par) + 8 : 0);
-    auto stage0 = [&](int s) {
+    auto stage0 = [&](int s) __attribute__((always_inline)) {
       if (s < nd) { issue_pair_part(xs_other, wp_other, (t >> 1) + 1, s); return; }
       s -= nd;
       if (!packed) return;
@@ -947,12 +960,11 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       }
       if (s < 8) lookup(s);
     };
-    // Phase 1 (k-step 1): the next tile's first fragments (every k-step 0
-    // MFMA has been issued, so their registers are free), the other lookups,
-    // the two weight writes.
+    // Phase 1: the next tile's X and first W fragments, the other lookups, the
+    // two weight writes.
     const int nd1 = MID && par ? AP + 2 : 0;
     const int ns1 = packed ? nd1 + 10 : 0;
-    auto stage1 = [&](int s) {
+    auto stage1 = [&](int s) __attribute__((always_inline)) {
       if (!packed) return;
       if (s < nd1) {
         if (s < AP) issue_pair_part(xs, wp, (t >> 1) + NS, s);
@@ -963,38 +975,42 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       if (s < 8) lookup(8 + s);
       else if (s < 10) write_weights(s_fill, s - 8);
     };
-    auto read0 = [&](int r) {
-      if (r < TN) read_w(1, r, wp, par, s_cur, 1);
-      else read_x(1, r - TN, xs, par, 1);
+    auto read0 = [&](int r) __attribute__((always_inline)) { read_w(HN + r, wp, par, s_cur); };
+    auto read1 = [&](int r) __attribute__((always_inline)) {
+      if (XB == 2 && r < TM) read_x(r, xs_n, par ^ 1);
+      else read_w(r - (XB == 2 ? TM : 0), wp_n, par ^ 1, s_nxt);
     };
-    auto read1 = [&](int r) {
-      if (r < TN) read_w(0, r, wp_n, par ^ 1, s_nxt, 0);
-      else read_x(0, r - TN, xs_n, par ^ 1, 0);
+    // X block m / HN behind its last MFMA of this tile, which is slot m of phase 1
+    auto read_x_behind = [&](int m) __attribute__((always_inline)) {
+      if (XB == 1 && m % HN == HN - 1) read_x(m / HN, xs_n, par ^ 1);
     };
-    // place k of a phase: a read at every third place while reads last, stage parts elsewhere
-    auto place = [&](int k, int ns, auto&& rd, auto&& st) {
-      if (k < 3 * NF) {
+    // place k of a phase of nf reads: a read at every third place while reads last, stage parts elsewhere
+    auto place = [&](int k, int nf, int ns, auto&& rd, auto&& st) __attribute__((always_inline)) {
+      if (k < 3 * nf) {
         if (k % 3 == 0) rd(k / 3);
         else if ((k / 3) * 2 + k % 3 - 1 < ns) st((k / 3) * 2 + k % 3 - 1);
-      } else if (k - NF < ns) {
-        st(k - NF);
+      } else if (k - nf < ns) {
+        st(k - nf);
       }
     };
     if constexpr (!packed) {
       // Plain fp16 weights: both operands arrive by transfer and nothing is written to LDS by the waves, so one
       // barrier per pair of K-tiles is enough, and it sits in the middle of the odd iteration: by then the pair in
-      // flight has had two iterations to land, the reads of this pair's last k-step were issued half an
-      // iteration ago, and what follows the barrier is exactly what needs it -- the first reads from the other
+      // flight has had two iterations to land, the reads of this pair's last operands were issued at the
+      // iteration's start, and what follows the barrier is exactly what needs it -- the first reads from the other
       // slot and the transfer of the pair after next into this one.
-      constexpr int RPS = (NF + NM - 1) / NM;            // fragment reads per MFMA, front-loaded
-      constexpr int PPS = (AP + BP + NM - 1) / NM;       // transfer parts per MFMA
+      constexpr int RPS0 = (NF0 + NM - 1) / NM, RPS1 = (NF1 + NM - 1) / NM;  // fragment reads per MFMA, front-loaded
+      constexpr int PPS = (AP + BP + NM - 1) / NM;                           // transfer parts per MFMA
+      // the 128 x 128 tile is bound by how soon its next pair arrives: all of the transfer goes out behind the barrier,
+      // ahead of the reads (1376 x 12288 -> 3072 141.5 / 124.5 us)
+      constexpr bool EARLY = BM == 128 && BN == 128;
 #pragma unroll
       for (int m = 0; m < NM; m++) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma(0, m / TM, m % TM);
+        mfma(0, m, par);
 #pragma unroll
-        for (int r = m * RPS; r < (m + 1) * RPS; r++)
-          if (r < NF) read0(r);
+        for (int r = m * RPS0; r < (m + 1) * RPS0; r++)
+          if (r < NF0) read0(r);
       }
       if (par) {
         __builtin_amdgcn_sched_barrier(0);
@@ -1004,11 +1020,16 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 #pragma unroll
       for (int m = 0; m < NM; m++) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma(1, m / TM, m % TM);
+        if (par && EARLY && m == 0) {
 #pragma unroll
-        for (int r = m * RPS; r < (m + 1) * RPS; r++)
-          if (r < NF) read1(r);
-        if (par) {
+          for (int q = 0; q < AP + BP; q++) issue_pair_part(xs, wp, (t >> 1) + NS, q);
+        }
+        mfma(1, m, par);
+        read_x_behind(m);
+#pragma unroll
+        for (int r = m * RPS1; r < (m + 1) * RPS1; r++)
+          if (r < NF1) read1(r);
+        if (par && !EARLY) {
           // this iteration's slot is free from the barrier on: pair q + NS goes into it
 #pragma unroll
           for (int q = m * PPS; q < (m + 1) * PPS; q++)
@@ -1018,14 +1039,14 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       return;
     }
-    const int n0 = NF + (ns0 > 2 * NF ? ns0 : 2 * NF);
-    const int n1 = NF + (ns1 > 2 * NF ? ns1 : 2 * NF);
+    const int n0 = NF0 + (ns0 > 2 * NF0 ? ns0 : 2 * NF0);
+    const int n1 = NF1 + (ns1 > 2 * NF1 ? ns1 : 2 * NF1);
 #pragma unroll
     for (int m = 0; m < NM; m++) {
       __builtin_amdgcn_sched_barrier(0);
-      mfma(0, m / TM, m % TM);
+      mfma(0, m, par);
 #pragma unroll
-      for (int k = m * n0 / NM; k < (m + 1) * n0 / NM; k++) place(k, ns0, read0, stage0);
+      for (int k = m * n0 / NM; k < (m + 1) * n0 / NM; k++) place(k, NF0, ns0, read0, stage0);
     }
     if (MID && par) {
       // the next pair and the indices of the one after it; this pair's slot is free from here on
@@ -1036,9 +1057,10 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 #pragma unroll
     for (int m = 0; m < NM; m++) {
       __builtin_amdgcn_sched_barrier(0);
-      mfma(1, m / TM, m % TM);
+      mfma(1, m, par);
+      read_x_behind(m);
 #pragma unroll
-      for (int k = m * n1 / NM; k < (m + 1) * n1 / NM; k++) place(k, ns1, read1, stage1);
+      for (int k = m * n1 / NM; k < (m + 1) * n1 / NM; k++) place(k, NF1, ns1, read1, stage1);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (par == 0 && !MID)
@@ -1052,37 +1074,47 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     s_fill = s;
   };
 
-  int t = SPLIT ? t_lo : 0;
-  if constexpr (NS > 2) {
-    // Rounds of NS pairs, so that every slot is a constant (us, slot addresses made in the loop / here, and with two slots:
-    // 1344 x 1920 -> 200 17.6 / 16.3, 16.3; 300 x 3904 -> 2 x 384 27.8 / 25.4, 39.1; 3175 x 5120 -> 3 x 256 45.3 / 42.5, 57.5).
-    const auto pair = [&](int t, int slot) __attribute__((always_inline)) {
-      const int next = slot + 1 < NS ? slot + 1 : 0;
-      half_t* const xs = XsA + slot * (XS_BYTES / 2);
-      half_t* const wp = WpA + slot * (WP_BYTES / 2);
-      half_t* const xn = XsA + next * (XS_BYTES / 2);
-      half_t* const wn_ = WpA + next * (WP_BYTES / 2);
-      iteration(t, 0, xs, wp, xn, wn_);
-      iteration(t + 1, 1, xs, wp, xn, wn_);
-    };
-    for (; t + 2 * NS <= nk; t += 2 * NS) {
+  const auto all_tiles = [&]() __attribute__((always_inline)) {
+    int t = SPLIT ? t_lo : 0;
+    if constexpr (NS > 2) {
+      // Rounds of NS pairs, so that every slot is a constant (us, slot addresses made in the loop / here, and with two slots:
+      // 1344 x 1920 -> 200 17.6 / 16.3, 16.3; 300 x 3904 -> 2 x 384 27.8 / 25.4, 39.1; 3175 x 5120 -> 3 x 256 45.3 / 42.5, 57.5).
+      const auto pair = [&](int t, int slot) __attribute__((always_inline)) {
+        const int next = slot + 1 < NS ? slot + 1 : 0;
+        half_t* const xs = XsA + slot * (XS_BYTES / 2);
+        half_t* const wp = WpA + slot * (WP_BYTES / 2);
+        half_t* const xn = XsA + next * (XS_BYTES / 2);
+        half_t* const wn_ = WpA + next * (WP_BYTES / 2);
+        iteration(t, 0, xs, wp, xn, wn_);
+        iteration(t + 1, 1, xs, wp, xn, wn_);
+      };
+      for (; t + 2 * NS <= nk; t += 2 * NS) {
 #pragma unroll
-      for (int slot = 0; slot < NS; slot++) pair(t + 2 * slot, slot);
+        for (int slot = 0; slot < NS; slot++) pair(t + 2 * slot, slot);
+      }
+#pragma unroll
+      for (int slot = 0; slot < NS - 1; slot++)
+        if (t + 2 * slot < nk) pair(t + 2 * slot, slot);
+    } else {
+      for (; t + 3 < nk; t += 4) {
+        iteration(t, 0, XsA, WpA, XsB, WpB);
+        iteration(t + 1, 1, XsA, WpA, XsB, WpB);
+        iteration(t + 2, 0, XsB, WpB, XsA, WpA, 1);
+        iteration(t + 3, 1, XsB, WpB, XsA, WpA, 1);
+      }
+      if (t < nk) {  // nk is even: two iterations left
+        iteration(t, 0, XsA, WpA, XsB, WpB);
+        iteration(t + 1, 1, XsA, WpA, XsB, WpB);
+      }
     }
-#pragma unroll
-    for (int slot = 0; slot < NS - 1; slot++)
-      if (t + 2 * slot < nk) pair(t + 2 * slot, slot);
+  };
+  // Where only half of the waves stage weights, each half has a loop of its own: straight-line code, where a test around
+  // every piece of staging had cut an iteration into twenty blocks.
+  if constexpr (MODE != kPlainF16 && BN == 128) {
+    if (stager) all_tiles();
+    else all_tiles();
   } else {
-    for (; t + 3 < nk; t += 4) {
-      iteration(t, 0, XsA, WpA, XsB, WpB);
-      iteration(t + 1, 1, XsA, WpA, XsB, WpB);
-      iteration(t + 2, 0, XsB, WpB, XsA, WpA, 1);
-      iteration(t + 3, 1, XsB, WpB, XsA, WpA, 1);
-    }
-    if (t < nk) {  // nk is even: two iterations left
-      iteration(t, 0, XsA, WpA, XsB, WpB);
-      iteration(t + 1, 1, XsA, WpA, XsB, WpB);
-    }
+    all_tiles();
   }
 
   if constexpr (MODE == kPlainF16 || MID) {
@@ -1090,11 +1122,17 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
     __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
     __syncthreads();
   }
+  // the last MFMAs' results are not interlocked against ordinary instructions, and the compiler does not know of them
+  asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+  for (int i = 0; i < TN; i++)
+#pragma unroll
+    for (int j = 0; j < TM; j++) asm volatile("" : "+v"(acc[i][j]));
   if constexpr (SPLIT) {
     if (split_tile >= 0) {
       __shared__ int s_seen;
       const int64_t slot_step = (int64_t)(a.total_tiles - a.whole_tiles) * (BM * BN);
-      // slot: [TN * TM * 16][512 threads] floats, so that a wave's access covers 256 consecutive bytes
+      // slot: [TN * TM * 4][512 threads] floats, so that a wave's access covers 256 consecutive bytes
       float* const slots = a.partials + (int64_t)split_tile * (BM * BN) + tid;
       int32_t* const counters = a.counters + split_tile * kSplitNodes;
       int node0 = 0;  // counters of this level
@@ -1111,8 +1149,8 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
 #pragma unroll
               for (int j = 0; j < TM; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++)
-                  __hip_atomic_store(own + ((i * TM + j) * 16 + v) * 512, acc[i][j][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int v = 0; v < 4; v++)
+                  __hip_atomic_store(own + ((i * TM + j) * 4 + v) * 512, acc[i][j][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // every wave's stores have been acknowledged before the barrier, hence before the count that publishes them
             __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
             __syncthreads();
@@ -1121,17 +1159,17 @@ __global__ void __launch_bounds__(512) dense_qx_kernel(const DenseArgs a) {
             if (s_seen == 0) return;  // uniform: the other one goes on
           }
           const float* const theirs = slots + (other << level) * slot_step;
-          constexpr int NH = TN * TM > 4 ? 2 : 1;  // in halves where a whole slot would not fit beside the sums
+          constexpr int NH = TN * TM > 16 ? 2 : 1;  // in halves where a whole slot would not fit beside the sums
 #pragma unroll
           for (int h = 0; h < NH; h++) {
-            float16_t got[TN / NH][TM];
+            float4_t got[TN / NH][TM];
 #pragma unroll
             for (int i = 0; i < TN / NH; i++)
 #pragma unroll
               for (int j = 0; j < TM; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++)
-                  got[i][j][v] = __hip_atomic_load(theirs + (((h * (TN / NH) + i) * TM + j) * 16 + v) * 512, __ATOMIC_RELAXED,
+                for (int v = 0; v < 4; v++)
+                  got[i][j][v] = __hip_atomic_load(theirs + (((h * (TN / NH) + i) * TM + j) * 4 + v) * 512, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
