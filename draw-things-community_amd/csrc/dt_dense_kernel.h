@@ -478,6 +478,43 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
   }
 }
 
+// Tile order: bands of 4 token tiles; inside a band feature tiles outermost,
+// token tiles innermost.  Workgroups are dealt round-robin to the 8 XCDs;
+// giving each XCD a contiguous run of that order makes the workgroups that
+// run together on an XCD cover a compact 2-D block of tiles (4 token tiles x 8
+// feature tiles at 32 CUs: an X slice is 16 KB per K-tile, a packed W slice 4-8 KB),
+// so every X and W panel slice is fetched into that XCD's L2 once per block
+// instead of once per tile column.
+__device__ __forceinline__ int xcd_order(int i, int total) {
+  const int per = total / 8;
+  return i < per * 8 ? (i & 7) * per + (i >> 3) : i;
+}
+struct TileAt {
+  int group, weight;
+  int tm, tn;  // token tile of the group, feature tile of the group's weights
+};
+__device__ __forceinline__ TileAt tile_at(const DenseArgs& a, int bid) {
+  TileAt t;
+  t.group = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxGroups; i++)
+    if (i < a.n_groups && bid >= a.g[i].tile_begin) t.group = i;
+  const DenseGroup& g = a.g[t.group];
+  bid -= g.tile_begin;
+  constexpr int GM = 4;
+  const int band_tiles = GM * g.tiles_n;
+  const int band = bid / band_tiles;
+  const int in_band = bid - band * band_tiles;
+  const int rows_in_band = (g.tiles_m - band * GM) < GM ? (g.tiles_m - band * GM) : GM;
+  t.tn = in_band / rows_in_band;
+  t.tm = band * GM + (in_band - t.tn * rows_in_band);
+  t.weight = g.w_begin;
+#pragma unroll
+  for (int i = 1; i < kMaxWeights; i++)
+    if (i > g.w_begin && i < g.w_end && t.tn >= a.w[i].tile_begin) t.weight = i;
+  return t;
+}
+
 // 512 threads = 8 waves, two per SIMD, all eight running MFMAs on a (BN/2) x
 // (BM/4) slice.  Every thread issues its share of the memory -> LDS transfer of
 // X and unpacks / looks up half a granule (16 weights) of one W row per
@@ -498,8 +535,8 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
 // shares of 80 tiles; two that meet take 7.)
 //
 // NS: pair slots.  Two, or more of them with plain fp16 weights: every pair then has NS - 1 pairs of K-tiles to arrive,
-// which a workgroup that has a compute unit to itself needs (128 x 128 tiles with two and with four slots: 2016 x 5120 ->
-// 1280 57.8 / 48.7 us, 4608 x 3072 -> 64 31.7 / 23.9; two tiles on a compute unit hide the latency for each other).
+// which a workgroup that has a compute unit to itself needs (two tiles on a compute unit hide the latency for each other;
+// 128 x 128 tiles of plain weights that have one to themselves run in dense_f16_kernel).
 //
 // Where two 128 x 128 tiles fit a compute unit's LDS, their registers have to leave room for both: four waves per SIMD.
 constexpr bool dense_two_per_cu(int Q, int BM, int BN, int mode, int NS) {
@@ -551,17 +588,6 @@ __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 
   const int lt = BN == 256 ? (tid & 255) : (lane + 64 * (wave & 1));
   const int wn = wave & 1, wm = ((wave >> 1) & 1) | ((wave >> 2) << 1);  // waves w and w+4 share a SIMD and take different m slices
 
-  // Tile order: bands of 4 token tiles; inside a band feature tiles outermost,
-  // token tiles innermost.  Workgroups are dealt round-robin to the 8 XCDs;
-  // giving each XCD a contiguous run of that order makes the workgroups that
-  // run together on an XCD cover a compact 2-D block of tiles (4 token tiles x 8
-  // feature tiles at 32 CUs: an X slice is 16 KB per K-tile, a packed W slice 4-8 KB),
-  // so every X and W panel slice is fetched into that XCD's L2 once per block
-  // instead of once per tile column.
-  auto xcd_order = [](int i, int total) __attribute__((always_inline)) {
-    const int per = total / 8;
-    return i < per * 8 ? (i & 7) * per + (i >> 3) : i;
-  };
   int bid = blockIdx.x, share = 0, split_tile = -1;  // share: which part of K (split tiles)
   if constexpr (SPLIT) {
     // split tiles follow the whole ones, share by share: the workgroups that run together on a die walk the same
@@ -578,28 +604,10 @@ __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 
   } else {
     bid = xcd_order(bid, a.total_tiles);
   }
-  int gi = 0;
-#pragma unroll
-  for (int i = 1; i < kMaxGroups; i++)
-    if (i < a.n_groups && bid >= a.g[i].tile_begin) gi = i;
-  const DenseGroup g = a.g[gi];
-  bid -= g.tile_begin;
-  int tm, tn;
-  {
-    constexpr int GM = 4;
-    const int band_tiles = GM * g.tiles_n;
-    const int band = bid / band_tiles;
-    const int in_band = bid - band * band_tiles;
-    const int rows_in_band = (g.tiles_m - band * GM) < GM ? (g.tiles_m - band * GM) : GM;
-    tn = in_band / rows_in_band;
-    tm = band * GM + (in_band - tn * rows_in_band);
-  }
-
-  int wi = g.w_begin;
-#pragma unroll
-  for (int i = 1; i < kMaxWeights; i++)
-    if (i > g.w_begin && i < g.w_end && tn >= a.w[i].tile_begin) wi = i;
-  const DenseWeight w = a.w[wi];
+  const TileAt at = tile_at(a, bid);
+  const DenseGroup g = a.g[at.group];
+  const DenseWeight w = a.w[at.weight];
+  const int tm = at.tm, tn = at.tn;
   const int n0 = (tn - w.tile_begin) * BN;
   const int m0 = tm * BM;
   const int K = a.k;

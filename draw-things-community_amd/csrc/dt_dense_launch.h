@@ -1,5 +1,6 @@
 // Launchers of the tiled Dense kernels, instantiated once per index width in dt_dense_q<Q>.hip.
 #pragma once
+#include "dt_dense_f16.h"
 #include "dt_dense_kernel.h"
 
 namespace dt {
@@ -14,12 +15,12 @@ static dt_status launch_tiled(hipStream_t s, const DenseArgs& a, int mode) {
   const int64_t rest = SPLIT ? a.total_tiles - a.whole_tiles : 0;
   dim3 grid((unsigned)(a.total_tiles - rest + rest * a.split)), block(512);
   if constexpr (Q == 16) {  // plain fp16 weight
-    // pair slots: as many as fit where a workgroup has a compute unit to itself (up to 256 tiles of 128 x 128; beyond,
-    // two slots let two of them share one)
+    // pair slots: as many as fit where a workgroup has a compute unit to itself (up to 256 tiles of 128 x 128 and K over 256: in
+    // a kernel of their own; else two slots let two of them share one)
     if constexpr (BM == 128 && BN == 256) {
       hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 3>), grid, block, 0, s, a);
     } else if constexpr (BM == 128 && BN == 128) {
-      if (grid.x <= 256) hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 4>), grid, block, 0, s, a);
+      if (grid.x <= 256 && a.k > 256) hipLaunchKernelGGL(dense_f16_kernel<POST>, grid, block, 0, s, a);
       else hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 2>), grid, block, 0, s, a);
     } else {
       hipLaunchKernelGGL((dense_qx_kernel<8, BM, BN, kPlainF16, POST, SPLIT, 2>), grid, block, 0, s, a);

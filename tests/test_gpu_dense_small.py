@@ -190,6 +190,25 @@ def test_dense_plain_pair_slots(dthip, oracle, K):
             check(dthip.dense_multi(dev(X), [head, w], [None, None], epilogues=[epi, None])[1].cpu().numpy(), X, W)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 8, 320), (128, 128, 384), (129, 257, 448), (300, 600, 512), (1000, 3900, 576)])
+def test_dense_plain_tile_per_compute_unit(dthip, oracle, M, N, K):
+    """Plain fp16 weights on up to 256 tiles of 128 x 128, five pairs of K-tiles and more: every remainder of the rounds of
+    four slots, ragged edges, two weights; and the kernel with the tail, whose tail does nothing, bit for bit."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    pairs = [make(dthip, oracle, rng, n, K, 16, 0) for n in (N, 128)]
+    ws, bias = [w for w, _ in pairs], dev((rng.standard_normal(N) * 0.1).astype(np.float16))
+    print("dense plain tile per compute unit", M, N, K, flush=True)
+    outs = dthip.dense_multi(dev(X), ws, [bias, None])
+    check(outs[0].cpu().numpy(), X, pairs[0][1], bias.cpu().numpy())
+    check(outs[1].cpu().numpy(), X, pairs[1][1])
+    zero = torch.zeros((M, N), dtype=torch.float16, device="cuda")
+    tails = dthip.dense_post(dev(X), ws, [bias, None], [dthip.DensePost(addend=zero), dthip.DensePost()])
+    assert all(torch.equal(a, b) for a, b in zip(outs, tails))
+
+
 @pytest.mark.parametrize("K", [64, 128, 192])
 def test_dense_plain_brief(dthip, oracle, K):
     """Many tiles of one or two K-tile pairs stay 128 x 128; with three they are 256 x 256."""
