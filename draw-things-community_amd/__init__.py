@@ -36,6 +36,8 @@ ABI_SYMBOLS = (
     "dt_dense_qx_grouped_f16",
     "dt_dense_workspace_bytes",
     "dt_dense_qx_grouped_ws_f16",
+    "dt_dense_scratch_bytes",
+    "dt_dense_qx_grouped_scratch_f16",
     "dt_dense_qx_post_f16",
     "dt_qk_norm_rope_f16",
     "dt_layernorm_modulate_f16",
@@ -145,6 +147,10 @@ def lib():
         L.dt_dense_workspace_bytes.argtypes = [i32, vp]
         L.dt_dense_qx_grouped_ws_f16.restype = i32
         L.dt_dense_qx_grouped_ws_f16.argtypes = [vp, i32, vp, ctypes.c_uint32, vp, ctypes.c_size_t]
+        L.dt_dense_scratch_bytes.restype = ctypes.c_size_t
+        L.dt_dense_scratch_bytes.argtypes = [i32, vp]
+        L.dt_dense_qx_grouped_scratch_f16.restype = i32
+        L.dt_dense_qx_grouped_scratch_f16.argtypes = L.dt_dense_qx_grouped_ws_f16.argtypes
         L.dt_qk_norm_rope_f16.argtypes = [vp, _View4, i32, i64, i32, i32, vp, f32, i32, vp, i64, f32]
         L.dt_layernorm_modulate_f16.restype = i32
         L.dt_layernorm_modulate_f16.argtypes = [vp, i64, i64, vp, i64, vp, vp, i32, f32, vp, i64]
@@ -451,13 +457,18 @@ def _scratch(like, need, least):
 
 def _enqueue_dense(problems, flags, stream):
     """Enqueues Dense problems -- (x, weights, biases, outs, epilogues, posts) each -- together, with the scratch memory
-    that lets the library cut tiles along K where there are too few of them for the chip.  Returns their outputs."""
+    that lets the library look palettized weights up ahead of the launch where X has many rows, and cut tiles along K where
+    there are too few of them for the chip.  Returns their outputs."""
     packed = [_marshal_dense(*p) for p in problems]
     groups = b"".join(g for _, g, _, _ in packed)  # (what they point to lives in `packed` until the call returns)
     n, L = len(packed), lib()
-    need = L.dt_dense_workspace_bytes(n, groups) if any(M > _ROWS_MAX for _, _, _, M in packed) else 0
+    need = L.dt_dense_scratch_bytes(n, groups) if any(M > _ROWS_MAX for _, _, _, M in packed) else 0
     ws, at, need = _scratch(problems[0][0], need, 0)
-    _check("dt_dense_qx_grouped_ws_f16", L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, at, need))
+    if need:
+        _check("dt_dense_qx_grouped_scratch_f16",
+               L.dt_dense_qx_grouped_scratch_f16(_stream_ptr(stream), n, groups, flags, at, need))
+    else:
+        _check("dt_dense_qx_grouped_ws_f16", L.dt_dense_qx_grouped_ws_f16(_stream_ptr(stream), n, groups, flags, None, 0))
     return [_shape_outs(p[0], M, outs, p[3] is None) for p, (_, _, outs, M) in zip(problems, packed)]
 
 

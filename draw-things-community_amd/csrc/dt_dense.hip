@@ -20,6 +20,7 @@
 #include "dt_dense_any.h"
 #include "dt_dense_launch.h"
 #include "dt_dense_rows.h"
+#include "dt_depalettize.h"
 
 namespace dt {
 
@@ -225,14 +226,21 @@ struct TilePlan {
   int64_t tiles = 0;
   int64_t whole = 0;  // tiles that stay whole; the rest is cut into `split` shares each
   int split = 1;
+  size_t expand_bytes = 0;  // > 0: the weights are written out as fp16 in front of the launch, to this much scratch
   // workspace of the split tiles: their counters, then their slots
   size_t counter_bytes() const { return split > 1 ? ((size_t)(tiles - whole) * kSplitNodes * 4 + 255) & ~(size_t)255 : 0; }
-  size_t bytes() const { return split > 1 ? counter_bytes() + (size_t)((tiles - whole) * split * dense_split_slot_bytes(BM, BN)) : 0; }
+  size_t split_bytes() const { return split > 1 ? counter_bytes() + (size_t)((tiles - whole) * split * dense_split_slot_bytes(BM, BN)) : 0; }
+  size_t bytes() const { return expand_bytes + split_bytes(); }
 };
 
 // Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
 constexpr int64_t kFillTiles = 192;
 constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
+// fp16 copies of a launch's weights.  Few rows do not pay for holding large ones: 512 x 5120 -> 5120 q6p 61 us and 46 on a
+// copy of 50 MB, 512 x 3072 -> 12288 67 and 57 on 72 MB, 512 x 5120 -> 2 x 5120 q5p 87 and 84 on 100 MB.
+constexpr size_t kDenseMaxExpand = (size_t)512 << 20;
+constexpr size_t kDenseFewRowsExpand = (size_t)48 << 20;
+constexpr int64_t kDenseFewRows = 640;
 
 // Estimated time (us) of a launch whose rows enter new blocks at every `step`-th K-tile at most: a fit to 930 launches of
 // 65 .. 4000 rows on the whole card (part of one would need costs of its own; the results do not depend on the layout
@@ -243,7 +251,8 @@ constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
 // turns; and cutting: the launch that zeroes the counters and, for each level of meetings, a way out and in for the sums.
 // (us, uncut / cut: 512 x 5120 -> 2 x 5120 q5p 117 / 88, 128 x 5120 -> 1152 q8p 90 / 37; and left whole because of these
 // terms: 3 x (571 x 4288 -> 7872) q7p 251 / 342, 1000 x 1792 -> 4096 q7p 42 / 48, 721 x 7168 -> 2560 fp16 46 / 52.)
-static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t step) {
+// `expanded`: plain weights that a launch of their own writes first, which also zeroes the counters.
+static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t step, bool expanded) {
   const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8, row = mode == kPalRow;
   const double entering = row ? (wide ? 0.70 : 0.33) / (double)step : 0.0;
   // one workgroup's K-tile with the share `busy` of the compute units at work
@@ -274,23 +283,24 @@ static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t 
   const int64_t shares = (p.tiles - p.whole) * p.split;
   const int levels = p.split > 4 ? 3 : p.split > 2 ? 2 : 1;
   const double mb = 1e-6 * (double)(shares * dense_split_slot_bytes(p.BM, p.BN));
-  return time(p.whole, nk) + time(shares, 2 * ((nk / 2 + p.split - 1) / p.split)) + 5.0 + levels * (3.5 + 0.095 * mb);
+  return time(p.whole, nk) + time(shares, 2 * ((nk / 2 + p.split - 1) / p.split)) + (expanded ? 0.0 : 5.0) + levels * (3.5 + 0.095 * mb);
 }
 
 // The best way to cut tiles of `base`'s shape that `ws_bytes` of workspace allow: all of them, or those of the last,
 // unfilled round of workgroups.  None of up to 32 K-tiles (K = 1024): a cut would gain a few us of 25 at most.
-static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, int64_t step, size_t ws_bytes, double* cost) {
+static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, int64_t step, bool expanded, size_t ws_bytes,
+                            double* cost) {
   TilePlan best = base;
   best.split = 1;
   best.whole = base.tiles;
-  *cost = plan_cost(best, qbits, mode, nk, step);
+  *cost = plan_cost(best, qbits, mode, nk, step, expanded);
   for (int s = 2; nk > 32 && s <= kMaxSplit && nk / s >= 8; s++)
     for (const int64_t whole : {(int64_t)0, base.tiles / kDenseCUs * kDenseCUs}) {
       TilePlan p = base;
       p.split = s;
       p.whole = whole;
       if (p.whole >= p.tiles || p.bytes() > ws_bytes || p.bytes() > kDenseMaxWorkspace) continue;
-      const double t = plan_cost(p, qbits, mode, nk, step);
+      const double t = plan_cost(p, qbits, mode, nk, step, expanded);
       if (t < (best.split > 1 ? 0.97 : 1.0) * *cost) {  // (a finer cut, of more memory, has to be worth it)
         *cost = t;
         best = p;
@@ -300,9 +310,10 @@ static TilePlan best_split(const TilePlan& base, int qbits, int mode, int nk, in
 }
 
 // The layout of one launch over problems hs[0 .. n) (weights [w_begin, w_end) of each; they share K and the weight
-// format).  `wide`: a fused head epilogue needs tiles of 256 features.
-static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws_bytes) {
-  const dt_qx_weight& w0 = hs[0].W[w_begin];
+// format, which w0 stands for; `expanded`: plain fp16, as the copies of palettized weights are).  `wide`: a fused head
+// epilogue needs tiles of 256 features.  *cost: its estimate.
+static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws_bytes,
+                            const dt_qx_weight& w0, bool expanded, double* cost) {
   const int64_t K = hs[0].K;
   const int nk = (int)(K / BK);
   const auto shape = [&](int tile, int BM, int BN) {
@@ -335,6 +346,9 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   const bool big = (((m_max >= 1024) && (n_max >= 256) && t256.tiles >= kFillTiles) && pal_fits_big && !brief) || wide;
   TilePlan base = big ? (m_max < 1024 ? tnarrow : t256) : (!pal_fits_big && tall_ok && m_max >= 1024 && n_max >= 128 && t256.tiles * 2 >= kFillTiles) ? ttall : tsmall;
   const auto pal_mode = [&](const TilePlan& p) { return choose_pal_mode(w0.qbits, w0.qbits == 16 ? 32 : w0.nib, K, p.BM, p.BN, p.tiles); };
+  const int64_t step = pal_step(K, w0.qbits == 16 ? 32 : w0.nib);
+  const double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step, expanded);
+  *cost = start;
   // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate, whose error
   // is up to a tenth, sees a clear gain.
   const char* knob = getenv("DT_DENSE_SPLIT");  // "never" | "always" (as often as can be; for tests); read at every call
@@ -347,17 +361,15 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
     return p.split > 1 && p.bytes() <= std::min(ws_bytes, kDenseMaxWorkspace) ? p : base;
   }
   TilePlan best = base;
-  const int64_t step = pal_step(K, w0.qbits == 16 ? 32 : w0.nib);
-  const double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step);
   // A clear gain: 5 %, and 8 us for launches of up to 30, since a cut's second launch and its workspace cost the host 7
   // beside the 17 of the call, which chains of short launches wait for (a UNet block of 702 tokens, 320 wide, whose
   // feed-forward would gain 6 of 32 us, took 228 us a pass with it and 220 without).
   double least = 0.95 * start;
   const auto consider = [&](const TilePlan& shape) {
     double t;
-    const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, step, ws_bytes, &t);
+    const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, step, expanded, ws_bytes, &t);
     if (t < least && (t > 30.0 || t < start - 8.0)) {
-      least = t;
+      least = *cost = t;
       best = p;
     }
   };
@@ -370,23 +382,110 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   return best;
 }
 
+// The layout of one launch on plain fp16 weights, the palettized ones among them copied to scratch first.  Returns false where
+// that cannot be, or is not wanted.
+static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, TilePlan* plan, double* cost) {
+  const char* knob = getenv("DT_DENSE_EXPAND");  // "never" | "always" (wherever it can be; for tests); read at every call
+  if ((knob && knob[0] == 'n') || (!knob && getenv("DT_DENSE_SPLIT"))) return false;
+  size_t bytes = 0;
+  int64_t weights = 0, m_max = 0;
+  for (int gi = 0; gi < n; gi++) {
+    m_max = std::max(m_max, hs[gi].M);
+    for (int j = w_begin; j < (n > 1 ? hs[gi].n_weights : w_end); j++) {
+      const dt_qx_weight& w = hs[gi].W[j];
+      if (w.qbits == 16) continue;
+      if (w.nib < kDepalMinNib || w.count > 0x7fffffff) return false;  // (the tiled kernel's 32-bit byte offsets)
+      bytes += ((size_t)w.count * 2 + 255) & ~(size_t)255;
+      weights += w.count;
+    }
+  }
+  if (weights == 0 || bytes > ws || bytes > kDenseMaxExpand || (bytes > kDenseFewRowsExpand && m_max <= kDenseFewRows && !knob)) return false;
+  dt_qx_weight f16 = hs[0].W[w_begin];
+  f16.qbits = 16;
+  *plan = plan_format(hs, n, w_begin, w_end, wide, std::min(ws - bytes, kDenseMaxWorkspace), f16, true, cost);
+  plan->expand_bytes = bytes;
+  // A copy costs 3.4 us and 0.44 per million weights, 0.65 where it outgrows the memory-side cache (28 M weights 13 us, 94 M
+  // 61), and the plain launch on it takes 0.93 of its estimate (medians of 700 launches of 65 .. 8192 rows).
+  const double m = 1e-6 * (double)weights;
+  *cost = 0.93 * *cost + 3.4 + 0.44 * m + 0.21 * std::max(0.0, m - 64.0);
+  return true;
+}
+
+// The layout of one launch with `ws` bytes of scratch, of which `expand` says whether fp16 copies of the weights may go
+// into them.
+// The tiled kernel on palettized weights looks every weight up once per tile of rows, at a cost that no schedule hides: 0.6
+// against 0.2 us a K-tile on 128 x 128 tiles, however few the rows.  us, packed / copied: 4608 x 3072 -> 3 x 3072 q6p 284 /
+// 227, 1376 x 3072 -> 12288 q8p 158 / 131, 512 x 3072 -> 3072 q8p 47 / 26; and the other way round 188 x 3840 -> 3 x 8192 q6p
+// 84 / 112, 579 x 256 -> 5376 q6p 9.8 / 12.1.  The gain has to be 5 %, and 6 us since the second launch costs the host as much
+// (a UNet block of short launches, which wait for the host, took 251 us a pass without copies and 279 with one for every
+// launch that the GPU alone would gain by).
+static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, bool expand, double* cost) {
+  const dt_qx_weight& w0 = hs[0].W[w_begin];
+  const TilePlan packed = plan_format(hs, n, w_begin, w_end, wide, std::min(ws, kDenseMaxWorkspace), w0, false, cost);
+  TilePlan plain;
+  double copied;
+  if (!expand || w0.qbits == 16 || !plan_copies(hs, n, w_begin, w_end, wide, ws, &plain, &copied)) return packed;
+  const char* knob = getenv("DT_DENSE_EXPAND");
+  if (!(knob && knob[0] == 'a') && !(copied < 0.95 * *cost && copied < *cost - 6.0)) return packed;
+  *cost = copied;
+  return plain;
+}
+
 // End of the run of weights from i on that share a launch: at most kMaxWeights, of one format, all within the tiled
-// kernels' alignment.  *fused: one of them wants its head epilogue fused.
-static int weight_run(const HostGroup& h, int i, bool* fused) {
-  const dt_qx_weight& w0 = h.W[i];
+// kernels' alignment.  *fused: one of them wants its head epilogue fused.  mixed: plain fp16 weights may be among palettized
+// ones of one format, all of which can be copied to fp16.
+static int weight_run(const HostGroup& h, int i, bool* fused, bool mixed = false) {
+  const dt_qx_weight* first = &h.W[i];
   int end = i;
   for (; end < h.n_weights && end - i < kMaxWeights; end++) {
     const dt_qx_weight& w = h.W[end];
-    if (w.qbits != w0.qbits || (w.qbits != 16 && w.nib != w0.nib) || !h.w_tiled(end)) break;
+    if (!h.w_tiled(end)) break;
+    if (mixed) {
+      if (w.qbits != 16 && (w.nib < kDepalMinNib || (first->qbits != 16 && (w.qbits != first->qbits || w.nib != first->nib)))) break;
+      if (first->qbits == 16) first = &w;
+    } else if (w.qbits != first->qbits || (w.qbits != 16 && w.nib != first->nib)) {
+      break;
+    }
     *fused = *fused || (h.wants_epi(end) && h.fusable(end));
   }
   return end;
+}
+
+// The weights from i on that go out in the next launch of the tiled kernel, and how.
+struct NextLaunch {
+  int end;
+  bool fused = false;
+  TilePlan plan;
+};
+static NextLaunch next_launch(const HostGroup& h, int i, size_t ws, bool expand) {
+  NextLaunch l;
+  double cost;
+  l.end = weight_run(h, i, &l.fused);
+  l.plan = plan_tiles(&h, 1, i, l.end, l.fused, ws, expand, &cost);
+  if (!expand) return l;
+  // Palettized weights and plain ones on the same X -- a LoRA layer's base and down projections -- in one launch, on copies of
+  // the palettized ones, where that is no slower than one launch after the other, each of which costs the host 5 us
+  // (4608 x 3072 -> 3072 q6p and 64 plain features: 91 and 18 us, together 82).
+  NextLaunch all;
+  all.end = weight_run(h, i, &all.fused, true);
+  double together;
+  if (all.end <= l.end || !plan_copies(&h, 1, i, all.end, all.fused, ws, &all.plan, &together)) return l;
+  for (int j = l.end; j < all.end;) {
+    bool fused = false;
+    const int end = std::min(weight_run(h, j, &fused), all.end);
+    double apart;
+    plan_tiles(&h, 1, j, end, fused, ws, true, &apart);
+    cost += apart + 5.0;
+    j = end;
+  }
+  return together < cost ? all : l;
 }
 
 // Scratch memory of a call, or none.
 struct Workspace {
   uint8_t* ptr = nullptr;
   size_t bytes = 0;
+  bool expand = false;  // also for fp16 copies of the weights
 };
 
 // Zeroes the counters of a K-split launch (a fill kernel, so that the launch can be captured in a graph).
@@ -395,17 +494,46 @@ __global__ void dense_zero_counters_kernel(int32_t* counters, int n) {
   if (i < n) counters[i] = 0;
 }
 
-static dt_status launch_plan(hipStream_t s, DenseArgs& a, const TilePlan& plan, const Workspace& ws, int qbits, int mode) {
+// qx: the launch's n_w weights.
+static dt_status launch_plan(hipStream_t s, DenseArgs& a, int n_w, const TilePlan& plan, const Workspace& ws,
+                             const dt_qx_weight* const* qx) {
   a.whole_tiles = (int32_t)plan.whole;
   a.split = plan.split;
   a.partials = nullptr;
   a.counters = nullptr;
+  const int n_counters = plan.split > 1 ? (int)(plan.tiles - plan.whole) * kSplitNodes : 0;
   if (plan.split > 1) {
-    a.counters = reinterpret_cast<int32_t*>(ws.ptr);
-    a.partials = reinterpret_cast<float*>(ws.ptr + plan.counter_bytes());
-    const int n = (int)(plan.tiles - plan.whole) * kSplitNodes;
-    hipLaunchKernelGGL(dense_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
-    if (const dt_status st = launch_status(); st != DT_OK) return st;
+    a.counters = reinterpret_cast<int32_t*>(ws.ptr + plan.expand_bytes);
+    a.partials = reinterpret_cast<float*>(ws.ptr + plan.expand_bytes + plan.counter_bytes());
+  }
+  int qbits = qx[0]->qbits, mode;
+  if (plan.expand_bytes > 0) {
+    DepalettizeMany d = {};
+    d.counters = a.counters;
+    d.n_counters = n_counters;
+    uint8_t* out = ws.ptr;
+    int64_t tiles = 0;
+    for (int i = 0; i < n_w; i++) {
+      if (qx[i]->qbits == 16) continue;
+      qbits = qx[i]->qbits;
+      d.nib = qx[i]->nib;
+      d.w[d.n++] = {a.w[i].data, reinterpret_cast<uint16_t*>(out), qx[i]->count / 32, (int32_t)tiles};
+      a.w[i].data = out;
+      tiles += (qx[i]->count / 32 + 255) / 256;
+      out += ((size_t)qx[i]->count * 2 + 255) & ~(size_t)255;
+    }
+    for (int i = n_w; i < kMaxWeights; i++) a.w[i] = a.w[0];
+    if (const dt_status st = depalettize_many_launch(s, qbits, d, (int)tiles); st != DT_OK) return st;
+    qbits = 16;
+    mode = kPlainF16;
+    a.nib = 32;
+    a.pal_step = 1;
+  } else {
+    mode = choose_pal_mode(qbits, a.nib, a.k, plan.BM, plan.BN, plan.tiles);
+    if (plan.split > 1) {
+      hipLaunchKernelGGL(dense_zero_counters_kernel, dim3((unsigned)((n_counters + 255) / 256)), dim3(256), 0, s, a.counters, n_counters);
+      if (const dt_status st = launch_status(); st != DT_OK) return st;
+    }
   }
   return launch_dense(s, a, plan.tile, qbits, mode);
 }
@@ -486,7 +614,8 @@ static dt_status run_group(hipStream_t s, const HostGroup& h, const Workspace& w
       if (st != DT_OK) return st;
       continue;
     }
-    const TilePlan plan = plan_tiles(&h, 1, i, run_end, any_fused, ws.bytes);
+    const NextLaunch next = next_launch(h, i, ws.bytes, ws.expand);
+    const TilePlan& plan = next.plan;
     const int BM = plan.BM, BN = plan.BN;
     const bool big = BN == 256;
     DenseArgs a;
@@ -499,14 +628,17 @@ static dt_status run_group(hipStream_t s, const HostGroup& h, const Workspace& w
     g.w_begin = 0;
     int tiles_n = 0, cnt = 0;
     const int first = i;
-    for (; i < run_end; i++, cnt++) tiles_n += add_weight(a, cnt, h, i, tiles_n, BN, big && h.wants_epi(i) && h.fusable(i));
+    const dt_qx_weight* qx[kMaxWeights];
+    for (; i < next.end; i++, cnt++) {
+      qx[cnt] = &h.W[i];
+      tiles_n += add_weight(a, cnt, h, i, tiles_n, BN, big && h.wants_epi(i) && h.fusable(i));
+    }
     g.w_end = cnt;
     g.tiles_n = tiles_n;
     if ((int64_t)g.tiles_m * tiles_n > 0x7fffffff) return DT_NO_KERNEL;
     a.total_tiles = g.tiles_m * tiles_n;
     finish_args(a, 1, cnt, K, w0);
-    const int mode = choose_pal_mode(w0.qbits, a.nib, K, BM, BN, plan.tiles);
-    dt_status st = launch_plan(s, a, plan, ws, w0.qbits, mode);
+    dt_status st = launch_plan(s, a, cnt, plan, ws, qx);
     if (st != DT_OK) return st;
     for (int j = first; j < i; j++)
       if (h.wants_epi(j) && !(big && h.fusable(j))) {
@@ -553,7 +685,9 @@ static bool groups_fuse(const HostGroup* hs, int n) {
 
 static dt_status run_groups_fused(hipStream_t s, const HostGroup* hs, int n, const Workspace& ws) {
   const dt_qx_weight& w0 = hs[0].W[0];
-  const TilePlan plan = plan_tiles(hs, n, 0, 0, true, ws.bytes);
+  double cost;
+  const TilePlan plan = plan_tiles(hs, n, 0, 0, true, ws.bytes, ws.expand, &cost);
+  const dt_qx_weight* qx[kMaxWeights];
   const int BM = plan.BM, BN = plan.BN;
   DenseArgs a;
   int cnt = 0;
@@ -568,24 +702,28 @@ static dt_status run_groups_fused(hipStream_t s, const HostGroup* hs, int n, con
     g.tile_begin = (int32_t)tiles;
     g.w_begin = cnt;
     int tiles_n = 0;
-    for (int i = 0; i < h.n_weights; i++, cnt++)
+    for (int i = 0; i < h.n_weights; i++, cnt++) {
+      qx[cnt] = &h.W[i];
       tiles_n += add_weight(a, cnt, h, i, tiles_n, BN, h.wants_epi(i) && h.fusable(i));
+    }
     g.w_end = cnt;
     g.tiles_n = tiles_n;
     tiles += (int64_t)g.tiles_m * tiles_n;
   }
   a.total_tiles = (int32_t)tiles;
   finish_args(a, n, cnt, hs[0].K, w0);
-  const int mode = choose_pal_mode(w0.qbits, a.nib, hs[0].K, BM, BN);
-  dt_status st = launch_plan(s, a, plan, ws, w0.qbits, mode);
+  dt_status st = launch_plan(s, a, cnt, plan, ws, qx);
   for (int gi = 0; gi < n && st == DT_OK; gi++)
     for (int i = 0; i < hs[gi].n_weights && st == DT_OK; i++)
       if (hs[gi].wants_epi(i) && !hs[gi].fusable(i)) st = epilogue_pass(s, hs[gi], i);
   return st;
 }
 
+// The most that a launch may ask for.
+static size_t scratch_limit(bool expand) { return kDenseMaxWorkspace + (expand ? kDenseMaxExpand : 0); }
+
 // The workspace that run_group would use for h.
-static size_t group_workspace(const HostGroup& h) {
+static size_t group_workspace(const HostGroup& h, bool expand) {
   size_t need = 0;
   if (!h.x_ok()) return 0;
   for (int i = 0; i < h.n_weights;) {
@@ -594,11 +732,14 @@ static size_t group_workspace(const HostGroup& h) {
       continue;
     }
     bool wide = false;
-    const int end = weight_run(h, i, &wide);
+    int end = weight_run(h, i, &wide);
     int64_t features = 0;
     for (int j = i; j < end; j++) features += h.W[j].count / h.K;
-    if (dense_rows_features(h.M, h.K, h.W[i].qbits, h.W[i].nib, features) == 0)
-      need = std::max(need, plan_tiles(&h, 1, i, end, wide, kDenseMaxWorkspace).bytes());
+    if (dense_rows_features(h.M, h.K, h.W[i].qbits, h.W[i].nib, features) == 0) {
+      const NextLaunch next = next_launch(h, i, scratch_limit(expand), expand);
+      need = std::max(need, next.plan.bytes());
+      end = next.end;
+    }
     i = end;
   }
   return need;
@@ -676,15 +817,26 @@ DT_EXPORT dt_status dt_dense_qx_grouped_f16(dt_stream stream, int32_t n_groups, 
   return dt::run_groups(stream, n_groups, groups, dt::Workspace{});
 }
 
-DT_EXPORT size_t dt_dense_workspace_bytes(int32_t n_groups, const dt_dense_group* groups) {
+static size_t groups_workspace(int32_t n_groups, const dt_dense_group* groups, bool expand) {
   using namespace dt;
   HostGroup hs[64];
   int n = 0;
   if (gather_groups(n_groups, groups, hs, n) != DT_OK || n == 0) return 0;
-  if (groups_fuse(hs, n)) return plan_tiles(hs, n, 0, 0, true, kDenseMaxWorkspace).bytes();
+  if (groups_fuse(hs, n)) {
+    double cost;
+    return plan_tiles(hs, n, 0, 0, true, scratch_limit(expand), expand, &cost).bytes();
+  }
   size_t need = 0;
-  for (int i = 0; i < n; i++) need = std::max(need, group_workspace(hs[i]));
+  for (int i = 0; i < n; i++) need = std::max(need, group_workspace(hs[i], expand));
   return need;
+}
+
+DT_EXPORT size_t dt_dense_workspace_bytes(int32_t n_groups, const dt_dense_group* groups) {
+  return groups_workspace(n_groups, groups, false);
+}
+
+DT_EXPORT size_t dt_dense_scratch_bytes(int32_t n_groups, const dt_dense_group* groups) {
+  return groups_workspace(n_groups, groups, true);
 }
 
 DT_EXPORT dt_status dt_dense_qx_grouped_ws_f16(dt_stream stream, int32_t n_groups, const dt_dense_group* groups,
@@ -692,5 +844,13 @@ DT_EXPORT dt_status dt_dense_qx_grouped_ws_f16(dt_stream stream, int32_t n_group
   (void)flags;
   if (reinterpret_cast<uintptr_t>(workspace) & 255) return DT_INVALID;
   return dt::run_groups(stream, n_groups, groups,
-                        dt::Workspace{static_cast<uint8_t*>(workspace), workspace ? workspace_bytes : 0});
+                        dt::Workspace{static_cast<uint8_t*>(workspace), workspace ? workspace_bytes : 0, false});
+}
+
+DT_EXPORT dt_status dt_dense_qx_grouped_scratch_f16(dt_stream stream, int32_t n_groups, const dt_dense_group* groups,
+                                                    uint32_t flags, void* scratch, size_t scratch_bytes) {
+  (void)flags;
+  if (reinterpret_cast<uintptr_t>(scratch) & 255) return DT_INVALID;
+  return dt::run_groups(stream, n_groups, groups,
+                        dt::Workspace{static_cast<uint8_t*>(scratch), scratch ? scratch_bytes : 0, true});
 }

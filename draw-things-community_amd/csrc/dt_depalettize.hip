@@ -1,6 +1,7 @@
 // K0: depalettize a packed tensor to fp16 (bit-exact table lookup).
 // HBM-bound byte work: reads count*q/8 + palettes, writes 2*count bytes.
 #include "dt_common.h"
+#include "dt_depalettize.h"
 #include "dt_layout.h"
 
 namespace dt {
@@ -46,34 +47,33 @@ __global__ void __launch_bounds__(256) depalettize32_kernel(const uint8_t* __res
 // instruction of a wave writes 1 KB of consecutive addresses (thread-per-granule stores are 64 bytes apart per lane).
 // Chunk c of thread t is staged at chunk 4 t + (c ^ (t / 4 % 4)): 16 consecutive lanes hit 16 different 16-byte
 // bank groups on the way in (stride of 4 chunks) and on the way out (consecutive chunks).
-constexpr int kDepalMinNib = 512;
+// A thread's indices are asked for ahead of the palettes, so that the two memory latencies are one.
+// tile: which 256 granules of the tensor.
 template <int Q>
-__global__ void __launch_bounds__(256) depalettize_tile_kernel(const uint8_t* __restrict__ packed, int nib,
-                                                             int64_t n_granules, uint16_t* __restrict__ out) {
+__device__ __forceinline__ void depalettize_tile(const uint8_t* __restrict__ packed, int nib, int64_t n_granules,
+                                                 int64_t tile, uint16_t* __restrict__ out) {
   constexpr int MAXP = 8192 / kDepalMinNib + 2;
   __shared__ uint16_t pal[MAXP << Q];
   __shared__ __attribute__((aligned(16))) uint4_t stage[256 * 4];
   const int t = threadIdx.x;
-  const int64_t g0 = (int64_t)blockIdx.x * 256;
+  const int64_t g0 = tile * 256;
   const QxLayout l = make_layout(Q, nib);
   const int64_t g_last = (g0 + 255 < n_granules ? g0 + 255 : n_granules - 1);
   const int64_t b_first = g0 * 32 / nib, b_last = (g_last * 32 + 31) / nib;
   const int n_pal = (int)(b_last - b_first + 1);
+  const int64_t g = g0 + t < n_granules ? g0 + t : g_last;
+  const int64_t b = b_first + (uint32_t)(g * 32 - b_first * nib) / (uint32_t)nib;  // (the difference is below 8192 + nib)
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(packed + index_byte_offset(l, b, g * 32 - b * nib));
+  uint32_t raw[Q];
+#pragma unroll
+  for (int i = 0; i < Q; i++) raw[i] = src[i];
   for (int i = t; i < n_pal << (Q - 1); i += 256) {
     const int p = i >> (Q - 1), e = i & ((1 << (Q - 1)) - 1);
     reinterpret_cast<uint32_t*>(pal)[i] =
         reinterpret_cast<const uint32_t*>(packed + palette_offset(l, b_first + p))[e];
   }
   __syncthreads();
-  const int64_t g = g0 + t;
-  if (g < n_granules) {
-    const int64_t e = g * 32;
-    const int64_t b = e / nib;
-    const int64_t r = e - b * nib;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(packed + index_byte_offset(l, b, r));
-    uint32_t raw[Q];
-#pragma unroll
-    for (int i = 0; i < Q; i++) raw[i] = src[i];
+  {
     uint32_t idx[32];
     unpack32<Q>(raw, idx);
     const uint16_t* mine = pal + ((int)(b - b_first) << Q);
@@ -94,6 +94,37 @@ __global__ void __launch_bounds__(256) depalettize_tile_kernel(const uint8_t* __
     const int src_t = L >> 2, c = L & 3;
     if (L < n_chunks) dst[L] = stage[4 * src_t + (c ^ ((src_t >> 2) & 3))];
   }
+}
+
+template <int Q>
+__global__ void __launch_bounds__(256) depalettize_tile_kernel(const uint8_t* __restrict__ packed, int nib,
+                                                             int64_t n_granules, uint16_t* __restrict__ out) {
+  depalettize_tile<Q>(packed, nib, n_granules, blockIdx.x, out);
+}
+
+// Several weights at once, and the counters of the launch behind it zeroed on the way.
+template <int Q>
+__global__ void __launch_bounds__(256) depalettize_many_kernel(const DepalettizeMany a) {
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < a.n_counters; i += 256) a.counters[i] = 0;
+  int wi = 0;
+#pragma unroll
+  for (int i = 1; i < kDepalMax; i++)
+    if (i < a.n && (int)blockIdx.x >= a.w[i].tile_begin) wi = i;
+  depalettize_tile<Q>(a.w[wi].packed, a.nib, a.w[wi].n_granules, (int)blockIdx.x - a.w[wi].tile_begin, a.w[wi].out);
+}
+
+dt_status depalettize_many_launch(hipStream_t s, int qbits, const DepalettizeMany& a, int tiles) {
+  const dim3 grid((unsigned)tiles), block(256);
+  switch (qbits) {
+    case 4: hipLaunchKernelGGL(depalettize_many_kernel<4>, grid, block, 0, s, a); break;
+    case 5: hipLaunchKernelGGL(depalettize_many_kernel<5>, grid, block, 0, s, a); break;
+    case 6: hipLaunchKernelGGL(depalettize_many_kernel<6>, grid, block, 0, s, a); break;
+    case 7: hipLaunchKernelGGL(depalettize_many_kernel<7>, grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL(depalettize_many_kernel<8>, grid, block, 0, s, a); break;
+    default: return DT_INVALID;
+  }
+  return launch_status();
 }
 
 template <int Q>

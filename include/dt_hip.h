@@ -287,6 +287,16 @@ dt_status dt_dense_qx_grouped_ws_f16(dt_stream stream, int32_t n_groups, const d
                                      uint32_t flags, void* workspace, size_t workspace_bytes);
 
 /*
+ * The same with scratch memory that may also take fp16 copies of the call's palettized weights: where X has rows enough
+ * to pay for it, the weights are looked up once, in a launch of their own, instead of once per tile of rows.  The values
+ * multiplied are the same.  dt_dense_scratch_bytes() says how much the call can use (copies take 2 bytes per weight,
+ * up to 512 MiB for the weights of one launch); with less, or none, it runs as with that much workspace.
+ */
+size_t dt_dense_scratch_bytes(int32_t n_groups, const dt_dense_group* groups);
+dt_status dt_dense_qx_grouped_scratch_f16(dt_stream stream, int32_t n_groups, const dt_dense_group* groups,
+                                          uint32_t flags, void* scratch, size_t scratch_bytes);
+
+/*
  * In place on a [B, S, H, D] view: optional RMSNorm, then optional RoPE.
  *   gamma       : RMSNorm weight, [D] when norm_per_head != 0 (Flux:
  *                 RMSNorm(axis: [3]), Models/Flux1.swift:165), [H*D] when 0

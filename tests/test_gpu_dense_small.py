@@ -353,6 +353,60 @@ def test_dense_c_entry_points_without_workspace(dthip, oracle, monkeypatch, M, q
         assert all(torch.equal(a, b) for a, b in zip(outs, want[kind]))
 
 
+@pytest.mark.parametrize("M,N,K,q,nib", [
+    (70, 8, 64, 6, 4096),                                # less than one block, two granules per row
+    (129, 257, 320, 4, 512), (200, 130, 448, 5, 1024),   # the smallest blocks; a last tile of granules that is not full
+    (300, 600, 704, 7, 8192), (1100, 520, 576, 8, 16384), (260, 300, 640, 8, 544),  # a block per 17 granules
+])
+def test_dense_on_copies_of_the_weights(dthip, oracle, monkeypatch, M, N, K, q, nib):
+    """Weights written out as fp16 ahead of the launch: the same bits as looked up in it, with every kind of tail; cut along K
+    as well; not with less scratch than the copies take; and replayed from a graph."""
+    import torch
+
+    rng = np.random.default_rng(M + N * 3 + K + q)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    pairs = [make(dthip, oracle, rng, n, K, q, nib) for n in (N, 128)]
+    ws, bias = [w for w, _ in pairs], dev((rng.standard_normal(N) * 0.1).astype(np.float16))
+    x, gamma = dev(X), dev((1 + 0.1 * rng.standard_normal(128)).astype(np.float16))
+    epi, res = [None, dthip.HeadEpilogue(gamma, None, 0)], torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    print("dense on copies", M, N, K, q, nib, flush=True)
+    outs = [torch.empty((M, w.shape[0]), dtype=torch.float16, device="cuda") for w in ws]
+    G, keep = _groups(dthip, x, ws, outs)
+    L, s = dthip.lib(), torch.cuda.current_stream().cuda_stream
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    got = {}
+    for knob in ("never", "always"):
+        monkeypatch.setenv("DT_DENSE_EXPAND", knob)
+        res.zero_()
+        got[knob] = dthip.dense_multi(x, ws, [bias, None]) + dthip.dense_multi(x, ws, [bias, None], epilogues=epi)
+        got[knob] += dthip.dense_post(x, ws, [bias, None], [dthip.DensePost(dthip.ACT_GELU_TANH, residual=res), None]) + [res.clone()]
+    check(got["always"][0].cpu().numpy(), X, pairs[0][1], bias.cpu().numpy())
+    assert all(torch.equal(a, b) for a, b in zip(got["always"], got["never"]))
+    need = L.dt_dense_scratch_bytes(1, G)
+    assert need == sum((w.count * 2 + 255) // 256 * 256 for w in ws) and L.dt_dense_workspace_bytes(1, G) == 0
+    scratch = torch.full((need + 256,), 0xff, dtype=torch.uint8, device="cuda")
+    at = (scratch.data_ptr() + 255) & ~255
+    assert L.dt_dense_qx_grouped_scratch_f16(s, 1, G, 0, at + 64, need) == dthip.DT_INVALID
+    assert L.dt_dense_qx_grouped_scratch_f16(s, 1, G, 0, at, need - 256) == 0 and bool((scratch == 0xff).all())
+    plain = dthip.dense_multi(x, ws, [None, None])
+    assert all(torch.equal(a, b) for a, b in zip(outs, plain))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        assert L.dt_dense_qx_grouped_scratch_f16(torch.cuda.current_stream().cuda_stream, 1, G, 0, at, need) == 0
+    for _ in range(3):
+        outs[0].zero_()
+        scratch.fill_(0xff)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, plain))
+    for w, copy in zip(ws, torch.split(scratch[at - scratch.data_ptr():][:need], [(w.count * 2 + 255) // 256 * 256 for w in ws])):
+        assert torch.equal(copy[:w.count * 2].view(torch.float16).view(w.shape), w.dequantize())
+    monkeypatch.setenv("DT_DENSE_SPLIT", "always")
+    cut = dthip.dense_multi(x, ws, [bias, None])
+    check(cut[0].cpu().numpy(), X, pairs[0][1], bias.cpu().numpy())
+    check(cut[1].cpu().numpy(), X, pairs[1][1])
+
+
 def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     """288 tiles: 256 stay whole, the 32 of the second round are cut; against the uncut launch, one fp16 rounding apart."""
     import torch

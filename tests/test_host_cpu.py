@@ -106,6 +106,28 @@ def test_dense_is_cut_where_that_is_faster(dthip, monkeypatch, M, K, N, n, q, ni
     assert (dthip.lib().dt_dense_workspace_bytes(1, G) > 0) == cut
 
 
+@pytest.mark.parametrize("M,K,N,n,q,nib,copied", [
+    (4608, 3072, 3072, 3, 6, 4096, True), (300, 3072, 3072, 1, 8, 16384, True), (2016, 1280, 5120, 1, 4, 512, True),
+    (512, 5120, 5120, 2, 5, 1024, False),    # 100 MB of copies for 512 rows
+    (4096, 320, 320, 1, 6, 4096, False),     # a second launch would cost more than it gains
+    (4608, 3072, 3072, 1, 6, 64, False),     # small blocks are not copied, nor are plain weights
+    (4608, 3072, 3072, 1, 16, 0, False), (64, 3072, 3072, 1, 6, 4096, False), (32760, 5120, 51200, 2, 6, 4096, False),
+])
+def test_dense_scratch_for_copies(dthip, monkeypatch, M, K, N, n, q, nib, copied):
+    """dt_dense_scratch_bytes asks for room for fp16 copies of the weights where the launch is estimated to gain by them."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    addr = ctypes.addressof
+    W = (dthip._QxWeight * n)(*[dthip._QxWeight(4096, q, nib, N * K)] * n)  # (addresses are not looked at)
+    Y, ldy = (ctypes.c_void_p * n)(*[4096] * n), (ctypes.c_int64 * n)(*[N] * n)
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), n, None, addr(Y), addr(ldy), None, None))
+    cut, scratch = dthip.lib().dt_dense_workspace_bytes(1, G), dthip.lib().dt_dense_scratch_bytes(1, G)
+    assert (scratch >= n * N * K * 2) == copied
+    assert copied or scratch == cut
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
+    assert dthip.lib().dt_dense_scratch_bytes(1, G) == cut
+
+
 def test_rows_that_need_no_workspace(dthip):
     """The operators do not ask for workspace up to the rows that the library's streaming kernel takes: one number, twice."""
     import re
