@@ -606,8 +606,8 @@ class LoRANetworkConfiguration:
 class LoRADense:
     """LoRADense(count:configuration:noBias:flags:name:) -- dense(x) + up(scale * down(x)) with the palettized base
     left packed and the fp16 low-rank pair applied beside it (Models/LoRA.swift:85-142; running the LoRA separately
-    is the preferred mode for quantized models, Models/UNetProtocol.swift:696-697).  Three launches of the Dense
-    kernel: down (with the scale in its epilogue) beside the base projection, then up, whose epilogue adds the base
+    is the preferred mode for quantized models, Models/UNetProtocol.swift:696-697).  The Dense kernel on the base and
+    the down projection (with the scale in its epilogue), then on the up projection, whose epilogue adds the base
     projection's result; every intermediate is rounded to fp16 as the reference's separate ops round.  With
     `highPrecision` the pair is fp32 (`down.data` / `up.data` float32 tensors): the branch is computed as
     fp16(up(scale * down(float(x)))) in fp32 throughout (Models/LoRA.swift:117-139) by dt_lora_branch_f32_f16 and added
@@ -663,30 +663,20 @@ class LoRADense:
         if self.configuration.highPrecision:
             return self._high_precision(x, b, p, stream)
         dn, up = self._padded()
-        # The down projection is a few dozen workgroups that wait on memory; the base projection does not depend on
-        # it.  They go out side by side on two streams, and the up projection, whose epilogue adds the base
-        # projection's result and then runs the tail, follows both.  (fp16(base) + fp16(branch) rounds the same
-        # whichever of the two is the addend.)
-        torch = _torch()
-        main = stream if stream is not None else torch.cuda.current_stream(x.device)
-        side = _side_stream(x.device)
-        side.wait_stream(main)
-        down = dense_post(x, [dn], [None], [DensePost(scale=self.configuration.scale)], stream=side)[0]
-        # (making a stream current that is so already costs 8 us)
-        at = stream if x.device.index == torch.cuda.current_device() else main
-        base = dense_multi(x, [self.weight], [b], flags=self.flags, stream=at)[0]
-        main.wait_stream(side)  # every use of x and `down` on the side stream is ordered before what follows on `main`
-        # `down` came from the side stream's pool and is read on `main`: its memory must not go back to that pool's
-        # next user before `main` has passed this point
-        down.record_stream(main)
+        # Base and down projection share x: one call, which puts them into one launch where the base weight is copied to
+        # fp16 for it (the down projection's few tiles then run on compute units that the base projection leaves idle).  The
+        # up projection's epilogue adds the base projection's result and then runs the tail.  (fp16(base) + fp16(branch)
+        # rounds the same whichever of the two is the addend.)
+        base, down = dense_post(x, [self.weight, dn], [b, None], [None, DensePost(scale=self.configuration.scale)],
+                                flags=self.flags, stream=stream)
         tail = DensePost(p.activation, p.gate, p.residual, p.keep_output, addend=base.reshape(-1, self.count))
-        out = dense_post(down, [up], [None], [tail], stream=at)[0]
+        out = dense_post(down, [up], [None], [tail], stream=stream)[0]
         return None if out is None else out.reshape(*x.shape[:-1], self.count)
 
 
 def _lora_high_precision(self, x, b, p, stream):
-    """out = dense(x) + fp16(up32(scale * down32(float(x)))), then the tail: the fp32 branch beside the base projection
-    on a second stream, the sum in the base projection's epilogue."""
+    """out = dense(x) + fp16(up32(scale * down32(float(x)))), then the tail: the fp32 branch, then the base projection with
+    the sum in its epilogue."""
     torch = _torch()
     dn, up = self.down.data, self.up.data
     if dn.dtype != torch.float32 or up.dtype != torch.float32 or not dn.is_contiguous() or not up.is_contiguous():
@@ -698,19 +688,14 @@ def _lora_high_precision(self, x, b, p, stream):
         x2 = x.reshape(-1, K)
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
-    M = x2.shape[0]
-    side = _side_stream(x.device)
-    side.wait_stream(main)
-    with torch.cuda.stream(side):
+        M = x2.shape[0]
+        # (on the caller's stream: the base projection waits for the branch, so there is nothing to run it beside)
         T = torch.empty((M, r), dtype=torch.float32, device=x.device)
         branch = torch.empty((M, self.count), dtype=torch.float16, device=x.device)
-        st = lib().dt_lora_branch_f32_f16(_stream_ptr(side), M, K, x2.data_ptr(), x2.stride(0), dn.data_ptr(), r,
+        st = lib().dt_lora_branch_f32_f16(_stream_ptr(main), M, K, x2.data_ptr(), x2.stride(0), dn.data_ptr(), r,
                                           up.data_ptr(), self.count, float(self.configuration.scale), T.data_ptr(),
                                           branch.data_ptr(), branch.stride(0))
         _check("dt_lora_branch_f32_f16", st)
-    main.wait_stream(side)
-    T.record_stream(main)
-    branch.record_stream(main)
     tail = DensePost(p.activation, p.gate, p.residual, p.keep_output, addend=branch)
     out = dense_post(x2, [self.weight], [b], [tail], flags=self.flags, stream=main)[0]
     return None if out is None else out.reshape(*x.shape[:-1], self.count)

@@ -407,6 +407,25 @@ def test_dense_on_copies_of_the_weights(dthip, oracle, monkeypatch, M, N, K, q, 
     check(cut[1].cpu().numpy(), X, pairs[1][1])
 
 
+@pytest.mark.parametrize("M,N,K,q,nib,rank", [(130, 260, 320, 6, 4096, 16), (300, 512, 448, 8, 16384, 64), (1100, 600, 704, 4, 512, 100)])
+def test_lora_base_and_down_in_one_launch(dthip, oracle, monkeypatch, M, N, K, q, nib, rank):
+    """The base projection on a copy of its weight and the plain down projection go out together: the same bits as one after
+    the other, with and without a tail."""
+    import torch
+
+    rng = np.random.default_rng(M + N + rank)
+    op = dthip.LoRADense(N, dthip.LoRANetworkConfiguration(rank, 0.75, False))
+    op.weight, op.bias = make(dthip, oracle, rng, N, K, q, nib)[0], dev((rng.standard_normal(N) * 0.1).astype(np.float16))
+    op.down, op.up = make(dthip, oracle, rng, rank, K, 16, 0)[0], make(dthip, oracle, rng, N, rank, 16, 0)[0]
+    x, got = dev(rng.standard_normal((M, K)).astype(np.float16)), {}
+    print("lora in one launch", M, N, K, q, nib, rank, flush=True)
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    for knob in ("never", "always"):
+        monkeypatch.setenv("DT_DENSE_EXPAND", knob)
+        got[knob] = [op(x), op(x, dthip.DensePost(dthip.ACT_SWISH))]
+    assert all(torch.equal(a, b) for a, b in zip(got["never"], got["always"]))
+
+
 def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     """288 tiles: 256 stay whole, the 32 of the second round are cut; against the uncut launch, one fp16 rounding apart."""
     import torch
