@@ -27,6 +27,7 @@ struct SdpaArgs {
   const uint16_t* q_rot;
   float q_eps;
   int32_t q_prep;  // any of the above is set
+  int32_t q_norm;  // any q_gamma is (filled by the launcher)
   // Key-split launch (optional; partials == nullptr runs one workgroup per task): workspace for the parts' partial
   // results and the counters of their meetings, sized and laid out by sdpa_split_plan().
   float* partials;

@@ -6,20 +6,29 @@
 // barrier per tile).
 //
 // Everything is computed transposed so that the query index is the MFMA
-// column (lane & 31) in every stage:
+// column in every stage:
 //   S^T = K Q^T          A = K tile rows from LDS, B = Q^T held in registers
-//   O^T = V^T P^T        A = V^T, B = P^T = the S^T accumulator itself
-// The accumulator of a 32x32 MFMA holds, for column q = lane & 31, rows
-// 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  Feeding it back as the B operand
-// only permutes the summation index, so the V^T operand is fetched with the
-// same permutation and P never leaves registers; the softmax row reductions
-// are in-lane plus one exchange with lane ^ 32.  V stays row-major in LDS:
-// the V^T operand (head dimension along lanes, keys along registers) comes
-// from ds_read_b64_tr_b16, which hands lane j of a 16-lane group the element
-// column (j % 4) of the rows addressed by lanes (j / 4) + {0, 4, 8, 12}.
+//   O^T = V^T P^T        A = V^T, B = P^T = the S^T accumulators themselves
+// With 32x32x16 MFMAs the column is lane & 31, and an accumulator holds rows
+// 8*(v/4) + 4*(lane/32) + (v%4), v = 0..15.  With 16x16x32 MFMAs (M16) it is
+// lane & 15 of two blocks of 16 queries, and an accumulator holds rows
+// 4*(lane/16) + v, v = 0..3; those of 32 keys go side by side into one operand.
+// Feeding accumulators back as the B operand only permutes the summation index,
+// so the V^T operand is fetched with the same permutation and P never leaves
+// registers; the softmax row reductions are in-lane plus exchanges between the
+// lane groups of a column.  V stays row-major in LDS: the V^T operand (head
+// dimension along lanes, keys along registers) comes from ds_read_b64_tr_b16,
+// which hands lane j of a 16-lane group the element column (j % 4) of the rows
+// addressed by lanes (j / 4) + {0, 4, 8, 12}.
+//
+// Which MFMA: for the same work 16x16x32 moves a fifth less through the register
+// file, which counts where the launch is limited by the card's power, but leaves
+// the exponentials of the SIMD's other wave 12 of every 16 issue clocks where
+// 32x32x16 leaves 28 of 32 (an exponential takes 8: one to a slot, not three).
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
+#include <type_traits>
 
 #include "dt_common.h"
 #include "dt_qkprep.h"
@@ -45,13 +54,38 @@ __device__ __forceinline__ int k_chunk_swz(int row, int c) {
   if constexpr (DP == 128) return c ^ (row & 15);
   return c ^ ((row >> 1) & 7);
 }
-// V tile: [64 keys][DP] halfs; the transposing read touches 4 consecutive key
-// rows x 64 contiguous bytes per 32 lanes, so 64-byte units are swizzled over
-// the row index.
-template <int DP>
+// V tile: [64 keys][DP] halfs; 32 lanes of the transposing read touch 4
+// consecutive key rows x 64 contiguous bytes (M16: 8 x 32), so units of that
+// many bytes are swizzled over the row index.
+template <int DP, bool M16>
 __device__ __forceinline__ int v_unit_swz(int row, int u) {
-  if constexpr (DP == 128) return u ^ (row & 3);
-  return u ^ ((row >> 1) & 1);
+  if constexpr (M16) return u ^ (DP == 128 ? row & 7 : (row >> 1) & 3);
+  return u ^ (DP == 128 ? row & 3 : (row >> 1) & 1);
+}
+
+// The lane groups of a wave -- two of 32, M16: four of 16 -- hold the same matrix columns: combine them without touching LDS.
+__device__ __forceinline__ void halves16(float v, float& even, float& odd) {  // groups {0, 0, 2, 2} and {1, 1, 3, 3}
+  uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
+  asm volatile("" : "+v"(b));  // (as in halves32)
+  auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  uint32_t x0 = r[0], x1 = r[1];
+  asm volatile("" : "+v"(x0), "+v"(x1));
+  even = __builtin_bit_cast(float, x0);
+  odd = __builtin_bit_cast(float, x1);
+}
+template <bool M16>
+__device__ __forceinline__ float max_groups(float v) {
+  if constexpr (!M16) return max32(v);
+  float a, b;
+  halves16(v, a, b);
+  return max32(fmaxf(a, b));
+}
+template <bool M16>
+__device__ __forceinline__ float sum_groups(float v) {
+  if constexpr (!M16) return sum32(v);
+  float a, b;
+  halves16(v, a, b);
+  return sum32(a + b);
 }
 
 // SPLIT: for launches whose task count -- a task being the 256 query rows of one (batch, head) -- leaves the last round
@@ -62,14 +96,22 @@ __device__ __forceinline__ int v_unit_swz(int row, int u) {
 // registers and goes on to the next meeting, the last of them to the output.  Nobody waits for anybody, and the fold is
 // the same whichever came first.  (Runs of several tasks' parts per workgroup, folded one after the other by the last
 // to arrive, balance better on paper; that kernel needed 370 registers, and its spills made a tile 1.8 times as long.)
-template <int DP, bool PREMUL, bool ONESEG, bool SPLIT>
+//
+// M16: 16x16x32 MFMAs.  DL: head dimension that is multiplied (M16: D rounded up to a block of 16; DP, what a tile row
+// holds, otherwise).
+template <int DP, int DL, bool M16, bool PREMUL, bool ONESEG, bool SPLIT>
 __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   constexpr int ROWB = DP * 2;                 // bytes per tile row
   constexpr int DCH = DP / 8;                  // 16-byte chunks per row
   constexpr int TILE_B = BKV * ROWB;           // bytes of one K (or V) tile
   constexpr int LOADS = BKV * DCH / 512;       // 16-byte chunks per thread per tile (2 at DP = 128)
-  constexpr int DB = DP / 32;                  // 32-wide blocks of the head dimension
-  constexpr int KS = DP / 16;                  // MFMA k-steps over the head dimension
+  constexpr int MB = M16 ? 16 : 32;            // rows and columns of an MFMA
+  constexpr int MK = M16 ? 32 : 16;            // its k-step
+  constexpr int QB = 32 / MB;                  // its blocks in a wave's 32 queries
+  constexpr int NV = M16 ? 4 : 16;             // its sums per lane
+  constexpr int DB = DL / MB;                  // its blocks of the head dimension
+  constexpr int KS = (DL + MK - 1) / MK;       // k-steps over the head dimension
+  typedef typename std::conditional<M16, float4_t, float16_t>::type sums_t;
   static_assert(LOADS >= 1, "tile");
 
   // Two stages each for K and V: a tile is read from one while the next is in
@@ -82,8 +124,8 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int l32 = lane & 31;
-  const int hi = lane >> 5;
+  const int col = lane & (MB - 1);  // row or column of an MFMA block
+  const int grp = lane / MB;        // lane group: which k
 
   // XCD-aware order: tiles of one (batch, head) are consecutive, and each XCD
   // gets a contiguous run, so a head's K/V stay in one XCD's L2.
@@ -116,7 +158,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     const int row = off / ROWB, pc = (off % ROWB) / 16;
     ld_row[i] = row;
     k_ch[i] = k_chunk_swz<DP>(row, pc);  // the swizzles are involutions
-    v_ch[i] = v_unit_swz<DP>(row, pc >> 2) * 4 + (pc & 3);
+    v_ch[i] = M16 ? v_unit_swz<DP, M16>(row, pc >> 1) * 2 + (pc & 1) : v_unit_swz<DP, M16>(row, pc >> 2) * 4 + (pc & 3);
   }
   // slots that no transfer will ever write must not hold NaN patterns
   if (D < DP || Skv % BKV != 0) {
@@ -130,19 +172,19 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   }
 
   // ---- per-lane LDS read offsets --------------------------------------------
-  // K operand: key row kb*32 + l32, chunk 2*ks + hi
+  // K operand: key row kb*MB + col, chunk of the group's 8 head-dim elements in k-step ks
   int k_rd[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) k_rd[ks] = l32 * ROWB + k_chunk_swz<DP>(l32, 2 * ks + hi) * 16;
-  // V^T operand through the transposing read: lane i of a 16-lane group addresses
-  // key row (i / 4) of a 4-key run and 4 head-dim elements at 4 * (i % 4); the
-  // two groups of a half-wave cover head-dim 0..15 and 16..31 of block db.
+  for (int ks = 0; ks < KS; ks++) k_rd[ks] = col * ROWB + k_chunk_swz<DP>(col, ks * (MK / 8) + grp) * 16;
+  // V^T operand through the transposing read: lane i of a 16-lane group addresses key row (i / 4) of a 4-key run and 4
+  // head-dim elements at 4 * (i % 4).  M16: the run is the group's, the elements those of block db.  Else: the run is the
+  // half-wave's, and its two groups cover head-dim 0..15 and 16..31 of block db.
   const int li = lane & 15, dg = (lane >> 4) & 1;
   int v_rd[DB];
 #pragma unroll
   for (int db = 0; db < DB; db++) {
-    const int row = 4 * hi + (li >> 2);  // + multiples of 4 per k-step: the swizzle depends on row & 3 (or (row >> 1) & 1) only
-    v_rd[db] = row * ROWB + v_unit_swz<DP>(row, db) * 64 + dg * 32 + (li & 3) * 8;
+    const int row = 4 * grp + (li >> 2);  // + multiples of 8 (M16: 16) per read: the swizzle depends on row & 3 (7) at most
+    v_rd[db] = row * ROWB + (M16 ? v_unit_swz<DP, M16>(row, db) * 32 : v_unit_swz<DP, M16>(row, db) * 64 + dg * 32) + (li & 3) * 8;
   }
   const float c = PREMUL ? 1.0f : a.scale_log2e;
 
@@ -164,10 +206,11 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   const int hk = h / a.group;
 
   // ---- Q^T fragments straight from global memory -----------------------
-  // B operand of K Q^T: lane holds query column l32, head-dim slots 16*ks + 8*hi + 0..7.
-  half8_t qf[KS];
-  {
-    int64_t qi = (int64_t)qt * QROWS + wave * 32 + l32;
+  // B operand of K Q^T: lane holds query column col of block qb, head-dim slots MK*ks + 8*grp + 0..7.
+  half8_t qf[QB][KS];
+#pragma unroll
+  for (int qb = 0; qb < QB; qb++) {
+    int64_t qi = (int64_t)qt * QROWS + wave * 32 + qb * MB + col;
     if (qi >= Sq) qi = Sq - 1;
     int sg = 0;
 #pragma unroll
@@ -177,16 +220,16 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     uint4_t qraw[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      const int d0 = ks * 16 + hi * 8;
+      const int d0 = ks * MK + grp * 8;
       qraw[ks] = uint4_t{0, 0, 0, 0};
       if (d0 < D) qraw[ks] = *reinterpret_cast<const uint4_t*>(qp + d0);
     }
     if (a.q_prep) {  // uniform
-      // RMSNorm over the head, then the rotation: the row's D elements sit in this lane and in lane ^ 32
+      // RMSNorm over the head, then the rotation: the row's D elements sit in the lanes of this column
       const uint16_t* gam = a.q_gamma[sg];
       const uint16_t* rrow = a.q_rot ? a.q_rot + qi * D : nullptr;
       float inv = 1.f;
-      if (gam) {
+      if (a.q_norm) {  // uniform: some segment has a norm weight, and the sum takes every lane
         float ss = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
@@ -195,8 +238,8 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
 #pragma unroll
           for (int e = 0; e < 8; e++) ss += x[e] * x[e];
         }
-        ss = sum32(ss);
-        inv = 1.0f / sqrtf(ss / (float)D + a.q_eps);
+        ss = sum_groups<M16>(ss);
+        if (gam) inv = 1.0f / sqrtf(ss / (float)D + a.q_eps);
       }
       auto chunk16 = [](const uint16_t* p) __attribute__((always_inline)) {
         if ((reinterpret_cast<uintptr_t>(p) & 15) == 0) return *reinterpret_cast<const uint4_t*>(p);
@@ -207,7 +250,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       };
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) {
-        const int d0 = ks * 16 + hi * 8;
+        const int d0 = ks * MK + grp * 8;
         if (d0 < D) {
           float x[8];
           unpack_chunk(qraw[ks], x);
@@ -218,7 +261,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       }
     }
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[ks] = __builtin_bit_cast(half8_t, qraw[ks]);
+    for (int ks = 0; ks < KS; ks++) qf[qb][ks] = __builtin_bit_cast(half8_t, qraw[ks]);
   }
 
   // ---- K / V tile loaders ------------------------------------------------
@@ -338,43 +381,64 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     }
   };
   // ---- running state -----------------------------------------------------
-  float16_t oacc[DB];
+  sums_t oacc[DB][QB];  // O^T: [block of the head dimension][block of queries]
 #pragma unroll
   for (int db = 0; db < DB; db++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) oacc[db][v] = 0.f;
-  float m_ref = -INFINITY;  // reference for the exponentials (raw score units); trails the true running maximum
-  float l_run = 0.f;        // this lane's share of the row sum
+    for (int qb = 0; qb < QB; qb++)
+#pragma unroll
+      for (int v = 0; v < NV; v++) oacc[db][qb][v] = 0.f;
+  float m_ref[QB];  // reference for the exponentials (raw score units); trails the true running maximum
+  float l_run[QB];  // this lane's share of the row sums
+#pragma unroll
+  for (int qb = 0; qb < QB; qb++) {
+    m_ref[qb] = -INFINITY;
+    l_run[qb] = 0.f;
+  }
 
-  float16_t sacc[2];   // S^T of the tile in flight (keys x queries)
-  half8_t pf[2][2];    // its probabilities, as the B operand of the second MFMA
+  constexpr int KB = BKV / MB;        // blocks of keys in a tile
+  constexpr int PK = M16 ? 32 : 16;   // keys of a second MFMA
+  sums_t sacc[KB][QB];                // S^T of the tile in flight: [block of keys][block of queries]
+  half8_t pf[BKV / PK][QB];           // its probabilities, as the B operand of the second MFMA
+  auto mfma = [](half8_t a, half8_t b, sums_t sum) __attribute__((always_inline)) {
+    if constexpr (M16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, sum, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, sum, 0, 0, 0);
+  };
 
   // S^T = K Q^T for the K tile in stage st
   auto s_phase = [&](const unsigned char* kt) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kb = 0; kb < 2; kb++)
+    for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-      for (int v = 0; v < 16; v++) sacc[kb][v] = 0.f;
-    // K fragments are read two k-steps (4 reads) ahead of the MFMAs that use them
+      for (int qb = 0; qb < QB; qb++)
+#pragma unroll
+        for (int v = 0; v < NV; v++) sacc[kb][qb][v] = 0.f;
+    // K fragments are read a group of four ahead of the MFMAs that use them: KB blocks of 4 / KB k-steps
+    constexpr int GS = 4 / KB;
     half8_t kf[2][4];
-    // (a k-step that lies wholly in the zero padding of a short head -- the fourth at D = 40 -- is left out)
-    auto live = [&](int ks) __attribute__((always_inline)) { return DP != 64 || ks * 16 < D; };
+    // (a k-step that lies wholly in the zero padding of a short head -- the fourth of 16 at D = 40 -- is left out)
+    auto live = [&](int ks) __attribute__((always_inline)) { return M16 || DP != 64 || ks * MK < D; };
     auto read_k = [&](int buf, int g) __attribute__((always_inline)) {
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (live(2 * g + (u >> 1)))
-          kf[buf][u] = *reinterpret_cast<const half8_t*>(kt + (u & 1) * 32 * ROWB + k_rd[2 * g + (u >> 1)]);
+      for (int u = 0; u < 4; u++) {
+        const int ks = g * GS + u / KB, kb = u % KB;
+        if (ks < KS && live(ks)) kf[buf][u] = *reinterpret_cast<const half8_t*>(kt + kb * MB * ROWB + k_rd[ks < KS ? ks : 0]);
+      }
     };
     read_k(0, 0);
 #pragma unroll
-    for (int g = 0; g < KS / 2; g++) {
+    for (int g = 0; g * GS < KS; g++) {
       __builtin_amdgcn_sched_barrier(0);
-      if (g + 1 < KS / 2) read_k((g + 1) & 1, g + 1);
+      if ((g + 1) * GS < KS) read_k((g + 1) & 1, g + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (live(2 * g + (u >> 1)))
-          sacc[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[g & 1][u], qf[2 * g + (u >> 1)], sacc[u & 1], 0, 0, 0);
+      for (int u = 0; u < 4; u++) {
+        const int ks = g * GS + u / KB, kb = u % KB;
+        if (ks < KS && live(ks)) {
+#pragma unroll
+          for (int qb = 0; qb < QB; qb++) sacc[kb][qb] = mfma(kf[g & 1][u], qf[qb][ks < KS ? ks : 0], sacc[kb][qb]);
+        }
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -385,89 +449,108 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     const bool ragged = rem < BKV;
     if (PREMUL || ragged) {
 #pragma unroll
-      for (int kb = 0; kb < 2; kb++)
+      for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-          float s = sacc[kb][v];
-          if (PREMUL) s *= a.scale_log2e;
-          if (ragged) {
-            const int kj = kb * 32 + 8 * (v >> 2) + 4 * hi + (v & 3);
-            if (kj >= rem) s = -INFINITY;
+        for (int qb = 0; qb < QB; qb++)
+#pragma unroll
+          for (int v = 0; v < NV; v++) {
+            float s = sacc[kb][qb][v];
+            if (PREMUL) s *= a.scale_log2e;
+            if (ragged) {
+              const int kj = kb * MB + 8 * (v >> 2) + 4 * grp + (v & 3);
+              if (kj >= rem) s = -INFINITY;
+            }
+            sacc[kb][qb][v] = s;
           }
-          sacc[kb][v] = s;
-        }
     }
-    // Probabilities against the current reference, and this lane's share of their row sum.  The tile's maximum is
-    // not looked for: as long as every lane's sum stays below 2^10 no probability exceeds that (fp16 holds 2^16),
+    // Probabilities against the current reference, and this lane's share of their row sums.  The tile's maximum is
+    // not looked for: as long as every lane's sums stay below 2^10 no probability exceeds that (fp16 holds 2^16),
     // which is all that the reference is there to ensure.
-    float psum;
+    float psum[QB];
     auto probabilities = [&]() __attribute__((always_inline)) {
-      const float mc = m_ref * c;
-      psum = 0.f;
+      float mc[QB];
 #pragma unroll
-      for (int kb = 0; kb < 2; kb++)
+      for (int qb = 0; qb < QB; qb++) {
+        mc[qb] = m_ref[qb] * c;
+        psum[qb] = 0.f;
+      }
 #pragma unroll
-        for (int tt = 0; tt < 2; tt++)
+      for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-          for (int e = 0; e < 8; e++) {
-            const float p = fast_exp2(__builtin_fmaf(sacc[kb][8 * tt + e], c, -mc));
-            psum += p;
-            pf[kb][tt][e] = (half_t)p;
+        for (int v = 0; v < NV; v++)
+#pragma unroll
+          for (int qb = 0; qb < QB; qb++) {
+            const float p = fast_exp2(__builtin_fmaf(sacc[kb][qb][v], c, -mc[qb]));
+            psum[qb] += p;
+            const int slot = kb * NV + v;  // of this lane's scores: eight to an operand
+            pf[slot >> 3][qb][slot & 7] = (half_t)p;
           }
     };
     probabilities();
-    // (the first tile arrives here with the reference at -inf: its sums are inf; a NaN fails the test too)
-    if (__builtin_amdgcn_ballot_w64(!(psum <= 1024.0f)) != 0) {
+    // (the first tile arrives here with the references at -inf: its sums are inf; a NaN fails the test too)
+    bool outgrown = !(psum[0] <= 1024.0f);
+    if constexpr (QB == 2) outgrown = outgrown || !(psum[1] <= 1024.0f);
+    if (__builtin_amdgcn_ballot_w64(outgrown) != 0) {
       // some row's scores have outgrown the reference: move every row's reference up to its running maximum,
       // rescale what has been accumulated, and redo this tile's probabilities
-      float mx = sacc[0][0];
 #pragma unroll
-      for (int kb = 0; kb < 2; kb++)
+      for (int qb = 0; qb < QB; qb++) {
+        float mx = sacc[0][qb][0];
 #pragma unroll
-        for (int v = (kb == 0 ? 1 : 0); v < 16; v++) mx = fmaxf(mx, sacc[kb][v]);
-      mx = max32(mx);
-      // (Finite even where every score so far is -inf -- keys masked through the dot product itself: against a
-      // reference of -inf the probabilities would be NaN, in a part of the keys that counts for nothing.  No finite
-      // score lies below: |q k| <= 128 * 65504^2 = 5.5e11, and PREMUL's own scale has the whole range of fp32.)
-      const float m_new = fmaxf(fmaxf(m_ref, mx), PREMUL ? -3e38f : -1e12f);
-      const float alpha = fast_exp2((m_ref - m_new) * c);  // first tile: exp2(-inf) = 0
-      m_ref = m_new;
-      l_run *= alpha;
+        for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-      for (int db = 0; db < DB; db++)
+          for (int v = (kb == 0 ? 1 : 0); v < NV; v++) mx = fmaxf(mx, sacc[kb][qb][v]);
+        mx = max_groups<M16>(mx);
+        // (Finite even where every score so far is -inf -- keys masked through the dot product itself: against a
+        // reference of -inf the probabilities would be NaN, in a part of the keys that counts for nothing.  No finite
+        // score lies below: |q k| <= 128 * 65504^2 = 5.5e11, and PREMUL's own scale has the whole range of fp32.)
+        const float m_new = fmaxf(fmaxf(m_ref[qb], mx), PREMUL ? -3e38f : -1e12f);
+        const float alpha = fast_exp2((m_ref[qb] - m_new) * c);  // first tile: exp2(-inf) = 0
+        m_ref[qb] = m_new;
+        l_run[qb] *= alpha;
 #pragma unroll
-        for (int v = 0; v < 16; v++) oacc[db][v] *= alpha;
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+          for (int v = 0; v < NV; v++) oacc[db][qb][v] *= alpha;
+      }
       probabilities();
     }
-    l_run += psum;
+#pragma unroll
+    for (int qb = 0; qb < QB; qb++) l_run[qb] += psum[qb];
   };
 
   // O^T += V^T P^T for the V tile in stage st.
-  // k-slot e of lane half `hi` in 16-key step s is key 16*s + 8*(e/4) + 4*hi + (e%4).
+  // k-slot e of lane group grp in step s of PK keys is key PK*s + (PK/2)*(e/4) + 4*grp + (e%4).
   auto pv_phase = [&](const unsigned char* vt) __attribute__((always_inline)) {
     typedef __attribute__((address_space(3))) short4_t lds_s4;
     typedef short short8_t __attribute__((ext_vector_type(8)));
-    // V^T fragments of the next 16-key step are read while the current step's MFMAs run
-    short4_t vlo[2][DB], vhi[2][DB];
-    auto read_v = [&](int buf, int step) __attribute__((always_inline)) {
-      const int koff = 16 * step * ROWB;
+    // V^T fragments (DB blocks per step) go in groups of up to four, the next group read while the current one's MFMAs run
+    constexpr int GF = M16 ? 4 : DB, NF = BKV / PK * DB, NG = (NF + GF - 1) / GF;
+    short4_t vlo[2][GF], vhi[2][GF];
+    auto read_v = [&](int buf, int g) __attribute__((always_inline)) {
 #pragma unroll
-      for (int db = 0; db < DB; db++) {
-        vlo[buf][db] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + koff + v_rd[db]));
-        vhi[buf][db] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + koff + 8 * ROWB + v_rd[db]));
+      for (int u = 0; u < GF; u++) {
+        const int f = g * GF + u, koff = PK * (f / DB) * ROWB;
+        if (f >= NF) continue;
+        vlo[buf][u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + koff + v_rd[f % DB]));
+        vhi[buf][u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + koff + PK / 2 * ROWB + v_rd[f % DB]));
       }
     };
     read_v(0, 0);
 #pragma unroll
-    for (int step = 0; step < 4; step++) {
+    for (int g = 0; g < NG; g++) {
       __builtin_amdgcn_sched_barrier(0);
-      if (step + 1 < 4) read_v((step + 1) & 1, step + 1);
+      if (g + 1 < NG) read_v((g + 1) & 1, g + 1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int db = 0; db < DB; db++) {
-        const short4_t lo = vlo[step & 1][db], h4 = vhi[step & 1][db];
+      for (int u = 0; u < GF; u++) {
+        const int f = g * GF + u;
+        if (f >= NF) continue;
+        const short4_t lo = vlo[g & 1][u], h4 = vhi[g & 1][u];
         const short8_t v8 = short8_t{lo[0], lo[1], lo[2], lo[3], h4[0], h4[1], h4[2], h4[3]};
-        oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, v8), pf[step >> 1][step & 1], oacc[db], 0, 0, 0);
+#pragma unroll
+        for (int qb = 0; qb < QB; qb++)
+          oacc[f % DB][qb] = mfma(__builtin_bit_cast(half8_t, v8), pf[f / DB][qb], oacc[f % DB][qb]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -520,38 +603,44 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   }
   __builtin_amdgcn_s_setprio(0);
 
+  // the row sums, the same in every group of lanes from here on
+#pragma unroll
+  for (int qb = 0; qb < QB; qb++) l_run[qb] = sum_groups<M16>(l_run[qb]);
+
   // ---- normalise and store O ----------------------------------------------
-  // O^T block db: lane holds query column l32 and head-dim 8*g + 4*hi + (0..3);
-  // swapping the odd groups of the low half-wave with the even groups of the
-  // high half-wave leaves every lane with runs of 8 consecutive head-dim
-  // elements (16-byte stores).
+  // Runs of 8 consecutive head-dim elements per lane (16-byte stores) out of its runs of four: 32x32 blocks hold head-dim
+  // 8*g + 4*grp + (0..3), and swapping the odd groups g of the low half-wave with the even ones of the high half-wave does
+  // it; 16x16 blocks hold 4*grp + (0..3), and the odd lane groups of one block are swapped with the even ones of the next.
   auto store_output = [&]() __attribute__((always_inline)) {
-    const int64_t qi = (int64_t)qt * QROWS + wave * 32 + l32;
-    const float l_tot = sum32(l_run);
-    const float inv = 1.0f / l_tot;
-    uint16_t* op = a.o + b * a.o_sb + (qi < Sq ? qi : 0) * a.o_ss + h * a.o_sh;
     const bool vec_ok = ((a.o_sb | a.o_ss | a.o_sh) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.o) & 15) == 0;
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
-      uint32_t pk[4][2];
+    for (int qb = 0; qb < QB; qb++) {
+      const int64_t qi = (int64_t)qt * QROWS + wave * 32 + qb * MB + col;
+      const float inv = 1.0f / l_run[qb];
+      uint16_t* op = a.o + b * a.o_sb + (qi < Sq ? qi : 0) * a.o_ss + h * a.o_sh;
+      constexpr int RUNS = DB * NV / 4;  // this lane's runs of four
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        pk[g][0] = (uint32_t)half_to_bits((half_t)(oacc[db][4 * g] * inv)) |
-                   ((uint32_t)half_to_bits((half_t)(oacc[db][4 * g + 1] * inv)) << 16);
-        pk[g][1] = (uint32_t)half_to_bits((half_t)(oacc[db][4 * g + 2] * inv)) |
-                   ((uint32_t)half_to_bits((half_t)(oacc[db][4 * g + 3] * inv)) << 16);
-      }
+      for (int r = 0; r < RUNS; r += 2) {
+        uint32_t pk[2][2];
 #pragma unroll
-      for (int gp = 0; gp < 2; gp++) {
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            const int n = (r + u < RUNS ? r + u : r) * 4 + 2 * e;  // (past the last block: never stored)
+            pk[u][e] = (uint32_t)half_to_bits((half_t)(oacc[n / NV][qb][n % NV] * inv)) |
+                       ((uint32_t)half_to_bits((half_t)(oacc[n / NV][qb][n % NV + 1] * inv)) << 16);
+          }
         uint32_t run[4];
 #pragma unroll
         for (int e = 0; e < 2; e++) {
-          auto r = __builtin_amdgcn_permlane32_swap(pk[2 * gp][e], pk[2 * gp + 1][e], false, false);
-          run[e] = r[0];
-          run[2 + e] = r[1];
+          uint32_t x = pk[0][e], y = pk[1][e];
+          if constexpr (RUNS % 2) asm volatile("" : "+v"(y));  // (the swap needs two distinct registers)
+          auto got = M16 ? __builtin_amdgcn_permlane16_swap(x, y, false, false) : __builtin_amdgcn_permlane32_swap(x, y, false, false);
+          run[e] = got[0];
+          run[2 + e] = got[1];
         }
-        const int d0 = db * 32 + 16 * gp + 8 * hi;
-        if (qi < Sq && d0 < D) {
+        const int d0 = M16 ? (r + (grp & 1)) * 16 + 8 * (grp >> 1) : r * 8 + 8 * grp;
+        if (qi < Sq && d0 < D && (M16 ? r + (grp & 1) < RUNS : true)) {
           if (vec_ok) {
             *reinterpret_cast<uint4_t*>(op + d0) = uint4_t{run[0], run[1], run[2], run[3]};
           } else {
@@ -566,8 +655,8 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   if constexpr (SPLIT) {
     if (!takes_whole) {
       __shared__ int s_seen;
-      // Slot layout (floats): [DB * 16 accumulators][512 threads], then [512] reference maxima, then [512] row-sum
-      // shares: a wave's access covers 256 consecutive bytes.  The parts of a task run on any compute units of the
+      // Slot layout (floats): [DP / 2 accumulators][512 threads] (those past DL unused), then [512]: for a wave, the
+      // reference maxima of its 32 queries and their row sums.  A wave's access covers 256 consecutive bytes.  The parts of a task run on any compute units of the
       // device, whose L2 caches (one per die) do not see each other's ordinary stores: slots are written and read with
       // device-scope accesses (relaxed atomics: write-through stores, loads that do not trust a die's cached copy)
       // instead of bracketing ordinary accesses with cache-wide write-backs and invalidations, which cost far more than
@@ -589,10 +678,12 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
 #pragma unroll
             for (int db = 0; db < DB; db++)
 #pragma unroll
-              for (int v = 0; v < 16; v++)
-                __hip_atomic_store(own + (db * 16 + v) * 512, oacc[db][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(own + DB * 16 * 512, m_ref, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(own + DB * 16 * 512 + 512, l_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              for (int qb = 0; qb < QB; qb++)
+#pragma unroll
+                for (int v = 0; v < NV; v++)
+                  __hip_atomic_store(own + ((db * QB + qb) * NV + v) * 512, oacc[db][qb][v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const float stat = lane & 32 ? (grp & (QB - 1) ? l_run[QB - 1] : l_run[0]) : (grp & (QB - 1) ? m_ref[QB - 1] : m_ref[0]);
+            __hip_atomic_store(own + DP / 2 * 512, stat, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             // every wave's stores have been acknowledged before the barrier, hence before the count that publishes them
             __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
             __syncthreads();
@@ -602,26 +693,38 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
           }
           const float* const theirs = slots + (other << level) * slot_step;
           auto ld = [&](int i) __attribute__((always_inline)) {
-            return __hip_atomic_load(theirs + i * 512, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return __hip_atomic_load(theirs + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           };
-          const float m_o = ld(DB * 16), l_o = ld(DB * 16 + 1);
-          const float m_new = fmaxf(m_ref, m_o);
-          const float wa = fast_exp2((m_ref - m_new) * c), wb = fast_exp2((m_o - m_new) * c);
-          // a wa + b wb with both products rounded: the same for either order
-          auto fold = [&](float mine, float got) __attribute__((always_inline)) {
-            float x = mine * wa, y = got * wb;
-            asm volatile("" : "+v"(x), "+v"(y));
-            return x + y;
-          };
-          m_ref = m_new;
-          l_run = fold(l_run, l_o);
+          // (theirs is this thread's place: - lane + col is its column's in the first group of lanes)
+          const int stats = DP / 2 * 512 - lane + col;
 #pragma unroll
-          for (int db = 0; db < DB; db++) {
-            float16_t got;
+          for (int qb = 0; qb < QB; qb++) {
+            const float m_o = ld(stats + MB * qb), l_o = ld(stats + 32 + MB * qb);
+            const float m_new = fmaxf(m_ref[qb], m_o);
+            const float wa = fast_exp2((m_ref[qb] - m_new) * c), wb = fast_exp2((m_o - m_new) * c);
+            // a wa + b wb with both products rounded: the same for either order
+            auto fold = [&](float mine, float got) __attribute__((always_inline)) {
+              float x = mine * wa, y = got * wb;
+              asm volatile("" : "+v"(x), "+v"(y));
+              return x + y;
+            };
+            m_ref[qb] = m_new;
+            l_run[qb] = fold(l_run[qb], l_o);
+            constexpr int AT = 16 / NV;  // blocks whose sums are asked for together
 #pragma unroll
-            for (int v = 0; v < 16; v++) got[v] = ld(db * 16 + v);
+            for (int d0 = 0; d0 < DB; d0 += AT) {
+              sums_t got[AT];
 #pragma unroll
-            for (int v = 0; v < 16; v++) oacc[db][v] = fold(oacc[db][v], got[v]);
+              for (int u = 0; u < AT; u++)
+                if (d0 + u < DB)
+#pragma unroll
+                  for (int v = 0; v < NV; v++) got[u][v] = ld((((d0 + u) * QB + qb) * NV + v) * 512);
+#pragma unroll
+              for (int u = 0; u < AT; u++)
+                if (d0 + u < DB)
+#pragma unroll
+                  for (int v = 0; v < NV; v++) oacc[d0 + u][qb][v] = fold(oacc[d0 + u][qb][v], got[u][v]);
+            }
           }
           __syncthreads();  // s_seen may be written again
         }
@@ -708,8 +811,10 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
   return true;
 }
 
-template <int DP>
+template <int DP, int DL, bool M16>
 static dt_status launch(hipStream_t s, SdpaArgs a) {
+  a.q_norm = 0;
+  for (int i = 0; i < a.n_qseg; i++) a.q_norm |= a.q_gamma[i] != nullptr;
   a.q_tiles = (int)((a.Sq + QROWS - 1) / QROWS);
   int64_t total = (int64_t)a.q_tiles * a.Hq * a.B;
   if (total > 0x7fffffff) return DT_NO_KERNEL;
@@ -719,8 +824,9 @@ static dt_status launch(hipStream_t s, SdpaArgs a) {
   const bool oneseg = a.n_kvseg == 1 && a.k[0].ss > 0 && a.v[0].ss > 0 && a.Skv < (1 << 30) &&
                       (a.Skv + 2 * BKV) * a.k[0].ss * 2 < 0x7fffffffLL && (a.Skv + 2 * BKV) * a.v[0].ss * 2 < 0x7fffffffLL;
   dim3 block(512);
-  if (a.partials) {
-    // key-split launch: the counters start at zero
+  if constexpr (DP == 64 || M16) if (a.partials) {
+    // key-split launch (never of the few long tasks that 32x32x16 MFMAs take at head sizes above 64): the counters start at
+    // zero
     if (!a.counters_zeroed) {
       const int n = a.cut_tasks * kSdpaSplitNodes;
       hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
@@ -729,29 +835,38 @@ static dt_status launch(hipStream_t s, SdpaArgs a) {
     a.total_blocks = a.cut_tasks * a.shares;  // (of the cut tasks)
     dim3 grid((unsigned)(a.whole_tasks + a.total_blocks));
     if (oneseg) {
-      if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, true, true, true>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((sdpa_kernel<DP, false, true, true>), grid, block, 0, s, a);
+      if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, true, true>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, true, true>), grid, block, 0, s, a);
     } else {
-      if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, true, false, true>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((sdpa_kernel<DP, false, false, true>), grid, block, 0, s, a);
+      if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, false, true>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, false, true>), grid, block, 0, s, a);
     }
     return launch_status();
   }
   dim3 grid((unsigned)total);
   if (oneseg) {
-    if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, true, true, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((sdpa_kernel<DP, false, true, false>), grid, block, 0, s, a);
+    if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, true, false>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, true, false>), grid, block, 0, s, a);
   } else {
-    if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, true, false, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((sdpa_kernel<DP, false, false, false>), grid, block, 0, s, a);
+    if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, false, false>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, false, false>), grid, block, 0, s, a);
   }
   return launch_status();
 }
 
 dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
   if (a.B <= 0 || a.Sq <= 0) return DT_OK;
-  if (a.D <= 64) return launch<64>(s, a);
-  return launch<128>(s, a);
+  // Head sizes up to 64 have an exponential for every two to four MFMAs and are bound by the exponentials (M16: 4096 queries,
+  // 16 heads of 40 73 us against 81, 20 heads of 64 113 against 122).  Above, 16x16x32 is ahead where the workgroups fill
+  // the card, whose power then is the limit, and behind where under seven tenths of the compute units have one and the clock
+  // stays up (us, 32x32x16 / 16x16x32, head size 128: 120 workgroups 34.8 / 36.9, 144 101 / 108, 168 47.2 / 48.3, 192 104
+  // / 99, 216 66.9 / 63.1, 264 cut along the keys 111 / 109, 432 250 / 235, 1440 of 141 key tiles 1495 / 1398; head size 80:
+  // 144 56.7 / 58.4, 256 113 / 96).
+  if (a.D <= 64) return launch<64, 64, false>(s, a);
+  const int64_t tasks = (a.Sq + QROWS - 1) / QROWS * a.Hq * a.B;
+  if (!a.partials && tasks * 10 < compute_units() * 7LL) return launch<128, 128, false>(s, a);
+  if (a.D <= 80) return launch<128, 80, true>(s, a);
+  return launch<128, 128, true>(s, a);
 }
 
 }  // namespace dt

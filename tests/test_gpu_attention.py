@@ -152,6 +152,36 @@ def test_sdpa_vs_oracle(dthip, oracle, torch_cuda, B, Sq, Skv, Hq, Hk, D):
     assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
 
 
+@pytest.mark.parametrize("D,Sq,Skv,n_seg,sign,prep", [
+    (72, 17, 65, 1, 1, False), (80, 33, 130, 2, 1, True), (88, 16, 64, 1, -1, False), (96, 20, 63, 2, -1, False),
+    (120, 31, 129, 1, 1, True), (128, 300, 70, 2, 1, False), (128, 1, 1, 1, 1, False), (128, 31, 191, 1, -1, True),
+])
+def test_sdpa_card_full_of_workgroups(dthip, oracle, torch_cuda, D, Sq, Skv, n_seg, sign, prep):
+    """Head sizes above 64 on enough workgroups for the 16x16x32 form (2 x 129 heads), against the oracle and, within a rounding
+    of the probabilities and one of the result, against the same heads one batch entry and a few at a time (32x32x16)."""
+    torch = torch_cuda
+    rng = np.random.default_rng(D * 1000 + Sq + Skv)
+    B, H, few = 2, 129, 3
+    q, k, v = rand_qkv(rng, B, Sq, Skv, H, H, D)
+    scale, cut = sign / np.sqrt(D), Skv // 3 + 1 if n_seg == 2 else Skv
+    qd, kd, vd = (to_dev(torch, t) for t in (q, k, v))
+    more, qn = {}, q
+    if prep:
+        gamma, rot = f16(1 + 0.1 * rng.standard_normal(D)), f16(rng.standard_normal((Sq, D)))
+        more = {"gamma_q": [to_dev(torch, gamma)], "rot_q": to_dev(torch, rot)}
+        qn = np.stack([oracle.C.cmul(oracle.C.rmsnorm(x, gamma, 1e-6), rot) for x in q])
+    print("sdpa card full", D, Sq, Skv, n_seg, sign, prep, flush=True)
+    call = lambda b, h: dthip.sdpa_segments([qd[b, :, h]], [t for t in (kd[b, :cut, h], kd[b, cut:, h]) if t.shape[1]],
+                                            [t for t in (vd[b, :cut, h], vd[b, cut:, h]) if t.shape[1]], scale, **more)
+    got = call(slice(None), slice(None))
+    some = call(slice(0, 1), slice(0, few))
+    torch.cuda.synchronize()
+    mx, rr = oracle.err_stats(got.cpu().numpy(), oracle.C.sdpa(qn, k, v, scale))
+    assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+    # |o| <= max |v| < 6: 2^-11 of it for the probabilities and half an ulp of a value below 8 for either result
+    assert float((got[:1, :, :few].float() - some.float()).abs().max()) <= 6 * 2.0 ** -10 + 2.0 ** -8
+
+
 def test_sdpa_invariants(dthip, oracle, torch_cuda):
     torch = torch_cuda
     rng = np.random.default_rng(5)
