@@ -66,8 +66,20 @@ __device__ __forceinline__ float act_gelu_tanh(float x) {
 __device__ __forceinline__ float act_swish(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
 }
-// 1 + erf(z) = erfc(-z): no cancellation for large negative x
-__device__ __forceinline__ float act_gelu_erf(float x) { return 0.5f * x * erfcf(x * -0.7071067811865476f); }
+// x Phi(x) = (x + |x| - 2 |x| Phi(-|x|)) / 2, and 2 Phi(-a) = erfc(a / sqrt 2) = 2^(a p(a)): its logarithm is so smooth that a
+// polynomial of degree 10 (least maximum error, fitted to float64 values) is as good as fp32 can hold, in 15 instructions without
+// a branch.  Behind a = 5.8 the result is below half of fp16's least value.  Over all fp16 x: relative error against float64 4.9e-8
+// rms, 8.2e-7 at most (erfcf: 6.3e-8, 1.1e-6); infinities and NaN come out as they do of x (1 + erf(x / sqrt 2)) / 2.
+// us, erfcf / this: 2016 x 1280 -> 5120 fp16 53.2 / 46.8, 8192 x 320 -> 1280 q6p 37.0 / 29.1 (39.0 and 22.7 without a tail).
+__device__ __forceinline__ float act_gelu_erf(float x) {
+  constexpr float kP[11] = {-0x1.26aecap+0f, -0x1.d63d8ap-2f, -0x1.ad94ap-5f, 0x1.c5ee4ap-8f, 0x1.398282p-15f, -0x1.477c1cp-12f,
+                            0x1.83bca8p-14f, -0x1.056702p-16f, 0x1.b7899ap-20f, -0x1.acf14p-24f, 0x1.73d6c8p-29f};
+  const float a = fminf(fabsf(x), 5.8f);
+  float p = kP[10];
+#pragma unroll
+  for (int i = 9; i >= 0; i--) p = __builtin_fmaf(p, a, kP[i]);
+  return 0.5f * __builtin_fmaf(-a, __builtin_amdgcn_exp2f(p * a), x + fabsf(x));
+}
 __device__ __forceinline__ float post_value(float v, float scale, bool has_add, float add, bool has_mul, float mul, int act,
                                             bool has_gate, float gate) {
   if (scale != 1.0f) v = round_f16(v * scale);

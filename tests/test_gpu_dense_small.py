@@ -560,3 +560,29 @@ def test_refused_dense_names_the_call_that_was_made(dthip, oracle):
     x, gamma = dev(rng.standard_normal((5, 64)).astype(np.float16)), dev(np.ones(130, np.float16))
     with pytest.raises(dthip.DtError, match="dt_dense_qx_grouped_ws_f16"):
         dthip.dense_multi(x, [w], [None], epilogues=[dthip.HeadEpilogue(gamma, head_dim=130)])
+
+
+@pytest.mark.parametrize("M", [1024, 16])  # the tiled kernel and the one for few rows
+def test_gelu_erf_of_every_fp16_value(dthip, M):
+    """The tail's GELU against float64 for every finite fp16 value, passed through a Dense with the identity; infinities and NaN
+    through its bias.  Bound: the exponent of erfc is below 28, so two roundings of it in fp32 weigh 2 x 2^-20 x ln 2 = 1.3e-6,
+    the polynomial 3e-8 and the other roundings 2e-7; then fp16's own rounding.  (Past -5.8: 1.9e-8 instead of less.)"""
+    import math
+
+    import torch
+
+    x = np.arange(1 << 16, dtype=np.uint16).view(np.float16).reshape(-1, M, 64)
+    x = np.where(np.isfinite(x), x, np.float16(0))
+    eye = dthip.QxTensor.from_f16(np.eye(64, dtype=np.float16))
+    tail = [dthip.DensePost(dthip.ACT_GELU_ERF)]
+    got = np.concatenate([dthip.dense_post(dev(p), [eye], [None], tail)[0].cpu().numpy() for p in x]).astype(np.float64).ravel()
+    x = x.astype(np.float64).ravel()
+    want = 0.5 * x * np.vectorize(math.erfc)(x * -math.sqrt(0.5))
+    slack = 2e-6 * np.abs(want) + np.where(x < -5.8, 2e-8, 0.0)
+    with np.errstate(over="ignore"):
+        lo, hi = (want - slack).astype(np.float16).astype(np.float64), (want + slack).astype(np.float16).astype(np.float64)
+    assert ((got >= lo) & (got <= hi)).all(), x[~((got >= lo) & (got <= hi))][:8]
+    bias = torch.zeros(64, dtype=torch.float16, device="cuda")
+    bias[:3] = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    out = dthip.dense_post(torch.zeros((M, 64), dtype=torch.float16, device="cuda"), [eye], [bias], tail)[0].cpu().numpy()
+    assert (out[:, 0] == np.inf).all() and np.isnan(out[:, 1:3]).all() and (out[:, 3:] == 0).all()
