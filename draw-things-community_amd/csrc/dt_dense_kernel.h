@@ -214,70 +214,81 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
   constexpr int CH = WN / 8;    // 16-byte chunks per parked row
   constexpr int RPI = 64 / CH;  // token rows per trip
   half_t* const park = reinterpret_cast<half_t*>(smem) + wave * (WM * WN);
-  {
-    // Accumulator block (i, j): lane holds token (lane & 15) of the block and
-    // features 4 (lane / 16) + (0..3).  Chunk c of token t is parked at chunk
-    // c ^ (t % CH): the 8-byte writes of 16 tokens spread over the banks.
+  const int c = lane & (CH - 1), rsub = lane / CH;
+  const int nn = nw + 8 * c;    // first of this lane's 8 features when it walks rows
+  auto lo16 = [](uint32_t v) { return (float)bits_to_half((uint16_t)v); };
+  auto hi16 = [](uint32_t v) { return (float)bits_to_half((uint16_t)(v >> 16)); };
+  // (a lane's 8 features lie inside the matrix or outside it, all of them, unless the slice ends in a width off the grid of 8)
+  const bool cols_in = nw + WN <= w.n, cols8 = cols_in || (w.n & 7) == 0;
+  const int nl = nn < w.n || !cols8 ? nn : w.n - 8;  // ... where the lane reads column data: the last ones in place of those outside
+  const bool aligned16 = (!w.y || (((w.ldy & 7) == 0) && (reinterpret_cast<uintptr_t>(w.y) & 15) == 0)) &&
+                         (!(head && w.rot) || (reinterpret_cast<uintptr_t>(w.rot) & 15) == 0) &&
+                         (!POST || ((!w.add || (((w.ld_add & 7) == 0) && (reinterpret_cast<uintptr_t>(w.add) & 15) == 0)) &&
+                                    (!w.mul || (((w.ld_mul & 7) == 0) && (reinterpret_cast<uintptr_t>(w.mul) & 15) == 0)) &&
+                                    (!w.res || (((w.ld_res & 3) == 0) && (reinterpret_cast<uintptr_t>(w.res) & 15) == 0))));
+  const bool fast = aligned16 && cols8;
+  const int rows = (int)(m_total - mw < WM ? m_total - mw : WM);  // of the slice's, those that exist (below 1: none)
+  // What the wave needs from memory for its columns and its first rows is asked for at once, ahead of the parking: bias,
+  // gate and gamma one after the other, each behind a test of its own, cost a trip to memory each.  (us, apart / at once: 2016 x
+  // 1280 -> 5120 fp16 39.1 / 38.5, with a multiplicand 45.0 / 43.1, with gate and residual 51.2 / 46.6; 9000 x 5120 -> 5120 q5p with
+  // fp32 gate and residual 456 / 436; with slices that end inside the matrix walked as vectors too, 333 x 640 -> 1000 fp16 8.4 /
+  // 7.3, with an addend 13.5 / 9.8.)  More rows ahead than one cost registers: two made the multiplicand's case 48.6, four spill.
+  uint2_t bb[TN];  // bias bits of features nw + 16 i + 4 quad + (0..3)
+  if (w.bias && cols8 && (reinterpret_cast<uintptr_t>(w.bias) & 7) == 0) {
 #pragma unroll
     for (int i = 0; i < TN; i++) {
-        const int nn = nw + i * 16 + 4 * quad;
-        float b4[4] = {0.f, 0.f, 0.f, 0.f};
-        if (w.bias) {
-          if (nn + 3 < w.n && (reinterpret_cast<uintptr_t>(w.bias) & 7) == 0) {
-            const uint2_t bb = *reinterpret_cast<const uint2_t*>(w.bias + nn);
-            b4[0] = (float)bits_to_half((uint16_t)bb[0]);
-            b4[1] = (float)bits_to_half((uint16_t)(bb[0] >> 16));
-            b4[2] = (float)bits_to_half((uint16_t)bb[1]);
-            b4[3] = (float)bits_to_half((uint16_t)(bb[1] >> 16));
-          } else {
+      const int ni = nw + i * 16 + 4 * quad;
+      bb[i] = *reinterpret_cast<const uint2_t*>(w.bias + (ni < w.n ? ni : w.n - 4));
+    }
+  } else {
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-              if (nn + e < w.n) b4[e] = (float)bits_to_half(w.bias[nn + e]);
-          }
-        }
+    for (int i = 0; i < TN; i++) {
+      const int ni = nw + i * 16 + 4 * quad;
+      bb[i] = uint2_t{0, 0};
+      if (w.bias) {
 #pragma unroll
-        for (int j = 0; j < TM; j++) {
-          const int t = j * 16 + l16;
-          const uint2_t pk = {pack_h2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]),
-                              pack_h2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
-          *reinterpret_cast<uint2_t*>(park + t * WN + (((i * 2 + (quad >> 1)) ^ (t & (CH - 1))) << 3) + 4 * (quad & 1)) = pk;
-        }
+        for (int e = 0; e < 4; e++)
+          if (ni + e < w.n) bb[i][e >> 1] |= (uint32_t)w.bias[ni + e] << (16 * (e & 1));
+      }
     }
   }
-  // a wave's LDS operations execute in order: its reads below see the writes above
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-  const int c = lane & (CH - 1), rsub = lane / CH;
-  const int nn = nw + 8 * c;    // first of this lane's 8 features
-  if (nw >= w.n) return;
-  // this lane's column data
   float gt[8];  // the gate, or the RMSNorm weight of a head tile
 #pragma unroll
   for (int e = 0; e < 8; e++) gt[e] = 1.f;
-  auto lo16 = [](uint32_t v) { return (float)bits_to_half((uint16_t)v); };
-  auto hi16 = [](uint32_t v) { return (float)bits_to_half((uint16_t)(v >> 16)); };
+  auto halfs8 = [&](const uint16_t* p) {
+    const uint4_t gg = *reinterpret_cast<const uint4_t*>(p);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      gt[2 * q] = lo16(gg[q]);
+      gt[2 * q + 1] = hi16(gg[q]);
+    }
+  };
   if (head && w.gamma) {
     if ((reinterpret_cast<uintptr_t>(w.gamma) & 15) == 0) {
-      const uint4_t gg = *reinterpret_cast<const uint4_t*>(w.gamma + 8 * c);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        gt[2 * q] = lo16(gg[q]);
-        gt[2 * q + 1] = hi16(gg[q]);
-      }
+      halfs8(w.gamma + 8 * c);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; e++) gt[e] = (float)bits_to_half(w.gamma[8 * c + e]);
     }
   }
   if constexpr (POST) {
+    if (w.gate && cols8 && (reinterpret_cast<uintptr_t>(w.gate) & 15) == 0) {
+      halfs8(w.gate + nl);
+    } else if (w.gate32 && cols8 && (reinterpret_cast<uintptr_t>(w.gate32) & 15) == 0) {
+      const float4_t g0 = *reinterpret_cast<const float4_t*>(w.gate32 + nl), g1 = *reinterpret_cast<const float4_t*>(w.gate32 + nl + 4);
 #pragma unroll
-    for (int e = 0; e < 8; e++)
-      if (nn + e < w.n) {
-        if (w.gate) gt[e] = (float)bits_to_half(w.gate[nn + e]);
-        if (w.gate32) gt[e] = w.gate32[nn + e];
+      for (int e = 0; e < 4; e++) {
+        gt[e] = g0[e];
+        gt[4 + e] = g1[e];
       }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        if (nn + e < w.n) {
+          if (w.gate) gt[e] = (float)bits_to_half(w.gate[nn + e]);
+          if (w.gate32) gt[e] = w.gate32[nn + e];
+        }
+    }
   }
   // what a row needs from memory before its arithmetic
   struct RowIn {
@@ -285,34 +296,60 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
     uint4_t mul;
     float4_t r0, r1;
   };
-  // FAST: the wave's slice lies inside the matrix and every row meets the vector alignment
+  auto fetch = [&](int it, RowIn& in) {
+    const int t = it * RPI + rsub;
+    const int64_t gm = mw + (t < rows ? t : rows - 1);  // (rows past the last read the last)
+    if (head && w.rot) in.add = *reinterpret_cast<const uint4_t*>(w.rot + (w.rot_pos0 + gm) * WN + 8 * c);
+    if constexpr (POST) {
+      if (w.add) in.add = *reinterpret_cast<const uint4_t*>(w.add + gm * w.ld_add + nl);
+      if (w.mul) in.mul = *reinterpret_cast<const uint4_t*>(w.mul + gm * w.ld_mul + nl);
+      if (w.res) {
+        in.r0 = *reinterpret_cast<const float4_t*>(w.res + gm * w.ld_res + nl);
+        in.r1 = *reinterpret_cast<const float4_t*>(w.res + gm * w.ld_res + nl + 4);
+      }
+    }
+  };
+  // Trips go in groups of GRP: the rows a group needs from memory are requested one group ahead, before the
+  // previous group's stores (a load behind a store waits for it), so a trip does not wait a memory round trip.
+  constexpr int TRIPS = WM / RPI;
+  constexpr int GRP = POST ? 1 : 4;
+  static_assert(TRIPS % GRP == 0, "trips per group");
+  RowIn first[GRP];
+  if (fast) {
+#pragma unroll
+    for (int j = 0; j < GRP; j++) fetch(j, first[j]);
+  }
+  {
+    // Accumulator block (i, j): lane holds token (lane & 15) of the block and
+    // features 4 (lane / 16) + (0..3).  Chunk c of token t is parked at chunk
+    // c ^ (t % CH): the 8-byte writes of 16 tokens spread over the banks.
+#pragma unroll
+    for (int i = 0; i < TN; i++) {
+      const float b4[4] = {lo16(bb[i][0]), hi16(bb[i][0]), lo16(bb[i][1]), hi16(bb[i][1])};
+#pragma unroll
+      for (int j = 0; j < TM; j++) {
+        const int t = j * 16 + l16;
+        const uint2_t pk = {pack_h2(acc[i][j][0] + b4[0], acc[i][j][1] + b4[1]),
+                            pack_h2(acc[i][j][2] + b4[2], acc[i][j][3] + b4[3])};
+        *reinterpret_cast<uint2_t*>(park + t * WN + (((i * 2 + (quad >> 1)) ^ (t & (CH - 1))) << 3) + 4 * (quad & 1)) = pk;
+      }
+    }
+  }
+  // a wave's LDS operations execute in order: its reads below see the writes above
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (nw >= w.n) return;
+  // FAST: a lane's 8 values of a row are one vector
   // ACT: the activation when it is known where the loop is instantiated (the fast form is instantiated once
   // per activation, so that its body holds one activation's code), or -1 = taken from the arguments at run time
   auto walk = [&](auto fast_tag, auto act_tag) {
     constexpr bool FAST = decltype(fast_tag)::value;
     constexpr int ACT = decltype(act_tag)::value;
-    auto fetch = [&](int it, RowIn& in) {
-      const int t = it * RPI + rsub;
-      const int64_t gm = mw + t;
-      if (head && w.rot) in.add = *reinterpret_cast<const uint4_t*>(w.rot + (w.rot_pos0 + gm) * WN + 8 * c);
-      if constexpr (POST) {
-        if (w.add) in.add = *reinterpret_cast<const uint4_t*>(w.add + gm * w.ld_add + nn);
-        if (w.mul) in.mul = *reinterpret_cast<const uint4_t*>(w.mul + gm * w.ld_mul + nn);
-        if (w.res) {
-          in.r0 = *reinterpret_cast<const float4_t*>(w.res + gm * w.ld_res + nn);
-          in.r1 = *reinterpret_cast<const float4_t*>(w.res + gm * w.ld_res + nn + 4);
-        }
-      }
-    };
-    // Trips go in groups of GRP: the rows a group needs from memory are requested one group ahead, before the
-    // previous group's stores (a load behind a store waits for it), so a trip does not wait a memory round trip.
-    constexpr int TRIPS = WM / RPI;
-    constexpr int GRP = (FAST && !POST) ? 4 : 1;
-    static_assert(TRIPS % GRP == 0, "trips per group");
     RowIn cur[GRP];
     if constexpr (FAST) {
 #pragma unroll
-      for (int j = 0; j < GRP; j++) fetch(j, cur[j]);
+      for (int j = 0; j < GRP; j++) cur[j] = first[j];
     }
     for (int it0 = 0; it0 < TRIPS; it0 += GRP) {
       RowIn nxt[GRP];
@@ -327,7 +364,7 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
       const int it = it0 + j;
       const int t = it * RPI + rsub;
       const int64_t gm = mw + t;
-      const bool row_ok = FAST || gm < m_total;
+      const bool row_ok = t < rows;
       const int64_t gmc = row_ok ? gm : 0;
       const uint4_t raw = *reinterpret_cast<const uint4_t*>(park + t * WN + ((c ^ (t & (CH - 1))) << 3));
       float v[8] = {lo16(raw[0]), hi16(raw[0]), lo16(raw[1]), hi16(raw[1]),
@@ -445,13 +482,15 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
       }
       const uint4_t out = {pack_h2(v[0], v[1]), pack_h2(v[2], v[3]), pack_h2(v[4], v[5]), pack_h2(v[6], v[7])};
       if constexpr (FAST) {
-        if constexpr (POST) {
-          if (w.res) {
-            *reinterpret_cast<float4_t*>(w.res + gm * w.ld_res + nn) = float4_t{res[0], res[1], res[2], res[3]};
-            *reinterpret_cast<float4_t*>(w.res + gm * w.ld_res + nn + 4) = float4_t{res[4], res[5], res[6], res[7]};
+        if (row_ok & (nn < w.n)) {
+          if constexpr (POST) {
+            if (w.res) {
+              *reinterpret_cast<float4_t*>(w.res + gm * w.ld_res + nn) = float4_t{res[0], res[1], res[2], res[3]};
+              *reinterpret_cast<float4_t*>(w.res + gm * w.ld_res + nn + 4) = float4_t{res[4], res[5], res[6], res[7]};
+            }
           }
+          if (w.y) *reinterpret_cast<uint4_t*>(w.y + gm * w.ldy + nn) = out;
         }
-        if (w.y) *reinterpret_cast<uint4_t*>(w.y + gm * w.ldy + nn) = out;
       } else if (row_ok) {
 #pragma unroll
         for (int e = 0; e < 8; e++)
@@ -469,12 +508,7 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
       }
     }
   };
-  const bool aligned16 = (!w.y || (((w.ldy & 7) == 0) && (reinterpret_cast<uintptr_t>(w.y) & 15) == 0)) &&
-                         (!(head && w.rot) || (reinterpret_cast<uintptr_t>(w.rot) & 15) == 0) &&
-                         (!POST || ((!w.add || (((w.ld_add & 7) == 0) && (reinterpret_cast<uintptr_t>(w.add) & 15) == 0)) &&
-                                    (!w.mul || (((w.ld_mul & 7) == 0) && (reinterpret_cast<uintptr_t>(w.mul) & 15) == 0)) &&
-                                    (!w.res || (((w.ld_res & 3) == 0) && (reinterpret_cast<uintptr_t>(w.res) & 15) == 0))));
-  if (aligned16 && nw + WN <= w.n && mw + WM <= m_total) {
+  if (fast) {
     if constexpr (POST) {
       switch (w.act) {
         case DT_ACT_GELU_TANH: walk(std::true_type{}, std::integral_constant<int, DT_ACT_GELU_TANH>{}); break;

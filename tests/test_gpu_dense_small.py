@@ -586,3 +586,53 @@ def test_gelu_erf_of_every_fp16_value(dthip, M):
     bias[:3] = torch.tensor([float("inf"), float("-inf"), float("nan")])
     out = dthip.dense_post(torch.zeros((M, 64), dtype=torch.float16, device="cuda"), [eye], [bias], tail)[0].cpu().numpy()
     assert (out[:, 0] == np.inf).all() and np.isnan(out[:, 1:3]).all() and (out[:, 3:] == 0).all()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (128, 128, 128),               # one whole tile
+    (129, 136, 128), (127, 120, 192),  # a row / eight features into the next tile, and as much short of one
+    (333, 652, 320),               # a width off the grid of 8 (it lies on that of 4)
+    (300, 1001, 128),              # an odd one
+    (200, 64, 320),                # half a tile of features
+    (4100, 3080, 128), (4099, 3076, 192),  # 256 x 256 tiles
+])
+@pytest.mark.parametrize("q", [16, 6])
+def test_dense_tails_at_the_edges(dthip, oracle, M, N, K, q):
+    """Bias and every tail on slices that end inside a row of tiles: the tails act on the Dense's own results, bit for bit, and
+    nothing behind a row or below the last one is written."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K + q)
+    X = rng.standard_normal((M, K)).astype(np.float16)
+    w, W = make(dthip, oracle, rng, N, K, q, 4096)
+    b = (rng.standard_normal(N) * 0.1).astype(np.float16)
+    x, bias = dev(X), dev(b)
+
+    def wide(dtype):  # [M, N] inside a buffer of sentinels, rows on the 16-byte grid
+        buf = torch.full((M + 3, (N + 15) // 8 * 8), -77.0, dtype=dtype, device="cuda")
+        return buf, buf[:M, :N]
+
+    def untouched(buf):
+        return bool((buf[M:] == -77).all()) and bool((buf[:, N:] == -77).all())
+
+    print("dense tails at the edges", M, N, K, q, flush=True)
+    buf, plain = wide(torch.float16)
+    dthip.dense_multi(x, [w], [bias], outs=[plain])
+    assert untouched(buf)
+    check(plain.cpu().numpy(), X, W, b)
+    rnd = lambda *s: dev(rng.standard_normal(s).astype(np.float16))
+    other, gate = rnd(M, N), rnd(N)
+    abuf, addend = wide(torch.float16)
+    addend.copy_(other)
+    res0 = rnd(M, N).float()
+    half = plain.float()
+    for post, want in ((dict(addend=addend), half + other.float()), (dict(multiplicand=addend), half * other.float()),
+                       (dict(gate=gate), half * gate.float())):
+        buf, y = wide(torch.float16)
+        dthip.dense_post(x, [w], [bias], [dthip.DensePost(**post)], outs=[y])
+        assert untouched(buf) and bool((y == want.half()).all()), post.keys()
+    for g, product in ((gate, (half * gate.float()).half().float()), (gate.float() + 2.0 ** -13, half * (gate.float() + 2.0 ** -13))):
+        rbuf, res = wide(torch.float32)
+        res.copy_(res0)
+        dthip.dense_post(x, [w], [bias], [dthip.DensePost(gate=g, residual=res, keep_output=False)])
+        assert untouched(rbuf) and bool((res == res0 + product).all())
