@@ -236,10 +236,12 @@ struct TilePlan {
 // Fewer 256 x 256 tiles than this leave too many of the 256 compute units idle: such launches take 128 x 128 tiles.
 constexpr int64_t kFillTiles = 192;
 constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
-// fp16 copies of a launch's weights.  Few rows do not pay for holding large ones: 512 x 5120 -> 5120 q6p 61 us and 46 on a
-// copy of 50 MB, 512 x 3072 -> 12288 67 and 57 on 72 MB, 512 x 5120 -> 2 x 5120 q5p 87 and 84 on 100 MB.
+// fp16 copies of a launch's weights.  Over 200 MiB they leave the memory-side cache (256 MB) before the launch has read them,
+// which launches of few rows, that wait for the weights, do not make up for (us, packed / copied: 373 x 10368 -> 2 x 6144 q5p, 255
+// MB, 180 / 218; 353 x 8832 -> 12352 q6p, 218 MB, 167 / 186; 468 x 12416 -> 2 x 5248 q8p, 261 MB, 243 / 289; below the line 512
+// x 5120 -> 5120 q6p, 52 MB, 71 / 52; 300 x 5120 -> 5120 q8p 56 / 49; 568 x 7488 -> 11648 q6p, 174 MB, 250 / 149).
 constexpr size_t kDenseMaxExpand = (size_t)512 << 20;
-constexpr size_t kDenseFewRowsExpand = (size_t)48 << 20;
+constexpr size_t kDenseFewRowsExpand = (size_t)200 << 20;
 constexpr int64_t kDenseFewRows = 640;
 
 // Estimated time (us) of a launch whose rows enter new blocks at every `step`-th K-tile at most: a fit to 930 launches of

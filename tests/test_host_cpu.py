@@ -128,6 +128,22 @@ def test_dense_scratch_for_copies(dthip, monkeypatch, M, K, N, n, q, nib, copied
     assert dthip.lib().dt_dense_scratch_bytes(1, G) == cut
 
 
+@pytest.mark.parametrize("K,N,n,q,nib,copied", [
+    (5120, 5120, 1, 6, 4096, True), (12288, 3072, 1, 8, 16384, True),  # 52 and 75 MB
+    (10368, 6144, 2, 5, 1024, False),                                  # 255 MB
+])
+def test_dense_scratch_for_copies_with_few_rows(dthip, monkeypatch, K, N, n, q, nib, copied):
+    """Few rows copy weights that the memory-side cache holds, larger ones do not."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    addr = ctypes.addressof
+    for M in (400, 512, 640):
+        W = (dthip._QxWeight * n)(*[dthip._QxWeight(4096, q, nib, N * K)] * n)  # (addresses are not looked at)
+        Y, ldy = (ctypes.c_void_p * n)(*[4096] * n), (ctypes.c_int64 * n)(*[N] * n)
+        G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), n, None, addr(Y), addr(ldy), None, None))
+        assert (dthip.lib().dt_dense_scratch_bytes(1, G) >= n * N * K * 2) == copied, M
+
+
 def test_rows_that_need_no_workspace(dthip):
     """The operators do not ask for workspace up to the rows that the library's streaming kernel takes: one number, twice."""
     import re
