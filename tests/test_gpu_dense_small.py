@@ -511,6 +511,7 @@ def test_optional_scratch_is_not_insisted_on(dthip, oracle, monkeypatch, kind):
 
     monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
     monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")  # (the uncut launch on copies of the weights gives the uncut one's bits)
     rng = np.random.default_rng(9)
     L = dthip.lib()
     staged = 0
