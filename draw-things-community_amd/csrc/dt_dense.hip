@@ -384,11 +384,17 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
   return best;
 }
 
+// DT_DENSE_EXPAND = "never" | "always" (wherever it can be) overrides the choice between packed weights and copies; for tests and
+// measurements, read at every call.  DT_DENSE_SPLIT has no say in it.
+static bool expand_knob(char first) {
+  const char* knob = getenv("DT_DENSE_EXPAND");
+  return knob && knob[0] == first;
+}
+
 // The layout of one launch on plain fp16 weights, the palettized ones among them copied to scratch first.  Returns false where
 // that cannot be, or is not wanted.
 static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, TilePlan* plan, double* cost) {
-  const char* knob = getenv("DT_DENSE_EXPAND");  // "never" | "always" (wherever it can be; for tests); read at every call
-  if ((knob && knob[0] == 'n') || (!knob && getenv("DT_DENSE_SPLIT"))) return false;
+  if (expand_knob('n')) return false;
   size_t bytes = 0;
   int64_t weights = 0, m_max = 0;
   for (int gi = 0; gi < n; gi++) {
@@ -401,7 +407,7 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
       weights += w.count;
     }
   }
-  if (weights == 0 || bytes > ws || bytes > kDenseMaxExpand || (bytes > kDenseFewRowsExpand && m_max <= kDenseFewRows && !knob)) return false;
+  if (weights == 0 || bytes > ws || bytes > kDenseMaxExpand || (bytes > kDenseFewRowsExpand && m_max <= kDenseFewRows && !expand_knob('a'))) return false;
   dt_qx_weight f16 = hs[0].W[w_begin];
   f16.qbits = 16;
   *plan = plan_format(hs, n, w_begin, w_end, wide, std::min(ws - bytes, kDenseMaxWorkspace), f16, true, cost);
@@ -427,8 +433,7 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   TilePlan plain;
   double copied;
   if (!expand || w0.qbits == 16 || !plan_copies(hs, n, w_begin, w_end, wide, ws, &plain, &copied)) return packed;
-  const char* knob = getenv("DT_DENSE_EXPAND");
-  if (!(knob && knob[0] == 'a') && !(copied < 0.95 * *cost && copied < *cost - 6.0)) return packed;
+  if (!expand_knob('a') && !(copied < 0.95 * *cost && copied < *cost - 6.0)) return packed;
   *cost = copied;
   return plain;
 }

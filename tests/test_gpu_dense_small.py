@@ -142,6 +142,7 @@ def test_dense_cut_along_k(dthip, oracle, monkeypatch, M, N, K, q, nib):
     gamma, rot = dev((1 + 0.1 * rng.standard_normal(128)).astype(np.float16)), dev(rng.standard_normal((M + 3, 128)).astype(np.float16))
     epi = [None, dthip.HeadEpilogue(gamma, rot, 3)]
     print("dense cut along K", M, N, K, q, nib, flush=True)
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
     monkeypatch.setenv("DT_DENSE_SPLIT", "never")
     whole = dthip.dense_multi(x, ws, [bias, None])
     monkeypatch.setenv("DT_DENSE_SPLIT", "always")
@@ -256,6 +257,7 @@ def test_dense_row_palettes_on_a_unit_of_ones_own(dthip, oracle, monkeypatch, K,
 
     rng = np.random.default_rng(K + q)
     monkeypatch.setenv("DT_DENSE_SPLIT", "never")  # (a cut tile's sums are added up in another order)
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
     nib = {7: 8192, 8: 16384}[q]
     N, few, many = 2433, 200, 1790  # 2 and 14 tiles by 20: 40 and 280
     X = rng.standard_normal((many, K)).astype(np.float16)
@@ -314,6 +316,7 @@ def test_dense_c_entry_points_without_workspace(dthip, oracle, monkeypatch, M, q
     import torch
 
     monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
     rng = np.random.default_rng(M + q)
     K, N = 320, 256
     x = dev(rng.standard_normal((M, K)).astype(np.float16))
@@ -434,6 +437,7 @@ def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     M, N, K = 1530, 12288, 3072
     w, _ = make(dthip, oracle, rng, N, K, 6, 4096)
     x = dev(rng.standard_normal((M, K)).astype(np.float16))
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
     monkeypatch.setenv("DT_DENSE_SPLIT", "never")
     whole = dthip.dense_multi(x, [w], [None])[0].float()
     monkeypatch.delenv("DT_DENSE_SPLIT")

@@ -128,6 +128,17 @@ def test_dense_scratch_for_copies(dthip, monkeypatch, M, K, N, n, q, nib, copied
     assert dthip.lib().dt_dense_scratch_bytes(1, G) == cut
 
 
+@pytest.mark.parametrize("split", ["never", "always", ""])
+def test_dense_copies_do_not_hang_on_the_knob_for_cuts(dthip, monkeypatch, split):
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    monkeypatch.setenv("DT_DENSE_SPLIT", split)
+    addr, M, K, N, n = ctypes.addressof, 4608, 3072, 3072, 3
+    W = (dthip._QxWeight * n)(*[dthip._QxWeight(4096, 6, 4096, N * K)] * n)  # (addresses are not looked at)
+    Y, ldy = (ctypes.c_void_p * n)(*[4096] * n), (ctypes.c_int64 * n)(*[N] * n)
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), n, None, addr(Y), addr(ldy), None, None))
+    assert dthip.lib().dt_dense_scratch_bytes(1, G) >= n * N * K * 2
+
+
 @pytest.mark.parametrize("K,N,n,q,nib,copied", [
     (5120, 5120, 1, 6, 4096, True), (12288, 3072, 1, 8, 16384, True),  # 52 and 75 MB
     (10368, 6144, 2, 5, 1024, False),                                  # 255 MB
