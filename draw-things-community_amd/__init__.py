@@ -607,8 +607,8 @@ class LoRADense:
     """LoRADense(count:configuration:noBias:flags:name:) -- dense(x) + up(scale * down(x)) with the palettized base
     left packed and the fp16 low-rank pair applied beside it (Models/LoRA.swift:85-142; running the LoRA separately
     is the preferred mode for quantized models, Models/UNetProtocol.swift:696-697).  The Dense kernel on the base and
-    the down projection (with the scale in its epilogue), then on the up projection, whose epilogue adds the base
-    projection's result; every intermediate is rounded to fp16 as the reference's separate ops round.  With
+    the down projection (with the scale in its epilogue), in one call or side by side, then on the up projection, whose
+    epilogue adds the base projection's result; every intermediate is rounded to fp16 as the reference's separate ops round.  With
     `highPrecision` the pair is fp32 (`down.data` / `up.data` float32 tensors): the branch is computed as
     fp16(up(scale * down(float(x)))) in fp32 throughout (Models/LoRA.swift:117-139) by dt_lora_branch_f32_f16 and added
     in the base projection's epilogue."""
@@ -645,6 +645,29 @@ class LoRADense:
             self._pad_key, self._pad = key, (dn, up)
         return self._pad
 
+    @staticmethod
+    def _down_beside_base(M, K, weight, rank, capturing) -> bool:
+        """Whether the down projection of M rows runs on a second stream beside the base projection.  On few workgroups it takes as
+        long as K is, 60 us at 64 x 13824, unless it shares the base projection's launch.  Two streams cost a captured graph 12
+        us, and a caller that waits for the host 65 (us, one call / two streams, rank 16: in a graph 64 x 13824 -> 5120 q6p 137 /
+        93, 64 x 5120 -> 5120 63 / 54, 48 x 5120 -> 5120 56 / 51, 1024 x 12288 -> 3072 in blocks of 128 200 / 178, 64 x 3072 -> 3072 39
+        / 39, and the other way round 32 x 13824 -> 5120 88 / 91, 48 x 3072 -> 3072 34 / 37, 1024 x 1280 -> 1280 in blocks of 256 48 / 53;
+        otherwise 64 x 13824 -> 5120 137 / 118, 1024 x 12288 -> 3072 in blocks of 128 190 / 170, and the other way round 48 x 12288 ->
+        3072 98 / 113, 1024 x 3072 -> 3072 in blocks of 256 86 / 123)."""
+        if weight.qbits == 16 or K < 3072 or M <= 32 or M * K < 64 * 3072:
+            return False
+        if not (M * K >= (48 * 13824 if M <= _ROWS_MAX else 8 << 20) or capturing()):
+            return False
+        if M <= _ROWS_MAX:
+            return True
+        # the call as the library sees it, as far as it looks at addresses
+        ws = (_QxWeight * 2)(_QxWeight(4096, weight.qbits, weight.nib, weight.count), _QxWeight(4096, 16, 0, rank * K))
+        ys, strides = (ctypes.c_void_p * 2)(4096, 4096), (ctypes.c_int64 * 2)(weight.shape[0], rank)
+        at = ctypes.addressof
+        group = (_DenseGroup * 1)(_DenseGroup(M, K, 4096, K, at(ws), 2, None, at(ys), at(strides), None, None))
+        # nothing is copied where the call has no use for more than the workspace that cutting takes
+        return lib().dt_dense_scratch_bytes(1, group) == lib().dt_dense_workspace_bytes(1, group)
+
     def __call__(self, x, post: Optional[DensePost] = None, stream=None):
         if self.weight is None:
             raise RuntimeError(f"LoRADense {self.name!r}: weight not loaded")
@@ -663,12 +686,27 @@ class LoRADense:
         if self.configuration.highPrecision:
             return self._high_precision(x, b, p, stream)
         dn, up = self._padded()
-        # Base and down projection share x: one call, which puts them into one launch where the base weight is copied to
-        # fp16 for it (the down projection's few tiles then run on compute units that the base projection leaves idle).  The
-        # up projection's epilogue adds the base projection's result and then runs the tail.  (fp16(base) + fp16(branch)
-        # rounds the same whichever of the two is the addend.)
-        base, down = dense_post(x, [self.weight, dn], [b, None], [None, DensePost(scale=self.configuration.scale)],
-                                flags=self.flags, stream=stream)
+        # Base and down projection share x.  One call puts them into one launch where the base weight is copied to fp16 for it (the
+        # down projection's few tiles then run on compute units that the base projection leaves idle), and where they are
+        # short the host has no time for more.  The up projection's epilogue adds the base projection's result and then runs
+        # the tail.  (fp16(base) + fp16(branch) rounds the same whichever of the two is the addend.)
+        down_post = DensePost(scale=self.configuration.scale)
+        K = _f16_cuda(x, "x").shape[-1]
+        if self._down_beside_base(x.numel() // max(K, 1), K, self.weight, dn.shape[0], lambda: _capturing(stream)):
+            torch = _torch()
+            main = stream if stream is not None else torch.cuda.current_stream(x.device)
+            side = _side_stream(x.device)
+            side.wait_stream(main)
+            down = dense_post(x, [dn], [None], [down_post], stream=side)[0]
+            # (making a stream current that is so already costs 8 us)
+            at = stream if x.device.index == torch.cuda.current_device() else main
+            base = dense_multi(x, [self.weight], [b], flags=self.flags, stream=at)[0]
+            main.wait_stream(side)  # every use of x and `down` on the side stream is ordered before what follows on `main`
+            # `down` came from the side stream's pool and is read on `main`: its memory must not go back to that pool's
+            # next user before `main` has passed this point
+            down.record_stream(main)
+        else:
+            base, down = dense_post(x, [self.weight, dn], [b, None], [None, down_post], flags=self.flags, stream=stream)
         tail = DensePost(p.activation, p.gate, p.residual, p.keep_output, addend=base.reshape(-1, self.count))
         out = dense_post(down, [up], [None], [tail], stream=stream)[0]
         return None if out is None else out.reshape(*x.shape[:-1], self.count)
@@ -713,6 +751,12 @@ def _side_stream(device):
     if key not in _SIDE_STREAMS:
         _SIDE_STREAMS[key] = torch.cuda.Stream(device=key)
     return _SIDE_STREAMS[key]
+
+
+def _capturing(stream) -> bool:
+    """Whether what is enqueued on `stream` (None: the current one) becomes part of a graph."""
+    with _on(stream):
+        return _torch().cuda.is_current_stream_capturing()
 
 
 def _view4(t) -> _View4:

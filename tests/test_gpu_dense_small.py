@@ -429,6 +429,32 @@ def test_lora_base_and_down_in_one_launch(dthip, oracle, monkeypatch, M, N, K, q
     assert all(torch.equal(a, b) for a, b in zip(got["never"], got["always"]))
 
 
+@pytest.mark.parametrize("M,N,K,q,nib", [(64, 256, 3072, 8, 16384), (64, 128, 13824, 6, 4096), (130, 260, 3072, 4, 256)])
+def test_lora_down_beside_the_base_in_a_graph(dthip, oracle, M, N, K, q, nib):
+    """The down projection on its own stream: captured, replayed and beside other work, the same bits as in one call."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    op = dthip.LoRADense(N, dthip.LoRANetworkConfiguration(16, 0.75, False))
+    op.weight, op.bias = make(dthip, oracle, rng, N, K, q, nib)[0], dev((rng.standard_normal(N) * 0.1).astype(np.float16))
+    op.down, op.up = make(dthip, oracle, rng, 16, K, 16, 0)[0], make(dthip, oracle, rng, N, 16, 16, 0)[0]
+    x = dev((0.1 * rng.standard_normal((M, K))).astype(np.float16))
+    print("lora side by side", M, N, K, q, nib, flush=True)
+    dn, up = op._padded()
+    base, down = dthip.dense_post(x, [op.weight, dn], [op.bias, None], [None, dthip.DensePost(scale=0.75)])
+    want = dthip.dense_post(down, [up], [None], [dthip.DensePost(addend=base)])[0]
+    assert torch.equal(op(x), want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = op(x)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert torch.equal(op(x), want)
+
+
 def test_dense_last_round_cut_along_k(dthip, oracle, monkeypatch):
     """288 tiles: 256 stay whole, the 32 of the second round are cut; against the uncut launch, one fp16 rounding apart."""
     import torch

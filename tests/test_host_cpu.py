@@ -155,6 +155,21 @@ def test_dense_scratch_for_copies_with_few_rows(dthip, monkeypatch, K, N, n, q, 
         assert (dthip.lib().dt_dense_scratch_bytes(1, G) >= n * N * K * 2) == copied, M
 
 
+@pytest.mark.parametrize("M,K,N,q,nib,captured,otherwise", [
+    (64, 13824, 5120, 6, 4096, True, True), (64, 5120, 5120, 8, 16384, True, False), (48, 12288, 3072, 8, 16384, True, False),
+    (32, 13824, 5120, 6, 4096, False, False), (48, 3072, 3072, 6, 4096, False, False), (64, 13824, 5120, 16, 0, False, False),
+    (1024, 12288, 3072, 6, 128, True, True), (1024, 3072, 3072, 6, 256, True, False), (4608, 1280, 1280, 6, 256, False, False),
+    (4608, 3072, 3072, 6, 4096, False, False), (512, 5120, 5120, 5, 1024, False, False),  # copied: one launch
+])
+def test_lora_down_projection_beside_the_base(dthip, monkeypatch, M, K, N, q, nib, captured, otherwise):
+    """The down projection gets a stream of its own where it is long and not part of the base projection's launch."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    w = dthip.QxTensor(None, q, nib, (N, K))
+    assert dthip.LoRADense._down_beside_base(M, K, w, 64, lambda: True) == captured
+    assert dthip.LoRADense._down_beside_base(M, K, w, 64, lambda: False) == otherwise
+
+
 def test_rows_that_need_no_workspace(dthip):
     """The operators do not ask for workspace up to the rows that the library's streaming kernel takes: one number, twice."""
     import re
