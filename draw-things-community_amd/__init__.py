@@ -652,11 +652,11 @@ class LoRADense:
         us, and a caller that waits for the host 65 (us, one call / two streams, rank 16: in a graph 64 x 13824 -> 5120 q6p 137 /
         93, 64 x 5120 -> 5120 63 / 54, 48 x 5120 -> 5120 56 / 51, 1024 x 12288 -> 3072 in blocks of 128 200 / 178, 64 x 3072 -> 3072 39
         / 39, and the other way round 32 x 13824 -> 5120 88 / 91, 48 x 3072 -> 3072 34 / 37, 1024 x 1280 -> 1280 in blocks of 256 48 / 53;
-        otherwise 64 x 13824 -> 5120 137 / 118, 1024 x 12288 -> 3072 in blocks of 128 190 / 170, and the other way round 48 x 12288 ->
-        3072 98 / 113, 1024 x 3072 -> 3072 in blocks of 256 86 / 123)."""
+        otherwise 64 x 13824 -> 5120 137 / 118, 1024 x 12288 -> 3072 in blocks of 128 190 / 170, and the other way round 64 x 12288 ->
+        3072 113 / 131, 1024 x 3072 -> 3072 in blocks of 256 86 / 123)."""
         if weight.qbits == 16 or K < 3072 or M <= 32 or M * K < 64 * 3072:
             return False
-        if not (M * K >= (48 * 13824 if M <= _ROWS_MAX else 8 << 20) or capturing()):
+        if not (M * K >= (60 * 13824 if M <= _ROWS_MAX else 8 << 20) or capturing()):
             return False
         if M <= _ROWS_MAX:
             return True

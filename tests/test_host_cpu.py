@@ -156,7 +156,7 @@ def test_dense_scratch_for_copies_with_few_rows(dthip, monkeypatch, K, N, n, q, 
 
 
 @pytest.mark.parametrize("M,K,N,q,nib,captured,otherwise", [
-    (64, 13824, 5120, 6, 4096, True, True), (64, 5120, 5120, 8, 16384, True, False), (48, 12288, 3072, 8, 16384, True, False),
+    (64, 13824, 5120, 6, 4096, True, True), (64, 5120, 5120, 8, 16384, True, False), (64, 12288, 3072, 8, 16384, True, False),
     (32, 13824, 5120, 6, 4096, False, False), (48, 3072, 3072, 6, 4096, False, False), (64, 13824, 5120, 16, 0, False, False),
     (1024, 12288, 3072, 6, 128, True, True), (1024, 3072, 3072, 6, 256, True, False), (4608, 1280, 1280, 6, 256, False, False),
     (4608, 3072, 3072, 6, 4096, False, False), (512, 5120, 5120, 5, 1024, False, False),  # copied: one launch
