@@ -67,13 +67,15 @@ __device__ __forceinline__ float act_swish(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * x));
 }
 // x Phi(x) = (x + |x| - 2 |x| Phi(-|x|)) / 2, and 2 Phi(-a) = erfc(a / sqrt 2) = 2^(a p(a)): its logarithm is so smooth that a
-// polynomial of degree 10 (least maximum error, fitted to float64 values) is as good as fp32 can hold, in 15 instructions without
-// a branch.  Behind a = 5.8 the result is below half of fp16's least value.  Over all fp16 x: relative error against float64 4.9e-8
-// rms, 8.2e-7 at most (erfcf: 6.3e-8, 1.1e-6); infinities and NaN come out as they do of x (1 + erf(x / sqrt 2)) / 2.
+// polynomial of degree 10 (least maximum error, fitted to float64 values, 5e-8) does, in 15 instructions without a branch.  Behind
+// a = 5.8 the result is below half of fp16's least value.  Relative error against float64 over all fp16 x >= -5.8, of which the
+// rounding of an exponent of up to 28 is the most: 7.6e-8 rms, 1.9e-6 at most (erfcf: 9.7e-8, 2.5e-6), where the result is a normal fp16
+// number 5.0e-8, 8.5e-7 (7.1e-8, 1.1e-6); infinities and NaN come out as they do of x (1 + erf(x / sqrt 2)) / 2.
+// (The exponent in two parts, -a^2 / 2 and a rest, each with its exponential: 4.8e-8, 1.3e-6, and 2 .. 5 % of the launch.)
 // us, erfcf / this: 2016 x 1280 -> 5120 fp16 53.2 / 46.8, 8192 x 320 -> 1280 q6p 37.0 / 29.1 (39.0 and 22.7 without a tail).
 __device__ __forceinline__ float act_gelu_erf(float x) {
-  constexpr float kP[11] = {-0x1.26aecap+0f, -0x1.d63d8ap-2f, -0x1.ad94ap-5f, 0x1.c5ee4ap-8f, 0x1.398282p-15f, -0x1.477c1cp-12f,
-                            0x1.83bca8p-14f, -0x1.056702p-16f, 0x1.b7899ap-20f, -0x1.acf14p-24f, 0x1.73d6c8p-29f};
+  constexpr float kP[11] = {-0x1.26aedap+0f, -0x1.d63b5p-2f, -0x1.adc97cp-5f, 0x1.c85c3ap-8f, 0x1.97be5p-18f, -0x1.36613p-12f,
+                            0x1.6cfc72p-14f, -0x1.e41dacp-17f, 0x1.8ed5fp-20f, -0x1.7cb02cp-24f, 0x1.428c4ep-29f};
   const float a = fminf(fabsf(x), 5.8f);
   float p = kP[10];
 #pragma unroll

@@ -170,6 +170,29 @@ def test_lora_down_projection_beside_the_base(dthip, monkeypatch, M, K, N, q, ni
     assert dthip.LoRADense._down_beside_base(M, K, w, 64, lambda: False) == otherwise
 
 
+def test_gelu_erf_polynomial_is_as_exact_as_erfcf():
+    """The tail's GELU in the kernel's fp32 steps, over every fp16 value from -5.8 on: no further from float64 than with the library
+    function (9.7e-8 rms, 2.49e-6 at most, measured on the GPU).  The steps leave out the exponential's own last bit."""
+    import math
+
+    src = open(os.path.join(ROOT, "draw-things-community_amd", "csrc", "dt_dense_kernel.h")).read()
+    coef = re.search(r"kP\[11\] = \{([^}]*)\}", src).group(1)
+    c = [np.float32(float.fromhex(t.strip().rstrip("f"))) for t in coef.split(",")]
+    x = np.arange(1 << 16, dtype=np.uint16).view(np.float16)
+    x = x[np.isfinite(x)].astype(np.float32)
+    x = x[(x >= -5.8) & (x != 0)]
+    fma = lambda u, v, w: (u.astype(np.float64) * v.astype(np.float64) + np.asarray(w, np.float64)).astype(np.float32)
+    a = np.minimum(np.abs(x), np.float32(5.8))
+    p = np.full_like(a, c[10])
+    for k in range(9, -1, -1):
+        p = fma(p, a, c[k])
+    e = np.exp2((p * a).astype(np.float64)).astype(np.float32)
+    got = (np.float32(0.5) * fma(-a, e, x + np.abs(x))).astype(np.float64)
+    want = np.array([0.5 * v * math.erfc(-v * math.sqrt(0.5)) for v in x.astype(np.float64)])
+    rel = np.abs(got - want) / np.abs(want)
+    assert np.sqrt((rel ** 2).mean()) <= 9e-8 and rel.max() <= 2.2e-6
+
+
 def test_rows_that_need_no_workspace(dthip):
     """The operators do not ask for workspace up to the rows that the library's streaming kernel takes: one number, twice."""
     import re
