@@ -824,9 +824,8 @@ static dt_status launch(hipStream_t s, SdpaArgs a) {
   const bool oneseg = a.n_kvseg == 1 && a.k[0].ss > 0 && a.v[0].ss > 0 && a.Skv < (1 << 30) &&
                       (a.Skv + 2 * BKV) * a.k[0].ss * 2 < 0x7fffffffLL && (a.Skv + 2 * BKV) * a.v[0].ss * 2 < 0x7fffffffLL;
   dim3 block(512);
-  if constexpr (DP == 64 || M16) if (a.partials) {
-    // key-split launch (never of the few long tasks that 32x32x16 MFMAs take at head sizes above 64): the counters start at
-    // zero
+  if (a.partials) {
+    // key-split launch: the counters start at zero
     if (!a.counters_zeroed) {
       const int n = a.cut_tasks * kSdpaSplitNodes;
       hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
@@ -860,11 +859,14 @@ dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
   // 16 heads of 40 73 us against 81, 20 heads of 64 113 against 122).  Above, 16x16x32 is ahead where the workgroups fill
   // the card, whose power then is the limit, and behind where under seven tenths of the compute units have one and the clock
   // stays up (us, 32x32x16 / 16x16x32, head size 128: 120 workgroups 34.8 / 36.9, 144 101 / 108, 168 47.2 / 48.3, 192 104
-  // / 99, 216 66.9 / 63.1, 264 cut along the keys 111 / 109, 432 250 / 235, 1440 of 141 key tiles 1495 / 1398; head size 80:
-  // 144 56.7 / 58.4, 256 113 / 96).
+  // / 99, 216 66.9 / 63.1, 432 250 / 235, 1440 of 141 key tiles 1495 / 1398; head size 80: 144 56.7 / 58.4, 256 113 / 96).
+  // Cut along the keys, launches of up to one round are too short to be limited by power, however many workgroups the parts
+  // are: 16x16x32 takes 1.06 times as long with under 100 of them, 1.05 up to 160, 1.00 .. 1.02 from 200 on (medians of 700
+  // launches of head sizes 88 .. 128; 12 heads, 323 x 1928 39.0 / 41.7), 0.97 behind whole rounds (264 tasks 111 / 109).
+  // Head sizes up to 80 multiply 80 columns in this form only, which decides for it wherever the launch is cut (0.83 .. 0.98).
   if (a.D <= 64) return launch<64, 64, false>(s, a);
   const int64_t tasks = (a.Sq + QROWS - 1) / QROWS * a.Hq * a.B;
-  if (!a.partials && tasks * 10 < compute_units() * 7LL) return launch<128, 128, false>(s, a);
+  if (a.partials ? a.D > 80 && a.whole_tasks == 0 : tasks * 10 < compute_units() * 7LL) return launch<128, 128, false>(s, a);
   if (a.D <= 80) return launch<128, 80, true>(s, a);
   return launch<128, 128, true>(s, a);
 }

@@ -182,6 +182,51 @@ def test_sdpa_card_full_of_workgroups(dthip, oracle, torch_cuda, D, Sq, Skv, n_s
     assert float((got[:1, :, :few].float() - some.float()).abs().max()) <= 6 * 2.0 ** -10 + 2.0 ** -8
 
 
+@pytest.mark.parametrize("D", [80, 128])
+@pytest.mark.parametrize("kind", ["large", "grouped", "strided", "segments3", "segments4", "one_norm", "unaligned"])
+def test_sdpa_card_full_beside_the_main_shape(dthip, oracle, torch_cuda, monkeypatch, kind, D):
+    """What small launches of other tests cover, on enough workgroups for the uncut 16x16x32 form (2 x 130 of them): scores that
+    outgrow the references tile after tile, grouped heads, outputs on the 8-byte grid, up to four segments, a norm weight on
+    one of two segments that share a wave, norm weights and tables off the 16-byte grid."""
+    torch = torch_cuda
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "never")
+    rng = np.random.default_rng(D + len(kind))
+    B, H, Sq, Skv, scale = 2, 130, 37, 210, 1 / np.sqrt(D)
+    q, k, v = rand_qkv(rng, B, Sq, Skv, H, 65 if kind == "grouped" else H, D)
+    if kind == "large":
+        q, k = f16(q * 4), f16(k * np.linspace(0.1, 30, Skv)[:, None, None])
+    cuts = {"segments3": [0, 64, 128, Skv], "segments4": [0, 5, 135, 136, Skv]}.get(kind, [0, Skv])
+    dev = lambda t: to_dev(torch, t)
+    parts = lambda t, at: [dev(t[:, a:b]) for a, b in zip(at, at[1:])]
+
+    def off(t):  # 4-byte, not 16-byte aligned
+        flat = torch.zeros(t.size + 2, dtype=torch.float16, device="cuda")
+        flat[2:] = dev(t).reshape(-1)
+        return flat[2:].view(*t.shape)
+
+    q_at, kw, qn = [0, Sq], {}, q
+    buf = torch.full((B, Sq, H * D + 4), -77.0, dtype=torch.float16, device="cuda")
+    if kind == "strided":
+        kw["out"] = buf[:, :, 4:].unflatten(2, (H, D))
+    if kind in ("one_norm", "unaligned"):
+        gamma, rot = f16(1 + 0.1 * rng.standard_normal(D)), f16(rng.standard_normal((Sq, D)))
+        normed = np.stack([oracle.C.rmsnorm(x, gamma, 1e-6) for x in q])
+        if kind == "one_norm":
+            q_at, normed[:, :17] = [0, 17, Sq], q[:, :17]
+            kw.update(gamma_q=[None, dev(gamma)], rot_q=dev(rot))
+        else:
+            kw.update(gamma_q=[off(gamma)], rot_q=off(rot))
+        qn = np.stack([oracle.C.cmul(x, rot) for x in normed])
+    print("sdpa card full, beside the main shape", kind, D, flush=True)
+    got = dthip.sdpa_segments(parts(q, q_at), parts(k, cuts), parts(v, cuts), scale, **kw)
+    mx, rr = oracle.err_stats(got.cpu().numpy(), oracle.C.sdpa(qn, k, v, scale))
+    assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+    if kind == "strided":
+        assert bool((buf[:, :, :4] == -77).all())
+    if kind.startswith("segments"):
+        assert torch.equal(got, dthip.sdpa_segments([dev(q)], [dev(k)], [dev(v)], scale))
+
+
 def test_sdpa_invariants(dthip, oracle, torch_cuda):
     torch = torch_cuda
     rng = np.random.default_rng(5)
@@ -723,6 +768,9 @@ SPLIT_CASES = [
     (1, 130, 1900, 4, 2, 64, 1),      # grouped heads
     (1, 520, 2100, 1, 1, 128, -1),    # a scale the kernel folds into the scores first (negative)
     (1, 1, 300, 1, 1, 128, 1),        # one query row, five key tiles in two pieces
+    (1, 300, 1000, 2, 2, 80, 1),      # 80 columns multiplied: an odd number of 16-wide blocks
+    (1, 130, 1900, 4, 2, 72, -1),     # the last of them half padding
+    (2, 256, 640, 3, 3, 96, 1),       # between 80 and 128
 ]
 
 
@@ -753,7 +801,8 @@ def test_sdpa_key_split_vs_oracle(dthip, oracle, torch_cuda, monkeypatch, B, Sq,
     assert float((got.float() - plain.float()).abs().max()) <= 2e-3
 
 
-@pytest.mark.parametrize("D,Skv,n_seg", [(128, 1100, 1), (128, 1100, 2), (64, 450, 1), (40, 130, 2)])
+@pytest.mark.parametrize("D,Skv,n_seg", [(128, 1100, 1), (128, 1100, 2), (64, 450, 1), (40, 130, 2),
+                                            (80, 1100, 1), (80, 450, 2), (72, 130, 2), (96, 450, 1)])
 def test_sdpa_key_split_last_round(dthip, oracle, torch_cuda, monkeypatch, D, Skv, n_seg):
     """264 tasks: 256 stay whole, the last 8 -- of the last head -- are cut into 8, 8, 4 and 2 parts."""
     torch = torch_cuda
@@ -777,7 +826,7 @@ def test_sdpa_key_split_last_round(dthip, oracle, torch_cuda, monkeypatch, D, Sk
     assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
 
 
-@pytest.mark.parametrize("D,n_seg,sign", [(128, 1, 1), (128, 2, 1), (64, 1, 1), (40, 2, 1), (128, 1, -1)])
+@pytest.mark.parametrize("D,n_seg,sign", [(128, 1, 1), (128, 2, 1), (64, 1, 1), (40, 2, 1), (128, 1, -1), (80, 1, 1), (80, 2, -1)])
 @pytest.mark.parametrize("masked", ["tail", "head"])
 def test_sdpa_key_split_masked_part(dthip, oracle, torch_cuda, monkeypatch, D, n_seg, sign, masked):
     """Keys masked through the dot product -- one component of -inf, so that their scores are -inf -- fill whole parts of
@@ -875,6 +924,26 @@ def test_sdpa_key_split_by_its_own_estimate(dthip, oracle, torch_cuda, monkeypat
     rows[0], rows[-1] = 0, S - 1
     want = oracle.C.sdpa(np.ascontiguousarray(q[:, rows]), k, v, scale)
     mx, rr = oracle.err_stats(got[:, rows], want)
+    assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+
+
+@pytest.mark.parametrize("B,H,D,S", [(1, 8, 80, 4096), (1, 8, 128, 4096)])
+def test_sdpa_key_split_of_blocks_of_few_heads(dthip, oracle, torch_cuda, monkeypatch, B, H, D, S):
+    """One image through a UNet block's self-attention (8 heads of 80), and 8 heads of 128: 128 workgroups, cut in two by
+    the library's own estimate; sampled rows against the oracle."""
+    torch = torch_cuda
+    monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
+    assert dthip.lib().dt_sdpa_workspace_bytes(B, H, H, D, S, S, 0, 0) > 0
+    rng = np.random.default_rng(S + D)
+    q, k, v = rand_qkv(rng, B, S, S, H, H, D)
+    scale = 1 / np.sqrt(D)
+    print("sdpa key split, few heads", B, H, D, S, flush=True)
+    args = [to_dev(torch, q)], [to_dev(torch, k)], [to_dev(torch, v)], scale
+    got = dthip.sdpa_segments(*args)
+    assert torch.equal(got, dthip.sdpa_segments(*args))
+    rows = np.sort(rng.choice(S, size=40, replace=False))
+    rows[0], rows[-1] = 0, S - 1
+    mx, rr = oracle.err_stats(got[:, rows].cpu().numpy(), oracle.C.sdpa(np.ascontiguousarray(q[:, rows]), k, v, scale))
     assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
 
 
