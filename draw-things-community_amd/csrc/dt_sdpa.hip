@@ -860,13 +860,16 @@ dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
   // the card, whose power then is the limit, and behind where under seven tenths of the compute units have one and the clock
   // stays up (us, 32x32x16 / 16x16x32, head size 128: 120 workgroups 34.8 / 36.9, 144 101 / 108, 168 47.2 / 48.3, 192 104
   // / 99, 216 66.9 / 63.1, 432 250 / 235, 1440 of 141 key tiles 1495 / 1398; head size 80: 144 56.7 / 58.4, 256 113 / 96).
-  // Cut along the keys, launches of up to one round are too short to be limited by power, however many workgroups the parts
-  // are: 16x16x32 takes 1.06 times as long with under 100 of them, 1.05 up to 160, 1.00 .. 1.02 from 200 on (medians of 700
-  // launches of head sizes 88 .. 128; 12 heads, 323 x 1928 39.0 / 41.7), 0.97 behind whole rounds (264 tasks 111 / 109).
+  // Cut along the keys, launches of up to one round are limited by power only where the parts are many and long: 16x16x32 takes
+  // 1.06 times as long with under 100 of them and 1.02 .. 1.03 with 220 .. 256 of up to 8 key tiles; from 200 parts of 16 key
+  // tiles on it takes 1.00 .. 0.97, behind whole rounds 0.97 (means of 1400 launches of head sizes 88 .. 128; us, 12 heads of 128, 323 x
+  // 1928 34.2 / 35.9, 4 heads, 4096 x 4096 60.3 / 58.0, 264 tasks 111 / 109).
   // Head sizes up to 80 multiply 80 columns in this form only, which decides for it wherever the launch is cut (0.83 .. 0.98).
   if (a.D <= 64) return launch<64, 64, false>(s, a);
   const int64_t tasks = (a.Sq + QROWS - 1) / QROWS * a.Hq * a.B;
-  if (a.partials ? a.D > 80 && a.whole_tasks == 0 : tasks * 10 < compute_units() * 7LL) return launch<128, 128, false>(s, a);
+  const int64_t cus = compute_units();
+  const auto short_parts = [&] { return (int64_t)a.cut_tasks * a.shares * 10 < cus * 8 || (a.Skv + BKV - 1) / BKV < 16 * a.shares; };
+  if (a.partials ? a.D > 80 && a.whole_tasks == 0 && short_parts() : tasks * 10 < cus * 7) return launch<128, 128, false>(s, a);
   if (a.D <= 80) return launch<128, 80, true>(s, a);
   return launch<128, 128, true>(s, a);
 }

@@ -927,9 +927,9 @@ def test_sdpa_key_split_by_its_own_estimate(dthip, oracle, torch_cuda, monkeypat
     assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
 
 
-@pytest.mark.parametrize("B,H,D,S", [(1, 8, 80, 4096), (1, 8, 128, 4096)])
+@pytest.mark.parametrize("B,H,D,S", [(1, 8, 80, 4096), (1, 8, 128, 4096), (1, 6, 128, 2560)])
 def test_sdpa_key_split_of_blocks_of_few_heads(dthip, oracle, torch_cuda, monkeypatch, B, H, D, S):
-    """One image through a UNet block's self-attention (8 heads of 80), and 8 heads of 128: 128 workgroups, cut in two by
+    """One image through a UNet block's self-attention (8 heads of 80), and heads of 128 in long and in short parts: cut by
     the library's own estimate; sampled rows against the oracle."""
     torch = torch_cuda
     monkeypatch.delenv("DT_SDPA_KEY_SPLIT", raising=False)
