@@ -463,7 +463,11 @@ def _enqueue_dense(problems, flags, stream):
     groups = b"".join(g for _, g, _, _ in packed)  # (what they point to lives in `packed` until the call returns)
     n, L = len(packed), lib()
     need = L.dt_dense_scratch_bytes(n, groups) if any(M > _ROWS_MAX for _, _, _, M in packed) else 0
-    ws, at, need = _scratch(problems[0][0], need, 0)
+    like = problems[0][0]
+    ws, at, got = _scratch(like, need, 0)
+    if need and not got:  # the device is too full for copies of the weights; cutting takes less
+        ws, at, got = _scratch(like, L.dt_dense_workspace_bytes(n, groups), 0)
+    need = got
     if need:
         _check("dt_dense_qx_grouped_scratch_f16",
                L.dt_dense_qx_grouped_scratch_f16(_stream_ptr(stream), n, groups, flags, at, need))

@@ -668,3 +668,35 @@ def test_dense_tails_at_the_edges(dthip, oracle, M, N, K, q):
         res.copy_(res0)
         dthip.dense_post(x, [w], [bias], [dthip.DensePost(gate=g, residual=res, keep_output=False)])
         assert untouched(rbuf) and bool((res == res0 + product).all())
+
+
+def test_cuts_where_copies_of_the_weights_do_not_fit(dthip, oracle, monkeypatch):
+    """512 x 5120 -> 5120 runs on a 52 MB copy of its weight; where the device has no room for that, the call is cut along K as it is
+    without copies, for which 27 MB do."""
+    import torch
+
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    rng = np.random.default_rng(10)
+    M, K, N = 512, 5120, 5120
+    w, _ = make(dthip, oracle, rng, N, K, 6, 4096)
+    x, out = dev(rng.standard_normal((M, K)).astype(np.float16)), torch.empty((M, N), dtype=torch.float16, device="cuda")
+    G, keep = _groups(dthip, x, [w], [out])
+    copies, cut = dthip.lib().dt_dense_scratch_bytes(1, G), dthip.lib().dt_dense_workspace_bytes(1, G)
+    assert copies >= 2 * N * K > cut > 0
+    call = lambda: dthip.dense_multi(x, [w], [None])[0]
+    print("scratch that takes cuts and no copies", flush=True)
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
+    want = call()
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    assert not torch.equal(call(), want)
+    monkeypatch.delenv("DT_DENSE_SPLIT")
+    monkeypatch.delenv("DT_DENSE_EXPAND")
+    asked, scratch = [], dthip._scratch
+
+    def tight(like, need, least):  # a device with room for `cut` bytes
+        asked.append(need)
+        return scratch(like, need if need <= cut else least, least)
+
+    monkeypatch.setattr(dthip, "_scratch", tight)
+    assert torch.equal(call(), want) and asked[0] == copies
