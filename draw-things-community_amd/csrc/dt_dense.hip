@@ -430,6 +430,9 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
 static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, bool expand, double* cost) {
   const dt_qx_weight& w0 = hs[0].W[w_begin];
   const TilePlan packed = plan_format(hs, n, w_begin, w_end, wide, std::min(ws, kDenseMaxWorkspace), w0, false, cost);
+  // (The estimate knows palettes in LDS.  Looked up in memory a launch takes four times as long, median of 1000 of them; priced like
+  // the others, 219 x 1024 -> 3 x 7808 in q8 blocks of 2048 with a head epilogue stayed packed, 169 us instead of 37.)
+  if (choose_pal_mode(w0.qbits, w0.nib, hs[0].K, packed.BM, packed.BN, packed.tiles) == kPalGlobal) *cost *= 4.0;
   TilePlan plain;
   double copied;
   if (!expand || w0.qbits == 16 || !plan_copies(hs, n, w_begin, w_end, wide, ws, &plain, &copied)) return packed;
