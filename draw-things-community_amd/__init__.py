@@ -655,12 +655,13 @@ class LoRADense:
         long as K is, 60 us at 64 x 13824, unless it shares the base projection's launch.  Two streams cost a captured graph 12
         us, and a caller that waits for the host 65 (us, one call / two streams, rank 16: in a graph 64 x 13824 -> 5120 q6p 137 /
         93, 64 x 5120 -> 5120 63 / 54, 48 x 5120 -> 5120 56 / 51, 1024 x 12288 -> 3072 in blocks of 128 200 / 178, 64 x 3072 -> 3072 39
-        / 39, and the other way round 32 x 13824 -> 5120 88 / 91, 48 x 3072 -> 3072 34 / 37, 1024 x 1280 -> 1280 in blocks of 256 48 / 53;
+        / 39, with over 64 rows and blocks too small to be copied, means over the other sizes: K = 2048 .. 2303 0.96 of the time, 2304 ..
+        3071 0.93, 1536 .. 2047 0.99; and the other way round 32 x 13824 -> 5120 88 / 91, 48 x 3072 -> 3072 34 / 37, 1024 x 1280 -> 1280 in blocks of 256 48 / 53;
         otherwise 64 x 13824 -> 5120 137 / 118, 1024 x 12288 -> 3072 in blocks of 128 190 / 170, and the other way round 64 x 12288 ->
         3072 113 / 131, 1024 x 3072 -> 3072 in blocks of 256 86 / 123)."""
-        if weight.qbits == 16 or K < 3072 or M <= 32 or M * K < 64 * 3072:
+        if weight.qbits == 16 or K < 2048 or M <= 32 or M * K < 64 * 3072:
             return False
-        if not (M * K >= (60 * 13824 if M <= _ROWS_MAX else 8 << 20) or capturing()):
+        if not (K >= 3072 and M * K >= (60 * 13824 if M <= _ROWS_MAX else 8 << 20) or capturing()):
             return False
         if M <= _ROWS_MAX:
             return True

@@ -173,6 +173,7 @@ def test_dense_scratch_for_copies_with_few_rows(dthip, monkeypatch, K, N, n, q, 
     (64, 13824, 5120, 6, 4096, True, True), (64, 5120, 5120, 8, 16384, True, False), (64, 12288, 3072, 8, 16384, True, False),
     (32, 13824, 5120, 6, 4096, False, False), (48, 3072, 3072, 6, 4096, False, False), (64, 13824, 5120, 16, 0, False, False),
     (1024, 12288, 3072, 6, 128, True, True), (1024, 3072, 3072, 6, 256, True, False), (4608, 1280, 1280, 6, 256, False, False),
+    (933, 2816, 1152, 6, 256, True, False), (4608, 2048, 1280, 6, 256, True, False), (1300, 1984, 640, 6, 256, False, False),
     (4608, 3072, 3072, 6, 4096, False, False), (512, 5120, 5120, 5, 1024, False, False),  # copied: one launch
 ])
 def test_lora_down_projection_beside_the_base(dthip, monkeypatch, M, K, N, q, nib, captured, otherwise):
