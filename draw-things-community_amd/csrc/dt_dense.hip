@@ -488,7 +488,7 @@ static NextLaunch next_launch(const HostGroup& h, int i, size_t ws, bool expand)
     cost += apart + 5.0;
     j = end;
   }
-  return together < cost ? all : l;
+  return together < cost || expand_knob('a') ? all : l;
 }
 
 // Scratch memory of a call, or none.

@@ -429,6 +429,35 @@ def test_lora_base_and_down_in_one_launch(dthip, oracle, monkeypatch, M, N, K, q
     assert all(torch.equal(a, b) for a, b in zip(got["never"], got["always"]))
 
 
+@pytest.mark.parametrize("formats,together", [
+    ([(16, 0), (6, 4096)], [1]),                          # the plain weight first: the launch's format is another weight's
+    ([(6, 4096), (16, 0), (6, 4096)], [0, 2]),
+    ([(6, 4096), (16, 0), (8, 16384), (16, 0), (8, 16384)], [2, 4]),  # two launches, a plain weight in each
+])
+def test_palettized_and_plain_weights_in_one_launch(dthip, oracle, monkeypatch, formats, together):
+    """One launch on the copies of all palettized weights and the plain ones between them, which the scratch asked for shows: the
+    same bits as one launch after the other; cut along K as well, the counters behind the copies."""
+    import torch
+
+    rng = np.random.default_rng(len(formats))
+    M, K = 300, 448
+    X, Ns = rng.standard_normal((M, K)).astype(np.float16), [260, 72, 130, 128, 300][:len(formats)]
+    pairs = [make(dthip, oracle, rng, n, K, q, nib) for n, (q, nib) in zip(Ns, formats)]
+    ws, bias = [w for w, _ in pairs], [(rng.standard_normal(n) * 0.1).astype(np.float16) for n in Ns]
+    x, b = dev(X), [dev(t) for t in bias]
+    print("palettized and plain weights in one launch", formats, flush=True)
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")
+    monkeypatch.setenv("DT_DENSE_EXPAND", "never")
+    apart = dthip.dense_multi(x, ws, b)
+    monkeypatch.setenv("DT_DENSE_EXPAND", "always")
+    G, keep = _groups(dthip, x, ws, apart)
+    assert dthip.lib().dt_dense_scratch_bytes(1, G) == sum((ws[i].count * 2 + 255) // 256 * 256 for i in together)
+    assert all(torch.equal(a, c) for a, c in zip(apart, dthip.dense_multi(x, ws, b)))
+    monkeypatch.setenv("DT_DENSE_SPLIT", "always")
+    for got, (_, W), t in zip(dthip.dense_multi(x, ws, b), pairs, bias):
+        check(got.cpu().numpy(), X, W, t)
+
+
 @pytest.mark.parametrize("M,N,K,q,nib", [(64, 256, 3072, 8, 16384), (64, 128, 13824, 6, 4096), (130, 260, 3072, 4, 256)])
 def test_lora_down_beside_the_base_in_a_graph(dthip, oracle, M, N, K, q, nib):
     """The down projection on its own stream: captured, replayed and beside other work, the same bits as in one call."""
