@@ -518,6 +518,7 @@ static dt_status launch_plan(hipStream_t s, DenseArgs& a, int n_w, const TilePla
   }
   int qbits = qx[0]->qbits, mode;
   if (plan.expand_bytes > 0) {
+    static_assert(kDepalMax >= kMaxWeights, "every weight of a launch may need a copy");
     DepalettizeMany d = {};
     d.counters = a.counters;
     d.n_counters = n_counters;

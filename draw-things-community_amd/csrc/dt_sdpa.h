@@ -39,8 +39,9 @@ struct SdpaArgs {
   int32_t q_tiles, total_blocks;  // filled by the launcher
 };
 
-// Floats of one partial-result slot of the key-split kernel: 512 threads x (DP / 32 * 16 accumulators + reference
-// maximum + row-sum share).
+// Floats of one partial-result slot of the key-split kernel: 512 threads x DP / 32 * 16 accumulators, then for each wave the 32
+// reference maxima and 32 row sums of its queries; the last 512 are spare, so that callers are asked for the room that they
+// always were.
 constexpr int sdpa_split_slot_floats(int dp) { return (dp / 32) * 16 * 512 + 2 * 512; }
 
 // Most parts of a task; their meetings are 4 + 2 + 1.

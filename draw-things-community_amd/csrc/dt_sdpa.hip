@@ -59,7 +59,8 @@ __device__ __forceinline__ int k_chunk_swz(int row, int c) {
 // many bytes are swizzled over the row index.
 template <int DP, bool M16>
 __device__ __forceinline__ int v_unit_swz(int row, int u) {
-  if constexpr (M16) return u ^ (DP == 128 ? row & 7 : (row >> 1) & 3);
+  static_assert(!M16 || DP == 128, "head sizes up to 64 are 32x32x16");
+  if constexpr (M16) return u ^ (row & 7);
   return u ^ (DP == 128 ? row & 3 : (row >> 1) & 1);
 }
 
