@@ -906,7 +906,9 @@ __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 
     const int i = half * HN + m % HN, j = m / HN;
     // (assembly because the sums have to stay where they are: the builtin's result may be any other four registers, and
     // with 176 of 256 taken by sums and operands the allocator spilled over the moving holes.  Operands come from LDS
-    // reads, whose waits the compiler inserts; a sum's next MFMA is a whole iteration away.)
+    // reads, whose waits the compiler inserts; a sum's next MFMA is a whole iteration away.  It depends on the compiler having no
+    // reason to copy, move or spill a sum before the s_nop behind the loop, which nothing would hold back until the MFMA is
+    // done: tests/test_matrix_sums_cpu.py looks through the built kernels for that.)
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(fw[i]), "v"(fx[XB == 2 ? par : 0][j]));
   };
 
