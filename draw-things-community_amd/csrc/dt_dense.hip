@@ -1,10 +1,13 @@
 // K1: Dense over palettized weights, Y = X W^T (+ bias), for gfx950.
 //
-// The packed weight never exists dequantized in memory: per K-tile two threads
+// The tiled kernel takes weights packed: per K-tile two threads
 // per weight row each pull half of a 32-index granule into registers, unpack
 // it, look the fp16 values up in palettes held in LDS, and write the fp16 row
 // slice into an LDS ring that v_mfma_f32_16x16x32_f16 then consumes; X (and a
-// plain fp16 weight) goes from memory straight into LDS.  fp32 accumulation,
+// plain fp16 weight) goes from memory straight into LDS.  Where many rows of X
+// would have it look every weight up once per tile of rows, and the caller has
+// scratch for them, fp16 copies of the weights are written first and the launch
+// runs on those (plan_copies).  fp32 accumulation,
 // one rounding to fp16, optional fused tails (per-head RMSNorm + RoPE, or
 // activation / gate / fp32 residual).
 //
@@ -246,7 +249,11 @@ constexpr int64_t kDenseFewRows = 640;
 
 // Estimated time (us) of a launch whose rows enter new blocks at every `step`-th K-tile at most: a fit to 930 launches of
 // 65 .. 4000 rows on the whole card (part of one would need costs of its own; the results do not depend on the layout
-// chosen beyond the order of the sums), nine tenths of them within a tenth.  Priced are: one workgroup's K-tile on each
+// chosen beyond the order of the sums), made on kernels with 32x32x16 instructions, nine tenths of them within a tenth then.  Against the
+// present ones (8100 launches of 65 .. 8192 rows of random sizes, replayed from graphs) it is high for uncut 128 x 128 tiles,
+// 1.29 times the measured time with packed weights and 1.41 with plain ones (medians; they take some 4 us less than the 7.7 outside the
+// K loop), and 0.94 .. 1.15 on the other shapes and on cuts.  The choice between packed weights and copies, which takes 0.93 of it for
+// these, falls on the slower by 5 % and 3 us in 346 of 6154 launches, 1.4 % of the time of all.  Priced are: one workgroup's K-tile on each
 // tile shape, the cheaper the more compute units idle (the card is limited as a whole); what entering new blocks adds to it
 // where every row has a table of its own to rewrite, most for 128 and 256 entries; the time outside the K loop; two
 // 128 x 128 tiles that share a compute unit, except with per-row tables of 32 or 64 KB beside the other 56, which take it in
@@ -351,8 +358,8 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
   const int64_t step = pal_step(K, w0.qbits == 16 ? 32 : w0.nib);
   const double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step, expanded);
   *cost = start;
-  // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate, whose error
-  // is up to a tenth, sees a clear gain.
+  // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate sees a
+  // clear gain.
   const char* knob = getenv("DT_DENSE_SPLIT");  // "never" | "always" (as often as can be; for tests); read at every call
   if (ws_bytes == 0 || (knob && knob[0] == 'n')) return base;
   if (knob && knob[0] == 'a') {
@@ -413,7 +420,8 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
   *plan = plan_format(hs, n, w_begin, w_end, wide, std::min(ws - bytes, kDenseMaxWorkspace), f16, true, cost);
   plan->expand_bytes = bytes;
   // A copy costs 3.4 us and 0.44 per million weights, 0.65 where it outgrows the memory-side cache (28 M weights 13 us, 94 M
-  // 61), and the plain launch on it takes 0.93 of its estimate (medians of 700 launches of 65 .. 8192 rows).
+  // 61), and the plain launch on it takes 0.93 of its estimate (medians of 700 launches of 65 .. 8192 rows; 0.87 over the larger set
+  // that plan_cost names).
   const double m = 1e-6 * (double)weights;
   *cost = 0.93 * *cost + 3.4 + 0.44 * m + 0.21 * std::max(0.0, m - 64.0);
   return true;

@@ -1135,8 +1135,9 @@ __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 
   const auto all_tiles = [&]() __attribute__((always_inline)) {
     int t = SPLIT ? t_lo : 0;
     if constexpr (NS > 2) {
-      // Rounds of NS pairs, so that every slot is a constant (us, slot addresses made in the loop / here, and with two slots:
-      // 1344 x 1920 -> 200 17.6 / 16.3, 16.3; 300 x 3904 -> 2 x 384 27.8 / 25.4, 39.1; 3175 x 5120 -> 3 x 256 45.3 / 42.5, 57.5).
+      // Rounds of NS pairs, so that every slot is a constant (on 128 x 128 tiles, which have a kernel of their own now, slot
+      // addresses made in the loop cost 7 .. 9 %).  us on 128 x 256 tiles, two slots / three: 500 x 3072 -> 3 x 3072 with a head epilogue
+      // 46.8 / 40.4, 900 x 5120 -> 2560 48.6 / 43.0; cut along K 200 x 8192 -> 3072 40.4 / 36.7.
       const auto pair = [&](int t, int slot) __attribute__((always_inline)) {
         const int next = slot + 1 < NS ? slot + 1 : 0;
         half_t* const xs = XsA + slot * (XS_BYTES / 2);

@@ -860,7 +860,8 @@ dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
   // 16 heads of 40 73 us against 81, 20 heads of 64 113 against 122).  Above, 16x16x32 is ahead where the workgroups fill
   // the card, whose power then is the limit, and behind where under seven tenths of the compute units have one and the clock
   // stays up (us, 32x32x16 / 16x16x32, head size 128: 120 workgroups 34.8 / 36.9, 144 101 / 108, 168 47.2 / 48.3, 192 104
-  // / 99, 216 66.9 / 63.1, 432 250 / 235, 1440 of 141 key tiles 1495 / 1398; head size 80: 144 56.7 / 58.4, 256 113 / 96).
+  // / 99, 216 66.9 / 63.1, 432 250 / 235 alone in a loop and 258 / 255 behind a block's projections, 1440 of 141 key tiles 1495 /
+  // 1398; head size 80: 144 56.7 / 58.4, 256 113 / 96).
   // Cut along the keys, launches of up to one round are limited by power only where the parts are many and long: 16x16x32 takes
   // 1.06 times as long with under 100 of them and 1.02 .. 1.03 with 220 .. 256 of up to 8 key tiles; from 200 parts of 16 key
   // tiles on it takes 1.00 .. 0.97, behind whole rounds 0.97 (means of 1400 launches of head sizes 88 .. 128; us, 12 heads of 128, 323 x
