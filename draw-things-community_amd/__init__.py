@@ -437,6 +437,10 @@ def _marshal_dense(x, weights, biases, outs, epilogues, posts):
 # not asked how much (0.5 us of a conditioning row's 22).  The few such calls that it gives to the tiled kernel after all
 # -- plain fp16 weights with over 16 rows and 8192 features, palettes that do not fit the LDS -- run uncut from here.
 _ROWS_MAX = 64
+# The smallest blocks and the most bytes of fp16 that the library copies palettized weights in (kDepalMinNib in
+# csrc/dt_depalettize.h, kDenseMaxExpand in csrc/dt_dense.hip).
+_COPIED_NIB, _COPIED_BYTES = 512, 512 << 20
+_BESIDE_INPUTS = 2048  # from which on a LoRA layer's down projection may get a stream of its own
 
 
 def _scratch(like, need, least):
@@ -659,12 +663,16 @@ class LoRADense:
         3071 0.93, 1536 .. 2047 0.99; and the other way round 32 x 13824 -> 5120 88 / 91, 48 x 3072 -> 3072 34 / 37, 1024 x 1280 -> 1280 in blocks of 256 48 / 53;
         otherwise 64 x 13824 -> 5120 137 / 118, 1024 x 12288 -> 3072 in blocks of 128 190 / 170, and the other way round 64 x 12288 ->
         3072 113 / 131, 1024 x 3072 -> 3072 in blocks of 256 86 / 123)."""
-        if weight.qbits == 16 or K < 2048 or M <= 32 or M * K < 64 * 3072:
+        if weight.qbits == 16 or K < _BESIDE_INPUTS or M <= 32 or M * K < 64 * 3072:
             return False
         if not (K >= 3072 and M * K >= (60 * 13824 if M <= _ROWS_MAX else 8 << 20) or capturing()):
             return False
-        if M <= _ROWS_MAX:
+        if M <= _ROWS_MAX or weight.nib < _COPIED_NIB or 2 * weight.count > _COPIED_BYTES:
             return True
+        # What can be copied mostly is, with that many rows, and asking takes the host 6 us of a layer that waits for it
+        # (2800 x 3072 -> 512: 42 us, 48 with the question).  A graph asks once.
+        if not capturing():
+            return False
         # the call as the library sees it, as far as it looks at addresses
         ws = (_QxWeight * 2)(_QxWeight(4096, weight.qbits, weight.nib, weight.count), _QxWeight(4096, 16, 0, rank * K))
         ys, strides = (ctypes.c_void_p * 2)(4096, 4096), (ctypes.c_int64 * 2)(weight.shape[0], rank)
@@ -696,8 +704,9 @@ class LoRADense:
         # short the host has no time for more.  The up projection's epilogue adds the base projection's result and then runs
         # the tail.  (fp16(base) + fp16(branch) rounds the same whichever of the two is the addend.)
         down_post = DensePost(scale=self.configuration.scale)
-        K = _f16_cuda(x, "x").shape[-1]
-        if self._down_beside_base(x.numel() // max(K, 1), K, self.weight, dn.shape[0], lambda: _capturing(stream)):
+        K = self.weight.shape[1]
+        if K >= _BESIDE_INPUTS and self._down_beside_base(_f16_cuda(x, "x").numel() // K, K, self.weight, dn.shape[0],
+                                                          lambda: _capturing(stream)):
             torch = _torch()
             main = stream if stream is not None else torch.cuda.current_stream(x.device)
             side = _side_stream(x.device)
@@ -760,6 +769,8 @@ def _side_stream(device):
 
 def _capturing(stream) -> bool:
     """Whether what is enqueued on `stream` (None: the current one) becomes part of a graph."""
+    if stream is None:
+        return _torch().cuda.is_current_stream_capturing()
     with _on(stream):
         return _torch().cuda.is_current_stream_capturing()
 

@@ -216,6 +216,18 @@ def test_rows_that_need_no_workspace(dthip):
     assert dthip._ROWS_MAX == int(re.search(r"kRowsMax = (\d+);", header).group(1))
 
 
+def test_eager_lora_layers_are_decided_without_the_library(dthip, monkeypatch):
+    """Its answer takes the host 6 us, which layers that wait for the host do not have; what it copies at most is stated twice."""
+    csrc = os.path.join(ROOT, "draw-things-community_amd", "csrc")
+    text = lambda name: open(os.path.join(csrc, name)).read()
+    assert dthip._COPIED_NIB == int(re.search(r"kDepalMinNib = (\d+);", text("dt_depalettize.h")).group(1))
+    assert dthip._COPIED_BYTES >> 20 == int(re.search(r"kDenseMaxExpand = \(size_t\)(\d+) << 20;", text("dt_dense.hip")).group(1))
+    monkeypatch.setattr(dthip, "lib", lambda: pytest.fail("the library was asked"))
+    for M, K, q, nib, beside in ((2800, 3072, 6, 4096, False), (4608, 12288, 8, 16384, False), (1024, 12288, 6, 256, True),
+                                 (64, 13824, 6, 4096, True), (64, 3072, 6, 4096, False)):
+        assert dthip.LoRADense._down_beside_base(M, K, dthip.QxTensor(None, q, nib, (512, K)), 64, lambda: False) == beside
+
+
 def test_missing_library_fails_loudly(dthip, monkeypatch):
     monkeypatch.setattr(dthip, "_lib", None)
     monkeypatch.setattr(dthip, "LIB_PATH", os.path.join(ROOT, "no_such_dir", "libdthip.so"))
