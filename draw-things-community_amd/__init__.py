@@ -704,10 +704,10 @@ class LoRADense:
         # short the host has no time for more.  The up projection's epilogue adds the base projection's result and then runs
         # the tail.  (fp16(base) + fp16(branch) rounds the same whichever of the two is the addend.)
         down_post = DensePost(scale=self.configuration.scale)
-        K = self.weight.shape[1]
-        if K >= _BESIDE_INPUTS and self._down_beside_base(_f16_cuda(x, "x").numel() // K, K, self.weight, dn.shape[0],
-                                                          lambda: _capturing(stream)):
-            torch = _torch()
+        torch, K = _torch(), self.weight.shape[1]
+        if K >= _BESIDE_INPUTS and self._down_beside_base(
+                _f16_cuda(x, "x").numel() // K, K, self.weight, dn.shape[0],
+                torch.cuda.is_current_stream_capturing if stream is None else lambda: _capturing(stream)):
             main = stream if stream is not None else torch.cuda.current_stream(x.device)
             side = _side_stream(x.device)
             side.wait_stream(main)
@@ -721,9 +721,10 @@ class LoRADense:
             down.record_stream(main)
         else:
             base, down = dense_post(x, [self.weight, dn], [b, None], [None, down_post], flags=self.flags, stream=stream)
-        tail = DensePost(p.activation, p.gate, p.residual, p.keep_output, addend=base.reshape(-1, self.count))
+        rows = x.dim() == 2  # (what has the shape already is not reshaped: 1 us each of 38)
+        tail = DensePost(p.activation, p.gate, p.residual, p.keep_output, addend=base if rows else base.reshape(-1, self.count))
         out = dense_post(down, [up], [None], [tail], stream=stream)[0]
-        return None if out is None else out.reshape(*x.shape[:-1], self.count)
+        return out if out is None or rows else out.reshape(*x.shape[:-1], self.count)
 
 
 def _lora_high_precision(self, x, b, p, stream):
@@ -737,7 +738,7 @@ def _lora_high_precision(self, x, b, p, stream):
     K, r = x.shape[-1], self.configuration.rank
     main = stream if stream is not None else torch.cuda.current_stream(x.device)
     with _on(main):  # a copy, if the view needs one, belongs on the caller's stream
-        x2 = x.reshape(-1, K)
+        x2 = x if x.dim() == 2 else x.reshape(-1, K)
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
         M = x2.shape[0]
@@ -750,7 +751,7 @@ def _lora_high_precision(self, x, b, p, stream):
         _check("dt_lora_branch_f32_f16", st)
     tail = DensePost(p.activation, p.gate, p.residual, p.keep_output, addend=branch)
     out = dense_post(x2, [self.weight], [b], [tail], flags=self.flags, stream=main)[0]
-    return None if out is None else out.reshape(*x.shape[:-1], self.count)
+    return out if out is None or x.dim() == 2 else out.reshape(*x.shape[:-1], self.count)
 
 
 LoRADense._high_precision = _lora_high_precision
@@ -768,9 +769,7 @@ def _side_stream(device):
 
 
 def _capturing(stream) -> bool:
-    """Whether what is enqueued on `stream` (None: the current one) becomes part of a graph."""
-    if stream is None:
-        return _torch().cuda.is_current_stream_capturing()
+    """Whether what is enqueued on `stream` becomes part of a graph."""
     with _on(stream):
         return _torch().cuda.is_current_stream_capturing()
 
