@@ -670,7 +670,7 @@ class LoRADense:
         if M <= _ROWS_MAX or weight.nib < _COPIED_NIB or 2 * weight.count > _COPIED_BYTES:
             return True
         # What can be copied mostly is, with that many rows, and asking takes the host 6 us of a layer that waits for it
-        # (2800 x 3072 -> 512: 42 us, 48 with the question).  A graph asks once.
+        # (2800 x 3072 -> 512: 38 us, 45 with the question).  A graph asks once.
         if not capturing():
             return False
         # the call as the library sees it, as far as it looks at addresses
@@ -736,6 +736,8 @@ def _lora_high_precision(self, x, b, p, stream):
         raise TypeError(f"LoRADense {self.name!r}: highPrecision takes contiguous float32 down / up weights")
     _f16_cuda(x, "x")
     K, r = x.shape[-1], self.configuration.rank
+    if dn.shape[1] != K or self.weight.shape[1] != K:  # (the branch goes out ahead of the Dense, which would say so)
+        raise ValueError(f"LoRADense {self.name!r}: weight or down do not match input width {K}")
     main = stream if stream is not None else torch.cuda.current_stream(x.device)
     with _on(main):  # a copy, if the view needs one, belongs on the caller's stream
         x2 = x if x.dim() == 2 else x.reshape(-1, K)

@@ -729,3 +729,17 @@ def test_cuts_where_copies_of_the_weights_do_not_fit(dthip, oracle, monkeypatch)
 
     monkeypatch.setattr(dthip, "_scratch", tight)
     assert torch.equal(call(), want) and asked[0] == copies
+
+
+@pytest.mark.parametrize("x_in,down_in", [(128, 64), (64, 128), (128, 128)])
+def test_lora_in_fp32_refuses_widths_that_differ(dthip, oracle, x_in, down_in):
+    """Inputs and down weights that are not as wide as the base weight (64) are refused before anything is launched on them."""
+    import torch
+
+    rng = np.random.default_rng(1)
+    op = dthip.LoRADense(128, dthip.LoRANetworkConfiguration(4, 0.75, True))
+    op.weight, op.bias = make(dthip, oracle, rng, 128, 64, 6, 4096)[0], None
+    op.down = dthip.QxTensor(torch.zeros((4, down_in), device="cuda"), 16, 0, (4, down_in))
+    op.up = dthip.QxTensor(torch.zeros((128, 4), device="cuda"), 16, 0, (128, 4))
+    with pytest.raises(ValueError, match="input width"):
+        op(torch.zeros((8, x_in), dtype=torch.float16, device="cuda"))
