@@ -27,7 +27,8 @@ struct SdpaArgs {
   const uint16_t* q_rot;
   float q_eps;
   int32_t q_prep;  // any of the above is set
-  int32_t q_norm;  // any q_gamma is (filled by the launcher)
+  int32_t q_norm;     // any q_gamma is (filled by the launcher)
+  int32_t q_aligned;  // q_rot and every q_gamma lie on 16 bytes (the same)
   // Key-split launch (optional; partials == nullptr runs one workgroup per task): workspace for the parts' partial
   // results and the counters of their meetings, sized and laid out by sdpa_split_plan().
   float* partials;

@@ -3,7 +3,8 @@
 // One 512-thread workgroup (8 waves, two per SIMD) owns 256 query rows of one
 // (batch, head); each wave owns 32 of them.  K/V arrive in tiles of 64 keys,
 // transferred from memory straight into LDS, row-major (double-buffered, one
-// barrier per tile).
+// barrier per tile).  Small launches take 128 rows, with two groups of waves
+// that share out the key tiles (KG).
 //
 // Everything is computed transposed so that the query index is the MFMA
 // column in every stage:
@@ -37,8 +38,12 @@
 namespace dt {
 
 constexpr int BKV = 64;     // keys per tile
-constexpr int QWAVES = 8;   // waves per workgroup, 32 query rows each
-constexpr int QROWS = QWAVES * 32;
+constexpr int WAVES = 8;    // waves per workgroup
+// Query rows of a workgroup whose waves, 32 rows each, fall into `key_groups` groups (see sdpa_kernel).
+constexpr int query_rows(int key_groups) { return WAVES / key_groups * 32; }
+// Two key groups at head sizes up to 64 leave registers and LDS for two workgroups on a compute unit: four waves on a SIMD, of 128
+// registers, which the loaders of several segments do not fit.
+constexpr bool sdpa_four_waves(int dp, bool oneseg, int key_groups) { return dp == 64 && oneseg && key_groups == 2; }
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
@@ -62,6 +67,13 @@ __device__ __forceinline__ int v_unit_swz(int row, int u) {
   static_assert(!M16 || DP == 128, "head sizes up to 64 are 32x32x16");
   if constexpr (M16) return u ^ (row & 7);
   return u ^ (DP == 128 ? row & 3 : (row >> 1) & 1);
+}
+
+// The larger of each half of three pairs of fp16; NaN wins.
+__device__ __forceinline__ uint32_t max3_h2(uint32_t x, uint32_t y, uint32_t z) {
+  uint32_t r;
+  asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "v"(z));
+  return r;
 }
 
 // The lane groups of a wave -- two of 32, M16: four of 16 -- hold the same matrix columns: combine them without touching LDS.
@@ -89,7 +101,12 @@ __device__ __forceinline__ float sum_groups(float v) {
   return sum32(a + b);
 }
 
-// SPLIT: for launches whose task count -- a task being the 256 query rows of one (batch, head) -- leaves the last round
+// KG: the waves of a workgroup fall into that many groups, which share the task's query rows and take every KG-th key tile each;
+// two meet through LDS at the end.
+// (VALU instructions of one wave run in the shadow of another's MFMAs only to a small degree, also with four waves on a SIMD: full
+// rounds gain nothing by this, small launches the finer tasks.)
+//
+// SPLIT: for launches whose task count -- a task being the query rows of a workgroup, of one (batch, head) -- leaves the last round
 // of workgroups mostly empty.  The first whole_tasks tasks, full rounds of them, go to a workgroup each; each of the
 // others is cut along its keys into `shares` equal parts.  A workgroup with a part holds its unnormalised fp32 output,
 // reference maximum and row sums, and the parts meet in pairs, the pairs in pairs, and so on: of two that meet, the
@@ -100,31 +117,38 @@ __device__ __forceinline__ float sum_groups(float v) {
 //
 // M16: 16x16x32 MFMAs.  DL: head dimension that is multiplied (M16: D rounded up to a block of 16; DP, what a tile row
 // holds, otherwise).
-template <int DP, int DL, bool M16, bool PREMUL, bool ONESEG, bool SPLIT>
-__global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
+template <int DP, int DL, bool M16, bool PREMUL, bool ONESEG, bool SPLIT, int KG>
+__global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)) sdpa_kernel(const SdpaArgs a) {
+  constexpr bool FOUR = sdpa_four_waves(DP, ONESEG, KG);
+  constexpr int QW = WAVES / KG;               // waves of a key group
+  constexpr int QROWS = query_rows(KG);
   constexpr int ROWB = DP * 2;                 // bytes per tile row
-  constexpr int DCH = DP / 8;                  // 16-byte chunks per row
   constexpr int TILE_B = BKV * ROWB;           // bytes of one K (or V) tile
-  constexpr int LOADS = BKV * DCH / 512;       // 16-byte chunks per thread per tile (2 at DP = 128)
+  constexpr int LOADS = TILE_B / (QW * 1024);  // 16-byte chunks per thread per tile
+  constexpr int LROWS = QW * 1024 / ROWB;      // rows of a tile that a load of all threads covers
+  constexpr bool ONES = DP == 64 && DL < DP;   // row sums come out of the second MFMA
   constexpr int MB = M16 ? 16 : 32;            // rows and columns of an MFMA
   constexpr int MK = M16 ? 32 : 16;            // its k-step
   constexpr int QB = 32 / MB;                  // its blocks in a wave's 32 queries
   constexpr int NV = M16 ? 4 : 16;             // its sums per lane
-  constexpr int DB = DL / MB;                  // its blocks of the head dimension
+  constexpr int DB = (DL + MB - 1) / MB;       // its blocks of the head dimension
   constexpr int KS = (DL + MK - 1) / MK;       // k-steps over the head dimension
   typedef typename std::conditional<M16, float4_t, float16_t>::type sums_t;
-  static_assert(LOADS >= 1, "tile");
+  static_assert(!SPLIT || KG == 1, "tasks are cut with one key group");
+  static_assert(LOADS >= 1 && LROWS % 16 == 0, "tile");
 
   // Two stages each for K and V: a tile is read from one while the next is in
   // flight into the other.
-  __shared__ __attribute__((aligned(1024))) unsigned char Ks0[TILE_B];
-  __shared__ __attribute__((aligned(1024))) unsigned char Ks1[TILE_B];
-  __shared__ __attribute__((aligned(1024))) unsigned char Vs0[TILE_B];
-  __shared__ __attribute__((aligned(1024))) unsigned char Vs1[TILE_B];
+  __shared__ __attribute__((aligned(1024))) unsigned char Ks0[KG * TILE_B];
+  __shared__ __attribute__((aligned(1024))) unsigned char Ks1[KG * TILE_B];
+  __shared__ __attribute__((aligned(1024))) unsigned char Vs0[KG * TILE_B];
+  __shared__ __attribute__((aligned(1024))) unsigned char Vs1[KG * TILE_B];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
+  const int qwave = wave & (QW - 1);                                      // which of the task's rows
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(wave / QW);  // key group
   const int col = lane & (MB - 1);  // row or column of an MFMA block
   const int grp = lane / MB;        // lane group: which k
 
@@ -141,7 +165,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   else bid = xcd_order(bid, a.total_blocks);
   const int64_t Sq = a.Sq, Skv = a.Skv;
   const int D = a.D;
-  const int n_tiles = (int)((Skv + BKV - 1) / BKV);
+  const int n_tiles = (int)((Skv + BKV - 1) / BKV), full_tiles = (int)(Skv / BKV);
 
   // ---- per-thread constants of the K / V tile loaders ---------------------
   // Tiles go from memory straight into LDS.  A wave's transfer instruction
@@ -151,23 +175,36 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   // (those slots keep the zeros they were given at the start), and so do, for
   // K, lanes whose row lies past the last key (their scores are masked whatever
   // the slot holds); V rows past the last key are zeroed (see zero_slot).
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  // One key group: a wave's loads cover consecutive rows, each with an offset
+  // in a register of its own.  Two, whose threads have twice as many: LROWS rows
+  // apart, whose chunk is the same (the swizzles depend on row % 16 at most), at
+  // one offset from bases that are.  (One offset costs one group 1 % of a launch.)
+  constexpr int OFFS = KG == 1 ? LOADS : 1;
+  const int qwave_u = __builtin_amdgcn_readfirstlane(qwave);
   int ld_row[LOADS], k_ch[LOADS], v_ch[LOADS];
+  auto v_chunk = [](int row, int pc) __attribute__((always_inline)) {  // (the swizzles are involutions)
+    return M16 ? v_unit_swz<DP, M16>(row, pc >> 1) * 2 + (pc & 1) : v_unit_swz<DP, M16>(row, pc >> 2) * 4 + (pc & 3);
+  };
+  auto place = [](int w, int i) __attribute__((always_inline)) { return (OFFS > 1 ? w * LOADS + i : i * QW + w) * 1024; };
 #pragma unroll
   for (int i = 0; i < LOADS; i++) {
-    const int off = (wave * LOADS + i) * 1024 + lane * 16;
+    const int off = place(qwave, OFFS > 1 ? i : 0) + lane * 16;
     const int row = off / ROWB, pc = (off % ROWB) / 16;
-    ld_row[i] = row;
-    k_ch[i] = k_chunk_swz<DP>(row, pc);  // the swizzles are involutions
-    v_ch[i] = M16 ? v_unit_swz<DP, M16>(row, pc >> 1) * 2 + (pc & 1) : v_unit_swz<DP, M16>(row, pc >> 2) * 4 + (pc & 3);
+    ld_row[i] = row + (OFFS > 1 ? 0 : i * LROWS);
+    k_ch[i] = k_chunk_swz<DP>(row, pc);
+    v_ch[i] = v_chunk(row, pc);
   }
-  // slots that no transfer will ever write must not hold NaN patterns
+  auto slot = [&](int i) __attribute__((always_inline)) { return (uint32_t)(kg * TILE_B + place(qwave_u, i)); };  // in a stage
+  // slots that no transfer will ever write must not hold NaN patterns; ONES: column D of V is ones
   if (D < DP || Skv % BKV != 0) {
-    for (int i = tid * 16; i < TILE_B; i += 512 * 16) {
-      *reinterpret_cast<uint4_t*>(Ks0 + i) = uint4_t{0, 0, 0, 0};
-      *reinterpret_cast<uint4_t*>(Ks1 + i) = uint4_t{0, 0, 0, 0};
-      *reinterpret_cast<uint4_t*>(Vs0 + i) = uint4_t{0, 0, 0, 0};
-      *reinterpret_cast<uint4_t*>(Vs1 + i) = uint4_t{0, 0, 0, 0};
+    for (int i = tid * 16; i < KG * TILE_B; i += 512 * 16) {
+      const uint4_t zero = {0, 0, 0, 0};
+      uint4_t v = zero;
+      if (ONES && v_chunk(i / ROWB, i % ROWB / 16) * 8 == D) v[0] = 0x3c00;
+      *reinterpret_cast<uint4_t*>(Ks0 + i) = zero;
+      *reinterpret_cast<uint4_t*>(Ks1 + i) = zero;
+      *reinterpret_cast<uint4_t*>(Vs0 + i) = v;
+      *reinterpret_cast<uint4_t*>(Vs1 + i) = v;
     }
     __syncthreads();
   }
@@ -176,7 +213,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   // K operand: key row kb*MB + col, chunk of the group's 8 head-dim elements in k-step ks
   int k_rd[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) k_rd[ks] = col * ROWB + k_chunk_swz<DP>(col, ks * (MK / 8) + grp) * 16;
+  for (int ks = 0; ks < KS; ks++) k_rd[ks] = kg * TILE_B + col * ROWB + k_chunk_swz<DP>(col, ks * (MK / 8) + grp) * 16;
   // V^T operand through the transposing read: lane i of a 16-lane group addresses key row (i / 4) of a 4-key run and 4
   // head-dim elements at 4 * (i % 4).  M16: the run is the group's, the elements those of block db.  Else: the run is the
   // half-wave's, and its two groups cover head-dim 0..15 and 16..31 of block db.
@@ -185,11 +222,11 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
 #pragma unroll
   for (int db = 0; db < DB; db++) {
     const int row = 4 * grp + (li >> 2);  // + multiples of 8 (M16: 16) per read: the swizzle depends on row & 3 (7) at most
-    v_rd[db] = row * ROWB + (M16 ? v_unit_swz<DP, M16>(row, db) * 32 : v_unit_swz<DP, M16>(row, db) * 64 + dg * 32) + (li & 3) * 8;
+    v_rd[db] = kg * TILE_B + row * ROWB + (M16 ? v_unit_swz<DP, M16>(row, db) * 32 : v_unit_swz<DP, M16>(row, db) * 64 + dg * 32) + (li & 3) * 8;
   }
   const float c = PREMUL ? 1.0f : a.scale_log2e;
 
-  // ---- the work of this workgroup: key tiles [t_lo, t_hi) of a task --------------------------------
+  // ---- the work of this workgroup: key tiles [t_lo, t_hi) of a task, dealt out to its key groups -----
   int task = bid, t_lo = 0, t_hi = n_tiles, share = 0;
   if constexpr (SPLIT) {
     if (!takes_whole) {
@@ -200,134 +237,84 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       t_hi = (int)((int64_t)(share + 1) * n_tiles / a.shares);
     }
   }
+  const int t0 = t_lo + kg;                         // this group's first
+  const int n_steps = (t_hi - t_lo + KG - 1) / KG;  // of the groups: the last one may be without a tile in its last step
   const int qt = task % a.q_tiles;
   const int bh = task / a.q_tiles;
   const int h = bh % a.Hq;
   const int b = bh / a.Hq;
   const int hk = h / a.group;
 
-  // ---- Q^T fragments straight from global memory -----------------------
-  // B operand of K Q^T: lane holds query column col of block qb, head-dim slots MK*ks + 8*grp + 0..7.
-  half8_t qf[QB][KS];
-#pragma unroll
-  for (int qb = 0; qb < QB; qb++) {
-    int64_t qi = (int64_t)qt * QROWS + wave * 32 + qb * MB + col;
-    if (qi >= Sq) qi = Sq - 1;
-    int sg = 0;
-#pragma unroll
-    for (int i = 1; i < kMaxSeg; i++)
-      if (i < a.n_qseg && qi >= a.q[i].start) sg = i;
-    const uint16_t* qp = a.q[sg].ptr + b * a.q[sg].sb + (qi - a.q[sg].start) * a.q[sg].ss + h * a.q[sg].sh;
-    uint4_t qraw[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      const int d0 = ks * MK + grp * 8;
-      qraw[ks] = uint4_t{0, 0, 0, 0};
-      if (d0 < D) qraw[ks] = *reinterpret_cast<const uint4_t*>(qp + d0);
-    }
-    if (a.q_prep) {  // uniform
-      // RMSNorm over the head, then the rotation: the row's D elements sit in the lanes of this column
-      const uint16_t* gam = a.q_gamma[sg];
-      const uint16_t* rrow = a.q_rot ? a.q_rot + qi * D : nullptr;
-      float inv = 1.f;
-      if (a.q_norm) {  // uniform: some segment has a norm weight, and the sum takes every lane
-        float ss = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-          float x[8];
-          unpack_chunk(qraw[ks], x);
-#pragma unroll
-          for (int e = 0; e < 8; e++) ss += x[e] * x[e];
-        }
-        ss = sum_groups<M16>(ss);
-        if (gam) inv = 1.0f / sqrtf(ss / (float)D + a.q_eps);
-      }
-      auto chunk16 = [](const uint16_t* p) __attribute__((always_inline)) {
-        if ((reinterpret_cast<uintptr_t>(p) & 15) == 0) return *reinterpret_cast<const uint4_t*>(p);
-        uint4_t v;
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = (uint32_t)p[2 * q] | ((uint32_t)p[2 * q + 1] << 16);
-        return v;
-      };
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        const int d0 = ks * MK + grp * 8;
-        if (d0 < D) {
-          float x[8];
-          unpack_chunk(qraw[ks], x);
-          const uint4_t g = gam ? chunk16(gam + d0) : uint4_t{0, 0, 0, 0};
-          const uint4_t r = rrow ? chunk16(rrow + d0) : uint4_t{0, 0, 0, 0};
-          qraw[ks] = finish_chunk(x, inv, gam != nullptr, g, rrow != nullptr, r, 1.0f);
-        }
-      }
-    }
-#pragma unroll
-    for (int ks = 0; ks < KS; ks++) qf[qb][ks] = __builtin_bit_cast(half8_t, qraw[ks]);
-  }
-
   // ---- K / V tile loaders ------------------------------------------------
   // ONESEG: K and V are one run of rows each and small enough for 32-bit byte
-  // offsets from a uniform base; a tile step adds a uniform stride.
+  // offsets from a uniform base, which a tile step moves.
   // Otherwise the segment of a tile is looked up once per tile (uniformly): a
   // tile that lies inside one segment is fetched from that segment's base with
   // per-lane 32-bit offsets, a tile that straddles segments row by row.
-  uint32_t k_off[LOADS], v_off[LOADS];
+  uint32_t k_off[OFFS], v_off[OFFS];  // of a thread's rows in a tile (of the first)
   const char* k_base = nullptr;
   const char* v_base = nullptr;
   uint32_t k_step = 0, v_step = 0;
-  const int64_t keys_ahead = Skv - (int64_t)t_lo * BKV;                     // keys from this piece's first tile on
+  const int64_t keys_ahead = Skv - (int64_t)t0 * BKV;                        // keys from this group's first tile on
   int rows_left = (int)(keys_ahead < 0x7fffffff ? keys_ahead : 0x7fffffff);  // ONESEG: keys from the next K tile on
   int rows_left_v = rows_left;
   if constexpr (ONESEG) {
-    k_base = reinterpret_cast<const char*>(a.k[0].ptr + b * a.k[0].sb + hk * a.k[0].sh);
-    v_base = reinterpret_cast<const char*>(a.v[0].ptr + b * a.v[0].sb + hk * a.v[0].sh);
     k_step = (uint32_t)(a.k[0].ss * BKV * 2);
     v_step = (uint32_t)(a.v[0].ss * BKV * 2);
+    k_base = reinterpret_cast<const char*>(a.k[0].ptr + b * a.k[0].sb + hk * a.k[0].sh) + (int64_t)t0 * k_step;
+    v_base = reinterpret_cast<const char*>(a.v[0].ptr + b * a.v[0].sb + hk * a.v[0].sh) + (int64_t)t0 * v_step;
 #pragma unroll
-    for (int i = 0; i < LOADS; i++) {
-      k_off[i] = (uint32_t)((ld_row[i] * a.k[0].ss + k_ch[i] * 8) * 2) + (uint32_t)t_lo * k_step;
-      v_off[i] = (uint32_t)((ld_row[i] * a.v[0].ss + v_ch[i] * 8) * 2) + (uint32_t)t_lo * v_step;
+    for (int i = 0; i < OFFS; i++) {
+      k_off[i] = (uint32_t)((ld_row[i] * a.k[0].ss + k_ch[i] * 8) * 2);
+      v_off[i] = (uint32_t)((ld_row[i] * a.v[0].ss + v_ch[i] * 8) * 2);
     }
   }
-  // General case: a uniform cursor holds the address of the next tile's first row, the step to the tile behind it and
+  // General case: a uniform cursor holds the address of the group's next tile's first row, the step to its tile behind it and
   // the first tile that does not lie wholly inside the segment.  Up to there a tile costs one scalar comparison and one
-  // addition, and its lanes fetch with 32-bit offsets from the cursor; a tile that straddles segments or ends the
-  // sequence goes row by row and moves the cursor to the segment the next tile starts in.
+  // addition, and its lanes fetch with 32-bit offsets from the cursor; from there on the cursor moves to the segment that the tile
+  // starts in, and where that does not hold all of it -- the tile straddles segments or ends the sequence -- it goes row by row.
   struct SegCursor {
     const char* base;
     int64_t step;
+    int rows;       // from a thread's row of a tile to its next
     int inside;  // tiles below this one lie inside the segment
   };
-  auto seek = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[LOADS], const int (&chs)[LOADS], int t)
+  auto seek = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[OFFS], const int (&chs)[LOADS], int t)
                   __attribute__((always_inline)) {
     const int64_t row0 = (int64_t)t * BKV;
     int sg = 0;
 #pragma unroll
     for (int i = 1; i < kMaxSeg; i++)
       if (i < a.n_kvseg && row0 >= segs[i].start) sg = i;
+    sg = __builtin_amdgcn_readfirstlane(sg);  // (comparisons of 64 bits leave uniform values in vector registers)
     const int64_t ss = segs[sg].ss, end = (sg + 1 < a.n_kvseg) ? segs[sg + 1].start : Skv;
-    c.inside = ss > 0 && ss < (1 << 24) ? (int)(end / BKV) : 0;
-    c.step = ss * (BKV * 2);
+    c.inside = __builtin_amdgcn_readfirstlane(ss > 0 && ss < (1 << 24) ? (int)(end / BKV) : 0);
+    c.step = ss * (KG * BKV * 2);
+    c.rows = (int)(ss * (LROWS * 2));  // (where `inside` says that the cursor is used)
     c.base = reinterpret_cast<const char*>(segs[sg].ptr + b * segs[sg].sb + hk * segs[sg].sh + (row0 - segs[sg].start) * ss);
 #pragma unroll
-    for (int i = 0; i < LOADS; i++) off[i] = (uint32_t)((ld_row[i] * ss + chs[i] * 8) * 2);
+    for (int i = 0; i < OFFS; i++) off[i] = (uint32_t)((ld_row[i] * ss + chs[i] * 8) * 2);
   };
-  SegCursor kcur{nullptr, 0, 0}, vcur{nullptr, 0, 0};
-  if constexpr (!ONESEG) {
-    seek(a.k, kcur, k_off, k_ch, t_lo);
-    seek(a.v, vcur, v_off, v_ch, t_lo);
-  }
+  SegCursor kcur{nullptr, 0, 0, 0}, vcur{nullptr, 0, 0, 0};
   // (zero_tail: rows of the tile past the last key get zeros instead of keeping an earlier tile's bytes -- for V,
   // whose stale rows would otherwise meet a probability of exactly zero in the second MFMA: 0 x Inf = NaN)
-  auto zero_slot = [&](unsigned char* dst, int i) __attribute__((always_inline)) {
-    *reinterpret_cast<uint4_t*>(dst + (wave * LOADS + i) * 1024 + lane * 16) = uint4_t{0, 0, 0, 0};
+  // What the paths that few tiles take derive from a thread's place is not to be kept in registers across the loop: they are short
+  // with four waves on a SIMD, and a reload from scratch waits for the transfers in flight.
+  auto opaque = [](int v) __attribute__((always_inline)) {
+    if constexpr (FOUR) asm volatile("" : "+v"(v));
+    return v;
   };
-  auto issue_general = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[LOADS], const int (&chs)[LOADS],
+  auto zero_slot = [&](unsigned char* dst, int i) __attribute__((always_inline)) {
+    *reinterpret_cast<uint4_t*>(dst + slot(i) + opaque(lane) * 16) = uint4_t{0, 0, 0, 0};
+  };
+  auto issue_general = [&](const SdpaSeg* segs, SegCursor& c, uint32_t (&off)[OFFS], const int (&chs)[LOADS],
                            unsigned char* dst, int t, bool zero_tail) __attribute__((always_inline)) {
-    if (t < c.inside) {  // uniform
+    if (t >= c.inside && t < full_tiles) seek(segs, c, off, chs, t);  // uniform
+    if (t < c.inside) {                                               // uniform
+      const int64_t rows = OFFS > 1 ? 0 : __builtin_amdgcn_readfirstlane(c.rows);
 #pragma unroll
       for (int i = 0; i < LOADS; i++)
-        if (chs[i] * 8 < D) load_to_lds_16(c.base, off[i], lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
+        if (chs[i] * 8 < D) load_to_lds_16(c.base + i * rows, off[OFFS > 1 ? i : 0], lds_address(dst) + slot(i));
       c.base += c.step;
       return;
     }
@@ -344,21 +331,26 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
           if (u < a.n_kvseg && kj >= segs[u].start) sl = u;
         const uint16_t* src =
             segs[sl].ptr + b * segs[sl].sb + (kj - segs[sl].start) * segs[sl].ss + hk * segs[sl].sh + chs[i] * 8;
-        load_to_lds_16(src, lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
+        load_to_lds_16(src, lds_address(dst) + slot(i));
       }
     }
-    if (t + 1 < n_tiles) seek(segs, c, off, chs, t + 1);
   };
-  // starts the transfer of the next K (or V) tile and moves on by one tile
+  auto advance = [](const char*& base, uint32_t (&off)[OFFS], uint32_t step) __attribute__((always_inline)) {
+    if constexpr (OFFS == 1) base += (int64_t)KG * step;
+    else {
+#pragma unroll
+      for (int i = 0; i < OFFS; i++) off[i] += step;
+    }
+  };
+  // starts the transfer of the group's next K (or V) tile and moves on to the one behind it
   auto issue_k = [&](unsigned char* dst, [[maybe_unused]] int t) __attribute__((always_inline)) {
     if constexpr (ONESEG) {
 #pragma unroll
-      for (int i = 0; i < LOADS; i++) {
+      for (int i = 0; i < LOADS; i++)
         if (ld_row[i] < rows_left && k_ch[i] * 8 < D)
-          load_to_lds_16(k_base, k_off[i], lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
-        k_off[i] += k_step;
-      }
-      rows_left -= BKV;
+          load_to_lds_16(k_base + (OFFS > 1 ? 0 : (int64_t)i * (k_step / BKV * LROWS)), k_off[OFFS > 1 ? i : 0], lds_address(dst) + slot(i));
+      advance(k_base, k_off, k_step);
+      rows_left -= KG * BKV;
     } else {
       issue_general(a.k, kcur, k_off, k_ch, dst, t, false);
     }
@@ -371,16 +363,88 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
           if (ld_row[i] >= rows_left_v) zero_slot(dst, i);
       }
 #pragma unroll
-      for (int i = 0; i < LOADS; i++) {
+      for (int i = 0; i < LOADS; i++)
         if (ld_row[i] < rows_left_v && v_ch[i] * 8 < D)
-          load_to_lds_16(v_base, v_off[i], lds_address(dst) + (uint32_t)((wave_u * LOADS + i) * 1024));
-        v_off[i] += v_step;
-      }
-      rows_left_v -= BKV;
+          load_to_lds_16(v_base + (OFFS > 1 ? 0 : (int64_t)i * (v_step / BKV * LROWS)), v_off[OFFS > 1 ? i : 0], lds_address(dst) + slot(i));
+      advance(v_base, v_off, v_step);
+      rows_left_v -= KG * BKV;
     } else {
       issue_general(a.v, vcur, v_off, v_ch, dst, t, true);
     }
   };
+  // ---- Q^T fragments straight from global memory -----------------------
+  // B operand of K Q^T: lane holds query column col of block qb, head-dim slots MK*ks + 8*grp + 0..7.  What the norm and the
+  // rotation need is asked for together with the rows (one after the other, behind tests of each chunk's alignment, 24 x 2637 tokens
+  // took 11 us for it).
+  half8_t qf[QB][KS];
+  {
+    uint4_t raw[QB][KS], gam[QB][KS], rot[QB][KS];
+    bool has_gam[QB];
+    const auto chunk = [](const uint16_t* p, bool aligned) __attribute__((always_inline)) {
+      if (aligned) return *reinterpret_cast<const uint4_t*>(p);  // uniform
+      uint4_t v;
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[q] = (uint32_t)p[2 * q] | ((uint32_t)p[2 * q + 1] << 16);
+      return v;
+    };
+#pragma unroll
+    for (int qb = 0; qb < QB; qb++) {
+      int64_t qi = (int64_t)qt * QROWS + qwave * 32 + qb * MB + col;
+      if (qi >= Sq) qi = Sq - 1;
+      // the row's segment, by selection: an index into the arguments that differs from lane to lane goes through memory
+      const uint16_t *ptr = a.q[0].ptr, *gp = a.q_gamma[0];
+      int64_t off = b * a.q[0].sb + h * a.q[0].sh, ss = a.q[0].ss;
+#pragma unroll
+      for (int i = 1; i < kMaxSeg; i++) {
+        const bool in = i < a.n_qseg && qi >= a.q[i].start;
+        ptr = in ? a.q[i].ptr : ptr;
+        off = in ? b * a.q[i].sb + h * a.q[i].sh - a.q[i].start * a.q[i].ss : off;
+        ss = in ? a.q[i].ss : ss;
+        gp = in ? a.q_gamma[i] : gp;
+      }
+      const uint16_t* const qp = ptr + (off + qi * ss);
+      has_gam[qb] = gp != nullptr;
+      if (!gp) gp = qp;  // (anything that can be read)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        const int d0 = ks * MK + grp * 8;
+        raw[qb][ks] = gam[qb][ks] = rot[qb][ks] = uint4_t{0, 0, 0, 0};
+        if (d0 < D) {
+          raw[qb][ks] = *reinterpret_cast<const uint4_t*>(qp + d0);
+          if (a.q_norm) gam[qb][ks] = chunk(gp + d0, a.q_aligned);  // uniform
+          if (a.q_rot) rot[qb][ks] = chunk(a.q_rot + qi * D + d0, a.q_aligned);
+        }
+      }
+    }
+#pragma unroll
+    for (int qb = 0; qb < QB; qb++) {
+      if (a.q_prep) {  // uniform
+        // RMSNorm over the head, then the rotation: the row's D elements sit in the lanes of this column
+        float inv = 1.f;
+        if (a.q_norm) {  // uniform: some segment has a norm weight, and the sum takes every lane
+          float ss = 0.f;
+#pragma unroll
+          for (int ks = 0; ks < KS; ks++) {
+            float x[8];
+            unpack_chunk(raw[qb][ks], x);
+#pragma unroll
+            for (int e = 0; e < 8; e++) ss += x[e] * x[e];
+          }
+          ss = sum_groups<M16>(ss);
+          if (has_gam[qb]) inv = 1.0f / sqrtf(ss / (float)D + a.q_eps);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          float x[8];
+          unpack_chunk(raw[qb][ks], x);
+          raw[qb][ks] = finish_chunk(x, inv, has_gam[qb], gam[qb][ks], a.q_rot != nullptr, rot[qb][ks], 1.0f);
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) qf[qb][ks] = __builtin_bit_cast(half8_t, raw[qb][ks]);
+    }
+  }
+
   // ---- running state -----------------------------------------------------
   sums_t oacc[DB][QB];  // O^T: [block of the head dimension][block of queries]
 #pragma unroll
@@ -414,11 +478,24 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       for (int qb = 0; qb < QB; qb++)
 #pragma unroll
         for (int v = 0; v < NV; v++) sacc[kb][qb][v] = 0.f;
+    if constexpr (FOUR) {  // (the waves hide the reads for each other)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+          sacc[kb][0] = mfma(*reinterpret_cast<const half8_t*>(kt + kb * MB * ROWB + k_rd[ks]), qf[0][ks], sacc[kb][0]);
+        if (ks & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      return;
+    }
     // K fragments are read a group of four ahead of the MFMAs that use them: KB blocks of 4 / KB k-steps
     constexpr int GS = 4 / KB;
     half8_t kf[2][4];
-    // (a k-step that lies wholly in the zero padding of a short head -- the fourth of 16 at D = 40 -- is left out)
-    auto live = [&](int ks) __attribute__((always_inline)) { return M16 || DP != 64 || ks * MK < D; };
+    // (A k-step that lies wholly in the zero padding of a head size is left out.  The test stays where no k-step does, at head size
+    // 64: the loop is 7 % slower without its branches, and at 40, where it is known, 4 % faster -- us, 2 x 10 x 4096 of 64 143 / 154, 2 x
+    // 8 x 4096 of 40 73.4 / 70.6.)
+    auto live = [&](int ks) __attribute__((always_inline)) { return M16 || DL != 64 || ks * MK < D; };
     auto read_k = [&](int buf, int g) __attribute__((always_inline)) {
 #pragma unroll
       for (int u = 0; u < 4; u++) {
@@ -466,8 +543,10 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     }
     // Probabilities against the current reference, and this lane's share of their row sums.  The tile's maximum is
     // not looked for: as long as every lane's sums stay below 2^10 no probability exceeds that (fp16 holds 2^16),
-    // which is all that the reference is there to ensure.
+    // which is all that the reference is there to ensure.  (ONES: the sums are the second MFMA's, and the largest of this lane's
+    // probabilities is looked at; as fp16 bits they order like integers, infinities and NaN last.)
     float psum[QB];
+    [[maybe_unused]] uint32_t pmax = 0;
     auto probabilities = [&]() __attribute__((always_inline)) {
       float mc[QB];
 #pragma unroll
@@ -482,14 +561,24 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
 #pragma unroll
           for (int qb = 0; qb < QB; qb++) {
             const float p = fast_exp2(__builtin_fmaf(sacc[kb][qb][v], c, -mc[qb]));
-            psum[qb] += p;
+            if constexpr (!ONES) psum[qb] += p;
             const int slot = kb * NV + v;  // of this lane's scores: eight to an operand
             pf[slot >> 3][qb][slot & 7] = (half_t)p;
+            if constexpr (FOUR)  // (operand by operand: 128 registers hold no more than one operand's probabilities in fp32)
+              if ((slot & 7) == 7) __builtin_amdgcn_sched_barrier(0);
           }
+      if constexpr (ONES) {
+        pmax = 0;
+#pragma unroll
+        for (int i = 0; i < BKV / PK; i++) {
+          const uint4_t two = __builtin_bit_cast(uint4_t, pf[i][0]);
+          pmax = max3_h2(max3_h2(pmax, two[0], two[1]), two[2], two[3]);
+        }
+      }
     };
     probabilities();
     // (the first tile arrives here with the references at -inf: its sums are inf; a NaN fails the test too)
-    bool outgrown = !(psum[0] <= 1024.0f);
+    bool outgrown = ONES ? (pmax & 0xffff) > 0x6400 || pmax > 0x6400ffff : !(psum[0] <= 1024.0f);
     if constexpr (QB == 2) outgrown = outgrown || !(psum[1] <= 1024.0f);
     if (__builtin_amdgcn_ballot_w64(outgrown) != 0) {
       // some row's scores have outgrown the reference: move every row's reference up to its running maximum,
@@ -517,7 +606,8 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
       probabilities();
     }
 #pragma unroll
-    for (int qb = 0; qb < QB; qb++) l_run[qb] += psum[qb];
+    for (int qb = 0; qb < QB; qb++)
+      if constexpr (!ONES) l_run[qb] += psum[qb];
   };
 
   // O^T += V^T P^T for the V tile in stage st.
@@ -525,6 +615,20 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   auto pv_phase = [&](const unsigned char* vt) __attribute__((always_inline)) {
     typedef __attribute__((address_space(3))) short4_t lds_s4;
     typedef short short8_t __attribute__((ext_vector_type(8)));
+    if constexpr (FOUR) {
+#pragma unroll
+      for (int s = 0; s < BKV / PK; s++) {
+        if (s % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int db = 0; db < DB; db++) {
+          const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + PK * s * ROWB + v_rd[db]));
+          const short4_t h4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(vt + (PK * s + PK / 2) * ROWB + v_rd[db]));
+          oacc[db][0] = mfma(__builtin_bit_cast(half8_t, short8_t{lo[0], lo[1], lo[2], lo[3], h4[0], h4[1], h4[2], h4[3]}), pf[s][0], oacc[db][0]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      return;
+    }
     // V^T fragments (DB blocks per step) go in groups of up to four, the next group read while the current one's MFMAs run
     constexpr int GF = M16 ? 4 : DB, NF = BKV / PK * DB, NG = (NF + GF - 1) / GF;
     short4_t vlo[2][GF], vhi[2][GF];
@@ -558,55 +662,145 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
   };
 
   // ---- pipeline ---------------------------------------------------------------
-  // Interval t (between two barriers) has K tile t and V tile t-1 readable in
-  // LDS while K tile t+1 and V tile t are written.  Every wave runs
-  //   O += V(t-1) P(t-1) ;  S(t) = K(t) Q ;  P(t) = softmax(S(t))
-  // per interval -- two MFMA phases back to back, then one VALU phase.  The two
-  // waves of a SIMD (w and w+4) run that cycle half a period apart: the second
-  // one starts each interval with the softmax of the scores it produced in the
-  // previous interval, so one wave's exponentials overlap the other's MFMAs.
-  const bool second = wave >= 4;
-  issue_k(Ks0, t_lo);
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the tile has landed
+  if (t0 < t_hi) {  // uniform
+    issue_k(Ks0, t0);
+    if constexpr (FOUR) issue_v(Vs0, t0);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the tiles has landed
   __syncthreads();
-
-  // interval t (key tiles t_lo .. t_hi - 1 of the task): K(t) is in k_cur, V(t-1) in v_prev; K(t+1) goes to
-  // k_next, V(t) to v_cur
-  auto interval = [&](int t, const unsigned char* k_cur, unsigned char* k_next, const unsigned char* v_prev,
-                      unsigned char* v_cur) __attribute__((always_inline)) {
-    if (t + 1 < t_hi) issue_k(k_next, t + 1);
-    if (t < t_hi) issue_v(v_cur, t);
-    // the wave doing softmax arithmetic gets issue priority: its exponentials only make progress in
-    // the gaps the other wave's MFMA stream leaves (measured: +1 %; the opposite assignment -2 %)
-    if (!second) {
-      __builtin_amdgcn_s_setprio(0);
-      if (t > t_lo) pv_phase(v_prev);
+  if constexpr (FOUR) {
+    // Step n (between two barriers) has the group's n-th K and V tiles readable in LDS while the next ones are written.  Four
+    // waves share a SIMD, and what one of them waits for -- the MFMA pipe, an exponential, LDS -- the others fill.
+    auto step = [&](int n, unsigned char* k_cur, unsigned char* k_next, unsigned char* v_cur, unsigned char* v_next)
+                    __attribute__((always_inline)) {
+      const int t = t0 + n * KG;
+      if (t + KG < t_hi) {
+        issue_k(k_next, t + KG);
+        issue_v(v_next, t + KG);
+      }
       if (t < t_hi) {
         s_phase(k_cur);
-        __builtin_amdgcn_s_setprio(2);
         softmax_phase(t);
+        pv_phase(v_cur);
       }
-    } else {
-      if (t > t_lo) {
-        __builtin_amdgcn_s_setprio(2);
-        softmax_phase(t - 1);
-        __builtin_amdgcn_s_setprio(0);
-        pv_phase(v_prev);
-      }
-      if (t < t_hi) s_phase(k_cur);
+      __builtin_amdgcn_s_waitcnt(0x0f70);
+      __syncthreads();
+    };
+    for (int n = 0; n < n_steps; n += 2) {
+      step(n, Ks0, Ks1, Vs0, Vs1);
+      if (n + 1 < n_steps) step(n + 1, Ks1, Ks0, Vs1, Vs0);
     }
-    __builtin_amdgcn_s_waitcnt(0x0f70);
-    __syncthreads();
-  };
-  for (int t = t_lo; t <= t_hi; t += 2) {
-    interval(t, Ks0, Ks1, Vs1, Vs0);
-    if (t + 1 <= t_hi) interval(t + 1, Ks1, Ks0, Vs0, Vs1);
+  } else {
+    // Interval n (between two barriers) has K tile n and V tile n-1 of the group readable in
+    // LDS while K tile n+1 and V tile n are written.  Every wave runs
+    //   O += V(n-1) P(n-1) ;  S(n) = K(n) Q ;  P(n) = softmax(S(n))
+    // per interval -- two MFMA phases back to back, then one VALU phase.  The two
+    // waves of a SIMD (w and w+4) run that cycle half a period apart: the second
+    // one starts each interval with the softmax of the scores it produced in the
+    // previous interval, so one wave's exponentials overlap the other's MFMAs.
+    const bool second = wave >= 4;
+    // K(n) is in k_cur, V(n-1) in v_prev; K(n+1) goes to k_next, V(n) to v_cur
+    auto interval = [&](int n, const unsigned char* k_cur, unsigned char* k_next, const unsigned char* v_prev,
+                        unsigned char* v_cur) __attribute__((always_inline)) {
+      const int t = t0 + n * KG;
+      if (t + KG < t_hi) issue_k(k_next, t + KG);
+      if (t < t_hi) issue_v(v_cur, t);
+      // (with scalar loads of the segments' places on their way, which may come out of order, the compiler would wait for all LDS
+      // reads in place of the next one: 3 % of a launch)
+      if constexpr (!ONESEG) __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+      const bool before = n > 0 && t - KG < t_hi;  // there is a tile n - 1
+      // the wave doing softmax arithmetic gets issue priority: its exponentials only make progress in
+      // the gaps the other wave's MFMA stream leaves (measured: +1 %; the opposite assignment -2 %)
+      if (!second) {
+        __builtin_amdgcn_s_setprio(0);
+        if (before) pv_phase(v_prev);
+        if (t < t_hi) {
+          s_phase(k_cur);
+          __builtin_amdgcn_s_setprio(2);
+          softmax_phase(t);
+        }
+      } else {
+        if (before) {
+          __builtin_amdgcn_s_setprio(2);
+          softmax_phase(t - KG);
+          __builtin_amdgcn_s_setprio(0);
+          pv_phase(v_prev);
+        }
+        if (t < t_hi) s_phase(k_cur);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0f70);
+      __syncthreads();
+    };
+    for (int n = 0; n <= n_steps; n += 2) {
+      interval(n, Ks0, Ks1, Vs1, Vs0);
+      if (n + 1 <= n_steps) interval(n + 1, Ks1, Ks0, Vs0, Vs1);
+    }
+    __builtin_amdgcn_s_setprio(0);
   }
-  __builtin_amdgcn_s_setprio(0);
 
   // the row sums, the same in every group of lanes from here on
 #pragma unroll
-  for (int qb = 0; qb < QB; qb++) l_run[qb] = sum_groups<M16>(l_run[qb]);
+  for (int qb = 0; qb < QB; qb++) {
+    if constexpr (ONES) {
+      // row D of O^T, which lane group 0 holds
+      float l = 0.f, other;
+#pragma unroll
+      for (int d = 0; d < DP; d += 8)
+        if (D == d) l = oacc[d / MB][0][d % MB / 2];
+      halves32(l, l_run[qb], other);
+    } else {
+      l_run[qb] = sum_groups<M16>(l_run[qb]);
+    }
+  }
+
+  // Where two hold partial results of the same rows, meet() takes in the other's reference and row sums and says how its sums are
+  // folded: mine a + got b with both products rounded, the same for either order.
+  struct Weights {
+    float a, b;
+    __device__ __forceinline__ float fold(float mine, float got) const {
+      float x = mine * a, y = got * b;
+      asm volatile("" : "+v"(x), "+v"(y));
+      return x + y;
+    }
+  };
+  auto meet = [&](int qb, float m_o, float l_o) __attribute__((always_inline)) {
+    const float m_new = fmaxf(m_ref[qb], m_o);
+    const Weights w{fast_exp2((m_ref[qb] - m_new) * c), fast_exp2((m_o - m_new) * c)};
+    m_ref[qb] = m_new;
+    l_run[qb] = w.fold(l_run[qb], l_o);
+    return w;
+  };
+  constexpr int SUMS = DB * QB * NV;  // of a lane
+  if constexpr (KG == 2) {
+    // the second key group hands its results to the first through the tiles' LDS (the loop ended with a barrier)
+    constexpr int QS = SUMS / 4;  // a quarter of the sums into each array
+    static_assert(SUMS % 4 == 0 && QS * 4 * 64 * QW <= KG * TILE_B, "room");
+    __shared__ float stats[QW][2 * QB][64];
+    float* const quarter[4] = {reinterpret_cast<float*>(Ks0), reinterpret_cast<float*>(Ks1), reinterpret_cast<float*>(Vs0), reinterpret_cast<float*>(Vs1)};
+    const int at = qwave * (QS * 64) + lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int i = 0; i < SUMS; i++) quarter[i / QS][at + i % QS * 64] = oacc[i / (QB * NV)][i / NV % QB][i % NV];
+#pragma unroll
+      for (int qb = 0; qb < QB; qb++) {
+        stats[qwave][2 * qb][lane] = m_ref[qb];
+        stats[qwave][2 * qb + 1][lane] = l_run[qb];
+      }
+    }
+    __syncthreads();
+    if (kg == 0) {
+      Weights w[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; qb++) w[qb] = meet(qb, stats[qwave][2 * qb][lane], stats[qwave][2 * qb + 1][lane]);
+#pragma unroll
+      for (int i = 0; i < SUMS; i++) {
+        sums_t& o = oacc[i / (QB * NV)][i / NV % QB];
+        o[i % NV] = w[i / NV % QB].fold(o[i % NV], quarter[i / QS][at + i % QS * 64]);
+      }
+    } else {
+      return;
+    }
+  }
 
   // ---- normalise and store O ----------------------------------------------
   // Runs of 8 consecutive head-dim elements per lane (16-byte stores) out of its runs of four: 32x32 blocks hold head-dim
@@ -616,7 +810,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
     const bool vec_ok = ((a.o_sb | a.o_ss | a.o_sh) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.o) & 15) == 0;
 #pragma unroll
     for (int qb = 0; qb < QB; qb++) {
-      const int64_t qi = (int64_t)qt * QROWS + wave * 32 + qb * MB + col;
+      const int64_t qi = (int64_t)qt * QROWS + qwave * 32 + qb * MB + col;
       const float inv = 1.0f / l_run[qb];
       uint16_t* op = a.o + b * a.o_sb + (qi < Sq ? qi : 0) * a.o_ss + h * a.o_sh;
       constexpr int RUNS = DB * NV / 4;  // this lane's runs of four
@@ -700,17 +894,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
           const int stats = DP / 2 * 512 - lane + col;
 #pragma unroll
           for (int qb = 0; qb < QB; qb++) {
-            const float m_o = ld(stats + MB * qb), l_o = ld(stats + 32 + MB * qb);
-            const float m_new = fmaxf(m_ref[qb], m_o);
-            const float wa = fast_exp2((m_ref[qb] - m_new) * c), wb = fast_exp2((m_o - m_new) * c);
-            // a wa + b wb with both products rounded: the same for either order
-            auto fold = [&](float mine, float got) __attribute__((always_inline)) {
-              float x = mine * wa, y = got * wb;
-              asm volatile("" : "+v"(x), "+v"(y));
-              return x + y;
-            };
-            m_ref[qb] = m_new;
-            l_run[qb] = fold(l_run[qb], l_o);
+            const Weights w = meet(qb, ld(stats + MB * qb), ld(stats + 32 + MB * qb));
             constexpr int AT = 16 / NV;  // blocks whose sums are asked for together
 #pragma unroll
             for (int d0 = 0; d0 < DB; d0 += AT) {
@@ -724,7 +908,7 @@ __global__ void __launch_bounds__(512) sdpa_kernel(const SdpaArgs a) {
               for (int u = 0; u < AT; u++)
                 if (d0 + u < DB)
 #pragma unroll
-                  for (int v = 0; v < NV; v++) oacc[d0 + u][qb][v] = fold(oacc[d0 + u][qb][v], got[u][v]);
+                  for (int v = 0; v < NV; v++) oacc[d0 + u][qb][v] = w.fold(oacc[d0 + u][qb][v], got[u][v]);
             }
           }
           __syncthreads();  // s_seen may be written again
@@ -769,7 +953,7 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
   const char* knob = getenv("DT_SDPA_KEY_SPLIT");
   const bool never = knob && knob[0] == 'n', always = knob && knob[0] == 'a';
   if (never) return false;
-  const int64_t tasks = (int64_t)B * Hq * ((Sq + QROWS - 1) / QROWS);
+  const int64_t tasks = (int64_t)B * Hq * ((Sq + query_rows(1) - 1) / query_rows(1));
   const int64_t n_tiles = (Skv + BKV - 1) / BKV;
   if (tasks > (1 << 20) || tasks * n_tiles >= (1LL << 31)) return false;  // (the kernel counts units in 32 bits)
   const int cus = compute_units();
@@ -812,46 +996,97 @@ bool sdpa_split_plan(int32_t B, int32_t Hq, int32_t D, int64_t Sq, int64_t Skv, 
   return true;
 }
 
-template <int DP, int DL, bool M16>
+static bool sdpa_premul(const SdpaArgs& a) { return !(a.scale_log2e > 0.f && a.scale_log2e < 1e30f); }
+// one K and one V segment whose rows lie within 2 GiB of the head's first row: 32-bit offsets
+static bool sdpa_oneseg(const SdpaArgs& a) {
+  return a.n_kvseg == 1 && a.k[0].ss > 0 && a.v[0].ss > 0 && a.Skv < (1 << 30) && (a.Skv + 2 * BKV) * a.k[0].ss * 2 < 0x7fffffffLL &&
+         (a.Skv + 2 * BKV) * a.v[0].ss * 2 < 0x7fffffffLL;
+}
+
+template <int DP, int DL, bool M16, int KG>
 static dt_status launch(hipStream_t s, SdpaArgs a) {
   a.q_norm = 0;
-  for (int i = 0; i < a.n_qseg; i++) a.q_norm |= a.q_gamma[i] != nullptr;
-  a.q_tiles = (int)((a.Sq + QROWS - 1) / QROWS);
+  a.q_aligned = (reinterpret_cast<uintptr_t>(a.q_rot) & 15) == 0;
+  for (int i = 0; i < a.n_qseg; i++) {
+    a.q_norm |= a.q_gamma[i] != nullptr;
+    a.q_aligned &= (reinterpret_cast<uintptr_t>(a.q_gamma[i]) & 15) == 0;
+  }
+  a.q_tiles = (int)((a.Sq + query_rows(KG) - 1) / query_rows(KG));
   int64_t total = (int64_t)a.q_tiles * a.Hq * a.B;
   if (total > 0x7fffffff) return DT_NO_KERNEL;
   a.total_blocks = (int)total;
-  const bool premul = !(a.scale_log2e > 0.f && a.scale_log2e < 1e30f);
-  // one K and one V segment whose rows lie within 2 GiB of the head's first row: 32-bit offsets
-  const bool oneseg = a.n_kvseg == 1 && a.k[0].ss > 0 && a.v[0].ss > 0 && a.Skv < (1 << 30) &&
-                      (a.Skv + 2 * BKV) * a.k[0].ss * 2 < 0x7fffffffLL && (a.Skv + 2 * BKV) * a.v[0].ss * 2 < 0x7fffffffLL;
+  const bool premul = sdpa_premul(a), oneseg = sdpa_oneseg(a);
   dim3 block(512);
-  if (a.partials) {
-    // key-split launch: the counters start at zero
-    if (!a.counters_zeroed) {
-      const int n = a.cut_tasks * kSdpaSplitNodes;
-      hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
-      if (const dt_status st = launch_status(); st != DT_OK) return st;
-    }
-    a.total_blocks = a.cut_tasks * a.shares;  // (of the cut tasks)
-    dim3 grid((unsigned)(a.whole_tasks + a.total_blocks));
-    if (oneseg) {
-      if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, true, true>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, true, true>), grid, block, 0, s, a);
-    } else {
-      if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, false, true>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, false, true>), grid, block, 0, s, a);
-    }
-    return launch_status();
-  }
   dim3 grid((unsigned)total);
-  if (oneseg) {
-    if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, true, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, true, false>), grid, block, 0, s, a);
-  } else {
-    if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, false, false>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, false, false>), grid, block, 0, s, a);
+  if constexpr (KG == 1) {
+    if (a.partials) {
+      // key-split launch: the counters start at zero
+      if (!a.counters_zeroed) {
+        const int n = a.cut_tasks * kSdpaSplitNodes;
+        hipLaunchKernelGGL(sdpa_zero_counters_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.counters, n);
+        if (const dt_status st = launch_status(); st != DT_OK) return st;
+      }
+      a.total_blocks = a.cut_tasks * a.shares;  // (of the cut tasks)
+      grid = dim3((unsigned)(a.whole_tasks + a.total_blocks));
+      if (oneseg) {
+        if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, true, true, 1>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, true, true, 1>), grid, block, 0, s, a);
+      } else {
+        if (premul) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, false, true, 1>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, false, true, 1>), grid, block, 0, s, a);
+      }
+      return launch_status();
+    }
+    if (premul) {
+      if (oneseg) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, true, false, 1>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, true, false, false, 1>), grid, block, 0, s, a);
+      return launch_status();
+    }
   }
+  if (oneseg) hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, true, false, KG>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((sdpa_kernel<DP, DL, M16, false, false, false, KG>), grid, block, 0, s, a);
   return launch_status();
+}
+
+// Estimated time (us) of a launch: `launch` once, and for every round of workgroups `round` and its steps, each of a key tile a
+// key group, which take `few` where few compute units are at work and `all` where all of them are.  Fits to 1000 launches of 256 ..
+// 5000 queries and 64 .. 5000 keys in two segments, 4 .. 24 heads, on the whole card: half of them within 4 %, nineteen of twenty within 12 %.
+// (Keys in one segment are 3 .. 10 % faster in either form; which form is taken does not depend on it, since results may not.)
+struct SdpaRate {
+  double few, all, round, launch;
+  double rounds(int64_t workgroups, int64_t steps, int cus) const {
+    const int64_t full = workgroups / cus, rest = workgroups % cus;
+    return (double)full * ((double)steps * all + round) + (rest ? (double)steps * (few + (all - few) * (double)rest / cus) + round : 0.0);
+  }
+};
+// head sizes up to 48, 64, 80, 128
+constexpr SdpaRate kOneGroup[4] = {{1.027, 1.087, 4.95, 1.946}, {1.02, 1.135, 6.472, 1.362}, {1.372, 1.511, 7.612, 1.745}, {1.326, 1.718, 9.237, 1.29}};
+constexpr SdpaRate kTwoGroups[4] = {{1.217, 1.244, 5.799, 2.19}, {1.279, 1.273, 6.058, 2.126}, {1.78, 1.844, 8.872, 1.35}, {1.662, 2.053, 9.644, 2.347}};
+
+// Whether a launch runs with two key groups to a workgroup.  Its tasks then are half as large, which fills the compute units where there
+// are few of them and wastes less of a last round: us, one group / two, head size 128, 12 x 1050 x 1050 30.8 / 23.8, 10 x 2472 x 2472 63.9 /
+// 43.8, 24 x 2637 x 2637 (in place of a cut last round) 109 / 93, 20 x 3160 x 545 43.3 / 36.4; 40 and 64, 4 x 1582 x 1582 26.7 / 20.1, 24 x 2637
+// x 2637 74 / 58.  But every key tile is fetched for half as many queries, and rounds of full-length tasks are slower: 40 x 8000 x 8000 1077 /
+// 1236, 24 x 4608 x 4608 232 / 290.  Taken where the estimate gains 3 %: 0.87 .. 0.92 of the time, by head size and segments, of 2000 random launches,
+// the worst of which takes 1.03.
+static bool sdpa_two_groups(const SdpaArgs& a) {
+  const char* knob = getenv("DT_SDPA_KEY_SPLIT");  // "groups": wherever it can be; "never" and "always" (sdpa_split_plan): no
+  if (knob && (knob[0] == 'n' || knob[0] == 'a' || knob[0] == 'g')) return knob[0] == 'g';
+  // a launch that was to be cut and got no workspace for it keeps the whole tasks that such calls have always had
+  if (!a.partials && sdpa_split_plan(a.B, a.Hq, a.D, a.Sq, a.Skv, nullptr)) return false;
+  const int size = a.D <= 48 ? 0 : a.D <= 64 ? 1 : a.D <= 80 ? 2 : 3;
+  const SdpaRate &one = kOneGroup[size], &two = kTwoGroups[size];
+  const int cus = compute_units();
+  const int64_t heads = (int64_t)a.B * a.Hq, n_tiles = (a.Skv + BKV - 1) / BKV;
+  const auto tasks = [&](int kg) { return heads * ((a.Sq + query_rows(kg) - 1) / query_rows(kg)); };
+  double t1 = one.launch;
+  if (a.partials) {  // (a cut costs another 16 us, 10 at head sizes up to 64)
+    const int64_t parts = (int64_t)a.cut_tasks * a.shares;
+    t1 += one.rounds(a.whole_tasks, n_tiles, cus) + one.rounds(parts, (n_tiles + a.shares - 1) / a.shares, cus) + (a.D <= 64 ? 10.0 : 16.0);
+  } else {
+    t1 += one.rounds(tasks(1), n_tiles, cus);
+  }
+  return two.launch + two.rounds(tasks(2), (n_tiles + 1) / 2, cus) < 0.97 * t1;
 }
 
 dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
@@ -867,13 +1102,23 @@ dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
   // tiles on it takes 1.00 .. 0.97, behind whole rounds 0.97 (means of 1400 launches of head sizes 88 .. 128; us, 12 heads of 128, 323 x
   // 1928 34.2 / 35.9, 4 heads, 4096 x 4096 60.3 / 58.0, 264 tasks 111 / 109).
   // Head sizes up to 80 multiply 80 columns in this form only, which decides for it wherever the launch is cut (0.83 .. 0.98).
-  if (a.D <= 64) return launch<64, 64, false>(s, a);
-  const int64_t tasks = (a.Sq + QROWS - 1) / QROWS * a.Hq * a.B;
+  // (a scale that is folded into the scores first has one key group)
+  if (!sdpa_premul(a) && sdpa_two_groups(a)) {
+    SdpaArgs u = a;
+    u.partials = nullptr;  // uncut, whatever the workspace
+    if (a.D <= 48) return launch<64, 48, false, 2>(s, u);
+    if (a.D <= 64) return launch<64, 64, false, 2>(s, u);
+    if (a.D <= 80) return launch<128, 80, true, 2>(s, u);
+    return launch<128, 128, false, 2>(s, u);  // (16x16x32 is 0 .. 7 % slower here, in launches of one round and of many)
+  }
+  if (a.D <= 48) return launch<64, 48, false, 1>(s, a);
+  if (a.D <= 64) return launch<64, 64, false, 1>(s, a);
+  const int64_t tasks = (a.Sq + query_rows(1) - 1) / query_rows(1) * a.Hq * a.B;
   const int64_t cus = compute_units();
   const auto short_parts = [&] { return (int64_t)a.cut_tasks * a.shares * 10 < cus * 8 || (a.Skv + BKV - 1) / BKV < 16 * a.shares; };
-  if (a.partials ? a.D > 80 && a.whole_tasks == 0 && short_parts() : tasks * 10 < cus * 7) return launch<128, 128, false>(s, a);
-  if (a.D <= 80) return launch<128, 80, true>(s, a);
-  return launch<128, 128, true>(s, a);
+  if (a.partials ? a.D > 80 && a.whole_tasks == 0 && short_parts() : tasks * 10 < cus * 7) return launch<128, 128, false, 1>(s, a);
+  if (a.D <= 80) return launch<128, 80, true, 1>(s, a);
+  return launch<128, 128, true, 1>(s, a);
 }
 
 }  // namespace dt

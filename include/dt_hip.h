@@ -341,7 +341,9 @@ dt_status dt_qk_norm_rope_f16(dt_stream stream, dt_view4 x, int32_t B, int64_t S
  *             nothing, such a launch runs unsplit: same results to within one
  *             rounding of the fp16 output, lower occupancy.
  *             Environment: DT_SDPA_KEY_SPLIT=never|always overrides the
- *             estimate (read at every call; for tests and measurements).
+ *             estimate (read at every call; for tests and measurements), and
+ *             so does "groups": a task's keys shared out over the waves of
+ *             one workgroup, which takes no workspace.
  * D in {40, 64, 128} (any D <= 128 that is a multiple of 8).
  * Inputs are expected to be finite.  A key whose V row holds Inf or NaN makes the output rows of its (batch, head)
  * non-finite, as in the reference (probability x Inf, and 0 x Inf = NaN where the probability underflows); it

@@ -998,3 +998,67 @@ def test_sdpa_key_split_replays_as_hip_graph(dthip, oracle, torch_cuda, monkeypa
         assert torch.equal(out, want)
         call()  # eager work between the replays
         torch.cuda.synchronize()
+
+
+# ------------------------------------------------------------------ K3, two key groups to a workgroup
+
+@pytest.mark.parametrize("B,Sq,Skv,Hq,Hk,D,cut", [
+    (1, 127, 64, 2, 2, 40, 0),     # one key tile: the second group has none
+    (1, 129, 1, 2, 2, 48, 0),      # one key
+    (2, 128, 65, 2, 1, 64, 0),     # a second tile of one key; grouped heads
+    (1, 1, 192, 3, 3, 40, 0),      # three tiles: the groups take two and one
+    (1, 300, 1000, 2, 2, 40, 77),  # keys in two segments, which straddle a tile; row sums out of the matrix instruction
+    (1, 260, 520, 2, 2, 56, 64),   # ... which begin with a tile; row sums added up
+    (2, 140, 700, 3, 3, 72, 333),
+    (1, 257, 450, 2, 2, 80, 0),
+    (1, 150, 330, 2, 2, 96, 130),
+    (1, 513, 777, 2, 2, 128, 0),
+    (1, 300, 1300, 2, 1, 128, 333),
+])
+@pytest.mark.parametrize("masked", [False, True])
+def test_sdpa_two_key_groups(dthip, oracle, torch_cuda, monkeypatch, B, Sq, Skv, Hq, Hk, D, cut, masked):
+    """Workgroups whose waves share out a task's key tiles in two groups: against the oracle, and within a rounding of one group.
+    masked: all keys but the first tile's are hidden through the dot product, which leaves the second group nothing that counts."""
+    torch = torch_cuda
+    rng = np.random.default_rng(Sq * 7 + Skv + D)
+    q, k, v = rand_qkv(rng, B, Sq, Skv, Hq, Hk, D)
+    scale = 1 / np.sqrt(D)
+    live = slice(0, Skv)
+    if masked:
+        live = slice(0, min(Skv, 64))
+        q[..., 0], k[..., 0] = 1, -np.inf
+        k[:, live, :, 0] = 0
+    want = oracle.C.sdpa(q, np.ascontiguousarray(k[:, live]), np.ascontiguousarray(v[:, live]), scale)
+    parts = lambda t: [to_dev(torch, np.ascontiguousarray(t[:, a:b])) for a, b in ([(0, Skv)] if not cut else [(0, cut), (cut, Skv)])]
+    args = ([to_dev(torch, q)], parts(k), parts(v), scale)
+    print("sdpa two key groups", B, Sq, Skv, Hq, Hk, D, cut, masked, flush=True)
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "groups")
+    got = dthip.sdpa_segments(*args)
+    whole = dthip.sdpa_segments([args[0][0]], [to_dev(torch, k)], [to_dev(torch, v)], scale)
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", "never")
+    one = dthip.sdpa_segments(*args)
+    mx, rr = oracle.err_stats(got.cpu().numpy(), want)
+    assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+    assert torch.equal(got, whole)  # however the keys are stored
+    assert float((got.float() - one.float()).abs().max()) <= 2e-3
+
+
+def test_sdpa_two_key_groups_with_prepared_queries(dthip, oracle, torch_cuda, monkeypatch):
+    """Norm weights and a rotation table that lie off 16 bytes, one segment without a norm weight: the same bits as aligned ones."""
+    torch = torch_cuda
+    rng = np.random.default_rng(77)
+    T, S, H, D = 70, 400, 2, 128
+    q, k, v = rand_qkv(rng, 1, S, S, H, H, D)
+    gam, rot = f16(1 + 0.05 * rng.standard_normal(D)), f16(dthip.WanRotaryPositionEmbedding(1, S, 1, channels=D))
+    off = lambda a: torch.cat([torch.zeros(1, dtype=torch.float16, device="cuda"), to_dev(torch, a).flatten()])[1:].view(a.shape)
+    seg = lambda t: [to_dev(torch, np.ascontiguousarray(t[:, :T])), to_dev(torch, np.ascontiguousarray(t[:, T:]))]
+    call = lambda place: dthip.sdpa_segments(seg(q), seg(k), seg(v), 1 / np.sqrt(D), gamma_q=[place(gam), None], rot_q=place(rot))
+    pq = np.concatenate([oracle.C.rmsnorm(q[0, :T], gam, 1e-6), q[0, T:]], axis=0)
+    want = oracle.C.sdpa(oracle.C.cmul(pq, rot)[None], k, v, 1 / np.sqrt(D))
+    for mode in ("never", "groups"):
+        monkeypatch.setenv("DT_SDPA_KEY_SPLIT", mode)
+        print("sdpa prepared queries", mode, flush=True)
+        got = call(lambda a: to_dev(torch, a))
+        assert torch.equal(got, call(off))
+        mx, rr = oracle.err_stats(got.cpu().numpy(), want)
+        assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
