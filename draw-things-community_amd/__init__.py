@@ -170,6 +170,27 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def _host():
+    """The operators' native way to the library (csrc/dt_host.cpp), or None where the library stands alone: everything it does
+    is done here as well, in more of the host's time."""
+    global _native
+    if _native is None:
+        _native = False
+        lib(), _torch()  # (whose libraries it is linked against)
+        path = os.path.join(_HERE, "_dthost.so")
+        if os.path.exists(path):
+            import importlib.util
+
+            spec = importlib.util.spec_from_file_location("_dthost", path)
+            _native = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(_native)
+            _native.classes(QxTensor, HeadEpilogue, DensePost)
+    return _native or None
+
+
 def _check(fn: str, status: int):
     if status != DT_OK:
         raise DtError(fn, status)
@@ -463,6 +484,13 @@ def _enqueue_dense(problems, flags, stream):
     """Enqueues Dense problems -- (x, weights, biases, outs, epilogues, posts) each -- together, with the scratch memory
     that lets the library look palettized weights up ahead of the launch where X has many rows, and cut tiles along K where
     there are too few of them for the chip.  Returns their outputs."""
+    host = _native or _host()
+    if host is not None:
+        got = host.dense(problems, flags, _scratch)
+        if type(got) is list:
+            return got
+        if got is not None:
+            _check(*(("dt_dense_qx_grouped_scratch_f16", got + 1000) if got < -500 else ("dt_dense_qx_grouped_ws_f16", got)))
     packed = [_marshal_dense(*p) for p in problems]
     groups = b"".join(g for _, g, _, _ in packed)  # (what they point to lives in `packed` until the call returns)
     n, L = len(packed), lib()
@@ -491,6 +519,8 @@ def dense_multi(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object
                 stream=None, epilogues: Optional[Sequence[Optional[HeadEpilogue]]] = None):
     """Several Dense ops that share the input, one launch (x_q / x_k / x_v).  `epilogues[i]` (optional) fuses the
     per-head RMSNorm / RoPE that follows projection i."""
+    if stream is None:
+        return _enqueue_dense([(x, weights, biases, outs, epilogues, None)], flags, None)[0]
     with _on(stream):
         return _enqueue_dense([(x, weights, biases, outs, epilogues, None)], flags, stream)[0]
 
@@ -571,6 +601,8 @@ def dense_post(x, weights: Sequence[QxTensor], biases: Sequence[Optional[object]
     """Dense ops sharing `x`, each followed by its DensePost tail inside the GEMM epilogue (the feed-forward's
     linear1 -> GELU and the gated residual additions of a transformer block).  Returns the fp16 outputs (None where
     a projection only accumulates into its residual)."""
+    if stream is None:
+        return _enqueue_dense([(x, weights, biases, outs, None, posts)], flags, None)[0]
     with _on(stream):
         return _enqueue_dense([(x, weights, biases, outs, None, posts)], flags, stream)[0]
 
@@ -866,6 +898,13 @@ def layernorm_modulate(x, scale=None, shift=None, epsilon: float = 1e-6, out=Non
 def layernorm16(x, weight=None, bias=None, epsilon: float = 1e-5, out=None, stream=None):
     """LayerNorm(epsilon:, axis: [last]) with fp16 affine `weight` / `bias` [C] on an fp16 tensor [..., C], fp16 out
     (the norms of a UNet transformer block, Models/UNet.swift:530, 544, 554)."""
+    host = _native or _host()
+    if host is not None and out is None:
+        got = host.layernorm16(x, weight, bias, epsilon)
+        if type(got) is int:
+            _check("dt_layernorm_f16", got)
+        if got is not None:
+            return got
     torch = _torch()
     _f16_cuda(x, "x")
     C = x.shape[-1]
@@ -957,6 +996,13 @@ def sdpa_segments(q_segs, k_segs, v_segs, scale, gamma_q=None, gamma_k=None, rot
     static_scratch: stage through the library's fixed per-GPU array (dt_sdpa_f16_static) instead of a workspace
     allocated here; with `out` given the call then allocates nothing.  Requests beyond STATIC_SCRATCH_BYTES raise
     DtError(DT_OOM); calls that may overlap on one GPU must not both use it."""
+    host = _native or _host()
+    if host is not None and not static_scratch and Wo is None and bo is None:
+        got = host.sdpa(q_segs, k_segs, v_segs, scale, gamma_q or None, gamma_k or None, rot_q, rot_k, eps, out, _scratch)
+        if type(got) is int:
+            _check("dt_sdpa_f16", got)
+        if got is not None:
+            return got
     torch = _torch()
     L = lib()
     for t in list(q_segs) + list(k_segs) + list(v_segs):
