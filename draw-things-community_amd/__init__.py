@@ -46,6 +46,8 @@ ABI_SYMBOLS = (
     "dt_sdpa_workspace_bytes",
     "dt_sdpa_f16_static",
     "dt_lora_branch_f32_f16",
+    "dt_lora_dense_scratch_bytes",
+    "dt_lora_dense_f16",
 )
 
 STATIC_SCRATCH_BYTES = 64 << 20  # DT_SDPA_STATIC_SCRATCH_BYTES
@@ -85,7 +87,12 @@ class _DenseGroup(ctypes.Structure):
                 ("post", ctypes.c_void_p)]
 
 
-# The same four as struct formats: a launch's arrays are packed in one go (a ctypes structure costs a microsecond each,
+class _LoraPair(ctypes.Structure):
+    _fields_ = [("down", ctypes.c_void_p), ("up", ctypes.c_void_p), ("ld_up", ctypes.c_int64), ("rank", ctypes.c_int32),
+                ("f32", ctypes.c_int32), ("scale", ctypes.c_float)]
+
+
+# The first four as struct formats: a launch's arrays are packed in one go (a ctypes structure costs a microsecond each,
 # which for a conditioning row's six projections is more than the kernel takes).
 _FMT_WEIGHT, _FMT_EPI, _FMT_POST, _FMT_GROUP = "Qiiq", "QQqfi", "i4xQQqf4xQqQQq", "qqQqQi4xQQQQQ"
 for _fmt, _cls in ((_FMT_WEIGHT, _QxWeight), (_FMT_EPI, _HeadEpilogue), (_FMT_POST, _DensePost), (_FMT_GROUP, _DenseGroup)):
@@ -164,6 +171,12 @@ def lib():
         L.dt_sdpa_f16_static.argtypes = L.dt_sdpa_f16.argtypes[:-2]
         L.dt_lora_branch_f32_f16.restype = i32
         L.dt_lora_branch_f32_f16.argtypes = [vp, i64, i64, vp, i64, vp, i32, vp, i64, f32, vp, vp, i64]
+        pair = [ctypes.POINTER(_DensePost), ctypes.POINTER(_LoraPair)]
+        L.dt_lora_dense_scratch_bytes.restype = ctypes.c_size_t
+        L.dt_lora_dense_scratch_bytes.argtypes = [i64, i64, vp, i64, ctypes.POINTER(_QxWeight), vp, i64, *pair]
+        L.dt_lora_dense_f16.restype = i32
+        L.dt_lora_dense_f16.argtypes = [vp, i64, i64, vp, i64, ctypes.POINTER(_QxWeight), vp, vp, i64, *pair, ctypes.c_uint32, vp,
+                                        ctypes.c_size_t]
         L.dt_sdpa_workspace_bytes.restype = ctypes.c_size_t
         L.dt_sdpa_workspace_bytes.argtypes = [i32, i32, i32, i32, i64, i64, i32, i32]
         _lib = L
@@ -646,12 +659,13 @@ class LoRANetworkConfiguration:
 class LoRADense:
     """LoRADense(count:configuration:noBias:flags:name:) -- dense(x) + up(scale * down(x)) with the palettized base
     left packed and the fp16 low-rank pair applied beside it (Models/LoRA.swift:85-142; running the LoRA separately
-    is the preferred mode for quantized models, Models/UNetProtocol.swift:696-697).  The Dense kernel on the base and
-    the down projection (with the scale in its epilogue), in one call or side by side, then on the up projection, whose
-    epilogue adds the base projection's result; every intermediate is rounded to fp16 as the reference's separate ops round.  With
+    is the preferred mode for quantized models, Models/UNetProtocol.swift:696-697).  dt_lora_dense_f16: the down
+    projection, then the Dense kernel on the base, whose epilogue multiplies with `up` and adds the branch.  What that does not take (few
+    rows, widths off the tiled kernels' grid, palettized pairs) goes out as Dense calls: base and down projection (with the
+    scale in its epilogue), in one call or side by side, then the up projection, whose epilogue adds the base projection's
+    result.  Every intermediate is rounded to fp16 as the reference's separate ops round, either way.  With
     `highPrecision` the pair is fp32 (`down.data` / `up.data` float32 tensors): the branch is computed as
-    fp16(up(scale * down(float(x)))) in fp32 throughout (Models/LoRA.swift:117-139) by dt_lora_branch_f32_f16 and added
-    in the base projection's epilogue."""
+    fp16(up(scale * down(float(x)))) in fp32 throughout (Models/LoRA.swift:117-139)."""
 
     def __init__(self, count: int, configuration: LoRANetworkConfiguration, noBias: bool = False, flags: int = 0,
                  name: str = ""):
@@ -713,6 +727,32 @@ class LoRADense:
         # nothing is copied where the call has no use for more than the workspace that cutting takes
         return lib().dt_dense_scratch_bytes(1, group) == lib().dt_dense_workspace_bytes(1, group)
 
+    def _fused(self, x, b, post, stream):
+        """The layer through dt_lora_dense_f16 as a list of its output, or None where it runs as Dense calls (us, those / this: 4608 x 3072
+        -> 3072 q6p, rank 16, 103 / 94; 300 x 1280 -> 1280 q8p 48 / 22, most of which is the host)."""
+        host = _native or _host()
+        if host is None or not isinstance(x, _torch().Tensor) or x.dim() < 1 or x.numel() <= _ROWS_MAX * x.shape[-1]:
+            return None
+        dn, up = (self.down, self.up) if self.configuration.highPrecision else self._padded()
+        K, rank = x.shape[-1], self.configuration.rank
+        if dn.shape[1] != K or dn.qbits not in (16, 32) or up.qbits not in (16, 32):
+            return None
+        if not self.configuration.highPrecision:
+            if dn.data.dtype != _torch().float16:
+                return None
+            rank = (rank + 15) // 16 * 16  # (of the padded pair's 64, 128, ...)
+        elif dn.data.dtype != _torch().float32:
+            return None
+        problem = (x, [self.weight], [b], None, None, None if post is None else [post])
+        if stream is None:
+            got = host.lora(problem, dn.data, up.data, rank, up.shape[1], self.configuration.scale, self.flags, _scratch)
+        else:
+            with _on(stream):
+                got = host.lora(problem, dn.data, up.data, rank, up.shape[1], self.configuration.scale, self.flags, _scratch)
+        if got is not None and type(got) is not list:
+            _check("dt_lora_dense_f16", got)
+        return got
+
     def __call__(self, x, post: Optional[DensePost] = None, stream=None):
         if self.weight is None:
             raise RuntimeError(f"LoRADense {self.name!r}: weight not loaded")
@@ -728,6 +768,9 @@ class LoRADense:
         p = post or DensePost()
         if p.scale != 1.0 or p.addend is not None or p.multiplicand is not None:
             raise ValueError(f"LoRADense {self.name!r}: the tail may carry an activation, a gate and a residual only")
+        got = self._fused(x, b, post, stream)
+        if got is not None:
+            return got[0]
         if self.configuration.highPrecision:
             return self._high_precision(x, b, p, stream)
         dn, up = self._padded()

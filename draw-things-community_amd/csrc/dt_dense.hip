@@ -24,6 +24,7 @@
 #include "dt_dense_launch.h"
 #include "dt_dense_rows.h"
 #include "dt_depalettize.h"
+#include "dt_lora.h"
 
 namespace dt {
 
@@ -36,7 +37,7 @@ extern template dt_status launch_dense_q<16>(hipStream_t, const DenseArgs&, int,
 
 // the kernel with the elementwise tail only when some weight of the launch asks for one
 static dt_status launch_dense(hipStream_t s, const DenseArgs& a, int tile, int qbits, int mode) {
-  bool post = false;
+  bool post = a.lora.up != nullptr;
   for (int i = 0; i < kMaxWeights; i++) post = post || a.w[i].act != DT_ACT_NONE || a.w[i].gate || a.w[i].res || a.w[i].add || a.w[i].mul || a.w[i].scale != 1.0f;
   switch (qbits) {
     case 4: return launch_dense_q<4>(s, a, tile, post, mode);
@@ -217,6 +218,7 @@ static void finish_args(DenseArgs& a, int n_groups, int n_w, int64_t K, const dt
   for (int j = n_w; j < kMaxWeights; j++) a.w[j] = a.w[0];
   for (int j = n_groups; j < kMaxGroups; j++) a.g[j] = a.g[0];
   a.n_groups = n_groups;
+  a.lora = DenseLora{};
   a.k = (int32_t)K;
   a.nib = w0.qbits == 16 ? 32 : w0.nib;
   a.pal_step = (int32_t)pal_step(K, a.nib);
@@ -512,9 +514,9 @@ __global__ void dense_zero_counters_kernel(int32_t* counters, int n) {
   if (i < n) counters[i] = 0;
 }
 
-// qx: the launch's n_w weights.
+// qx: the launch's n_w weights.  down: a LoRA layer's down projection to go out ahead of it, or null.
 static dt_status launch_plan(hipStream_t s, DenseArgs& a, int n_w, const TilePlan& plan, const Workspace& ws,
-                             const dt_qx_weight* const* qx) {
+                             const dt_qx_weight* const* qx, const LoraDownArgs* down = nullptr) {
   a.whole_tiles = (int32_t)plan.whole;
   a.split = plan.split;
   a.partials = nullptr;
@@ -532,23 +534,28 @@ static dt_status launch_plan(hipStream_t s, DenseArgs& a, int n_w, const TilePla
     d.n_counters = n_counters;
     uint8_t* out = ws.ptr;
     int64_t tiles = 0;
+    const int granules = down ? kLoraCopyGranules : 256;  // of a tile
     for (int i = 0; i < n_w; i++) {
       if (qx[i]->qbits == 16) continue;
       qbits = qx[i]->qbits;
       d.nib = qx[i]->nib;
       d.w[d.n++] = {a.w[i].data, reinterpret_cast<uint16_t*>(out), qx[i]->count / 32, (int32_t)tiles};
       a.w[i].data = out;
-      tiles += (qx[i]->count / 32 + 255) / 256;
+      tiles += (qx[i]->count / 32 + granules - 1) / granules;
       out += ((size_t)qx[i]->count * 2 + 255) & ~(size_t)255;
     }
     for (int i = n_w; i < kMaxWeights; i++) a.w[i] = a.w[0];
-    if (const dt_status st = depalettize_many_launch(s, qbits, d, (int)tiles); st != DT_OK) return st;
+    if (const dt_status st = down ? lora_down_copies_launch(s, *down, qbits, d, (int)tiles) : depalettize_many_launch(s, qbits, d, (int)tiles);
+        st != DT_OK)
+      return st;
     qbits = 16;
     mode = kPlainF16;
     a.nib = 32;
     a.pal_step = 1;
   } else {
     mode = choose_pal_mode(qbits, a.nib, a.k, plan.BM, plan.BN, plan.tiles);
+    if (down)
+      if (const dt_status st = lora_down_launch(s, *down); st != DT_OK) return st;
     if (plan.split > 1) {
       hipLaunchKernelGGL(dense_zero_counters_kernel, dim3((unsigned)((n_counters + 255) / 256)), dim3(256), 0, s, a.counters, n_counters);
       if (const dt_status st = launch_status(); st != DT_OK) return st;
@@ -666,6 +673,63 @@ static dt_status run_group(hipStream_t s, const HostGroup& h, const Workspace& w
       }
   }
   return DT_OK;
+}
+
+// ---- a LoRA layer -------------------------------------------------------------------------------------------------
+// The intermediate of the low-rank branch, ahead of everything else in scratch.
+static size_t lora_t_bytes(int64_t M, const dt_lora_pair& p) { return ((size_t)M * p.rank * (p.f32 ? 4 : 2) + 255) & ~(size_t)255; }
+
+// Whether the layer is one launch of a tiled kernel with the branch in its epilogue, behind its down projection.  (Few rows, and what is
+// off the tiled kernels' alignment, run as Dense calls of their own; so do fp16 pairs of ranks that are no multiple of 16.)
+// In fp16 the down projection of many ranks over many inputs reads more than a compute unit's L1 can deliver, where the tiled kernel shares
+// it in LDS, and the Dense calls run it beside the base projection.  us, Dense calls / here, the calls bound by the host below 50:
+//   rank 16: 4608 x 3072 -> 3072 103 / 96, 1376 x 3072 -> 3072 57 / 52, 512 x 3072 -> 3072 51 / 38, 300 x 1280 -> 1280 48 / 22, 4096 x 320 ->
+//   320 47 / 17, 100 x 5120 -> 1280 51 / 53; rank 64: 2016 x 1280 -> 1280 47 / 31, 512 x 3072 -> 3072 50 / 42, and the other way round 2500 x
+//   1024 -> 4096 56 / 67, 1376 x 3072 -> 3072 57 / 64; rank 128: 2016 x 1280 -> 1280 47 / 40, 512 x 3072 -> 3072 50 / 51.
+// In fp32, rank 32: 4608 x 3072 -> 3072 124 / 115, 512 x 3072 -> 3072 55 / 43, 300 x 1280 -> 1280 53 / 26; rank 128: 198 / 185, 68 / 55, 53 / 38, and the
+// other way round 2500 x 1024 -> 4096 106 / 114, which is all output.
+static bool lora_fusable(const HostGroup& h, const dt_lora_pair& p) {
+  if (h.M <= 0 || !h.x_ok() || !h.w_tiled(0)) return false;
+  if (dense_rows_features(h.M, h.K, h.W[0].qbits, h.W[0].nib, h.W[0].count / h.K) > 0) return false;
+  if (p.f32) return h.M <= 0x3fffffff && p.rank <= 4096 && !(p.rank > 64 && h.K < 2048 && h.M * (h.W[0].count / h.K) > 6000000);
+  if (p.rank > 32 && (double)h.M * (double)h.W[0].count * p.rank > 5e11) return false;
+  if (h.M < 512 && h.K > 4096) return false;
+  return p.rank % 16 == 0 && p.rank <= 128 && p.ld_up % 4 == 0 && (reinterpret_cast<uintptr_t>(p.down) & 15) == 0 &&
+         (reinterpret_cast<uintptr_t>(p.up) & 7) == 0;
+}
+
+static dt_status validate_lora(const HostGroup& h, const dt_lora_pair* p) {
+  if (const dt_status st = validate_group(h); st != DT_OK) return st;
+  if (!p || !p->down || !p->up || p->rank <= 0 || p->ld_up < p->rank || (p->f32 != 0 && p->f32 != 1)) return DT_INVALID;
+  if (!(p->scale == p->scale) || p->scale - p->scale != 0.f) return DT_INVALID;
+  const uintptr_t odd = p->f32 ? 3 : 1;
+  if ((reinterpret_cast<uintptr_t>(p->down) & odd) || (reinterpret_cast<uintptr_t>(p->up) & odd)) return DT_INVALID;
+  if (h.post && (h.post->addend || h.post->multiplicand || post_scale(h, 0) != 1.0f)) return DT_INVALID;
+  return DT_OK;
+}
+
+static dt_status run_lora(hipStream_t s, const HostGroup& h, const dt_lora_pair& p, uint8_t* scratch, size_t bytes) {
+  const size_t t_bytes = lora_t_bytes(h.M, p);
+  const Workspace ws{scratch + t_bytes, bytes - t_bytes, true};
+  double cost;
+  const TilePlan plan = plan_tiles(&h, 1, 0, 1, false, ws.bytes, true, &cost);
+  DenseArgs a;
+  DenseGroup& g = a.g[0];
+  g.x = h.X;
+  g.ldx = h.ldx;
+  g.m = (int32_t)h.M;
+  g.tiles_m = (int)((h.M + plan.BM - 1) / plan.BM);
+  g.tile_begin = 0;
+  g.w_begin = 0;
+  g.w_end = 1;
+  g.tiles_n = add_weight(a, 0, h, 0, 0, plan.BN, false);
+  if ((int64_t)g.tiles_m * g.tiles_n > 0x7fffffff) return DT_NO_KERNEL;
+  a.total_tiles = g.tiles_m * g.tiles_n;
+  finish_args(a, 1, 1, h.K, h.W[0]);
+  a.lora = DenseLora{scratch, p.up, p.rank, p.ld_up, p.rank, p.f32};
+  const LoraDownArgs down{h.X, h.ldx, h.M, h.K, p.down, p.rank, p.f32, p.scale, scratch};
+  const dt_qx_weight* const qx[1] = {h.W};
+  return launch_plan(s, a, 1, plan, ws, qx, &down);
 }
 
 // All problems in one launch, when every X and weight meets the tiled kernel's alignment, they share K and the weight
@@ -872,4 +936,28 @@ DT_EXPORT dt_status dt_dense_qx_grouped_scratch_f16(dt_stream stream, int32_t n_
   if (reinterpret_cast<uintptr_t>(scratch) & 255) return DT_INVALID;
   return dt::run_groups(stream, n_groups, groups,
                         dt::Workspace{static_cast<uint8_t*>(scratch), scratch ? scratch_bytes : 0, true});
+}
+
+DT_EXPORT size_t dt_lora_dense_scratch_bytes(int64_t M, int64_t K, const uint16_t* X, int64_t ldx, const dt_qx_weight* W, uint16_t* Y,
+                                             int64_t ldy, const dt_dense_post* post, const dt_lora_pair* pair) {
+  using namespace dt;
+  const HostGroup h{M, K, X, ldx, W, 1, nullptr, &Y, &ldy, nullptr, post};
+  if (validate_lora(h, pair) != DT_OK || !lora_fusable(h, *pair)) return 0;
+  double cost;
+  return lora_t_bytes(M, *pair) + plan_tiles(&h, 1, 0, 1, false, scratch_limit(true), true, &cost).bytes();
+}
+
+DT_EXPORT dt_status dt_lora_dense_f16(dt_stream stream, int64_t M, int64_t K, const uint16_t* X, int64_t ldx, const dt_qx_weight* W,
+                                      const uint16_t* bias, uint16_t* Y, int64_t ldy, const dt_dense_post* post, const dt_lora_pair* pair,
+                                      uint32_t flags, void* scratch, size_t scratch_bytes) {
+  using namespace dt;
+  (void)flags;
+  const HostGroup h{M, K, X, ldx, W, 1, &bias, &Y, &ldy, nullptr, post};
+  if (const dt_status st = validate_lora(h, pair); st != DT_OK) return st;
+  if (M == 0) return DT_OK;
+  if (!lora_fusable(h, *pair)) return DT_NO_KERNEL;
+  if (reinterpret_cast<uintptr_t>(scratch) & 255) return DT_INVALID;
+  if (!scratch || scratch_bytes < lora_t_bytes(M, *pair)) return DT_OOM;
+  if (const dt_status ready = device_ready(); ready != DT_OK) return ready;
+  return run_lora(as_stream(stream), h, *pair, static_cast<uint8_t*>(scratch), scratch_bytes);
 }

@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(512, 2) dense_f16_kernel(const DenseArgs a) {
 
   __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);  // nothing is in flight into LDS any more
   __syncthreads();
-  dense_epilogue<64, 32, POST>(acc, smem, wave, lane, n0 + wn * 64, (int64_t)m0 + wm * 32, w, g.m);
+  dense_epilogue<64, 32, POST>(acc, smem, wave, lane, n0 + wn * 64, (int64_t)m0 + wm * 32, w, g.m, a.lora);
 }
 
 }  // namespace dt

@@ -41,77 +41,24 @@ __global__ void __launch_bounds__(256) depalettize32_kernel(const uint8_t* __res
   }
 }
 
-// The same granule-per-thread unpacking for blocks of 512 elements and more, with both sides of the lookup moved
-// into LDS: the palettes of the (at most 8192 / nib + 2) blocks that a workgroup's 256 granules touch are loaded once,
-// and the 64 bytes a thread produces go through a [thread][4 chunks] staging array, so that every store
-// instruction of a wave writes 1 KB of consecutive addresses (thread-per-granule stores are 64 bytes apart per lane).
-// Chunk c of thread t is staged at chunk 4 t + (c ^ (t / 4 % 4)): 16 consecutive lanes hit 16 different 16-byte
-// bank groups on the way in (stride of 4 chunks) and on the way out (consecutive chunks).
-// A thread's indices are asked for ahead of the palettes, so that the two memory latencies are one.
-// tile: which 256 granules of the tensor.
-template <int Q>
-__device__ __forceinline__ void depalettize_tile(const uint8_t* __restrict__ packed, int nib, int64_t n_granules,
-                                                 int64_t tile, uint16_t* __restrict__ out) {
-  constexpr int MAXP = 8192 / kDepalMinNib + 2;
-  __shared__ uint16_t pal[MAXP << Q];
-  __shared__ __attribute__((aligned(16))) uint4_t stage[256 * 4];
-  const int t = threadIdx.x;
-  const int64_t g0 = tile * 256;
-  const QxLayout l = make_layout(Q, nib);
-  const int64_t g_last = (g0 + 255 < n_granules ? g0 + 255 : n_granules - 1);
-  const int64_t b_first = g0 * 32 / nib, b_last = (g_last * 32 + 31) / nib;
-  const int n_pal = (int)(b_last - b_first + 1);
-  const int64_t g = g0 + t < n_granules ? g0 + t : g_last;
-  const int64_t b = b_first + (uint32_t)(g * 32 - b_first * nib) / (uint32_t)nib;  // (the difference is below 8192 + nib)
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(packed + index_byte_offset(l, b, g * 32 - b * nib));
-  uint32_t raw[Q];
-#pragma unroll
-  for (int i = 0; i < Q; i++) raw[i] = src[i];
-  for (int i = t; i < n_pal << (Q - 1); i += 256) {
-    const int p = i >> (Q - 1), e = i & ((1 << (Q - 1)) - 1);
-    reinterpret_cast<uint32_t*>(pal)[i] =
-        reinterpret_cast<const uint32_t*>(packed + palette_offset(l, b_first + p))[e];
-  }
-  __syncthreads();
-  {
-    uint32_t idx[32];
-    unpack32<Q>(raw, idx);
-    const uint16_t* mine = pal + ((int)(b - b_first) << Q);
-    uint32_t o[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) o[j] = (uint32_t)mine[idx[2 * j]] | ((uint32_t)mine[idx[2 * j + 1]] << 16);
-#pragma unroll
-    for (int c = 0; c < 4; c++)
-      stage[4 * t + (c ^ ((t >> 2) & 3))] = uint4_t{o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]};
-  }
-  __syncthreads();
-  // chunk L of the workgroup's 16 KB (L = 4 * thread + c) leaves through lane L % 256 of trip L / 256
-  uint4_t* dst = reinterpret_cast<uint4_t*>(out + g0 * 32);
-  const int64_t n_chunks = (g_last - g0 + 1) * 4;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int L = j * 256 + t;
-    const int src_t = L >> 2, c = L & 3;
-    if (L < n_chunks) dst[L] = stage[4 * src_t + (c ^ ((src_t >> 2) & 3))];
-  }
-}
-
 template <int Q>
 __global__ void __launch_bounds__(256) depalettize_tile_kernel(const uint8_t* __restrict__ packed, int nib,
                                                              int64_t n_granules, uint16_t* __restrict__ out) {
-  depalettize_tile<Q>(packed, nib, n_granules, blockIdx.x, out);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[depalettize_lds(Q, 256)];
+  depalettize_tile<Q, 256>(packed, nib, n_granules, blockIdx.x, out, smem);
 }
 
 // Several weights at once, and the counters of the launch behind it zeroed on the way.
 template <int Q>
 __global__ void __launch_bounds__(256) depalettize_many_kernel(const DepalettizeMany a) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[depalettize_lds(Q, 256)];
   if (blockIdx.x == 0)
     for (int i = threadIdx.x; i < a.n_counters; i += 256) a.counters[i] = 0;
   int wi = 0;
 #pragma unroll
   for (int i = 1; i < kDepalMax; i++)
     if (i < a.n && (int)blockIdx.x >= a.w[i].tile_begin) wi = i;
-  depalettize_tile<Q>(a.w[wi].packed, a.nib, a.w[wi].n_granules, (int)blockIdx.x - a.w[wi].tile_begin, a.w[wi].out);
+  depalettize_tile<Q, 256>(a.w[wi].packed, a.nib, a.w[wi].n_granules, (int)blockIdx.x - a.w[wi].tile_begin, a.w[wi].out, smem);
 }
 
 dt_status depalettize_many_launch(hipStream_t s, int qbits, const DepalettizeMany& a, int tiles) {

@@ -320,6 +320,41 @@ PyObject* dense(Py_ssize_t n_args, PyObject* const* args) {
   return all;
 }
 
+// lora(problem, down, up, rank, ld_up, scale, flags, scratch): a list of the output of the problem's only weight with the low-rank branch
+// added, or a status that is not DT_OK as an int, or None.  down, up: both fp16, or both fp32, contiguous.
+PyObject* lora(Py_ssize_t n_args, PyObject* const* args) {
+  if (n_args != 8) throw Fallback{};
+  const at::Tensor &down = tensor(args[1]), &up = tensor(args[2]);
+  const bool f32 = down.scalar_type() == at::kFloat;
+  for (const at::Tensor* t : {&down, &up})
+    if (!t->is_cuda() || !t->is_contiguous() || t->scalar_type() != (f32 ? at::kFloat : at::kHalf)) throw Fallback{};
+  Problem p;
+  read_problem(args[0], p);
+  if (p.w.size() != 1 || !p.epi.empty()) throw Fallback{};
+  const dt_lora_pair pair{ptr<const void>(down), ptr<const void>(up), as_int(args[4]), as_int32(args[3]), f32 ? 1 : 0, as_float(args[5])};
+  // (the ones that the library may read: `rank` rows of each half, in up's case columns)
+  if (pair.rank <= 0 || down.numel() < pair.rank * p.K || up.numel() < p.ldy[0] * pair.ld_up || p.w[0].count != p.ldy[0] * p.K) throw Fallback{};
+  const uint32_t flags = (uint32_t)as_int32(args[6]);
+  const uint16_t* const x = ptr<const uint16_t>(*p.x);
+  const int64_t ldx = p.x->dim() == 2 && p.M > 1 ? p.x->stride(0) : p.K;
+  const dt_dense_post* const post = p.post.empty() ? nullptr : p.post.data();
+  const size_t need = dt_lora_dense_scratch_bytes(p.M, p.K, x, ldx, p.w.data(), p.y[0], p.ldy[0], post, &pair);
+  if (need == 0) throw Fallback{};
+  Scratch scratch;  // (on a device too full for copies of the weights: the intermediate alone)
+  scratch.ask(args[7], PyTuple_GET_ITEM(args[0], 0), need, ((size_t)p.M * pair.rank * (f32 ? 4 : 2) + 255) & ~(size_t)255);
+  const dt_stream stream = current_stream();
+  dt_status st;
+  Py_BEGIN_ALLOW_THREADS;
+  st = dt_lora_dense_f16(stream, p.M, p.K, x, ldx, p.w.data(), p.bias[0], p.y[0], p.ldy[0], post, &pair, flags, scratch.at, scratch.bytes);
+  Py_END_ALLOW_THREADS;
+  if (st != DT_OK) return PyLong_FromLong((long)st);
+  PyObject* const out = p.outs[0].defined() ? THPVariable_Wrap(std::move(p.outs[0])) : Py_NewRef(Py_None);
+  PyObject* const all = out ? PyList_New(1) : nullptr;
+  if (!all) Py_XDECREF(out);
+  else PyList_SET_ITEM(all, 0, out);
+  return all;
+}
+
 dt_view4 view4(const at::Tensor& t) {
   if (t.dim() != 4 || t.stride(3) != 1) throw Fallback{};
   return dt_view4{t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
@@ -420,6 +455,7 @@ PyObject* classes(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 PyMethodDef methods[] = {{"classes", (PyCFunction)(void*)classes, METH_FASTCALL, nullptr},
                          {"dense", (PyCFunction)(void*)guarded<dense>, METH_FASTCALL, nullptr},
+                         {"lora", (PyCFunction)(void*)guarded<lora>, METH_FASTCALL, nullptr},
                          {"sdpa", (PyCFunction)(void*)guarded<sdpa>, METH_FASTCALL, nullptr},
                          {"layernorm16", (PyCFunction)(void*)guarded<layernorm16>, METH_FASTCALL, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
