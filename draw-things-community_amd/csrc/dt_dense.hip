@@ -231,6 +231,7 @@ struct TilePlan {
   int64_t tiles = 0;
   int64_t whole = 0;  // tiles that stay whole; the rest is cut into `split` shares each
   int split = 1;
+  bool act = false;  // some weight's tail has an activation
   size_t expand_bytes = 0;  // > 0: the weights are written out as fp16 in front of the launch, to this much scratch
   // workspace of the split tiles: their counters, then their slots
   size_t counter_bytes() const { return split > 1 ? ((size_t)(tiles - whole) * kSplitNodes * 4 + 255) & ~(size_t)255 : 0; }
@@ -270,12 +271,16 @@ static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t 
   const auto k_tile = [&](double busy) -> double {
     switch (p.tile) {
       case kTile256x256: return plain ? 0.37 + 0.44 * busy : (wide ? 0.71 + 0.47 * busy : 0.73 + 0.27 * busy) + entering;
+      case kTile192x256: return 0.30 + 0.30 * busy;
       case kTile128x256: return plain ? 0.28 + 0.14 * busy : wide ? 0.85 + 0.10 * busy : (row ? 0.60 : 0.78) + 0.17 * busy + entering;
       case kTile128x128: return plain ? 0.145 + 0.09 * busy : row ? 0.49 + 0.06 * busy + entering : wide ? 0.575 + 0.065 * busy : 0.56 + 0.09 * busy;
     }
     return 0.51 + 0.195 * busy + entering;
   };
-  const double outside = p.tile == kTile256x256 ? 11.3 : p.tile == kTile128x128 ? 7.7 : 7.1;
+  double outside = p.tile == kTile256x256 ? 11.3 : p.tile == kTile192x256 ? 12.3 : p.tile == kTile128x128 ? 7.7 : 7.1;
+  // an activation's arithmetic (us, none / GELU, plain weights: one round of 256 x 256 tiles 33.4 / 42.4 and 48.6 / 56.7, of 192 x 256 45.9 / 51.2
+  // and 94.4 / 97.6; 2.5 rounds of 128 x 256 33.8 / 45.9, of two 128 x 128 a compute unit 26.9 / 34.8)
+  if (p.act) outside += p.tile == kTile256x256 ? 9.0 : p.tile == kTile192x256 ? 5.0 : p.tile == kTile128x128 ? 3.3 : 4.5;
   const bool pairs_of_tiles = p.tile == kTile128x128 && !(row && wide);
   // `n` workgroups of `kt` K-tiles each
   const auto time = [&](int64_t n, int kt) -> double {
@@ -333,8 +338,10 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
     p.BM = BM;
     p.BN = BN;
     for (int gi = 0; gi < n; gi++)
-      for (int j = w_begin; j < (n > 1 ? hs[gi].n_weights : w_end); j++)
+      for (int j = w_begin; j < (n > 1 ? hs[gi].n_weights : w_end); j++) {
+        p.act = p.act || (hs[gi].post && hs[gi].post[j].activation != DT_ACT_NONE);
         p.tiles += ((hs[gi].M + BM - 1) / BM) * ((hs[gi].W[j].count / K + BN - 1) / BN);
+      }
     p.whole = p.tiles;
     return p;
   };
@@ -358,7 +365,24 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
   TilePlan base = big ? (m_max < 1024 ? tnarrow : t256) : (!pal_fits_big && tall_ok && m_max >= 1024 && n_max >= 128 && t256.tiles * 2 >= kFillTiles) ? ttall : tsmall;
   const auto pal_mode = [&](const TilePlan& p) { return choose_pal_mode(w0.qbits, w0.qbits == 16 ? 32 : w0.nib, K, p.BM, p.BN, p.tiles); };
   const int64_t step = pal_step(K, w0.qbits == 16 ? 32 : w0.nib);
-  const double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step, expanded);
+  double start = plan_cost(base, w0.qbits, pal_mode(base), nk, step, expanded);
+  // Plain weights: tiles of 192 tokens where the rounds of the others come out badly filled, and under an activation, which big tiles do with
+  // nothing beside it on the compute unit, small ones, whose estimate is high.  The sums are the same on every tile.  us, without
+  // / with these, of 130 launches of random sizes the slowest by 3 % and half of them faster by 3 % and more: 1 x (2304 x 2048 -> 5120) fp16 57.2 / 45.9
+  // (240 tiles, 720 of 128 x 128), 3394 x 4544 -> 3200 q8p 115.8 / 97.2, 4108 x 2048 -> 2816 q8p 64.9 / 53.3, 2 x (576 x 2368 -> 10368) q6p 128.9 /
+  // 77.0, with GELU 2016 x 1280 -> 5120 fp16 44.2 / 38.2, 2 x (4531 x 448 -> 5888) q6p 121.1 / 102.7, 3 x (5454 x 320 -> 960) q8p 54.2 / 39.1; left as
+  // they were: 3500 x 1280 -> 3840 fp16 36.6 on 210 tiles of 256 x 256, 54.6 on 285, 1376 x 3072 -> 12288 134 on 288, 117 cut, 112 on 384.
+  if (w0.qbits == 16 && !brief) {
+    const auto instead = [&](const TilePlan& p, double factor) {
+      const double t = factor * plan_cost(p, 16, kPlainF16, nk, step, expanded);
+      if (t < 0.95 * start) {
+        start = t;
+        base = p;
+      }
+    };
+    if (m_max > 128 && n_max >= 256) instead(shape(kTile192x256, 192, 256), 1.0);
+    if (base.act && !wide && base.tile != kTile128x128) instead(tsmall, 1.0 / 1.15);
+  }
   *cost = start;
   // Without workspace the rules above stand.  With it, another shape or a cut is taken where the estimate sees a
   // clear gain.

@@ -626,7 +626,7 @@ __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 
   constexpr int NST = 3;                         // ring depth of the unpacked weight tiles
   constexpr int B_STAGE = BN * BK;
   constexpr int PROW = 2 * BK;                   // halfs per row of a pair slot
-  static_assert(BM % 128 == 0 && BN % 128 == 0 && BN <= 256, "tile");
+  static_assert((BM % 128 == 0 || (BM == 192 && MODE == kPlainF16)) && BN % 128 == 0 && BN <= 256, "tile");
   static_assert(NS == 2 || (MODE == kPlainF16 && NS > 2 && (NS - 1) * (AP + BP) < 16), "pair slots");
 
   // One LDS array, carved up by hand so that the epilogue can reuse all of it.  The palettes come first:

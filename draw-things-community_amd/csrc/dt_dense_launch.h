@@ -7,8 +7,9 @@ namespace dt {
 
 // Tile shapes the host side chooses between.
 // (tokens x features; 256 x 128 exists for the palettes that only fit beside a 128-feature tile -- per-row tables of
-// 128 and 256 entries -- and is instantiated for those index widths only)
-enum DenseTile : int { kTile128x128 = 0, kTile128x256 = 1, kTile256x256 = 2, kTile256x128 = 3 };
+// 128 and 256 entries -- and is instantiated for those index widths only; 192 x 256 for plain fp16 weights, where its rounds of
+// workgroups come out fuller)
+enum DenseTile : int { kTile128x128 = 0, kTile128x256 = 1, kTile256x256 = 2, kTile256x128 = 3, kTile192x256 = 4 };
 
 template <int Q, int BM, int BN, bool POST, bool SPLIT>
 static dt_status launch_tiled(hipStream_t s, const DenseArgs& a, int mode) {
@@ -60,6 +61,9 @@ static dt_status launch_dense_qp(hipStream_t s, const DenseArgs& a, int tile, in
       } else {
         return DT_NO_KERNEL;  // the host side picks this tile for 7- and 8-bit indices only
       }
+    case kTile192x256:
+      if constexpr (Q == 16) return a.partials ? DT_NO_KERNEL : launch_tiled<Q, 192, 256, POST, false>(s, a, mode);  // (never cut)
+      else return DT_NO_KERNEL;
     default:
       return a.partials ? launch_tiled<Q, 256, 256, POST, true>(s, a, mode) : launch_tiled<Q, 256, 256, POST, false>(s, a, mode);
   }

@@ -1,0 +1,45 @@
+"""GPU: tiles of 192 tokens, which plain fp16 weights and fp16 copies take where they fill the chip better than others.  Every tile sums
+over K in the same order, so a launch that is not cut has to give the bits of the same rows in calls of few enough of them to run on other tiles."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+# (rows and features at the ends of tiles and off them; sizes at which the estimates take the tile)
+@pytest.mark.parametrize("M,N,K,q", [(3174, 3590, 512, 16), (3265, 3584, 512, 16), (2304, 5120, 2048, 16), (2305, 5121, 1984, 16), (4108, 2816, 2048, 8),
+                                     (1900, 5504, 2176, 6)])
+def test_tiles_of_192_tokens(dthip, oracle, monkeypatch, M, N, K, q):
+    import torch
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    rng = np.random.default_rng(M + N)
+    if q == 16:
+        w = dthip.QxTensor.from_f16((rng.standard_normal((N, K)) * 0.05).astype(np.float16))
+    else:
+        w = dthip.QxTensor.from_packed(oracle.synth_qx_weight(rng, N, K, q, 4096, 0.05)[0], q, 4096, (N, K))
+    wf = w.dequantize() if q != 16 else w.data.view(N, K)
+    dev = lambda a: torch.from_numpy(a.astype(np.float16)).cuda()
+    x, b, gate = dev(rng.standard_normal((M, K))), dev(rng.standard_normal(N) * 0.1), dev(1 + 0.3 * rng.standard_normal(N))
+    res = torch.from_numpy(rng.standard_normal((M, N)).astype(np.float32)).cuda()
+    print("dense 192", M, N, K, q, flush=True)
+    monkeypatch.setenv("DT_DENSE_SPLIT", "never")  # (what is cut along K adds its shares up otherwise)
+    ends = [M * i // (M // 100) for i in range(M // 100 + 1)]  # 100 .. 110 rows each: more than the kernel for few rows takes
+    parts = list(zip(ends, ends[1:]))
+    plain = dthip.dense_multi(x, [w], [b])[0]
+    want = torch.cat([dthip.dense_multi(x[i:j], [dthip.QxTensor(wf, 16, 0, (N, K))], [b])[0] for i, j in parts])
+    assert torch.equal(plain, want)
+    exact = x[:64].double() @ wf.double().T + b.double()
+    assert float((plain[:64].double() - exact).abs().max()) <= 2.0 ** -10 * float(exact.abs().max())
+    r, rw = res.clone(), res.clone()
+    got = dthip.dense_post(x, [w], [b], [dthip.DensePost(dthip.ACT_GELU_TANH, gate=gate, residual=r)])[0]
+    want = torch.cat([dthip.dense_post(x[i:j], [dthip.QxTensor(wf, 16, 0, (N, K))], [b],
+                                       [dthip.DensePost(dthip.ACT_GELU_TANH, gate=gate, residual=rw[i:j])])[0] for i, j in parts])
+    assert torch.equal(got, want) and torch.equal(r, rw)
+    if N % 128 == 0:  # norm and rotation fused
+        gamma, rot = dev(1 + 0.1 * rng.standard_normal(128)), dev(rng.standard_normal((M + 3, 128)))
+        epi = lambda p: dthip.HeadEpilogue(gamma, rot, p, 1e-6, 128)
+        got = dthip.dense_multi(x, [w], [b], epilogues=[epi(3)])[0]
+        want = torch.cat([dthip.dense_multi(x[i:j], [dthip.QxTensor(wf, 16, 0, (N, K))], [b], epilogues=[epi(3 + i)])[0] for i, j in parts])
+        assert torch.equal(got, want)
