@@ -396,14 +396,12 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
     return p.split > 1 && p.bytes() <= std::min(ws_bytes, kDenseMaxWorkspace) ? p : base;
   }
   TilePlan best = base;
-  // A clear gain: 5 %, and 8 us for launches of up to 30, since a cut's second launch and its workspace cost the host 7
-  // beside the 17 of the call, which chains of short launches wait for (a UNet block of 702 tokens, 320 wide, whose
-  // feed-forward would gain 6 of 32 us, took 228 us a pass with it and 220 without).
+  // A clear gain: 5 %, and 4 us for launches of up to 30, where the second launch and the workspace of a cut cost the host some of it.
   double least = 0.95 * start;
   const auto consider = [&](const TilePlan& shape) {
     double t;
     const TilePlan p = best_split(shape, w0.qbits, pal_mode(shape), nk, step, expanded, ws_bytes, &t);
-    if (t < least && (t > 30.0 || t < start - 8.0)) {
+    if (t < least && (t > 30.0 || t < start - 4.0)) {
       least = *cost = t;
       best = p;
     }
@@ -458,9 +456,10 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
 // The tiled kernel on palettized weights looks every weight up once per tile of rows, at a cost that no schedule hides: 0.6
 // against 0.2 us a K-tile on 128 x 128 tiles, however few the rows.  us, packed / copied: 4608 x 3072 -> 3 x 3072 q6p 284 /
 // 227, 1376 x 3072 -> 12288 q8p 158 / 131, 512 x 3072 -> 3072 q8p 47 / 26; and the other way round 188 x 3840 -> 3 x 8192 q6p
-// 84 / 112, 579 x 256 -> 5376 q6p 9.8 / 12.1.  The gain has to be 5 %, and 6 us since the second launch costs the host as much
-// (a UNet block of short launches, which wait for the host, took 251 us a pass without copies and 279 with one for every
-// launch that the GPU alone would gain by).
+// 84 / 112, 579 x 256 -> 5376 q6p 9.8 / 12.1.  The gain has to be 5 % and 6 us, or 7 % and 2 us of the
+// second launch on the host (512 x 5120 -> 2 x 5120 q5p, 105 MB of copies, gains less than 6).  (us, 6 and 8 for a cut / 2 and 4: UNet blocks 43 x 19 tokens, 640 wide, q8p 198 / 181, 50 x 50 q6p 236 / 222, LoRA
+// layers 464 x 704 -> 3008 q8p 34 / 27, 407 x 512 -> 1280 q4p 20.0 / 15.6, 6 x (995 x 256 -> 1344) q8p 22.4 / 20.8; 60 calls of random sizes 0.966 of
+// the time, none over 1.01.  Before the calls were made natively, second launches cost more of the host than they gained.)
 static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, bool expand, double* cost) {
   const dt_qx_weight& w0 = hs[0].W[w_begin];
   const TilePlan packed = plan_format(hs, n, w_begin, w_end, wide, std::min(ws, kDenseMaxWorkspace), w0, false, cost);
@@ -470,7 +469,7 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   TilePlan plain;
   double copied;
   if (!expand || w0.qbits == 16 || !plan_copies(hs, n, w_begin, w_end, wide, ws, &plain, &copied)) return packed;
-  if (!expand_knob('a') && !(copied < 0.95 * *cost && copied < *cost - 6.0)) return packed;
+  if (!expand_knob('a') && !(copied < 0.95 * *cost && copied < *cost - (copied < 0.93 * *cost ? 2.0 : 6.0))) return packed;
   *cost = copied;
   return plain;
 }
