@@ -2,10 +2,11 @@
 // no multiple of 32, rows or weights off the 16-byte grid -- on the matrix instruction all the same.
 //
 // What bounds it: the launches are small (odd widths come with small layers), so it is latency: of the index and X
-// loads, hidden by fetching a K-tile ahead into registers, and of the K loop, kept short by giving the four waves of a
-// small tile a quarter of every K-tile each (their sums meet in LDS).  231 x 1000 -> 1001 q8p: 12.6 us (8.0 with plain
-// fp16 weights), where one thread per output, walking K on its own, took 1105.  (Fetching two to four K-tiles ahead changes
-// nothing: 13.0 - 13.2 us; what is left is the unpacking of a tile's indices, one wave to a SIMD.)
+// loads, hidden by fetching a K-tile ahead into registers, of the unpacking of a tile's indices, and of the K loop, kept short by
+// giving the four waves of a small tile a quarter of every K-tile each and, where compute units have a workgroup to themselves, by
+// groups of four waves that take every second or fourth K-tile (their sums meet in LDS).  231 x 1000 -> 1001 q8p: 8.6 us (13.3 with one
+// group, 10.1 with two; 6.8 / 8.6 / 7.4 with plain fp16 weights), where one thread per output, walking K on its own, took 1105.
+// (One group that fetches two to four K-tiles ahead changes nothing: 13.0 - 13.2 us.)
 #include "dt_dense_any.h"
 
 #include "dt_dense_kernel.h"
@@ -42,20 +43,23 @@ __device__ __forceinline__ void load_halfs16(const uint16_t* p, int left, uint32
 // BT x BT outputs per 256-thread workgroup (BT = 64: 2 x 2 waves of 32 x 32; BT = 32: every wave computes the whole
 // tile over its own quarter of each K-tile).  A K-tile is 4096 / BT wide, so that a thread always stages 16 consecutive
 // k of one X row and of one weight row.
-template <int Q, int BT>
-__global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
+// G groups of 256 threads take every G-th K-tile each, and their sums meet in LDS.
+template <int Q, int BT, int G>
+__global__ void __launch_bounds__(256 * G) dense_any_kernel(const DenseAnyArgs a) {
   constexpr int BKA = 4096 / BT, RUNS = BKA / 16;
   constexpr int LDR = BKA + 8;                 // halfs per LDS row: 16 consecutive rows start on 16 different bank groups
   constexpr int BUF = BT * LDR;                // halfs per operand and stage
   constexpr int HW = Q == 16 ? 8 : (Q + 1) / 2;  // dwords that hold a thread's 16 weights or indices
   constexpr int NRAW = Q == 16 ? 8 : HW + 1;     // ... at any byte offset
   constexpr int OUT_LD = BT + 1;
-  constexpr int OUT_BYTES = (BT == 32 ? 4 : 1) * BT * OUT_LD * 4;
-  static_assert(OUT_BYTES <= 4 * BUF * 2, "the output tile reuses the operand buffers");
-  __shared__ __attribute__((aligned(16))) half_t tiles[4 * BUF];
+  constexpr int PARTS = (BT == 32 ? 4 : 1) * G;  // sums of every output
+  static_assert(PARTS * BT * OUT_LD * 4 <= G * 4 * BUF * 2, "the output tile reuses the operand buffers");
+  __shared__ __attribute__((aligned(16))) half_t all_tiles[G * 4 * BUF];
   __shared__ __attribute__((aligned(4))) uint16_t pal_lds[Q == 16 ? 2 : kAnyPalBytes / 2];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  half_t* const tiles = all_tiles + group * 4 * BUF;
   const int l32 = lane & 31, hi = lane >> 5;
   const int64_t m0 = (blockIdx.x % a.tiles_m) * BT, n0 = (blockIdx.x / a.tiles_m) * BT;
   const int row = tid / RUNS, run = tid % RUNS;
@@ -65,7 +69,7 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
   const int nib = lay.nib;
 
   // the output feature that this thread finishes (in several rows), and its bias
-  const int of = tid % BT;
+  const int of = threadIdx.x % BT;
   const float bias = a.bias && n0 + of < a.n ? (float)bits_to_half(a.bias[n0 + of]) : 0.f;
 
   // palettes of every block the tile's rows touch, asked for four dwords at a time: one trip to memory, not one for each
@@ -77,23 +81,23 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
       const AnyBlocks held = any_blocks(n0, BT, a.n, a.k, nib);
       blk0 = held.first;
       const int n_pal = held.count << (Q - 1);
-      for (int i0 = tid; i0 < n_pal; i0 += 4 * 256) {
+      for (int i0 = threadIdx.x; i0 < n_pal; i0 += 4 * 256 * G) {
         uint32_t v[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-          const int i = i0 + 256 * j < n_pal ? i0 + 256 * j : i0;
+          const int i = i0 + 256 * G * j < n_pal ? i0 + 256 * G * j : i0;
           v[j] = reinterpret_cast<const u32_any*>(a.w + palette_offset(lay, blk0 + (i >> (Q - 1))))[i & ((1 << (Q - 1)) - 1)];
         }
 #pragma unroll
         for (int j = 0; j < 4; j++)
-          if (i0 + 256 * j < n_pal) reinterpret_cast<uint32_t*>(pal_lds)[i0 + 256 * j] = v[j];
+          if (i0 + 256 * G * j < n_pal) reinterpret_cast<uint32_t*>(pal_lds)[i0 + 256 * G * j] = v[j];
       }
     }
   }
 
   const bool runs_ok = any_by_words(NRAW, a.w_bytes, nib);  // (otherwise index by index)
   AnyCursor next = {0, 0};  // this thread's next weight run
-  if constexpr (Q != 16) next = any_cursor(gn, a.k, run * 16, nib);
+  if constexpr (Q != 16) next = any_cursor(gn, a.k, group * BKA + run * 16, nib);
 
   // NRAW dwords from byte p of the packed buffer on; the result is the number of bytes by which they are early.
   auto load_raw = [&](int64_t p, uint32_t (&raw)[NRAW]) {
@@ -153,7 +157,7 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
           early2 = load_raw(bit >> 3, wraw2);
         }
       }
-      any_advance(next, BKA, nib);
+      any_advance(next, G * BKA, nib);
     }
   };
   auto stage = [&](int buf) {
@@ -220,14 +224,14 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
   const int wn = BT == 64 ? wave & 1 : 0, wm = BT == 64 ? wave >> 1 : 0;
   const int ks0 = BT == 64 ? 0 : 2 * wave;
   constexpr int NKS = BT == 64 ? 4 : 2;
-  const int nkt = (int)((a.k + BKA - 1) / BKA);
-  fetch(0);
+  const int nkt = (int)((a.k + BKA - 1) / BKA), rounds = (nkt + G - 1) / G;  // (a K-tile past the end is zeros)
+  fetch(group);
   __syncthreads();  // palettes visible
   stage(0);
   __syncthreads();
-  for (int kt = 0; kt < nkt; kt++) {
-    const bool more = kt + 1 < nkt;
-    if (more) fetch(kt + 1);
+  for (int kt = 0; kt < rounds; kt++) {
+    const bool more = kt + 1 < rounds;
+    if (more) fetch((kt + 1) * G + group);
     const half_t* xs = tiles + (kt & 1) * 2 * BUF + (wm * 32 + l32) * LDR + 8 * hi;
     const half_t* ws = tiles + (kt & 1) * 2 * BUF + BUF + (wn * 32 + l32) * LDR + 8 * hi;
 #pragma unroll
@@ -239,19 +243,19 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
   }
 
   // Sums to LDS as [token][feature], then element by element with consecutive features in consecutive lanes.
-  float* outs = reinterpret_cast<float*>(tiles) + (BT == 32 ? wave * BT * OUT_LD : 0);
+  float* outs = reinterpret_cast<float*>(all_tiles) + (BT == 32 ? group * 4 + wave : group) * BT * OUT_LD;
 #pragma unroll
   for (int v = 0; v < 16; v++)
     outs[(wm * 32 + l32) * OUT_LD + wn * 32 + 8 * (v >> 2) + 4 * hi + (v & 3)] = acc[v];
   __syncthreads();
-  const float* sums = reinterpret_cast<const float*>(tiles);
-  for (int t = tid / BT; t < BT; t += 256 / BT) {
+  const float* sums = reinterpret_cast<const float*>(all_tiles);
+  for (int t = threadIdx.x / BT; t < BT; t += 256 * G / BT) {
     const int64_t mi = m0 + t, ni = n0 + of;
     if (mi >= a.m || ni >= a.n) continue;
     float s = sums[t * OUT_LD + of];
-    if constexpr (BT == 32) {
+    if constexpr (PARTS > 1) {
 #pragma unroll
-      for (int p = 1; p < 4; p++) s += sums[(p * BT + t) * OUT_LD + of];
+      for (int p = 1; p < PARTS; p++) s += sums[(p * BT + t) * OUT_LD + of];
     }
     if (a.bias) s += bias;
     store_post(a, mi, ni, round_f16(s));
@@ -259,31 +263,45 @@ __global__ void __launch_bounds__(256) dense_any_kernel(const DenseAnyArgs a) {
 }
 
 template <int Q>
-static void launch_any(hipStream_t s, const DenseAnyArgs& a, bool big, unsigned grid) {
-  if (big) hipLaunchKernelGGL((dense_any_kernel<Q, 64>), dim3(grid), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((dense_any_kernel<Q, 32>), dim3(grid), dim3(256), 0, s, a);
+static void launch_any(hipStream_t s, const DenseAnyArgs& a, bool big, int groups, unsigned grid) {
+  const dim3 block(256 * (unsigned)groups);
+  if (big) {
+    if (groups == 4) hipLaunchKernelGGL((dense_any_kernel<Q, 64, 4>), dim3(grid), block, 0, s, a);
+    else hipLaunchKernelGGL((dense_any_kernel<Q, 64, 1>), dim3(grid), block, 0, s, a);
+  } else {
+    if (groups == 4) hipLaunchKernelGGL((dense_any_kernel<Q, 32, 4>), dim3(grid), block, 0, s, a);
+    else if (groups == 2) hipLaunchKernelGGL((dense_any_kernel<Q, 32, 2>), dim3(grid), block, 0, s, a);
+    else hipLaunchKernelGGL((dense_any_kernel<Q, 32, 1>), dim3(grid), block, 0, s, a);
+  }
 }
 
 dt_status dense_any_launch(hipStream_t s, DenseAnyArgs a) {
   if (a.m <= 0 || a.n <= 0) return DT_OK;
   const auto tiles = [&](int t) { return ((a.m + t - 1) / t) * ((a.n + t - 1) / t); };
-  // The 64 x 64 tile halves what is read and unpacked per output but takes twice as long for a K-tile pair; it wins once
-  // there is one for every compute unit.  1000 -> 1001, 32 against 64 wide, us: 500 rows (128 tiles of 64) 14.9 / 23.9
-  // q8p and 9.7 / 14.8 fp16; 1000 rows (256 tiles) 26.2 / 24.0 and 15.2 / 15.1; 2000 rows (512) 48.2 / 27.7 and
-  // 31.7 / 18.6.
-  const bool big = tiles(64) >= 256;
+  // The 64 x 64 tile halves what is read and unpacked per output but takes twice as long for a K-tile pair; with one group of waves it
+  // wins once there are more of them than compute units.  Up to there groups share K out: as many as K is long enough for where 32 x 32
+  // tiles have a compute unit each, and on 64 x 64 tiles where there are more of the small ones.  us, q8p (fp16):
+  //   small tiles, 1 / 2 / 4 groups: 231 x 1000 -> 1001 13.3 / 10.1 / 8.6 (8.6 / 7.4 / 6.8), 130 x 700 -> 500 11.2 / 8.9 / 8.8 (7.7 / 6.7 / 7.3), 1 x 2555 ->
+  //     2555 23.6 / 17.3 / 15.0 (13.3 / 10.8 / 9.8), 70 x 100 -> 96 5.6 / 5.7 / 6.3; where they share compute units 500 x 1000 -> 1001 15.4 / 18.1 / 15.4
+  //   small ones / 64 wide, 1 / 4 groups: 500 x 1000 -> 1001 15.4 / 24.6 / 13.4 (10.3 / 15.4 / 9.9), 1000 rows 26.9 / 24.9 / 13.7 (15.9 / 15.8 / 10.4), 100
+  //     x 300 -> 2200 9.1 / 13.7 / 10.2, 333 x 90 -> 1500 7.7 / 10.8 / 8.1; over 256 of them 1000 x 2500 -> 2500 112 / 70.6 / 73.9, 700 x 300 -> 2200 19.3
+  //     / 16.3 / 18.9
+  const int64_t small_tiles = tiles(32), k_tiles = (a.k + 127) / 128;
+  const bool shared_out = tiles(64) <= 256 && small_tiles > 256 && a.k > 512;
+  const bool big = shared_out || tiles(64) >= 256;
+  const int groups = shared_out ? 4 : big || small_tiles > 256 || k_tiles < 2 ? 1 : k_tiles >= (a.qbits == 16 ? 8 : 6) ? 4 : 2;
   const int BT = big ? 64 : 32;
   const int64_t grid = tiles(BT);
   if (grid > 0x7fffffff) return DT_NO_KERNEL;
   a.tiles_m = (a.m + BT - 1) / BT;
   a.pal_shared = a.qbits != 16 && any_pal_shared(BT, a.k, a.qbits, a.nib);
   switch (a.qbits) {
-    case 4: launch_any<4>(s, a, big, (unsigned)grid); break;
-    case 5: launch_any<5>(s, a, big, (unsigned)grid); break;
-    case 6: launch_any<6>(s, a, big, (unsigned)grid); break;
-    case 7: launch_any<7>(s, a, big, (unsigned)grid); break;
-    case 8: launch_any<8>(s, a, big, (unsigned)grid); break;
-    case 16: launch_any<16>(s, a, big, (unsigned)grid); break;
+    case 4: launch_any<4>(s, a, big, groups, (unsigned)grid); break;
+    case 5: launch_any<5>(s, a, big, groups, (unsigned)grid); break;
+    case 6: launch_any<6>(s, a, big, groups, (unsigned)grid); break;
+    case 7: launch_any<7>(s, a, big, groups, (unsigned)grid); break;
+    case 8: launch_any<8>(s, a, big, groups, (unsigned)grid); break;
+    case 16: launch_any<16>(s, a, big, groups, (unsigned)grid); break;
     default: return DT_INVALID;
   }
   return launch_status();

@@ -5,7 +5,7 @@
 
 namespace dt {
 
-constexpr int kAnyPalBytes = 16384;  // LDS for the palettes of a tile's rows (with the tiles used: three workgroups per CU)
+constexpr int kAnyPalBytes = 16384;  // LDS for the palettes of a tile's rows (with a group's tiles: three workgroups per CU; with four groups' 64 x 64 tiles all of it)
 
 // Rows past the last one read the last one: the only row that is sure to lie among the palettes of their tile.
 DT_HD int64_t any_row(int64_t row, int64_t n) { return row < n ? row : n - 1; }
