@@ -729,20 +729,19 @@ class LoRADense:
 
     def _fused(self, x, b, post, stream):
         """The layer through dt_lora_dense_f16 as a list of its output, or None where it runs as Dense calls (us, those / this: 4608 x 3072
-        -> 3072 q6p, rank 16, 103 / 94; 300 x 1280 -> 1280 q8p 48 / 22, most of which is the host)."""
+        -> 3072 q6p, rank 16, 104 / 95; 300 x 1280 -> 1280 q8p 28 / 22)."""
+        high, rank = self.configuration.highPrecision, self.configuration.rank
         host = _native or _host()
-        if host is None or not isinstance(x, _torch().Tensor) or x.dim() < 1 or x.numel() <= _ROWS_MAX * x.shape[-1]:
+        # (what the library would answer no to by its widths alone is not asked: 4 us of a small layer's 22)
+        if host is None or not (high or rank <= 32) or not isinstance(x, _torch().Tensor) or x.dim() < 1 \
+                or x.numel() <= _ROWS_MAX * x.shape[-1] or x.shape[-1] % 64:
             return None
-        dn, up = (self.down, self.up) if self.configuration.highPrecision else self._padded()
-        K, rank = x.shape[-1], self.configuration.rank
-        if dn.shape[1] != K or dn.qbits not in (16, 32) or up.qbits not in (16, 32):
+        dn, up = (self.down, self.up) if high else self._padded()
+        if dn.shape[1] != x.shape[-1] or dn.qbits not in (16, 32) or up.qbits not in (16, 32) \
+                or dn.data.dtype != (_torch().float32 if high else _torch().float16):
             return None
-        if not self.configuration.highPrecision:
-            if dn.data.dtype != _torch().float16:
-                return None
-            rank = (rank + 15) // 16 * 16  # (of the padded pair's 64, 128, ...)
-        elif dn.data.dtype != _torch().float32:
-            return None
+        if not high:
+            rank = (rank + 15) // 16 * 16  # (of the padded pair's 64)
         problem = (x, [self.weight], [b], None, None, None if post is None else [post])
         if stream is None:
             got = host.lora(problem, dn.data, up.data, rank, up.shape[1], self.configuration.scale, self.flags, _scratch)

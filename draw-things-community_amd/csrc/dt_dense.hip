@@ -705,20 +705,20 @@ static size_t lora_t_bytes(int64_t M, const dt_lora_pair& p) { return ((size_t)M
 
 // Whether the layer is one launch of a tiled kernel with the branch in its epilogue, behind its down projection.  (Few rows, and what is
 // off the tiled kernels' alignment, run as Dense calls of their own; so do fp16 pairs of ranks that are no multiple of 16.)
-// In fp16 the down projection of many ranks over many inputs reads more than a compute unit's L1 can deliver, where the tiled kernel shares
-// it in LDS, and the Dense calls run it beside the base projection.  us, Dense calls / here, the calls bound by the host below 50:
-//   rank 16: 4608 x 3072 -> 3072 103 / 96, 1376 x 3072 -> 3072 57 / 52, 512 x 3072 -> 3072 51 / 38, 300 x 1280 -> 1280 48 / 22, 4096 x 320 ->
-//   320 47 / 17, 100 x 5120 -> 1280 51 / 53; rank 64: 2016 x 1280 -> 1280 47 / 31, 512 x 3072 -> 3072 50 / 42, and the other way round 2500 x
-//   1024 -> 4096 56 / 67, 1376 x 3072 -> 3072 57 / 64; rank 128: 2016 x 1280 -> 1280 47 / 40, 512 x 3072 -> 3072 50 / 51.
-// In fp32, rank 32: 4608 x 3072 -> 3072 124 / 115, 512 x 3072 -> 3072 55 / 43, 300 x 1280 -> 1280 53 / 26; rank 128: 198 / 185, 68 / 55, 53 / 38, and the
-// other way round 2500 x 1024 -> 4096 106 / 114, which is all output.
+// In fp16 the down projection of many ranks, or of long rows, reads more than a compute unit's L1 can deliver, where the tiled kernel
+// shares it in LDS, and the Dense calls run it beside the base projection.  us, Dense calls / here:
+//   rank 16 (32): 4608 x 3072 -> 3072 q6p 104 / 95 (105 / 100), 1376 x 3072 -> 3072 q8p 58 / 52 (58 / 54), 512 x 3072 -> 3072 q6p 42 / 38 (42 / 39), 2016 x
+//   1280 -> 1280 q6p 30 / 24 (30 / 27), 300 x 1280 -> 1280 q8p 28 / 22 (28 / 24), 4096 x 320 -> 320 q6p 22 / 17 (22 / 19), and the other way round, rank 32, 2206
+//   x 4928 -> 320 45 / 53, rank 16, 100 x 5120 -> 1280 51 / 53; rank 64 and 128, with kernels for them: 929 x 3456 -> 704 40 / 54, 1432 x 832 -> 640 24
+//   / 25, 1571 x 704 -> 832 24 / 32.
+//   fp32, rank 32 (128): 4608 x 3072 -> 3072 128 / 113 (203 / 184), 512 x 3072 -> 3072 50 / 43 (54 / 54), 300 x 1280 -> 1280 44 / 26 (44 / 38), and the other way
+//   round, rank 128, 2500 x 1024 -> 4096 106 / 114, which is all output.
 static bool lora_fusable(const HostGroup& h, const dt_lora_pair& p) {
   if (h.M <= 0 || !h.x_ok() || !h.w_tiled(0)) return false;
   if (dense_rows_features(h.M, h.K, h.W[0].qbits, h.W[0].nib, h.W[0].count / h.K) > 0) return false;
   if (p.f32) return h.M <= 0x3fffffff && p.rank <= 4096 && !(p.rank > 64 && h.K < 2048 && h.M * (h.W[0].count / h.K) > 6000000);
-  if (p.rank > 32 && (double)h.M * (double)h.W[0].count * p.rank > 5e11) return false;
-  if (h.M < 512 && h.K > 4096) return false;
-  return p.rank % 16 == 0 && p.rank <= 128 && p.ld_up % 4 == 0 && (reinterpret_cast<uintptr_t>(p.down) & 15) == 0 &&
+  if (h.K > 4096 && (h.M < 512 || p.rank > 16)) return false;
+  return p.rank % 16 == 0 && p.rank <= 32 && p.ld_up % 4 == 0 && (reinterpret_cast<uintptr_t>(p.down) & 15) == 0 &&
          (reinterpret_cast<uintptr_t>(p.up) & 7) == 0;
 }
 

@@ -116,7 +116,7 @@ template <int MT, int RT>
 constexpr int lora_down_f16_lds = MT * RT * 256 * 4;
 template <int MT, int RT>
 __device__ __forceinline__ void lora_down_f16(const LoraDownArgs& a, int block_m, int block_r, unsigned char* smem) {
-  constexpr int NW = 8, S = MT + RT <= 3 ? 6 : MT + RT <= 5 ? 4 : 2;
+  constexpr int NW = 8, S = MT + RT <= 3 ? 6 : 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, c = lane >> 4;
   float* const sums = reinterpret_cast<float*>(smem) + lane;  // [MT * RT][4][64 lanes]
   const int64_t m = (int64_t)block_m * 16 * MT + l16;
@@ -269,15 +269,15 @@ __global__ void __launch_bounds__(256) lora_up_kernel(const LoraUpArgs a) {
 
 // Rows (16 MT) and ranks (16 RT) of a workgroup, handed to run(F32, MT, RT, blocks of rows, blocks): the shape for which a compute unit
 // reads least.  A step of 32 k takes one read for 16 rows of X and one, in fp32 two, for 16 ranks of `down`; what several
-// workgroups on a compute unit read adds up.  (us, the whole layer, all ranks up to 64 in a workgroup / by this rule, rank 64 in fp16: 4608 x 3072 -> 3072 q6p 130 / 117, 1024 x 5120
-// -> 5120 q5p 109 / 98, 512 x 3072 -> 3072 q6p 52 / 42, 300 x 1280 -> 1280 q8p 33 / 28; in fp32 141 / 141, 124 / 103, 62 / 46, 37 / 30.)
+// workgroups on a compute unit read adds up.  (us, the whole layer, all ranks up to 64 in a workgroup / by this rule, rank 32 in fp16: 4608 x 3072 -> 3072 q6p 106 / 101, 1376 x
+// 3072 -> 3072 q8p 57 / 54, 512 x 3072 -> 3072 q6p 42 / 38; rank 64 in fp32: 141 / 141, 82 / 70, 62 / 46.)
 template <typename F>
 static dt_status with_down_shape(const LoraDownArgs& a, const F& run) {
   using std::integral_constant;
   int MT = 1, RT = 1;
   int64_t bm = 0, br = 0, least = INT64_MAX;
   for (int mt = 1; mt <= 2; mt++)
-    for (int rt = 1; rt <= 4; rt *= 2) {
+    for (int rt = 1; rt <= (a.f32 ? 4 : 2); rt *= 2) {  // (fp16: ranks up to 32)
       const int64_t m = (a.m + 16 * mt - 1) / (16 * mt), r = (a.rank + 16 * rt - 1) / (16 * rt);
       const int64_t reads = (mt + (a.f32 ? 2 : 1) * rt) * ((m * r + 255) / 256);
       if (reads < least) {
@@ -290,7 +290,7 @@ static dt_status with_down_shape(const LoraDownArgs& a, const F& run) {
   const auto ranks = [&](auto f32, auto mt) {
     if (RT == 1) run(f32, mt, integral_constant<int, 1>{}, blocks_m, blocks);
     else if (RT == 2) run(f32, mt, integral_constant<int, 2>{}, blocks_m, blocks);
-    else run(f32, mt, integral_constant<int, 4>{}, blocks_m, blocks);
+    else if constexpr (decltype(f32)::value) run(f32, mt, integral_constant<int, 4>{}, blocks_m, blocks);
   };
   const auto rows = [&](auto f32) {
     if (MT == 2) ranks(f32, integral_constant<int, 2>{});

@@ -7,7 +7,7 @@
 
 namespace dt {
 
-// T and up of a layer, both fp16 (`rank` a multiple of 16, all rows 8-byte aligned) or both fp32 (any rank).
+// T and up of a layer, both fp16 (`rank` 16 or 32, all rows 8-byte aligned) or both fp32 (any rank).
 struct DenseLora {
   const void* t;   // [M, rank], scale included, row stride ld_t
   const void* up;  // [N, rank], row stride ld_up; null = no branch
@@ -92,10 +92,8 @@ __device__ __forceinline__ void low_rank_sums(float4_t (&s)[TN][TM], const Dense
 #pragma unroll 1
     for (; r0 < l.rank; r0 += 16) steps(std::true_type{}, std::integral_constant<int, 1>{}, r0);
   } else {
-#pragma unroll 1
-    for (; r0 + 64 <= l.rank; r0 += 64) steps(std::false_type{}, std::integral_constant<int, 4>{}, r0);
-#pragma unroll 1
-    for (; r0 < l.rank; r0 += 16) steps(std::false_type{}, std::integral_constant<int, 1>{}, r0);
+    if (l.rank > 16) steps(std::false_type{}, std::integral_constant<int, 2>{}, 0);
+    else steps(std::false_type{}, std::integral_constant<int, 1>{}, 0);
   }
 }
 

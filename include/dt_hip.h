@@ -251,7 +251,7 @@ dt_status dt_lora_branch_f32_f16(dt_stream stream, int64_t M, int64_t K, const u
  * A whole LoRADense (Models/LoRA.swift:85-142) on up to two launches: Y = tail(dense(x) + up(scale * down(x))), the branch rounded to fp16
  * and added to the base projection's fp16 result in its epilogue.  fp16 pairs round the intermediate to fp16 before and behind
  * `scale`, fp32 ones (highPrecision) keep it in fp32; results are those of the Dense calls that the layer consists of, bit for bit.
- *   pair : f32 = 0: `down` [rank, K] and `up` [N, rank] (row stride ld_up) in fp16, rank padded with zeros to a multiple of 16, at most 128
+ *   pair : f32 = 0: `down` [rank, K] and `up` [N, rank] (row stride ld_up) in fp16, rank padded with zeros to 16 or 32
  *          f32 = 1: fp32, any rank up to 4096
  *   post : as for dt_dense_qx_post_f16 without scale, addend and multiplicand; NULL = no tail
  * dt_lora_dense_scratch_bytes: the scratch memory (256-byte aligned) that the call takes, with less of it the weight stays packed, but at

@@ -38,9 +38,9 @@ def pair_of(dthip, op):
 
 
 @pytest.mark.parametrize("M,N,K,q,nib,rank,high", [
-    (65, 130, 64, 6, 512, 1, False), (129, 257, 128, 8, 4096, 17, False), (300, 512, 832, 4, 1024, 48, False),   # part of a wave's steps, of the waves
-    (1100, 640, 1536, 6, 4096, 64, False), (257, 384, 1600, 5, 2048, 128, False), (4099, 256, 448, 16, 0, 33, False),  # whole rounds, a round and a share
-    (4099, 300, 192, 7, 4096, 128, False), (16400, 128, 128, 6, 4096, 20, False), (70, 320, 192, 8, 256, 16, False),   # 32 rows a workgroup; blocks too small to copy
+    (65, 130, 64, 6, 512, 1, False), (129, 257, 128, 8, 4096, 17, False), (300, 512, 832, 4, 1024, 32, False),   # part of a wave's steps, of the waves
+    (1100, 640, 1536, 6, 4096, 32, False), (257, 384, 1600, 5, 2048, 8, False), (4099, 256, 448, 16, 0, 16, False),  # whole rounds, a round and a share
+    (4099, 300, 192, 7, 4096, 31, False), (16400, 128, 128, 6, 4096, 20, False), (70, 320, 192, 8, 256, 16, False),   # 32 rows a workgroup; blocks too small to copy
     (65, 130, 64, 6, 512, 1, True), (300, 257, 832, 4, 1024, 20, True), (1100, 512, 192, 8, 4096, 33, True),    # ranks of no multiple of 16, of 4
     (4099, 256, 320, 16, 0, 70, True), (16400, 130, 128, 6, 4096, 31, True), (129, 256, 256, 5, 512, 130, True),
 ])
