@@ -69,13 +69,6 @@ __device__ __forceinline__ int v_unit_swz(int row, int u) {
   return u ^ (DP == 128 ? row & 3 : (row >> 1) & 1);
 }
 
-// The larger of each half of three pairs of fp16; NaN wins.
-__device__ __forceinline__ uint32_t max3_h2(uint32_t x, uint32_t y, uint32_t z) {
-  uint32_t r;
-  asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(x), "v"(y), "v"(z));
-  return r;
-}
-
 // The lane groups of a wave -- two of 32, M16: four of 16 -- hold the same matrix columns: combine them without touching LDS.
 __device__ __forceinline__ void halves16(float v, float& even, float& odd) {  // groups {0, 0, 2, 2} and {1, 1, 3, 3}
   uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
@@ -126,7 +119,6 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
   constexpr int TILE_B = BKV * ROWB;           // bytes of one K (or V) tile
   constexpr int LOADS = TILE_B / (QW * 1024);  // 16-byte chunks per thread per tile
   constexpr int LROWS = QW * 1024 / ROWB;      // rows of a tile that a load of all threads covers
-  constexpr bool ONES = DP == 64 && DL < DP;   // row sums come out of the second MFMA
   constexpr int MB = M16 ? 16 : 32;            // rows and columns of an MFMA
   constexpr int MK = M16 ? 32 : 16;            // its k-step
   constexpr int QB = 32 / MB;                  // its blocks in a wave's 32 queries
@@ -182,29 +174,23 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
   constexpr int OFFS = KG == 1 ? LOADS : 1;
   const int qwave_u = __builtin_amdgcn_readfirstlane(qwave);
   int ld_row[LOADS], k_ch[LOADS], v_ch[LOADS];
-  auto v_chunk = [](int row, int pc) __attribute__((always_inline)) {  // (the swizzles are involutions)
-    return M16 ? v_unit_swz<DP, M16>(row, pc >> 1) * 2 + (pc & 1) : v_unit_swz<DP, M16>(row, pc >> 2) * 4 + (pc & 3);
-  };
   auto place = [](int w, int i) __attribute__((always_inline)) { return (OFFS > 1 ? w * LOADS + i : i * QW + w) * 1024; };
 #pragma unroll
   for (int i = 0; i < LOADS; i++) {
     const int off = place(qwave, OFFS > 1 ? i : 0) + lane * 16;
     const int row = off / ROWB, pc = (off % ROWB) / 16;
     ld_row[i] = row + (OFFS > 1 ? 0 : i * LROWS);
-    k_ch[i] = k_chunk_swz<DP>(row, pc);
-    v_ch[i] = v_chunk(row, pc);
+    k_ch[i] = k_chunk_swz<DP>(row, pc);  // (the swizzles are involutions)
+    v_ch[i] = M16 ? v_unit_swz<DP, M16>(row, pc >> 1) * 2 + (pc & 1) : v_unit_swz<DP, M16>(row, pc >> 2) * 4 + (pc & 3);
   }
   auto slot = [&](int i) __attribute__((always_inline)) { return (uint32_t)(kg * TILE_B + place(qwave_u, i)); };  // in a stage
-  // slots that no transfer will ever write must not hold NaN patterns; ONES: column D of V is ones
+  // slots that no transfer will ever write must not hold NaN patterns
   if (D < DP || Skv % BKV != 0) {
     for (int i = tid * 16; i < KG * TILE_B; i += 512 * 16) {
-      const uint4_t zero = {0, 0, 0, 0};
-      uint4_t v = zero;
-      if (ONES && v_chunk(i / ROWB, i % ROWB / 16) * 8 == D) v[0] = 0x3c00;
-      *reinterpret_cast<uint4_t*>(Ks0 + i) = zero;
-      *reinterpret_cast<uint4_t*>(Ks1 + i) = zero;
-      *reinterpret_cast<uint4_t*>(Vs0 + i) = v;
-      *reinterpret_cast<uint4_t*>(Vs1 + i) = v;
+      *reinterpret_cast<uint4_t*>(Ks0 + i) = uint4_t{0, 0, 0, 0};
+      *reinterpret_cast<uint4_t*>(Ks1 + i) = uint4_t{0, 0, 0, 0};
+      *reinterpret_cast<uint4_t*>(Vs0 + i) = uint4_t{0, 0, 0, 0};
+      *reinterpret_cast<uint4_t*>(Vs1 + i) = uint4_t{0, 0, 0, 0};
     }
     __syncthreads();
   }
@@ -543,10 +529,10 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
     }
     // Probabilities against the current reference, and this lane's share of their row sums.  The tile's maximum is
     // not looked for: as long as every lane's sums stay below 2^10 no probability exceeds that (fp16 holds 2^16),
-    // which is all that the reference is there to ensure.  (ONES: the sums are the second MFMA's, and the largest of this lane's
-    // probabilities is looked at; as fp16 bits they order like integers, infinities and NaN last.)
+    // which is all that the reference is there to ensure.  (The sums are of the fp32 probabilities at every head size.  A column of
+    // ones in V's padding, which has the second MFMA add up the fp16 ones, is 3 us of 72 faster at 2 x 8 heads of 40, 4096 x 4096, and
+    // loses what lies below 2^-25 of the reference: 16383 such keys beside one took a result from 0.9995 to 1.)
     float psum[QB];
-    [[maybe_unused]] uint32_t pmax = 0;
     auto probabilities = [&]() __attribute__((always_inline)) {
       float mc[QB];
 #pragma unroll
@@ -561,24 +547,16 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
 #pragma unroll
           for (int qb = 0; qb < QB; qb++) {
             const float p = fast_exp2(__builtin_fmaf(sacc[kb][qb][v], c, -mc[qb]));
-            if constexpr (!ONES) psum[qb] += p;
+            psum[qb] += p;
             const int slot = kb * NV + v;  // of this lane's scores: eight to an operand
             pf[slot >> 3][qb][slot & 7] = (half_t)p;
             if constexpr (FOUR)  // (operand by operand: 128 registers hold no more than one operand's probabilities in fp32)
               if ((slot & 7) == 7) __builtin_amdgcn_sched_barrier(0);
           }
-      if constexpr (ONES) {
-        pmax = 0;
-#pragma unroll
-        for (int i = 0; i < BKV / PK; i++) {
-          const uint4_t two = __builtin_bit_cast(uint4_t, pf[i][0]);
-          pmax = max3_h2(max3_h2(pmax, two[0], two[1]), two[2], two[3]);
-        }
-      }
     };
     probabilities();
     // (the first tile arrives here with the references at -inf: its sums are inf; a NaN fails the test too)
-    bool outgrown = ONES ? (pmax & 0xffff) > 0x6400 || pmax > 0x6400ffff : !(psum[0] <= 1024.0f);
+    bool outgrown = !(psum[0] <= 1024.0f);
     if constexpr (QB == 2) outgrown = outgrown || !(psum[1] <= 1024.0f);
     if (__builtin_amdgcn_ballot_w64(outgrown) != 0) {
       // some row's scores have outgrown the reference: move every row's reference up to its running maximum,
@@ -607,7 +585,7 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
     }
 #pragma unroll
     for (int qb = 0; qb < QB; qb++)
-      if constexpr (!ONES) l_run[qb] += psum[qb];
+      l_run[qb] += psum[qb];
   };
 
   // O^T += V^T P^T for the V tile in stage st.
@@ -740,18 +718,7 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
 
   // the row sums, the same in every group of lanes from here on
 #pragma unroll
-  for (int qb = 0; qb < QB; qb++) {
-    if constexpr (ONES) {
-      // row D of O^T, which lane group 0 holds
-      float l = 0.f, other;
-#pragma unroll
-      for (int d = 0; d < DP; d += 8)
-        if (D == d) l = oacc[d / MB][0][d % MB / 2];
-      halves32(l, l_run[qb], other);
-    } else {
-      l_run[qb] = sum_groups<M16>(l_run[qb]);
-    }
-  }
+  for (int qb = 0; qb < QB; qb++) l_run[qb] = sum_groups<M16>(l_run[qb]);
 
   // Where two hold partial results of the same rows, meet() takes in the other's reference and row sums and says how its sums are
   // folded: mine a + got b with both products rounded, the same for either order.

@@ -1007,8 +1007,8 @@ def test_sdpa_key_split_replays_as_hip_graph(dthip, oracle, torch_cuda, monkeypa
     (1, 129, 1, 2, 2, 48, 0),      # one key
     (2, 128, 65, 2, 1, 64, 0),     # a second tile of one key; grouped heads
     (1, 1, 192, 3, 3, 40, 0),      # three tiles: the groups take two and one
-    (1, 300, 1000, 2, 2, 40, 77),  # keys in two segments, which straddle a tile; row sums out of the matrix instruction
-    (1, 260, 520, 2, 2, 56, 64),   # ... which begin with a tile; row sums added up
+    (1, 300, 1000, 2, 2, 40, 77),  # keys in two segments, which straddle a tile; 48 of 64 columns multiplied
+    (1, 260, 520, 2, 2, 56, 64),   # ... which begin with a tile; all of them
     (2, 140, 700, 3, 3, 72, 333),
     (1, 257, 450, 2, 2, 80, 0),
     (1, 150, 330, 2, 2, 96, 130),
@@ -1062,3 +1062,19 @@ def test_sdpa_two_key_groups_with_prepared_queries(dthip, oracle, torch_cuda, mo
         assert torch.equal(got, call(off))
         mx, rr = oracle.err_stats(got.cpu().numpy(), want)
         assert mx <= MAX_ABS and rr <= REL_RMS, (mx, rr)
+
+
+@pytest.mark.parametrize("mode", ["never", "always", "groups"])
+@pytest.mark.parametrize("D", [40, 48, 64, 80, 128])
+def test_sdpa_row_sums_hold_small_probabilities(dthip, torch_cuda, monkeypatch, D, mode):
+    """One key at 1 and 16383 at 2^-25.05 of it, which fp16 does not hold: they are 4.7e-4 of the row's sum all the same.  The result
+    is within half an fp16 step below 1 (2^-12) of the exact one, and 2^-16 for the sums and exponentials in fp32."""
+    torch = torch_cuda
+    n, low = 16384, -25.046875  # (a value of fp16)
+    q, k, v = (torch.zeros((1, s, 1, D), dtype=torch.float16, device="cuda") for s in (5, n, n))
+    q[..., 0], k[:, 1:, :, 0], v[:, 0] = 1, low, 1
+    print("sdpa small probabilities", D, mode, flush=True)
+    monkeypatch.setenv("DT_SDPA_KEY_SPLIT", mode)
+    got = dthip.sdpa_segments([q], [k], [v], float(np.log(2.0)))
+    exact = 1.0 / (1.0 + (n - 1) * 2.0 ** low)
+    assert float((got.double() - exact).abs().max()) <= 2.0 ** -12 + 2.0 ** -16
