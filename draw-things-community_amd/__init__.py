@@ -743,6 +743,8 @@ class LoRADense:
         if not high:
             rank = (rank + 15) // 16 * 16  # (of the padded pair's 64)
         problem = (x, [self.weight], [b], None, None, None if post is None else [post])
+        if stream is None and x.is_cuda and x.device.index != _torch().cuda.current_device():
+            stream = _torch().cuda.current_stream(x.device)  # (a layer runs where x is)
         if stream is None:
             got = host.lora(problem, dn.data, up.data, rank, up.shape[1], self.configuration.scale, self.flags, _scratch)
         else:

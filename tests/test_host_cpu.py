@@ -403,3 +403,43 @@ int main(int argc, char** argv) {
         shapes.append((n, k, int(rng.integers(4, 9)), nib))
     out = subprocess.run([str(exe)] + [str(v) for s in shapes for v in s], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+@pytest.mark.parametrize("high", [False, True])
+@pytest.mark.parametrize("current", [0, 1])
+def test_lora_layer_runs_where_its_input_is(dthip, monkeypatch, high, current):
+    """x on the second device, whichever is current: the layer is enqueued on the current stream of x's device, made current for the
+    call where its device is not.  (The tensors are host ones that say they are there, the native call a stand-in.)"""
+    import contextlib
+
+    import torch
+
+    class There(torch.Tensor):
+        is_cuda = property(lambda self: True)
+        device = property(lambda self: torch.device("cuda", 1))
+
+    entered, calls = [], []
+
+    @contextlib.contextmanager
+    def on(stream):
+        entered.append(stream)
+        yield
+        entered.pop()
+
+    class Host:
+        @staticmethod
+        def lora(*args):
+            calls.append(list(entered))
+            return ["out"]
+
+    monkeypatch.setattr(dthip, "_native", Host)
+    monkeypatch.setattr(dthip, "_on", on)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: ("stream of", str(device)))
+    dtype = torch.float32 if high else torch.float16
+    op = dthip.LoRADense(128, dthip.LoRANetworkConfiguration(16, 0.5, high))
+    op.weight = dthip.QxTensor(torch.zeros((128, 64), dtype=torch.float16), 16, 0, (128, 64))
+    op.down, op.up = (dthip.QxTensor(torch.zeros(s, dtype=dtype), 16, 0, s) for s in ((16, 64), (128, 16)))
+    x = torch.zeros((80, 64), dtype=torch.float16).as_subclass(There)
+    assert op(x) == "out" and op(x, stream="mine") == "out"
+    assert calls == [[] if current == 1 else [("stream of", "cuda:1")], ["mine"]]
