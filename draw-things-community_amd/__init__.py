@@ -766,6 +766,8 @@ class LoRADense:
             return dense_post(x, [self.weight], [b], [post], flags=self.flags, stream=stream)[0]
         if self.down.shape[0] != self.configuration.rank or self.up.shape != (self.count, self.configuration.rank):
             raise ValueError(f"LoRADense {self.name!r}: down / up shapes do not match rank and count")
+        if self.weight.shape[0] != self.count:
+            raise ValueError(f"LoRADense {self.name!r}: weight has {self.weight.shape[0]} rows, count is {self.count}")
         p = post or DensePost()
         if p.scale != 1.0 or p.addend is not None or p.multiplicand is not None:
             raise ValueError(f"LoRADense {self.name!r}: the tail may carry an activation, a gate and a residual only")

@@ -332,8 +332,8 @@ PyObject* lora(Py_ssize_t n_args, PyObject* const* args) {
   read_problem(args[0], p);
   if (p.w.size() != 1 || !p.epi.empty()) throw Fallback{};
   const dt_lora_pair pair{ptr<const void>(down), ptr<const void>(up), as_int(args[4]), as_int32(args[3]), f32 ? 1 : 0, as_float(args[5])};
-  // (the ones that the library may read: `rank` rows of each half, in up's case columns)
-  if (pair.rank <= 0 || down.numel() < pair.rank * p.K || up.numel() < p.ldy[0] * pair.ld_up || p.w[0].count != p.ldy[0] * p.K) throw Fallback{};
+  // (of the pair's padded halves the first `rank` rows are read, in up's case columns)
+  if (pair.rank <= 0 || down.numel() < pair.rank * p.K || up.numel() != p.ldy[0] * pair.ld_up) throw Fallback{};
   const uint32_t flags = (uint32_t)as_int32(args[6]);
   const uint16_t* const x = ptr<const uint16_t>(*p.x);
   const int64_t ldx = p.x->dim() == 2 && p.M > 1 ? p.x->stride(0) : p.K;

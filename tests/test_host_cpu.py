@@ -443,3 +443,30 @@ def test_lora_layer_runs_where_its_input_is(dthip, monkeypatch, high, current):
     x = torch.zeros((80, 64), dtype=torch.float16).as_subclass(There)
     assert op(x) == "out" and op(x, stream="mine") == "out"
     assert calls == [[] if current == 1 else [("stream of", "cuda:1")], ["mine"]]
+
+
+@pytest.mark.parametrize("high", [False, True])
+@pytest.mark.parametrize("rows", [64, 192])
+def test_lora_layer_refuses_a_weight_of_other_rows_than_count(dthip, monkeypatch, high, rows):
+    """Before anything is enqueued: the base projection's result and the branch have to be of one width."""
+    import torch
+
+    class Host:
+        @staticmethod
+        def lora(*args):
+            return ["out"]
+
+        @staticmethod
+        def dense(*args):
+            return [["plain"]]
+
+    monkeypatch.setattr(dthip, "_native", Host)
+    dtype = torch.float32 if high else torch.float16
+    op = dthip.LoRADense(128, dthip.LoRANetworkConfiguration(16, 0.5, high))
+    op.weight = dthip.QxTensor(torch.zeros((rows, 64), dtype=torch.float16), 16, 0, (rows, 64))
+    op.down, op.up = (dthip.QxTensor(torch.zeros(s, dtype=dtype), 16, 0, s) for s in ((16, 64), (128, 16)))
+    x = torch.zeros((80, 64), dtype=torch.float16)
+    with pytest.raises(ValueError, match="rows"):
+        op(x)
+    op.configuration.scale = 0  # no branch: a plain Dense, of whatever rows its weight has
+    assert op(x) == "plain"
