@@ -104,8 +104,8 @@ class _Segment(ctypes.Structure):
 
 
 def build(verbose: bool = False) -> str:
-    """Compile libdthip.so for gfx950 with the Makefile under csrc/ (always recompiles)."""
-    cmd = ["make", "-C", CSRC, "-B", "-j8"]
+    """Compile libdthip.so for gfx950, and these operators' way to it, with the Makefile under csrc/ (always recompiles)."""
+    cmd = ["make", "-C", CSRC, "-B", "-j8", "python"]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if verbose or res.returncode != 0:
         print(res.stdout)
@@ -123,7 +123,7 @@ def lib():
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(
-                f"{LIB_PATH} is missing: build it with __graft_entry__.build() or `make -C {CSRC}`; "
+                f"{LIB_PATH} is missing: build it with __graft_entry__.build() or `make -C {CSRC} python`; "
                 "this package has no CPU or PyTorch fallback"
             )
         L = ctypes.CDLL(LIB_PATH)

@@ -235,6 +235,18 @@ def test_missing_library_fails_loudly(dthip, monkeypatch):
         dthip.lib()
 
 
+def test_library_builds_without_python(dthip):
+    """What a C, C++ or Swift host runs names neither Python nor torch; the package's own build makes its native calls as well."""
+    import subprocess
+
+    recipe = lambda *goals: subprocess.run(["make", "-n", "-B", "-C", dthip.CSRC, "PYTHON=no-such-python", *goals], capture_output=True, text=True,
+                                           check=True).stdout
+    plain = recipe()
+    assert "libdthip.so" in plain and "dt_cpp_check" in plain
+    assert "no-such-python" not in plain and "torch" not in plain
+    assert "no-such-python" in recipe("python") and "libdthip.so" in recipe("python")
+
+
 @pytest.mark.parametrize("q", [4, 5, 6, 7, 8])
 def test_host_packer_matches_oracle(dthip, oracle, q):
     rng = np.random.default_rng(q)
