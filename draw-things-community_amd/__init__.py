@@ -13,6 +13,7 @@ import ctypes
 import os
 import struct
 import subprocess
+import warnings
 from dataclasses import dataclass
 from typing import Optional, Sequence
 
@@ -187,20 +188,25 @@ _native = None
 
 
 def _host():
-    """The operators' native way to the library (csrc/dt_host.cpp), or None where the library stands alone: everything it does
-    is done here as well, in more of the host's time."""
+    """The operators' native way to the library (csrc/dt_host.cpp), or None where there is none that loads beside this torch: every
+    operator's results are the same without it, in more of the host's time and, for LoRA layers, more launches."""
     global _native
     if _native is None:
-        _native = False
         lib(), _torch()  # (whose libraries it is linked against)
-        path = os.path.join(_HERE, "_dthost.so")
+        path, host = os.path.join(_HERE, "_dthost.so"), False
         if os.path.exists(path):
             import importlib.util
 
-            spec = importlib.util.spec_from_file_location("_dthost", path)
-            _native = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(_native)
-            _native.classes(QxTensor, HeadEpilogue, DensePost)
+            try:
+                spec = importlib.util.spec_from_file_location("_dthost", path)
+                host = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(host)
+                host.classes(QxTensor, HeadEpilogue, DensePost)
+            except ImportError as e:
+                host = False
+                warnings.warn(f"{path} does not load ({e}); calls go through ctypes.  Build it against this torch: "
+                              f"`make -C {CSRC} python`", RuntimeWarning)
+        _native = host  # (whole: another thread may be looking)
     return _native or None
 
 

@@ -235,6 +235,42 @@ def test_missing_library_fails_loudly(dthip, monkeypatch):
         dthip.lib()
 
 
+def test_native_calls_that_do_not_load(dthip, monkeypatch, tmp_path):
+    """A module built against another torch: said once, and every call goes through ctypes, the first one too."""
+    import warnings
+
+    (tmp_path / "_dthost.so").write_bytes(b"no library")
+    monkeypatch.setattr(dthip, "_HERE", str(tmp_path))
+    monkeypatch.setattr(dthip, "_native", None)
+    with pytest.warns(RuntimeWarning, match="_dthost.so does not load"):
+        assert dthip._host() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert dthip._host() is None
+
+
+def test_native_calls_are_seen_whole(dthip, monkeypatch):
+    """Threads that come while the module is being loaded find nothing, or all of it."""
+    import importlib.util
+    import types
+
+    seen = []
+
+    class Loader:
+        create_module = staticmethod(lambda spec: None)
+
+        @staticmethod
+        def exec_module(module):
+            seen.append(dthip._native)
+            module.classes = lambda *c: seen.append(dthip._native)
+
+    spec = lambda name, path: importlib.util.spec_from_loader(name, Loader())
+    monkeypatch.setattr(importlib.util, "spec_from_file_location", spec)
+    monkeypatch.setattr(dthip, "_native", None)
+    host = dthip._host()
+    assert isinstance(host, types.ModuleType) and host is dthip._native and not any(seen) and len(seen) == 2
+
+
 def test_library_builds_without_python(dthip):
     """What a C, C++ or Swift host runs names neither Python nor torch; the package's own build makes its native calls as well."""
     import subprocess
