@@ -174,12 +174,12 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
   constexpr int OFFS = KG == 1 ? LOADS : 1;
   const int qwave_u = __builtin_amdgcn_readfirstlane(qwave);
   int ld_row[LOADS], k_ch[LOADS], v_ch[LOADS];
-  auto place = [](int w, int i) __attribute__((always_inline)) { return (OFFS > 1 ? w * LOADS + i : i * QW + w) * 1024; };
+  auto place = [](int w, int i) __attribute__((always_inline)) { return (KG == 1 ? w * LOADS + i : i * QW + w) * 1024; };
 #pragma unroll
   for (int i = 0; i < LOADS; i++) {
-    const int off = place(qwave, OFFS > 1 ? i : 0) + lane * 16;
+    const int off = place(qwave, KG == 1 ? i : 0) + lane * 16;
     const int row = off / ROWB, pc = (off % ROWB) / 16;
-    ld_row[i] = row + (OFFS > 1 ? 0 : i * LROWS);
+    ld_row[i] = row + (KG == 1 ? 0 : i * LROWS);
     k_ch[i] = k_chunk_swz<DP>(row, pc);  // (the swizzles are involutions)
     v_ch[i] = M16 ? v_unit_swz<DP, M16>(row, pc >> 1) * 2 + (pc & 1) : v_unit_swz<DP, M16>(row, pc >> 2) * 4 + (pc & 3);
   }
@@ -231,9 +231,49 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
   const int b = bh / a.Hq;
   const int hk = h / a.group;
 
+  // ---- Q^T fragments straight from global memory -----------------------
+  // B operand of K Q^T: lane holds query column col of block qb, head-dim slots MK*ks + 8*grp + 0..7.  What the norm and the
+  // rotation need is asked for together with the rows (one after the other, behind tests of each chunk's alignment, 24 x 2637 tokens
+  // took 11 us for it), all of it ahead of what the loaders need, which hides the way to the rows: us, 24 heads of 64 / 128, 1344 tokens in
+  // two segments, asked for behind it 28.9 / 39.7, here 28.6 / 39.3.  A lane's segment is an index into the arguments: selecting
+  // among all eight takes some 0.6 us of arithmetic.
+  half8_t qf[QB][KS];
+  uint4_t raw[QB][KS], gam[QB][KS], rot[QB][KS];
+  bool has_gam[QB];
+  const auto chunk = [](const uint16_t* p, bool aligned) __attribute__((always_inline)) {
+    if (aligned) return *reinterpret_cast<const uint4_t*>(p);  // uniform
+    uint4_t v;
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = (uint32_t)p[2 * q] | ((uint32_t)p[2 * q + 1] << 16);
+    return v;
+  };
+#pragma unroll
+  for (int qb = 0; qb < QB; qb++) {
+    int64_t qi = (int64_t)qt * QROWS + qwave * 32 + qb * MB + col;
+    if (qi >= Sq) qi = Sq - 1;
+    int sg = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxSeg; i++)
+      if (i < a.n_qseg && qi >= a.q[i].start) sg = i;
+    const uint16_t* const qp = a.q[sg].ptr + b * a.q[sg].sb + (qi - a.q[sg].start) * a.q[sg].ss + h * a.q[sg].sh;
+    const uint16_t* gp = a.q_gamma[sg];
+    has_gam[qb] = gp != nullptr;
+    if (!gp) gp = qp;  // (anything that can be read)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      const int d0 = ks * MK + grp * 8;
+      raw[qb][ks] = gam[qb][ks] = rot[qb][ks] = uint4_t{0, 0, 0, 0};
+      if (d0 < D) {
+        raw[qb][ks] = *reinterpret_cast<const uint4_t*>(qp + d0);
+        if (a.q_norm) gam[qb][ks] = chunk(gp + d0, a.q_aligned);  // uniform
+        if (a.q_rot) rot[qb][ks] = chunk(a.q_rot + qi * D + d0, a.q_aligned);
+      }
+    }
+  }
+
   // ---- K / V tile loaders ------------------------------------------------
   // ONESEG: K and V are one run of rows each and small enough for 32-bit byte
-  // offsets from a uniform base, which a tile step moves.
+  // offsets from a uniform base; a tile step moves these (two key groups: that).
   // Otherwise the segment of a tile is looked up once per tile (uniformly): a
   // tile that lies inside one segment is fetched from that segment's base with
   // per-lane 32-bit offsets, a tile that straddles segments row by row.
@@ -281,7 +321,11 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
 #pragma unroll
     for (int i = 0; i < OFFS; i++) off[i] = (uint32_t)((ld_row[i] * ss + chs[i] * 8) * 2);
   };
-  SegCursor kcur{nullptr, 0, 0, 0}, vcur{nullptr, 0, 0, 0};
+  SegCursor kcur{}, vcur{};
+  if constexpr (!ONESEG) {
+    seek(a.k, kcur, k_off, k_ch, t0);
+    seek(a.v, vcur, v_off, v_ch, t0);
+  }
   // (zero_tail: rows of the tile past the last key get zeros instead of keeping an earlier tile's bytes -- for V,
   // whose stale rows would otherwise meet a probability of exactly zero in the second MFMA: 0 x Inf = NaN)
   // What the paths that few tiles take derive from a thread's place is not to be kept in registers across the loop: they are short
@@ -297,10 +341,10 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
                            unsigned char* dst, int t, bool zero_tail) __attribute__((always_inline)) {
     if (t >= c.inside && t < full_tiles) seek(segs, c, off, chs, t);  // uniform
     if (t < c.inside) {                                               // uniform
-      const int64_t rows = OFFS > 1 ? 0 : __builtin_amdgcn_readfirstlane(c.rows);
+      const int64_t rows = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(c.rows);
 #pragma unroll
       for (int i = 0; i < LOADS; i++)
-        if (chs[i] * 8 < D) load_to_lds_16(c.base + i * rows, off[OFFS > 1 ? i : 0], lds_address(dst) + slot(i));
+        if (chs[i] * 8 < D) load_to_lds_16(c.base + i * rows, off[KG == 1 ? i : 0], lds_address(dst) + slot(i));
       c.base += c.step;
       return;
     }
@@ -322,7 +366,7 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
     }
   };
   auto advance = [](const char*& base, uint32_t (&off)[OFFS], uint32_t step) __attribute__((always_inline)) {
-    if constexpr (OFFS == 1) base += (int64_t)KG * step;
+    if constexpr (KG > 1) base += (int64_t)KG * step;
     else {
 #pragma unroll
       for (int i = 0; i < OFFS; i++) off[i] += step;
@@ -334,7 +378,7 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
 #pragma unroll
       for (int i = 0; i < LOADS; i++)
         if (ld_row[i] < rows_left && k_ch[i] * 8 < D)
-          load_to_lds_16(k_base + (OFFS > 1 ? 0 : (int64_t)i * (k_step / BKV * LROWS)), k_off[OFFS > 1 ? i : 0], lds_address(dst) + slot(i));
+          load_to_lds_16(k_base + (KG == 1 ? 0 : (int64_t)i * (k_step / BKV * LROWS)), k_off[KG == 1 ? i : 0], lds_address(dst) + slot(i));
       advance(k_base, k_off, k_step);
       rows_left -= KG * BKV;
     } else {
@@ -351,84 +395,40 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
 #pragma unroll
       for (int i = 0; i < LOADS; i++)
         if (ld_row[i] < rows_left_v && v_ch[i] * 8 < D)
-          load_to_lds_16(v_base + (OFFS > 1 ? 0 : (int64_t)i * (v_step / BKV * LROWS)), v_off[OFFS > 1 ? i : 0], lds_address(dst) + slot(i));
+          load_to_lds_16(v_base + (KG == 1 ? 0 : (int64_t)i * (v_step / BKV * LROWS)), v_off[KG == 1 ? i : 0], lds_address(dst) + slot(i));
       advance(v_base, v_off, v_step);
       rows_left_v -= KG * BKV;
     } else {
       issue_general(a.v, vcur, v_off, v_ch, dst, t, true);
     }
   };
-  // ---- Q^T fragments straight from global memory -----------------------
-  // B operand of K Q^T: lane holds query column col of block qb, head-dim slots MK*ks + 8*grp + 0..7.  What the norm and the
-  // rotation need is asked for together with the rows (one after the other, behind tests of each chunk's alignment, 24 x 2637 tokens
-  // took 11 us for it).
-  half8_t qf[QB][KS];
-  {
-    uint4_t raw[QB][KS], gam[QB][KS], rot[QB][KS];
-    bool has_gam[QB];
-    const auto chunk = [](const uint16_t* p, bool aligned) __attribute__((always_inline)) {
-      if (aligned) return *reinterpret_cast<const uint4_t*>(p);  // uniform
-      uint4_t v;
+  // ---- the queries' norm and rotation --------------------------------------
 #pragma unroll
-      for (int q = 0; q < 4; q++) v[q] = (uint32_t)p[2 * q] | ((uint32_t)p[2 * q + 1] << 16);
-      return v;
-    };
-#pragma unroll
-    for (int qb = 0; qb < QB; qb++) {
-      int64_t qi = (int64_t)qt * QROWS + qwave * 32 + qb * MB + col;
-      if (qi >= Sq) qi = Sq - 1;
-      // the row's segment, by selection: an index into the arguments that differs from lane to lane goes through memory
-      const uint16_t *ptr = a.q[0].ptr, *gp = a.q_gamma[0];
-      int64_t off = b * a.q[0].sb + h * a.q[0].sh, ss = a.q[0].ss;
-#pragma unroll
-      for (int i = 1; i < kMaxSeg; i++) {
-        const bool in = i < a.n_qseg && qi >= a.q[i].start;
-        ptr = in ? a.q[i].ptr : ptr;
-        off = in ? b * a.q[i].sb + h * a.q[i].sh - a.q[i].start * a.q[i].ss : off;
-        ss = in ? a.q[i].ss : ss;
-        gp = in ? a.q_gamma[i] : gp;
-      }
-      const uint16_t* const qp = ptr + (off + qi * ss);
-      has_gam[qb] = gp != nullptr;
-      if (!gp) gp = qp;  // (anything that can be read)
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        const int d0 = ks * MK + grp * 8;
-        raw[qb][ks] = gam[qb][ks] = rot[qb][ks] = uint4_t{0, 0, 0, 0};
-        if (d0 < D) {
-          raw[qb][ks] = *reinterpret_cast<const uint4_t*>(qp + d0);
-          if (a.q_norm) gam[qb][ks] = chunk(gp + d0, a.q_aligned);  // uniform
-          if (a.q_rot) rot[qb][ks] = chunk(a.q_rot + qi * D + d0, a.q_aligned);
-        }
-      }
-    }
-#pragma unroll
-    for (int qb = 0; qb < QB; qb++) {
-      if (a.q_prep) {  // uniform
-        // RMSNorm over the head, then the rotation: the row's D elements sit in the lanes of this column
-        float inv = 1.f;
-        if (a.q_norm) {  // uniform: some segment has a norm weight, and the sum takes every lane
-          float ss = 0.f;
-#pragma unroll
-          for (int ks = 0; ks < KS; ks++) {
-            float x[8];
-            unpack_chunk(raw[qb][ks], x);
-#pragma unroll
-            for (int e = 0; e < 8; e++) ss += x[e] * x[e];
-          }
-          ss = sum_groups<M16>(ss);
-          if (has_gam[qb]) inv = 1.0f / sqrtf(ss / (float)D + a.q_eps);
-        }
+  for (int qb = 0; qb < QB; qb++) {
+    if (a.q_prep) {  // uniform
+      // RMSNorm over the head, then the rotation: the row's D elements sit in the lanes of this column
+      float inv = 1.f;
+      if (a.q_norm) {  // uniform: some segment has a norm weight, and the sum takes every lane
+        float ss = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
           float x[8];
           unpack_chunk(raw[qb][ks], x);
-          raw[qb][ks] = finish_chunk(x, inv, has_gam[qb], gam[qb][ks], a.q_rot != nullptr, rot[qb][ks], 1.0f);
+#pragma unroll
+          for (int e = 0; e < 8; e++) ss += x[e] * x[e];
         }
+        ss = sum_groups<M16>(ss);
+        if (has_gam[qb]) inv = 1.0f / sqrtf(ss / (float)D + a.q_eps);
       }
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) qf[qb][ks] = __builtin_bit_cast(half8_t, raw[qb][ks]);
+      for (int ks = 0; ks < KS; ks++) {
+        float x[8];
+        unpack_chunk(raw[qb][ks], x);
+        raw[qb][ks] = finish_chunk(x, inv, has_gam[qb], gam[qb][ks], a.q_rot != nullptr, rot[qb][ks], 1.0f);
+      }
     }
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qf[qb][ks] = __builtin_bit_cast(half8_t, raw[qb][ks]);
   }
 
   // ---- running state -----------------------------------------------------
@@ -478,9 +478,9 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
     // K fragments are read a group of four ahead of the MFMAs that use them: KB blocks of 4 / KB k-steps
     constexpr int GS = 4 / KB;
     half8_t kf[2][4];
-    // (A k-step that lies wholly in the zero padding of a head size is left out.  The test stays where no k-step does, at head size
-    // 64: the loop is 7 % slower without its branches, and at 40, where it is known, 4 % faster -- us, 2 x 10 x 4096 of 64 143 / 154, 2 x
-    // 8 x 4096 of 40 73.4 / 70.6.)
+    // (A k-step that lies wholly in the zero padding of a head size is left out.  One key group tests for it at all head sizes up to
+    // 64: where no k-step does, the loop is 7 % slower without the branches, and at 40 a kernel that knows is no faster -- us, 2 x 10 x 4096 of 64
+    // 143 / 154, 2 x 8 x 4096 of 40 74.4 / 74.6, 24 x 1344 of 40 26.6 / 27.3.)
     auto live = [&](int ks) __attribute__((always_inline)) { return M16 || DL != 64 || ks * MK < D; };
     auto read_k = [&](int buf, int g) __attribute__((always_inline)) {
 #pragma unroll
@@ -686,7 +686,7 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
       // (with scalar loads of the segments' places on their way, which may come out of order, the compiler would wait for all LDS
       // reads in place of the next one: 3 % of a launch)
       if constexpr (!ONESEG) __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-      const bool before = n > 0 && t - KG < t_hi;  // there is a tile n - 1
+      const bool before = n > 0 && (KG == 1 || t - KG < t_hi);  // there is a tile n - 1
       // the wave doing softmax arithmetic gets issue priority: its exponentials only make progress in
       // the gaps the other wave's MFMA stream leaves (measured: +1 %; the opposite assignment -2 %)
       if (!second) {
@@ -1078,7 +1078,6 @@ dt_status sdpa_launch(hipStream_t s, const SdpaArgs& a) {
     if (a.D <= 80) return launch<128, 80, true, 2>(s, u);
     return launch<128, 128, false, 2>(s, u);  // (16x16x32 is 0 .. 7 % slower here, in launches of one round and of many)
   }
-  if (a.D <= 48) return launch<64, 48, false, 1>(s, a);
   if (a.D <= 64) return launch<64, 64, false, 1>(s, a);
   const int64_t tasks = (a.Sq + query_rows(1) - 1) / query_rows(1) * a.Hq * a.B;
   const int64_t cus = compute_units();
