@@ -232,6 +232,7 @@ struct TilePlan {
   int64_t whole = 0;  // tiles that stay whole; the rest is cut into `split` shares each
   int split = 1;
   bool act = false;  // some weight's tail has an activation
+  int64_t x_bytes = 0;  // of all problems' rows
   size_t expand_bytes = 0;  // > 0: the weights are written out as fp16 in front of the launch, to this much scratch
   // workspace of the split tiles: their counters, then their slots
   size_t counter_bytes() const { return split > 1 ? ((size_t)(tiles - whole) * kSplitNodes * 4 + 255) & ~(size_t)255 : 0; }
@@ -249,6 +250,7 @@ constexpr size_t kDenseMaxWorkspace = (size_t)128 << 20;
 constexpr size_t kDenseMaxExpand = (size_t)512 << 20;
 constexpr size_t kDenseFewRowsExpand = (size_t)200 << 20;
 constexpr int64_t kDenseFewRows = 640;
+constexpr int64_t kDenseNearX = (int64_t)48 << 20;
 
 // Estimated time (us) of a launch whose rows enter new blocks at every `step`-th K-tile at most: a fit to 930 launches of
 // 65 .. 4000 rows on the whole card (part of one would need costs of its own; the results do not depend on the layout
@@ -267,11 +269,16 @@ constexpr int64_t kDenseFewRows = 640;
 static double plan_cost(const TilePlan& p, int qbits, int mode, int nk, int64_t step, bool expanded) {
   const bool plain = qbits == 16, wide = qbits == 7 || qbits == 8, row = mode == kPalRow;
   const double entering = row ? (wide ? 0.70 : 0.33) / (double)step : 0.0;
+  // An X so large that it has left the memory-side cache when the copies behind it are written: a workgroup that has a compute unit to
+  // itself and two K-tiles on their way waits for memory, however few of them there are.  (us, 12288 -> 3072 in Flux blocks, 192 x 256 /
+  // 256 x 256 / 128 x 256 cut: 2577 rows 265 / 297 / 190, 2777 274 / 296 / 244, 3377 284 / 304 / 265, 3677 283 / 310 / 291, 4608 382 / 313 / 349; by itself,
+  // with X in the cache, 3112 rows 212 / 222 / 220.)
+  const bool far = plain && expanded && p.x_bytes > kDenseNearX;
   // one workgroup's K-tile with the share `busy` of the compute units at work
   const auto k_tile = [&](double busy) -> double {
     switch (p.tile) {
-      case kTile256x256: return plain ? 0.37 + 0.44 * busy : (wide ? 0.71 + 0.47 * busy : 0.73 + 0.27 * busy) + entering;
-      case kTile192x256: return 0.30 + 0.30 * busy;
+      case kTile256x256: return far ? 0.66 + 0.15 * busy : plain ? 0.37 + 0.44 * busy : (wide ? 0.71 + 0.47 * busy : 0.73 + 0.27 * busy) + entering;
+      case kTile192x256: return far ? 0.58 + 0.13 * busy : 0.30 + 0.30 * busy;
       case kTile128x256: return plain ? 0.28 + 0.14 * busy : wide ? 0.85 + 0.10 * busy : (row ? 0.60 : 0.78) + 0.17 * busy + entering;
       case kTile128x128: return plain ? 0.145 + 0.09 * busy : row ? 0.49 + 0.06 * busy + entering : wide ? 0.575 + 0.065 * busy : 0.56 + 0.09 * busy;
     }
@@ -337,11 +344,13 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
     p.tile = tile;
     p.BM = BM;
     p.BN = BN;
-    for (int gi = 0; gi < n; gi++)
+    for (int gi = 0; gi < n; gi++) {
+      p.x_bytes += 2 * hs[gi].M * K;
       for (int j = w_begin; j < (n > 1 ? hs[gi].n_weights : w_end); j++) {
         p.act = p.act || (hs[gi].post && hs[gi].post[j].activation != DT_ACT_NONE);
         p.tiles += ((hs[gi].M + BM - 1) / BM) * ((hs[gi].W[j].count / K + BN - 1) / BN);
       }
+    }
     p.whole = p.tiles;
     return p;
   };

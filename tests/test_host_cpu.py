@@ -128,6 +128,25 @@ def test_dense_scratch_for_copies(dthip, monkeypatch, M, K, N, n, q, nib, copied
     assert dthip.lib().dt_dense_scratch_bytes(1, G) == cut
 
 
+@pytest.mark.parametrize("M,q,cut", [
+    (3112, 8, True), (2791, 6, True),  # 238 against 269 on tiles of 192 x 256, 244 against 274
+    (4608, 6, False),                  # 349 against 313 on tiles of 256 x 256
+    (3112, 16, False),                 # no copies come between the launch and its X: 220 against 212
+])
+def test_dense_on_copies_with_an_x_that_left_the_cache(dthip, monkeypatch, M, q, cut):
+    """Big tiles wait for an X of over 48 MB that was written ahead of the copies: a Flux block's second feed-forward projection (us in the
+    block, cut first) is cut on 128 x 256 tiles, which have more on their way."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    addr, K, N, nib = ctypes.addressof, 12288, 3072, 0 if q == 16 else 16384 if q == 8 else 4096
+    W = (dthip._QxWeight * 1)(dthip._QxWeight(4096, q, nib, N * K))  # (addresses are not looked at)
+    Y, ldy = (ctypes.c_void_p * 1)(4096), (ctypes.c_int64 * 1)(N)
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), 1, None, addr(Y), addr(ldy), None, None))
+    copies = 0 if q == 16 else N * K * 2
+    scratch = dthip.lib().dt_dense_scratch_bytes(1, G)
+    assert scratch >= copies and (scratch > copies) == cut
+
+
 @pytest.mark.parametrize("M,K,N", [(219, 1024, 7808), (103, 1536, 10240), (108, 1024, 7296)])
 def test_dense_copies_where_palettes_would_be_looked_up_in_memory(dthip, monkeypatch, M, K, N):
     """A head epilogue needs tiles of 256 features, and q8 palettes of small blocks do not fit the LDS beside one: looked up in
