@@ -37,7 +37,7 @@ extern template dt_status launch_dense_q<16>(hipStream_t, const DenseArgs&, int,
 
 // the kernel with the elementwise tail only when some weight of the launch asks for one
 static dt_status launch_dense(hipStream_t s, const DenseArgs& a, int tile, int qbits, int mode) {
-  bool post = a.lora.up != nullptr;
+  bool post = false;
   for (int i = 0; i < kMaxWeights; i++) post = post || a.w[i].act != DT_ACT_NONE || a.w[i].gate || a.w[i].res || a.w[i].add || a.w[i].mul || a.w[i].scale != 1.0f;
   switch (qbits) {
     case 4: return launch_dense_q<4>(s, a, tile, post, mode);

@@ -17,7 +17,7 @@ namespace dt {
 // 2048 15.8 / 13.6.  Over 256 tiles two workgroups per compute unit are ahead (264 tiles, K = 3072 35.2 / 44.3).  (Waves
 // w and w + 4 on one K-tile of each pair, 64 x 64 slices: eight operand reads per pair instead of twelve, but the sums then
 // meet in LDS behind the loop: K = 1280 10.8, K = 2048 13.2, K = 256 6.5.)
-template <bool POST>
+template <bool POST, bool LORA>
 __global__ void __launch_bounds__(512, 2) dense_f16_kernel(const DenseArgs a) {
   constexpr int BM = 128, BN = 128;
   constexpr int NS = 4;                     // slots
@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(512, 2) dense_f16_kernel(const DenseArgs a) {
 
   __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);  // nothing is in flight into LDS any more
   __syncthreads();
-  dense_epilogue<64, 32, POST>(acc, smem, wave, lane, n0 + wn * 64, (int64_t)m0 + wm * 32, w, g.m, a.lora);
+  dense_epilogue<64, 32, POST, LORA>(acc, smem, wave, lane, n0 + wn * 64, (int64_t)m0 + wm * 32, w, g.m, a.lora);
 }
 
 }  // namespace dt

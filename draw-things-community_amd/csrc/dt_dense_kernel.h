@@ -121,7 +121,7 @@ struct DenseArgs {
   int32_t split;
   float* partials;
   int32_t* counters;
-  DenseLora lora;  // of w[0], the launch's only weight (kernels with a tail only)
+  DenseLora lora;  // of w[0], the launch's only weight
 };
 
 constexpr int kMaxSplit = 8;
@@ -197,7 +197,7 @@ __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
 // acc: the wave's WN x WM slice as TN x TM blocks of 16 x 16 (rows = features, columns = tokens).  nw / mw: first
 // feature (inside weight w) and first token of the slice; m_total: rows of X.  smem: the workgroup's LDS, free
 // for reuse (the caller's K loop ended with a barrier); the wave parks its slice at smem + wave * WM * WN halfs.
-template <int WN, int WM, bool POST>
+template <int WN, int WM, bool POST, bool LORA>
 __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16], unsigned char* smem, int wave, int lane,
                                                int nw, int64_t mw, const DenseWeight& w, int m_total, const DenseLora& lora) {
   constexpr int TN = WN / 16, TM = WM / 16;
@@ -340,27 +340,25 @@ __device__ __forceinline__ void dense_epilogue(float4_t (&acc)[WN / 16][WM / 16]
     }
   }
   if (nw >= w.n) return;
-  if constexpr (POST) {
+  if constexpr (LORA) {
     // The low-rank branch of a LoRA layer: its own sums, rounded to fp16, are added to what each lane has parked, which is rounded
     // again -- as a launch of its own with the base projection for its addend would, without that trip of the output to memory
     // and back.  (4608 x 3072, rank 16: 18 us for such a launch, 3 for this.)
     // Half of the features at a time, which keeps every kernel's occupancy what it is without.
-    if (lora.up) {  // uniform
 #pragma unroll 1
-      for (int i0 = 0; i0 < TN; i0 += TN / 2) {
-        float4_t low[TN / 2][TM];
-        low_rank_sums<TN / 2, TM>(low, lora, nw + 16 * i0, w.n, mw, m_total, lane);
+    for (int i0 = 0; i0 < TN; i0 += TN / 2) {
+      float4_t low[TN / 2][TM];
+      low_rank_sums<TN / 2, TM>(low, lora, nw + 16 * i0, w.n, mw, m_total, lane);
 #pragma unroll
-        for (int i = 0; i < TN / 2; i++)
+      for (int i = 0; i < TN / 2; i++)
 #pragma unroll
-          for (int j = 0; j < TM; j++) {
-            const int t = j * 16 + l16;
-            uint2_t* const p = reinterpret_cast<uint2_t*>(park + t * WN + ((((i0 + i) * 2 + (quad >> 1)) ^ (t & (CH - 1))) << 3) + 4 * (quad & 1));
-            const uint2_t base = *p;
-            *p = uint2_t{pack_h2(lo16(base[0]) + round_f16(low[i][j][0]), hi16(base[0]) + round_f16(low[i][j][1])),
-                         pack_h2(lo16(base[1]) + round_f16(low[i][j][2]), hi16(base[1]) + round_f16(low[i][j][3]))};
-          }
-      }
+        for (int j = 0; j < TM; j++) {
+          const int t = j * 16 + l16;
+          uint2_t* const p = reinterpret_cast<uint2_t*>(park + t * WN + ((((i0 + i) * 2 + (quad >> 1)) ^ (t & (CH - 1))) << 3) + 4 * (quad & 1));
+          const uint2_t base = *p;
+          *p = uint2_t{pack_h2(lo16(base[0]) + round_f16(low[i][j][0]), hi16(base[0]) + round_f16(low[i][j][1])),
+                       pack_h2(lo16(base[1]) + round_f16(low[i][j][2]), hi16(base[1]) + round_f16(low[i][j][3]))};
+        }
     }
   }
   // a wave's LDS operations execute in order: its reads below see the writes above
@@ -596,7 +594,7 @@ __device__ __forceinline__ TileAt tile_at(const DenseArgs& a, int bid) {
 // are spread evenly over all waves and between their MFMAs.  The accumulators
 // are held transposed (rows = output features n, columns = tokens m) so that
 // each lane ends up with runs of consecutive n for one token: 16-byte stores.
-// POST selects the epilogue with the elementwise tail.
+// POST selects the epilogue with the elementwise tail, LORA that with a LoRA layer's branch ahead of it.
 //
 // SPLIT: launches whose tiles do not fill the compute units (or fill them a little more than once) cut the tiles of
 // the unfilled round along K.  A workgroup then holds the fp32 sums of a share of K-tile pairs, and the shares meet in
@@ -615,7 +613,7 @@ __device__ __forceinline__ TileAt tile_at(const DenseArgs& a, int bid) {
 constexpr bool dense_two_per_cu(int Q, int BM, int BN, int mode, int NS) {
   return BM == 128 && BN == 128 && (mode == kPalShared || (mode == kPalRow && Q <= 6) || (mode == kPlainF16 && NS == 2));
 }
-template <int Q, int BM, int BN, int MODE, bool POST, bool SPLIT, int NS>
+template <int Q, int BM, int BN, int MODE, bool POST, bool SPLIT, int NS, bool LORA>
 __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 4 : 2)) dense_qx_kernel(const DenseArgs a) {
   constexpr int WN = BN / 2, WM = BM / 4;   // per-wave slice: WN features x WM tokens
   constexpr int TN = WN / 16, TM = WM / 16;  // its 16 x 16 blocks
@@ -1268,7 +1266,7 @@ __global__ void __launch_bounds__(512, (dense_two_per_cu(Q, BM, BN, MODE, NS) ? 
       }
     }
   }
-  dense_epilogue<WN, WM, POST>(acc, smem, wave, lane, n0 + wn * WN, (int64_t)m0 + wm * WM, w, g.m, a.lora);
+  dense_epilogue<WN, WM, POST, LORA>(acc, smem, wave, lane, n0 + wn * WN, (int64_t)m0 + wm * WM, w, g.m, a.lora);
 }
 
 }  // namespace dt
