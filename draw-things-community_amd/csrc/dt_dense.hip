@@ -234,6 +234,7 @@ struct TilePlan {
   bool act = false;  // some weight's tail has an activation
   int64_t x_bytes = 0;  // of all problems' rows
   size_t expand_bytes = 0;  // > 0: the weights are written out as fp16 in front of the launch, to this much scratch
+  int expanded = 0;         // that many of them
   // workspace of the split tiles: their counters, then their slots
   size_t counter_bytes() const { return split > 1 ? ((size_t)(tiles - whole) * kSplitNodes * 4 + 255) & ~(size_t)255 : 0; }
   size_t split_bytes() const { return split > 1 ? counter_bytes() + (size_t)((tiles - whole) * split * dense_split_slot_bytes(BM, BN)) : 0; }
@@ -438,6 +439,7 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
   if (expand_knob('n')) return false;
   size_t bytes = 0;
   int64_t weights = 0, m_max = 0;
+  int copies = 0;
   for (int gi = 0; gi < n; gi++) {
     m_max = std::max(m_max, hs[gi].M);
     for (int j = w_begin; j < (n > 1 ? hs[gi].n_weights : w_end); j++) {
@@ -446,6 +448,7 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
       if (w.nib < kDepalMinNib || w.count > 0x7fffffff) return false;  // (the tiled kernel's 32-bit byte offsets)
       bytes += ((size_t)w.count * 2 + 255) & ~(size_t)255;
       weights += w.count;
+      copies++;
     }
   }
   if (weights == 0 || bytes > ws || bytes > kDenseMaxExpand || (bytes > kDenseFewRowsExpand && m_max <= kDenseFewRows && !expand_knob('a'))) return false;
@@ -453,6 +456,7 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
   f16.qbits = 16;
   *plan = plan_format(hs, n, w_begin, w_end, wide, std::min(ws - bytes, kDenseMaxWorkspace), f16, true, cost);
   plan->expand_bytes = bytes;
+  plan->expanded = copies;
   // A copy costs 3.4 us and 0.44 per million weights, 0.65 where it outgrows the memory-side cache (28 M weights 13 us, 94 M
   // 61), and the plain launch on it takes 0.93 of its estimate (medians of 700 launches of 65 .. 8192 rows; 0.87 over the larger set
   // that plan_cost names).
@@ -466,11 +470,13 @@ static bool plan_copies(const HostGroup* hs, int n, int w_begin, int w_end, bool
 // The tiled kernel on palettized weights looks every weight up once per tile of rows, at a cost that no schedule hides: 0.6
 // against 0.2 us a K-tile on 128 x 128 tiles, however few the rows.  us, packed / copied: 4608 x 3072 -> 3 x 3072 q6p 284 /
 // 227, 1376 x 3072 -> 12288 q8p 158 / 131, 512 x 3072 -> 3072 q8p 47 / 26; and the other way round 188 x 3840 -> 3 x 8192 q6p
-// 84 / 112, 579 x 256 -> 5376 q6p 9.8 / 12.1.  The gain has to be 5 % and 6 us, or 7 % and 2 us of the
-// second launch on the host (512 x 5120 -> 2 x 5120 q5p, 105 MB of copies, gains less than 6).  (us, 6 and 8 for a cut / 2 and 4: UNet blocks 43 x 19 tokens, 640 wide, q8p 198 / 181, 50 x 50 q6p 236 / 222, LoRA
-// layers 464 x 704 -> 3008 q8p 34 / 27, 407 x 512 -> 1280 q4p 20.0 / 15.6, 6 x (995 x 256 -> 1344) q8p 22.4 / 20.8; 60 calls of random sizes 0.966 of
-// the time, none over 1.01.  Before the calls were made natively, second launches cost more of the host than they gained.)
-static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, bool expand, double* cost) {
+// 84 / 112, 579 x 256 -> 5376 q6p 9.8 / 12.1.  The gain has to be 5 %, and 2 us, which are the host's for a second launch, and more where
+// the estimate of so small a gain does not hold: 0.75 us for each of the weights, with several of which a short call waits for the host,
+// and 0.25 for every million of them, which with few rows take longer to copy; 6 at most.  (840 calls of random sizes whose estimate lies between 3
+// and 6 us: with 2 for all 0.936 of the time of 6 for all, but one in five slower by 2 % and more, up to 1.49 -- us, 91 x 448 -> 6 x 64 q8p 18.8 /
+// 12.6, 127 x 1024 -> 3 x 3776 q5p 27.7 / 19.7 --; with this 0.928 and one in twenty.)  Behind a LoRA layer's down projection, whose launch is made
+// anyway, 2 us do (0.963 of the time of 6, 890 layers: 464 x 704 -> 3008 q8p 34 / 27).
+static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, bool wide, size_t ws, bool expand, double* cost, bool beside_down = false) {
   const dt_qx_weight& w0 = hs[0].W[w_begin];
   const TilePlan packed = plan_format(hs, n, w_begin, w_end, wide, std::min(ws, kDenseMaxWorkspace), w0, false, cost);
   // (The estimate knows palettes in LDS.  Looked up in memory a launch takes four times as long, median of 1000 of them; priced like
@@ -479,7 +485,8 @@ static TilePlan plan_tiles(const HostGroup* hs, int n, int w_begin, int w_end, b
   TilePlan plain;
   double copied;
   if (!expand || w0.qbits == 16 || !plan_copies(hs, n, w_begin, w_end, wide, ws, &plain, &copied)) return packed;
-  if (!expand_knob('a') && !(copied < 0.95 * *cost && copied < *cost - (copied < 0.93 * *cost ? 2.0 : 6.0))) return packed;
+  const double least = beside_down ? 2.0 : std::min(6.0, 2.0 + 0.75 * plain.expanded + 0.125e-6 * (double)plain.expand_bytes);
+  if (!expand_knob('a') && !(copied < 0.95 * *cost && copied < *cost - least)) return packed;
   *cost = copied;
   return plain;
 }
@@ -745,7 +752,7 @@ static dt_status run_lora(hipStream_t s, const HostGroup& h, const dt_lora_pair&
   const size_t t_bytes = lora_t_bytes(h.M, p);
   const Workspace ws{scratch + t_bytes, bytes - t_bytes, true};
   double cost;
-  const TilePlan plan = plan_tiles(&h, 1, 0, 1, false, ws.bytes, true, &cost);
+  const TilePlan plan = plan_tiles(&h, 1, 0, 1, false, ws.bytes, true, &cost, true);
   DenseArgs a;
   DenseGroup& g = a.g[0];
   g.x = h.X;
@@ -977,7 +984,7 @@ DT_EXPORT size_t dt_lora_dense_scratch_bytes(int64_t M, int64_t K, const uint16_
   const HostGroup h{M, K, X, ldx, W, 1, nullptr, &Y, &ldy, nullptr, post};
   if (validate_lora(h, pair) != DT_OK || !lora_fusable(h, *pair)) return 0;
   double cost;
-  return lora_t_bytes(M, *pair) + plan_tiles(&h, 1, 0, 1, false, scratch_limit(true), true, &cost).bytes();
+  return lora_t_bytes(M, *pair) + plan_tiles(&h, 1, 0, 1, false, scratch_limit(true), true, &cost, true).bytes();
 }
 
 DT_EXPORT dt_status dt_lora_dense_f16(dt_stream stream, int64_t M, int64_t K, const uint16_t* X, int64_t ldx, const dt_qx_weight* W,

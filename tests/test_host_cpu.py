@@ -147,6 +147,23 @@ def test_dense_on_copies_with_an_x_that_left_the_cache(dthip, monkeypatch, M, q,
     assert scratch >= copies and (scratch > copies) == cut
 
 
+@pytest.mark.parametrize("M,K,N,n,q,nib,copied", [
+    (91, 448, 64, 6, 8, 16384, False), (1215, 448, 128, 6, 8, 16384, False),  # 18.8 against 12.6, 19.3 against 13.8: the host
+    (127, 1024, 3776, 3, 5, 1024, False), (346, 704, 3264, 6, 5, 1024, False),  # 27.7 against 19.7, 40.0 against 32.5: the copies
+    (3795, 640, 192, 1, 5, 1024, True), (82, 640, 192, 2, 5, 1024, True), (203, 704, 1664, 1, 6, 4096, True),  # 11.1 against 15.6, 11.2 / 15.3, 12.7 / 16.2
+])
+def test_dense_copies_for_small_gains(dthip, monkeypatch, M, K, N, n, q, nib, copied):
+    """Calls whose estimated gain is a few us: what the copies cost beyond the estimate grows with the weights and their size (us a call
+    at the right, copied first)."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    addr = ctypes.addressof
+    W = (dthip._QxWeight * n)(*[dthip._QxWeight(4096, q, nib, N * K)] * n)  # (addresses are not looked at)
+    Y, ldy = (ctypes.c_void_p * n)(*[4096] * n), (ctypes.c_int64 * n)(*[N] * n)
+    G = (dthip._DenseGroup * 1)(dthip._DenseGroup(M, K, 4096, K, addr(W), n, None, addr(Y), addr(ldy), None, None))
+    assert (dthip.lib().dt_dense_scratch_bytes(1, G) >= n * N * K * 2) == copied
+
+
 @pytest.mark.parametrize("M,K,N", [(219, 1024, 7808), (103, 1536, 10240), (108, 1024, 7296)])
 def test_dense_copies_where_palettes_would_be_looked_up_in_memory(dthip, monkeypatch, M, K, N):
     """A head epilogue needs tiles of 256 features, and q8 palettes of small blocks do not fit the LDS beside one: looked up in
