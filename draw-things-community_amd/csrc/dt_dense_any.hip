@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(256 * G) dense_any_kernel(const DenseAnyArgs a
   __shared__ __attribute__((aligned(16))) half_t all_tiles[G * 4 * BUF];
   __shared__ __attribute__((aligned(4))) uint16_t pal_lds[Q == 16 ? 2 : kAnyPalBytes / 2];
 
-  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+  const int tid = G == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   half_t* const tiles = all_tiles + group * 4 * BUF;
   const int l32 = lane & 31, hi = lane >> 5;
@@ -286,10 +286,14 @@ dt_status dense_any_launch(hipStream_t s, DenseAnyArgs a) {
   //   small ones / 64 wide, 1 / 4 groups: 500 x 1000 -> 1001 15.4 / 24.6 / 13.4 (10.3 / 15.4 / 9.9), 1000 rows 26.9 / 24.9 / 13.7 (15.9 / 15.8 / 10.4), 100
   //     x 300 -> 2200 9.1 / 13.7 / 10.2, 333 x 90 -> 1500 7.7 / 10.8 / 8.1; over 256 of them 1000 x 2500 -> 2500 112 / 70.6 / 73.9, 700 x 300 -> 2200 19.3
   //     / 16.3 / 18.9
-  const int64_t small_tiles = tiles(32), k_tiles = (a.k + 127) / 128;
-  const bool shared_out = tiles(64) <= 256 && small_tiles > 256 && a.k > 512;
+  //   ... and up to two of the small ones for a compute unit one or two groups on these hold their own: on plain weights against the wide ones, which
+  //     wait for memory (702 x 2452 -> 476 15.3 with two / 24.4, 265 x 2141 -> 1494 19.5 / 24.6, 240 x 1474 -> 1595 14.3 / 12.3; up to 1152 inputs with one, 233 x 547 ->
+  //     2006 9.8 / 11.5), and otherwise where the wide ones' last round of K-tiles is short (159 x 1052 -> 1650 15.0 with one / 16.5, 1000 inputs 13.8 / 13.6)
+  const int64_t small_tiles = tiles(32), k_tiles = (a.k + 127) / 128, wide_rounds = ((a.k + 63) / 64 + 3) / 4;
+  const bool two_each = small_tiles > 256 && small_tiles <= 512, plain = a.qbits == 16;
+  const bool shared_out = tiles(64) <= 256 && small_tiles > 256 && a.k > 512 && !(two_each && (plain || 20 * k_tiles <= 37 * wide_rounds));
   const bool big = shared_out || tiles(64) >= 256;
-  const int groups = shared_out ? 4 : big || small_tiles > 256 || k_tiles < 2 ? 1 : k_tiles >= (a.qbits == 16 ? 8 : 6) ? 4 : 2;
+  const int groups = shared_out ? 4 : big || k_tiles < 2 ? 1 : small_tiles > 256 ? (two_each && plain && a.k > 1152 ? 2 : 1) : k_tiles >= (plain ? 8 : 6) ? 4 : 2;
   const int BT = big ? 64 : 32;
   const int64_t grid = tiles(BT);
   if (grid > 0x7fffffff) return DT_NO_KERNEL;

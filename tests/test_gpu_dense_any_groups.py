@@ -10,6 +10,7 @@ pytestmark = pytest.mark.gpu
     (33, 65, 129), (70, 96, 257), (31, 130, 641), (5, 33, 767), (64, 100, 1025), (231, 1001, 1000),  # 32 x 32: two groups, four, a tile short of both
     (515, 1001, 519), (700, 1001, 1153), (1020, 1010, 770),                                          # 64 x 64, four groups: 9, 19, 13 K-tiles
     (515, 1001, 511), (1030, 1030, 600),                                                             # ... and where one group has all of K
+    (300, 1001, 1155), (297, 1030, 1051), (290, 1001, 1000), (512, 513, 1153),                       # 257 .. 512 small tiles: one or two groups on them, or 64 x 64
 ])
 @pytest.mark.parametrize("q,nib", [(16, 0), (4, 1024), (8, 4096), (6, 50), (5, 8)])
 def test_groups_of_waves_share_out_k(dthip, oracle, M, N, K, q, nib):
