@@ -26,13 +26,26 @@ def test_native_module_leaves_other_calls_alone(dthip):
 
 @pytest.fixture
 def both(dthip, monkeypatch):
-    """call -> its results the native way and the other one."""
+    """call -> its results the native way, which has to have been taken (natively=False: nowhere), and the other one."""
     import torch
 
-    def run(call):
+    def run(call, natively=True):
         native = dthip._host()
         assert native is not None
+        answers = []
+
+        class Watched:
+            def __getattr__(self, name):
+                def called(*args):
+                    answers.append(getattr(native, name)(*args))
+                    return answers[-1]
+
+                return called
+
+        monkeypatch.setattr(dthip, "_native", Watched())
         got = call()
+        monkeypatch.undo()
+        assert answers and all((a is not None) == natively for a in answers), answers
         monkeypatch.setattr(dthip, "_native", False)
         monkeypatch.setattr(dthip, "_host", lambda: None)
         want = call()
@@ -83,7 +96,9 @@ def test_dense_calls(dthip, oracle, both, shape):
 
     both(accumulated)
     both(lambda: dthip.dense_grouped([dict(x=x, weights=ws, biases=[b]), dict(x=x, weights=ws[:1], biases=[None], posts=[None])]))
-    both(lambda: dthip.dense_multi(x.transpose(0, 1) if x.dim() == 3 else x[:, ::1], ws, [b]))  # (a copy is the other way's)
+    # (a copy is the other way's)
+    for view in (x.transpose(0, 1) if x.dim() == 3 else x[:, ::1], dev(K, 70).t()):
+        both(lambda: dthip.dense_multi(view, ws, [b]), natively=view.is_contiguous())
 
 
 @pytest.mark.gpu
@@ -111,7 +126,14 @@ def test_refusals_are_the_same(dthip, oracle, monkeypatch):
     rng = np.random.default_rng(8)
     w = _weights(dthip, oracle, rng, 256, 128, 6, 4096)[0]
     x = torch.zeros((70, 128), dtype=torch.float16, device="cuda")
-    calls = [lambda: dthip.dense_multi(x.float(), [w], [None]), lambda: dthip.dense_multi(x[:, :64], [w], [None]),
+    layers = []
+    for high in (False, True):  # (a base weight of fewer rows than the layer's)
+        op = dthip.LoRADense(320, dthip.LoRANetworkConfiguration(16, 0.5, high))
+        dtype = torch.float32 if high else torch.float16
+        op.down, op.up = (dthip.QxTensor(torch.zeros(s, dtype=dtype, device="cuda"), 16, 0, s) for s in ((16, 128), (320, 16)))
+        op.weight = w
+        layers.append(op)
+    calls = [lambda: layers[0](x), lambda: layers[1](x), lambda: dthip.dense_multi(x.float(), [w], [None]), lambda: dthip.dense_multi(x[:, :64], [w], [None]),
              lambda: dthip.dense_multi(x, [w], [None, None]), lambda: dthip.dense_multi(x, [w], [x.float()]),
              lambda: dthip.dense_multi(x, [w], [None], epilogues=[dthip.HeadEpilogue(x[0], x[:1])]),
              lambda: dthip.dense_multi(x, [w], [None], epilogues=[dthip.HeadEpilogue(x[0, :100].contiguous(), None, head_dim=100)]),
