@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(256) lora_up_kernel(const LoraUpArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t m0 = (int64_t)blockIdx.x * TM, n0 = (int64_t)blockIdx.y * TN;
   float4_t acc[2][4];
-  low_rank_sums<2, 4>(acc, a.l, n0 + wave * 32, a.n, m0, a.m, lane);
+  low_rank_sums<2, 4, true>(acc, a.l, n0 + wave * 32, a.n, m0, a.m, lane);
 #pragma unroll
   for (int i = 0; i < 2; i++)
 #pragma unroll

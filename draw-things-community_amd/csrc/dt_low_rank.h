@@ -19,7 +19,7 @@ struct DenseLora {
 // s[i][j] = sums of features n0 + 16 i .. + 15 (rows: lane holds 4 (lane / 16) .. + 3) and tokens m0 + 16 j .. + 15 (column lane % 16);
 // what lies outside reads the last row.  fp16: v_mfma_f32_16x16x16_f16 from rank 0 up, two of which give the same bits as the
 // v_mfma_f32_16x16x32_f16 of the tiled kernels does (65536 sums of random operands: none differs).  The operands come straight from memory: they are read once or twice from a cache, and a launch is a few K-tiles long.
-template <int TN, int TM>
+template <int TN, int TM, bool KEEP = false>
 __device__ __forceinline__ void low_rank_sums(float4_t (&s)[TN][TM], const DenseLora& l, int64_t n0, int64_t n, int64_t m0, int64_t m, int lane) {
   typedef float float4_a4 __attribute__((ext_vector_type(4), aligned(4)));
   typedef half_t half4_t __attribute__((ext_vector_type(4)));
@@ -31,7 +31,8 @@ __device__ __forceinline__ void low_rank_sums(float4_t (&s)[TN][TM], const Dense
   // RS steps of 16 ranks, all of whose operands are asked for at once: a trip to memory takes longer than the multiplications
   const auto steps = [&](auto f32, auto count, int r0) {
     constexpr int RS = decltype(count)::value;
-    asm volatile("" : "+v"(lane));  // (keeps the rows' addresses out of the registers that live across a loop)
+    // (the rows' addresses out of the registers that live across a loop)
+    if constexpr (!KEEP) asm volatile("" : "+v"(lane));
     const int l16 = lane & 15, r = r0 + 4 * (lane >> 4);
     if constexpr (!decltype(f32)::value) {
       const half_t *const T = static_cast<const half_t*>(l.t) + r, *const U = static_cast<const half_t*>(l.up) + r;
