@@ -727,12 +727,19 @@ static size_t lora_t_bytes(int64_t M, const dt_lora_pair& p) { return ((size_t)M
 //   1280 -> 1280 q6p 30 / 24 (30 / 27), 300 x 1280 -> 1280 q8p 28 / 22 (28 / 24), 4096 x 320 -> 320 q6p 22 / 17 (22 / 19), and the other way round, rank 32, 2206
 //   x 4928 -> 320 45 / 53, rank 16, 100 x 5120 -> 1280 51 / 53; rank 64 and 128, with kernels for them: 929 x 3456 -> 704 40 / 54, 1432 x 832 -> 640 24
 //   / 25, 1571 x 704 -> 832 24 / 32.
-//   fp32, rank 32 (128): 4608 x 3072 -> 3072 128 / 113 (203 / 184), 512 x 3072 -> 3072 50 / 43 (54 / 54), 300 x 1280 -> 1280 44 / 26 (44 / 38), and the other way
-//   round, rank 128, 2500 x 1024 -> 4096 106 / 114, which is all output.
+//   fp32, rank 32 (128): 4608 x 3072 -> 3072 128 / 113 (203 / 184), 512 x 3072 -> 3072 50 / 43 (54 / 54), 300 x 1280 -> 1280 44 / 26 (44 / 38).  With many ranks the
+//   epilogue is most of it, and where few compute units have a second tile they are alone with its fp32 products: rank 128, 1331 x 1088 -> 3072 q6p
+//   (264 tiles of 128 x 128) 51 / 65, 2305 x 1536 -> 1856 fp16 (285) 69 / 79, 1617 x 320 -> 3712 q6p (377) 50 / 57; of 256 x 256 4371 x 640 -> 4672 rank 96 (342) 127 / 143; and
+//   otherwise 1334 x 832 -> 2816 q6p (242 of 128 x 128) 44 / 42, 2182 x 384 -> 3008 (432) 53 / 49, 3844 x 960 -> 4096 (992) 121 / 111: 0.92 of the time up to 256
+//   tiles, level above 384.
 static bool lora_fusable(const HostGroup& h, const dt_lora_pair& p) {
   if (h.M <= 0 || !h.x_ok() || !h.w_tiled(0)) return false;
   if (dense_rows_features(h.M, h.K, h.W[0].qbits, h.W[0].nib, h.W[0].count / h.K) > 0) return false;
-  if (p.f32) return h.M <= 0x3fffffff && p.rank <= 4096 && !(p.rank > 64 && h.K < 2048 && h.M * (h.W[0].count / h.K) > 6000000);
+  if (p.f32) {
+    const auto tiles = [&](int64_t t) { return ((h.M + t - 1) / t) * ((h.W[0].count / h.K + t - 1) / t); };
+    if (p.rank > 64 && ((h.K < 2560 && tiles(128) > kDenseCUs && tiles(128) <= kDenseCUs * 3 / 2) || (h.K < 1024 && tiles(256) > kDenseCUs))) return false;
+    return h.M <= 0x3fffffff && p.rank <= 4096;
+  }
   if (h.K > 4096 && (h.M < 512 || p.rank > 16)) return false;
   return p.rank % 16 == 0 && p.rank <= 32 && p.ld_up % 4 == 0 && (reinterpret_cast<uintptr_t>(p.down) & 15) == 0 &&
          (reinterpret_cast<uintptr_t>(p.up) & 7) == 0;

@@ -554,3 +554,18 @@ def test_lora_layer_refuses_a_weight_of_other_rows_than_count(dthip, monkeypatch
         op(x)
     op.configuration.scale = 0  # no branch: a plain Dense, of whatever rows its weight has
     assert op(x) == "plain"
+
+
+@pytest.mark.parametrize("M,K,N,rank,fused", [
+    (1334, 832, 2816, 128, True), (2182, 384, 3008, 96, True), (3844, 960, 4096, 128, True), (1331, 1088, 3072, 64, True),  # 42 against 44, 49 / 53, 111 / 121
+    (1331, 1088, 3072, 128, False), (2305, 1536, 1856, 128, False), (1617, 320, 3712, 128, False), (4371, 640, 4672, 96, False),  # 65 / 51, 79 / 69, 57 / 50, 143 / 127
+])
+def test_lora_layers_in_high_precision_that_run_as_calls(dthip, monkeypatch, M, K, N, rank, fused):
+    """Many ranks stay Dense calls where few compute units have a second tile and are alone with the fp32 products of its epilogue (us, in
+    one call first)."""
+    monkeypatch.delenv("DT_DENSE_SPLIT", raising=False)
+    monkeypatch.delenv("DT_DENSE_EXPAND", raising=False)
+    w = dthip._QxWeight(4096, 6, 4096, N * K)  # (addresses are not looked at)
+    pair = dthip._LoraPair(4096, 4096, rank, rank, 1, 0.5)
+    got = dthip.lib().dt_lora_dense_scratch_bytes(M, K, 4096, K, ctypes.byref(w), 4096, N, None, ctypes.byref(pair))
+    assert (got > 0) == fused
