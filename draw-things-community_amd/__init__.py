@@ -4,8 +4,9 @@ Mirrors the operator surface the reference's model builders use
 (`Dense`, `RMSNorm`, `Functional.cmul`, `ScaledDotProductAttention`,
 the rotary-table builders) on top of the C-ABI HIP library `libdthip.so`
 declared in `include/dt_hip.h`.  torch is used for device memory and streams
-only; every operator below runs a hand-written gfx950 kernel through ctypes
-and raises if the library is missing or a call fails.  There is no CPU path.
+only; every operator below runs hand-written gfx950 kernels, the common calls
+through `_dthost.so` (csrc/dt_host.cpp), all others through ctypes, and raises
+if the library is missing or a call fails.  There is no CPU path.
 """
 from __future__ import annotations
 
@@ -667,7 +668,7 @@ class LoRADense:
     left packed and the fp16 low-rank pair applied beside it (Models/LoRA.swift:85-142; running the LoRA separately
     is the preferred mode for quantized models, Models/UNetProtocol.swift:696-697).  dt_lora_dense_f16: the down
     projection, then the Dense kernel on the base, whose epilogue multiplies with `up` and adds the branch.  What that does not take (few
-    rows, widths off the tiled kernels' grid, palettized pairs) goes out as Dense calls: base and down projection (with the
+    rows, widths off the tiled kernels' grid, ranks for which it is slower, palettized pairs) goes out as Dense calls: base and down projection (with the
     scale in its epilogue), in one call or side by side, then the up projection, whose epilogue adds the base projection's
     result.  Every intermediate is rounded to fp16 as the reference's separate ops round, either way.  With
     `highPrecision` the pair is fp32 (`down.data` / `up.data` float32 tensors): the branch is computed as

@@ -380,8 +380,8 @@ static TilePlan plan_format(const HostGroup* hs, int n, int w_begin, int w_end, 
   // nothing beside it on the compute unit, small ones, whose estimate is high.  The sums are the same on every tile.  us, without
   // / with these, of 130 launches of random sizes the slowest by 3 % and half of them faster by 3 % and more: 1 x (2304 x 2048 -> 5120) fp16 57.2 / 45.9
   // (240 tiles, 720 of 128 x 128), 3394 x 4544 -> 3200 q8p 115.8 / 97.2, 4108 x 2048 -> 2816 q8p 64.9 / 53.3, 2 x (576 x 2368 -> 10368) q6p 128.9 /
-  // 77.0, with GELU 2016 x 1280 -> 5120 fp16 44.2 / 38.2, 2 x (4531 x 448 -> 5888) q6p 121.1 / 102.7, 3 x (5454 x 320 -> 960) q8p 54.2 / 39.1; left as
-  // they were: 3500 x 1280 -> 3840 fp16 36.6 on 210 tiles of 256 x 256, 54.6 on 285, 1376 x 3072 -> 12288 134 on 288, 117 cut, 112 on 384.
+  // 77.0, with GELU 2016 x 1280 -> 5120 fp16 44.2 / 38.2, 2 x (4531 x 448 -> 5888) q6p 121.1 / 102.7, 3 x (5454 x 320 -> 960) q8p 54.2 / 39.1, 1376 x 3072 -> 12288
+  // 134 on 288 tiles of 256 x 256, 117 cut, 112 on 384 of these; left as it was: 3500 x 1280 -> 3840 fp16 36.6 on 210 tiles of 256 x 256, 54.6 on 285.
   if (w0.qbits == 16 && !brief) {
     const auto instead = [&](const TilePlan& p, double factor) {
       const double t = factor * plan_cost(p, 16, kPlainF16, nk, step, expanded);

@@ -329,7 +329,8 @@ __global__ void __launch_bounds__(512, (sdpa_four_waves(DP, ONESEG, KG) ? 4 : 2)
   // (zero_tail: rows of the tile past the last key get zeros instead of keeping an earlier tile's bytes -- for V,
   // whose stale rows would otherwise meet a probability of exactly zero in the second MFMA: 0 x Inf = NaN)
   // What the paths that few tiles take derive from a thread's place is not to be kept in registers across the loop: they are short
-  // with four waves on a SIMD, and a reload from scratch waits for the transfers in flight.
+  // with four waves on a SIMD, and a reload from scratch waits for the transfers in flight.  (Nine registers at head sizes over 48 and four
+  // below do go to scratch; they come back behind the loop and where a ragged tile's rows are zeroed, nowhere else.)
   auto opaque = [](int v) __attribute__((always_inline)) {
     if constexpr (FOUR) asm volatile("" : "+v"(v));
     return v;
@@ -1026,7 +1027,7 @@ struct SdpaRate {
     return (double)full * ((double)steps * all + round) + (rest ? (double)steps * (few + (all - few) * (double)rest / cus) + round : 0.0);
   }
 };
-// head sizes up to 48, 64, 80, 128
+// head sizes up to 48 (whose kernels were some 3 % faster then, in either form), 64, 80, 128
 constexpr SdpaRate kOneGroup[4] = {{1.027, 1.087, 4.95, 1.946}, {1.02, 1.135, 6.472, 1.362}, {1.372, 1.511, 7.612, 1.745}, {1.326, 1.718, 9.237, 1.29}};
 constexpr SdpaRate kTwoGroups[4] = {{1.217, 1.244, 5.799, 2.19}, {1.279, 1.273, 6.058, 2.126}, {1.78, 1.844, 8.872, 1.35}, {1.662, 2.053, 9.644, 2.347}};
 

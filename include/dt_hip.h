@@ -248,15 +248,16 @@ dt_status dt_lora_branch_f32_f16(dt_stream stream, int64_t M, int64_t K, const u
                                  float* T, uint16_t* out, int64_t ldo);
 
 /*
- * A whole LoRADense (Models/LoRA.swift:85-142) on up to two launches: Y = tail(dense(x) + up(scale * down(x))), the branch rounded to fp16
- * and added to the base projection's fp16 result in its epilogue.  fp16 pairs round the intermediate to fp16 before and behind
- * `scale`, fp32 ones (highPrecision) keep it in fp32; results are those of the Dense calls that the layer consists of, bit for bit.
+ * A whole LoRADense (Models/LoRA.swift:85-142) in two launches, three where the weight stays packed and its tiles are cut along K:
+ * Y = tail(dense(x) + up(scale * down(x))), the branch rounded to fp16 and added to the base projection's fp16 result in its epilogue.
+ * fp16 pairs round the intermediate to fp16 before and behind `scale`, fp32 ones (highPrecision) keep it in fp32: every value is rounded
+ * where the Dense calls that the layer consists of round it, and the sums are in fp32.
  *   pair : f32 = 0: `down` [rank, K] and `up` [N, rank] (row stride ld_up) in fp16, rank padded with zeros to 16 or 32
  *          f32 = 1: fp32, any rank up to 4096
  *   post : as for dt_dense_qx_post_f16 without scale, addend and multiplicand; NULL = no tail
  * dt_lora_dense_scratch_bytes: the scratch memory (256-byte aligned) that the call takes, with less of it the weight stays packed, but at
  * least M x rank values of the pair's type, rounded up to 256 bytes (DT_OOM); 0 where the layer has to run as Dense calls of its
- * own (few rows, sizes or addresses off the tiled kernels' alignment; DT_NO_KERNEL).
+ * own (few rows, sizes or addresses off the tiled kernels' alignment, ranks for which those are faster; DT_NO_KERNEL).
  */
 typedef struct {
   const void* down;
